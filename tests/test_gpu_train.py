@@ -99,6 +99,19 @@ def test_scaled_add_sgd_sum_axis0_bit_exact(ag, dtype):
     assert np.array_equal(ag.Tensor.from_array(a).sum_axis0().into_array(), orc.sum_axis0(a))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("rows", [0, 1, 9, 128, 129, 255, 256, 257, 511, 512, 513, 769, 1025])
+def test_sum_axis0_chunk_and_column_edges(ag, dtype, rows):
+    # up to 128 rows one thread adds a column, beyond that rows go through LDS in chunks of 256 (two in flight), 64 columns
+    # a workgroup: bit for bit the serial sum either way
+    rng = np.random.default_rng(rows)
+    for cols in (1, 63, 64, 65, 130):
+        a = to_dtype(rng.standard_normal((rows, cols)) * 4, dtype)
+        assert np.array_equal(ag.Tensor.from_array(a).sum_axis0().into_array(), orc.sum_axis0(a)), cols
+
+
+
 def _view_of(ag, t, a, base):
     """The device Tensor that shows the same elements of `t` (uploaded from `base`) as the numpy view `a` of `base`."""
     es = base.itemsize
