@@ -98,9 +98,26 @@ struct DirectLoad {
                 const int pc = lane % CPR;
                 const uint32_t m = rslot_br<BR>((uint32_t)(pc >> 1), (uint32_t)kr);
                 int rowg = r0 + (int)(2 * m + (pc & 1)) * 8;
-                if (rowg >= NR) rowg = NR - 8;
+                // a group of 8 rows behind the last row reads one that exists (NR need not be a multiple of 8 for the
+                // unaligned kernel: its last group of each k-row but the last runs on into the next k-row)
+                if (rowg >= NR) rowg = NR % 8 ? NR / 8 * 8 : NR - 8;
                 off[i] = ((int64_t)kr * ks + rowg) * 2;
             }
+        }
+    }
+    // Unaligned kernel, last k-tile: elements by which the 16 bytes of load i must be moved down so that they do not pass
+    // the end of the row (LD_K) or of the last k-row (LD_R); what they then hold of the element wanted first is shifted
+    // back by funnel_shift, zeros coming in from behind.
+    static __device__ __forceinline__ int overhang(int i, int r0, int NR, int wave, int lane, int rem) {
+        const int inst = wave * NL + i;
+        if constexpr (MODE == LD_K) {
+            const int row = inst * 8 + (lane >> 3), k = ((lane & 7) ^ (int)swz((uint32_t)row)) * 8;
+            return k < rem && k + 8 > rem ? k + 8 - rem : 0;
+        } else {
+            const int kr = (int)krow_pos<BR>((uint32_t)(inst * KRPI + lane / CPR)), pc = lane % CPR;
+            int rowg = r0 + (int)(2 * rslot_br<BR>((uint32_t)(pc >> 1), (uint32_t)kr) + (pc & 1)) * 8;
+            if (rowg >= NR) rowg = NR % 8 ? NR / 8 * 8 : NR - 8;
+            return kr == rem - 1 && rowg + 8 > NR ? rowg + 8 - NR : 0;
         }
     }
     // whether this lane's 16 bytes of load i lie below k = rem within a k-tile (rem < 64: the last, shorter tile)
@@ -114,6 +131,21 @@ struct DirectLoad {
         }
     }
 };
+
+// 16 bytes at any element address: one global_load_dwordx4 (the device runs in unaligned access mode)
+typedef uint32_t any16_t __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ uint4 load_any16(const void *p) {
+    const any16_t v = *(const any16_t __attribute__((address_space(1))) *)p;
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+// the 128-bit value moved down by n elements of two bytes (0 <= n < 8), zeros from above
+__device__ __forceinline__ uint4 funnel_shift(const uint4 &v, int n) {
+    const uint64_t lo = (uint64_t)v.y << 32 | v.x, hi = (uint64_t)v.w << 32 | v.z;
+    const int b = (n & 3) * 16;
+    const uint64_t up = b ? hi << (64 - b) : 0;
+    const uint64_t slo = n & 4 ? hi >> b : (lo >> b) | up, shi = n & 4 ? 0 : hi >> b;
+    return make_uint4((uint32_t)slo, (uint32_t)(slo >> 32), (uint32_t)shi, (uint32_t)(shi >> 32));
+}
 
 // what the lanes of a shorter last k-tile read in place of elements at k >= K: both operands are zero there, so the
 // products vanish whatever lies behind the end of a row
@@ -159,8 +191,17 @@ struct FragRead {
 // NS: LDS stages.  Two serve wherever the CU's matrix pipes are kept busy by a second workgroup or by a k-tile long
 // enough to cover a load's latency; a 128 x 128 workgroup alone on its CU (a grid of at most one per CU) multiplies a
 // k-tile in 512 cycles, a quarter of that latency, and runs a ring of four.
-template <int BP, int BQ, int WGP, int WGQ, int LP, int LQ, bool STAGED, int NS = 2>
-__global__ __launch_bounds__(WGP *WGQ * 64) void gemm_bf16_dl_kernel(Args g) {
+//
+// DEPTH > 0: the form for operands that the direct loads cannot take (rows that do not start on 16-byte boundaries, k or a
+// row count that is no multiple of 8).  Same tiles, LDS layout, fragments and sums; the operand chunks travel through
+// registers instead: 16-byte loads from element addresses, DEPTH k-tiles in flight in as many register sets, each set
+// written to the LDS stage (two of them) one k-tile before it is multiplied.  What bounds it is the rate at
+// which a CU's L1 serves 16-byte loads that cross cache lines, about 60 cycles an instruction (16 when aligned).  The last k-tile is the only one in which a 16-byte chunk can pass the end of a row or of the
+// operand: its addresses are moved back by the overhang.  Against
+// the element-wise loaders: 1999x2047x1001 99 -> 25.8 us, 4099x4101x4103 1344 -> 238, 1058x4544x699 111 -> 24.1,
+// 8191x333x127 (transposed) 15.9 -> 6.5.
+template <int BP, int BQ, int WGP, int WGQ, int LP, int LQ, bool STAGED, int NS = 2, int DEPTH = 0>
+__global__ __launch_bounds__(WGP *WGQ * 64, DEPTH > 0 ? 2 : 1) void gemm_bf16_dl_kernel(Args g) {
     typedef uint16_t T;
     constexpr int NW = WGP * WGQ;
     constexpr int BK = 64;
@@ -186,8 +227,12 @@ __global__ __launch_bounds__(WGP *WGQ * 64) void gemm_bf16_dl_kernel(Args g) {
     const int split = blockIdx.y;
     const int kbeg = split * g.k_per_split;
     const int kend = min(g.K, kbeg + g.k_per_split);
-    const int KT = kend > kbeg ? (kend - kbeg) / BK : 0;     // whole k-tiles
-    const int rem = kend > kbeg ? (kend - kbeg) % BK : 0;    // depth of a shorter last one (the last split's only)
+    // whole k-tiles; depth of a shorter last one (the last split's only).  DEPTH > 0: all k-tiles, the last one of all
+    // (tile KT - 1 where `cut`) `rem` deep.
+    const int kspan = kend > kbeg ? kend - kbeg : 0;
+    const int KT = DEPTH > 0 ? (kspan + BK - 1) / BK : kspan / BK;
+    const int rem = DEPTH > 0 ? kspan - (KT - 1) * BK : kspan - KT * BK;
+    const bool cut = DEPTH > 0 && kend == g.K && KT > 0;
 
     int64_t offp[DlP::NL], offq[DlQ::NL];
     DlP::offsets(offp, g.ps, g.pk, p0, g.NP, wave, lane);
@@ -221,6 +266,45 @@ __global__ __launch_bounds__(WGP *WGQ * 64) void gemm_bf16_dl_kernel(Args g) {
             gq[l - NLP] += adv_q;
         }
     };
+    // DEPTH > 0: chunk l of a k-tile from memory to its register, and from there to its place in a stage (the place a
+    // direct load would put it)
+    constexpr int ND = DEPTH > 0 ? DEPTH : 1;
+    uint4 held[ND][DEPTH > 0 ? NLT : 1];
+    auto fetch = [&](uint4 (&set)[DEPTH > 0 ? NLT : 1], auto lc, int64_t adv_p, int64_t adv_q) __attribute__((always_inline)) {
+        constexpr int l = decltype(lc)::value;
+        if constexpr (l < NLP) {
+            set[l] = load_any16(gp[l]);
+            gp[l] += adv_p;
+        } else {
+            set[l] = load_any16(gq[l - NLP]);
+            gq[l - NLP] += adv_q;
+        }
+    };
+    // The pointers move on to the last k-tile of all: chunks that would pass the end of a row (of the operand) are read from
+    // addresses moved back by the overhang, chunks behind k = K are read from a block of zeros.  mend() writes the tile to
+    // LDS once more with the chunks of the first kind moved to their place, zeros coming in from behind (the registers
+    // stay as they are: changed behind a branch they would be copied, and every copy waits for its load).
+    auto aim_last = [&]() __attribute__((always_inline)) {
+        static_for<(DEPTH > 0 ? NLT : 0)>([&](auto lc) {
+            constexpr int l = decltype(lc)::value;
+            if constexpr (l < NLP) gp[l] = DlP::below(l, wave, lane, rem) ? gp[l] - 2 * DlP::overhang(l, p0, g.NP, wave, lane, rem) : (const unsigned char *)kZeroChunk;
+            else gq[l - NLP] = DlQ::below(l - NLP, wave, lane, rem) ? gq[l - NLP] - 2 * DlQ::overhang(l - NLP, q0, g.NQ, wave, lane, rem) : (const unsigned char *)kZeroChunk;
+        });
+    };
+    auto place = [&](unsigned char *stage, const uint4 &v, auto lc) __attribute__((always_inline)) {
+        constexpr int l = decltype(lc)::value;
+        if constexpr (l < NLP) *(uint4 *)(stage + (wave * NLP + l) * 1024 + lane * 16) = v;
+        else *(uint4 *)(stage + P_BYTES + (wave * NLQ + (l - NLP)) * 1024 + lane * 16) = v;
+    };
+    auto mend = [&](unsigned char *stage, const uint4 (&set)[DEPTH > 0 ? NLT : 1]) __attribute__((always_inline)) {
+        static_for<(DEPTH > 0 ? NLT : 0)>([&](auto lc) {
+            constexpr int l = decltype(lc)::value;
+            int over;
+            if constexpr (l < NLP) over = DlP::overhang(l, p0, g.NP, wave, lane, rem);
+            else over = DlQ::overhang(l - NLP, q0, g.NQ, wave, lane, rem);
+            place(stage, funnel_shift(set[l], over), lc);
+        });
+    };
 
     // two fragment sets of TP + TQ fragments each (one 32-deep substep of the wave's 128 x 128 tile)
     uint4 pfa[TP], qfa[TQ], pfb[TP], qfb[TQ];
@@ -252,6 +336,33 @@ __global__ __launch_bounds__(WGP *WGQ * 64) void gemm_bf16_dl_kernel(Args g) {
     constexpr int LSTEP = NM / NLT > 0 ? NM / NLT : 1;                // one direct load every LSTEP MFMAs
     static_assert(NU * RSTEP <= NM, "fragment reads must fit behind the MFMAs of one substep");
     static_assert(NB + LSTEP * NLT <= 2 * NM, "the loads of a tile must go out within the tile");
+    // DEPTH > 0: `set` holds tile kt+1, which goes to `nxt` (free since the last barrier) behind the first MFMAs; behind the
+    // barrier tile kt+1+DEPTH is requested into it.
+    constexpr int PSTEP = NB / NLT > 0 ? NB / NLT : 1;  // one LDS write every PSTEP MFMAs
+    static_assert(DEPTH == 0 || PSTEP * NLT <= NB, "the LDS writes of a tile must go out before the barrier");
+    auto step_held = [&](unsigned char *cur, unsigned char *nxt, uint4 (&set)[DEPTH > 0 ? NLT : 1], bool adv, bool last) __attribute__((always_inline)) {
+        const int64_t ap = adv ? stepP : 0, aq = adv ? stepQ : 0;
+        if constexpr (DEPTH > 0) static_for<2 * NM>([&](auto nc) {
+            constexpr int n = decltype(nc)::value, ph = n / NM, m = n % NM, i = m / TQ, j = m % TQ;
+            if constexpr (n == NB) {
+                if (last) mend(nxt, set);  // wave-uniform
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if constexpr (ph == 0) {
+                mma(acc[i][j], pfa[i], qfa[j]);
+                if constexpr (m % RSTEP == 0 && m / RSTEP < NU) read_unit(pfb, qfb, cur, std::integral_constant<int, 1>{}, std::integral_constant<int, m / RSTEP>{});
+            } else {
+                mma(acc[i][j], pfb[i], qfb[j]);
+                if constexpr (m % RSTEP == 0 && m / RSTEP < NU) read_unit(pfa, qfa, nxt, std::integral_constant<int, 0>{}, std::integral_constant<int, m / RSTEP>{});
+            }
+            if constexpr (n < NB && n % PSTEP == PSTEP - 1 && n / PSTEP < NLT)
+                place(nxt, set[n / PSTEP], std::integral_constant<int, n / PSTEP>{});
+            if constexpr (n >= NB && (n - NB) % LSTEP == LSTEP - 1 && (n - NB) / LSTEP < NLT)
+                fetch(set, std::integral_constant<int, (n - NB) / LSTEP>{}, ap, aq);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
     auto step = [&](unsigned char *cur, unsigned char *nxt, bool adv) __attribute__((always_inline)) {
         const uint32_t cur_addr = __builtin_amdgcn_readfirstlane(lds_address(cur));
         const int64_t ap = adv ? stepP : 0, aq = adv ? stepQ : 0;
@@ -276,31 +387,65 @@ __global__ __launch_bounds__(WGP *WGQ * 64) void gemm_bf16_dl_kernel(Args g) {
         });
     };
 
-    if (KT > 0) {
-        // tile min(t, KT-1) -> stage t
-        const uint32_t a0 = __builtin_amdgcn_readfirstlane(lds_address(stage0));
-        static_for<NS * NLT>([&](auto nc) {
-            constexpr int t = decltype(nc)::value / NLT, l = decltype(nc)::value % NLT;
-            issue_load(a0 + t * STAGE_BYTES, std::integral_constant<int, l>{}, KT > t + 1 ? stepP : 0, KT > t + 1 ? stepQ : 0);
-        });
-        static_assert((NS - 1) * NLT < 64, "the wait counter holds six bits");
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * NLT) : "memory");  // tile 0 has landed
-        __syncthreads();
-        static_for<NU>([&](auto uc) { read_unit(pfa, qfa, stage0, std::integral_constant<int, 0>{}, uc); });
-    }
-    int kt = 0;
-    for (; kt + NS <= KT; kt += NS)  // step kt requests tile kt+NS and moves on if a tile kt+NS+1 exists
-        static_for<NS>([&](auto sc) {
+    if constexpr (DEPTH > 0) {
+        static_assert(DEPTH % 2 == 0 && NS == 2, "set and stage of a tile are named by constants");
+        // a fetch of tile t (the last one again where t > KT - 1) leaves the pointers at tile t + 1
+        auto fetch_tile = [&](uint4 (&set)[NLT], int t) __attribute__((always_inline)) {
+            if (cut && t == KT - 1) aim_last();
+            const bool adv = t + 1 < KT;
+            static_for<NLT>([&](auto lc) { fetch(set, lc, adv ? stepP : 0, adv ? stepQ : 0); });
+        };
+        // Step kt multiplies tile kt, publishes tile kt+1 and requests tile kt+1+DEPTH.
+        auto turn = [&](int kt, auto sc) __attribute__((always_inline)) {
             constexpr int s = decltype(sc)::value;
-            step(stages[s], stages[(s + 1) % NS], kt + s + NS + 1 < KT);
+            if (cut && kt + 1 + DEPTH == KT - 1) aim_last();
+            step_held(stages[s & 1], stages[(s + 1) & 1], held[(s + 1) % DEPTH], kt + 2 + DEPTH < KT, cut && kt + 1 == KT - 1);
+        };
+        if (KT > 0) {
+            // tile 0 to stage 0, tile t = 1 .. DEPTH into set t % DEPTH
+            static_for<DEPTH>([&](auto tc) { fetch_tile(held[decltype(tc)::value], decltype(tc)::value); });
+            static_for<NLT>([&](auto lc) { place(stage0, held[0][decltype(lc)::value], lc); });
+            if (cut && KT == 1) mend(stage0, held[0]);
+            fetch_tile(held[0], DEPTH);
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            static_for<NU>([&](auto uc) { read_unit(pfa, qfa, stage0, std::integral_constant<int, 0>{}, uc); });
+        }
+        // (no branch around a step in the loop: where paths meet, the compiler waits for the loads of the path with the
+        // fewest in flight)
+        int kt = 0;
+        for (; kt + DEPTH <= KT; kt += DEPTH)
+            static_for<DEPTH>([&](auto sc) { turn(kt + decltype(sc)::value, sc); });
+        static_for<DEPTH - 1>([&](auto sc) {
+            if (kt + decltype(sc)::value < KT) turn(kt + decltype(sc)::value, sc);
         });
-    static_for<NS - 1>([&](auto sc) {
-        constexpr int s = decltype(sc)::value;
-        if (kt + s < KT) step(stages[s], stages[(s + 1) % NS], false);
-    });
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (rem > 0) {
+        __syncthreads();
+    } else {
+        if (KT > 0) {
+            // tile min(t, KT-1) -> stage t
+            const uint32_t a0 = __builtin_amdgcn_readfirstlane(lds_address(stage0));
+            static_for<NS * NLT>([&](auto nc) {
+                constexpr int t = decltype(nc)::value / NLT, l = decltype(nc)::value % NLT;
+                issue_load(a0 + t * STAGE_BYTES, std::integral_constant<int, l>{}, KT > t + 1 ? stepP : 0, KT > t + 1 ? stepQ : 0);
+            });
+            static_assert((NS - 1) * NLT < 64, "the wait counter holds six bits");
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * NLT) : "memory");  // tile 0 has landed
+            __syncthreads();
+            static_for<NU>([&](auto uc) { read_unit(pfa, qfa, stage0, std::integral_constant<int, 0>{}, uc); });
+        }
+        int kt = 0;
+        for (; kt + NS <= KT; kt += NS)  // step kt requests tile kt+NS and moves on if a tile kt+NS+1 exists
+            static_for<NS>([&](auto sc) {
+                constexpr int s = decltype(sc)::value;
+                step(stages[s], stages[(s + 1) % NS], kt + s + NS + 1 < KT);
+            });
+        static_for<NS - 1>([&](auto sc) {
+            constexpr int s = decltype(sc)::value;
+            if (kt + s < KT) step(stages[s], stages[(s + 1) % NS], false);
+        });
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    }
+    if (DEPTH == 0 && rem > 0) {
         // The shorter last k-tile, outside the pipeline (one load latency per workgroup, once): the same direct loads
         // into stage 0, lanes whose bytes lie at k >= K reading zeros instead.  After the loop the pointers stand at
         // the last whole tile (at this tile when there is none).
@@ -334,10 +479,11 @@ __global__ __launch_bounds__(WGP *WGQ * 64) void gemm_bf16_dl_kernel(Args g) {
     const int pw0 = pwb + (int)lg * 4, qw0 = qwb + (int)l16;
     T *D = (T *)g.D + (int64_t)blockIdx.z * g.batch_d;
     const T *bias = (const T *)g.bias;
-    const int mode = STAGED ? (int)ST_STAGED : g.store_mode;
+    const int mode = STAGED ? (int)ST_STAGED : g.store_mode == ST_STAGED_ANY ? (int)ST_STAGED : g.store_mode;
+    const bool any_c = !STAGED && g.store_mode == ST_STAGED_ANY;  // C's rows start anywhere, NP is any number
     const bool has_bias = g.has_bias != 0, bias_p = g.bias_on_p != 0;
     if (mode == ST_STAGED) {
-        // beta == 0, D rows 16-byte aligned, NP a multiple of 8.  A lane holds 4 consecutive p of ONE q row and the
+        // beta == 0, D rows 16-byte aligned, NP a multiple of 8 (ST_STAGED_ANY: neither, p still C's unit-stride axis).  A lane holds 4 consecutive p of ONE q row and the
         // 16 lanes of a group hold 16 different q rows, so storing straight from the accumulators would write 8 bytes
         // into each of 64 different cache lines per instruction.  Instead each wave transposes 32 q rows (two tile
         // columns) at a time through its own LDS region and stores whole 16-byte chunks of contiguous row segments.
@@ -410,7 +556,17 @@ __global__ __launch_bounds__(WGP *WGQ * 64) void gemm_bf16_dl_kernel(Args g) {
                     }
                     // streaming store: C is not read again by this launch, and keeping it out of the last-level
                     // cache leaves that cache to the operand panels, which every tile row / column re-reads
-                    if (qq < g.NQ && pp < g.NP)
+                    if (any_c) {  // wave-uniform
+                        T *dst = D + (int64_t)qq * g.dq + pp;
+                        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+                        if (qq < g.NQ && pp + 8 <= g.NP) {
+                            *(any16_t *)dst = any16_t{v.x, v.y, v.z, v.w};
+                        } else if (qq < g.NQ) {
+#pragma unroll
+                            for (int e = 0; e < 7; ++e)
+                                if (pp + e < g.NP) dst[e] = (T)(w[e >> 1] >> (16 * (e & 1)));
+                        }
+                    } else if (qq < g.NQ && pp < g.NP)
                         __builtin_nontemporal_store(u32x4_t{v.x, v.y, v.z, v.w}, (u32x4_t *)(D + (int64_t)qq * g.dq + pp));
                 });
             });

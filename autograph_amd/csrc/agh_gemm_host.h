@@ -55,6 +55,10 @@ int launch_one(const Args &g, int splits) {
 // (one translation unit per tile shape, so they compile in parallel)
 template <int BP, int BQ, int WGP, int WGQ, int LP, int LQ, int NS>
 int launch_one_dl(const Args &g, int splits);
+// the form of the same kernel for operands at any element address, k and row counts of any size
+// (agh_gemm_bf16_any_<tile>.hip)
+template <int BP, int BQ, int WGP, int WGQ, int LP, int LQ>
+int launch_one_any(const Args &g, int splits);
 #endif
 
 inline int env_int(const char *name, int dflt);
@@ -115,7 +119,7 @@ int launch_f32_dl(const Args &g, int splits) {
 #endif
 
 template <typename T, int BP, int BQ, int WGP, int WGQ, bool SCALAR_OK>
-int launch_loaders(const Args &g, int splits, int lp, int lq, bool direct) {
+int launch_loaders(const Args &g, int splits, int lp, int lq, bool direct, bool any) {
 #ifdef AGH_GEMM_WITH_F32_DIRECT
     if constexpr (std::is_same<T, float>::value && BP % 64 == 0 && BQ % 64 == 0) {
         // both operands vector-loadable (any k: a last k-tile shorter than 32 is loaded with zeros behind k = K)
@@ -135,6 +139,17 @@ int launch_loaders(const Args &g, int splits, int lp, int lq, bool direct) {
     }
 #endif
 #ifdef AGH_GEMM_WITH_BF16_DIRECT
+    if constexpr (std::is_same<T, uint16_t>::value && BP == BQ && BP <= 128) {
+        if (any) {
+            switch (lp * 3 + lq) {
+                case LD_K * 3 + LD_K: return launch_one_any<BP, BQ, WGP, WGQ, LD_K, LD_K>(g, splits);
+                case LD_K * 3 + LD_R: return launch_one_any<BP, BQ, WGP, WGQ, LD_K, LD_R>(g, splits);
+                case LD_R * 3 + LD_K: return launch_one_any<BP, BQ, WGP, WGQ, LD_R, LD_K>(g, splits);
+                case LD_R * 3 + LD_R: return launch_one_any<BP, BQ, WGP, WGQ, LD_R, LD_R>(g, splits);
+                default: break;
+            }
+        }
+    }
     if constexpr (std::is_same<T, uint16_t>::value && (!SCALAR_OK || (BP == 64 && BQ == 64))) {
         if (direct && lp != LD_S && lq != LD_S) {
             switch (lp * 3 + lq) {
@@ -168,15 +183,15 @@ int launch_loaders(const Args &g, int splits, int lp, int lq, bool direct) {
 }
 
 template <typename T>
-int launch_cfg(int cfg, const Args &g, int splits, int lp, int lq, bool direct) {
+int launch_cfg(int cfg, const Args &g, int splits, int lp, int lq, bool direct, bool any) {
     switch (cfg) {
-        case 0: return launch_loaders<T, 256, 256, 2, 2, false>(g, splits, lp, lq, direct);
-        case 1: return launch_loaders<T, 128, 256, 2, 2, false>(g, splits, lp, lq, direct);
-        case 2: return launch_loaders<T, 256, 128, 2, 2, false>(g, splits, lp, lq, direct);
-        case 3: return launch_loaders<T, 128, 128, 2, 2, false>(g, splits, lp, lq, direct);
-        case 4: return launch_loaders<T, 64, 64, 2, 2, true>(g, splits, lp, lq, direct);
-        case 5: return launch_loaders<T, 32, 128, 1, 4, true>(g, splits, lp, lq, false);
-        case 6: return launch_loaders<T, 128, 32, 4, 1, true>(g, splits, lp, lq, false);
+        case 0: return launch_loaders<T, 256, 256, 2, 2, false>(g, splits, lp, lq, direct, any);
+        case 1: return launch_loaders<T, 128, 256, 2, 2, false>(g, splits, lp, lq, direct, any);
+        case 2: return launch_loaders<T, 256, 128, 2, 2, false>(g, splits, lp, lq, direct, any);
+        case 3: return launch_loaders<T, 128, 128, 2, 2, false>(g, splits, lp, lq, direct, any);
+        case 4: return launch_loaders<T, 64, 64, 2, 2, true>(g, splits, lp, lq, direct, any);
+        case 5: return launch_loaders<T, 32, 128, 1, 4, true>(g, splits, lp, lq, false, any);
+        case 6: return launch_loaders<T, 128, 32, 4, 1, true>(g, splits, lp, lq, false, any);
         default: return fail(AGH_EINVAL, "gemm: bad tile config %d", cfg);
     }
 }
@@ -190,6 +205,17 @@ int pick_loader(const void *base, int64_t rs, int64_t ks, int NR, int K) {
     if (!aligned(base, 16)) return LD_S;
     if (ks == 1 && K % EPC == 0 && (rs % EPC == 0 || NR == 1)) return LD_K;
     if (rs == 1 && NR % EPC == 0 && (ks % EPC == 0 || K == 1)) return LD_R;
+    return LD_S;
+}
+
+// The same for the bf16 kernel that reads 16 bytes from any element address: no multiple of anything is needed, but
+// k >= 8 (a last chunk is read from up to 7 elements further down its row), and for rows as the unit-stride axis k-rows
+// that follow each other upwards at least 8 elements apart (a chunk that runs past the last row of a k-row stays inside the
+// operand's memory).
+inline int pick_loader_any(int64_t rs, int64_t ks, int K) {
+    if (K < 8) return LD_S;
+    if (ks == 1) return LD_K;
+    if (rs == 1 && ks >= 8) return LD_R;
     return LD_S;
 }
 
@@ -258,6 +284,14 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
     // every matrix of a batch must satisfy the same alignment as the first
     const bool batch_aligned = batch == 1 || (g.batch_p % EPC == 0 && g.batch_q % EPC == 0);
     if (!batch_aligned) lp = lq = LD_S;
+    // bf16 operands that are no whole 16-byte vectors but have a unit-stride axis each take the direct-to-LDS kernel's form
+    // for any element address (tiles 128 x 128 and 64 x 64); what is left has the element-wise loader
+    int lp_any = LD_S, lq_any = LD_S;
+    if (sizeof(T) == 2 && (lp == LD_S || lq == LD_S) && k > 0 && env_int("AGH_GEMM_DIRECT", 1) != 0) {
+        lp_any = pick_loader_any(g.ps, g.pk, g.K);
+        lq_any = pick_loader_any(g.qs, g.qk, g.K);
+    }
+    const bool any_addr = lp_any != LD_S && lq_any != LD_S;
     const bool any_scalar = (lp == LD_S || lq == LD_S);
     const bool vec_store = g.dp == 1 && g.NP % 4 == 0 && (g.dq % 4 == 0 || g.NQ == 1) && aligned(C, 4 * sizeof(T)) &&
                            (batch == 1 || g.batch_d % 4 == 0);
@@ -272,12 +306,12 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
     // ---- tile shape: minimise (rounds of workgroups) x (tile area) / efficiency ----
     const int cus = compute_units() > 0 ? compute_units() : 256;
     // (any k: a last k-tile shorter than 64 is loaded with zeros behind k = K)
-    const bool direct_ok = sizeof(T) == 2 && !any_scalar && g.K > 0 && env_int("AGH_GEMM_DIRECT", 1) != 0;
+    const bool direct_ok = sizeof(T) == 2 && (!any_scalar || any_addr) && g.K > 0 && env_int("AGH_GEMM_DIRECT", 1) != 0;
     int best = -1;
     double best_cost = 0;
     for (int i = 0; i < kNumCfgs; ++i) {
         const TileCfg &t = kCfgs[i];
-        if (any_scalar && !t.scalar_ok) continue;
+        if (any_addr ? i != 3 && i != 4 : any_scalar && !t.scalar_ok) continue;
         const int64_t tiles = (int64_t)((g.NP + t.bp - 1) / t.bp) * ((g.NQ + t.bq - 1) / t.bq) * batch;
         if (tiles > 0x7FFFFFFF) continue;
         // a CU works through ceil(tiles / CUs) tiles; co-resident workgroups share its MFMA rate
@@ -337,10 +371,19 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
             const double per_tile = (double)t.bp * t.bq / (tiles <= cus ? kDirect64Alone : kDirect64Shared);
             cost = (double)((tiles + slots - 1) / slots) * (tiles <= cus ? 1 : 2) * per_tile * (kt + 6.0) / kt;
         }
+        // Operands at any element address: bound by the L1s, whatever the clock.  Microseconds a k-tile, a workgroup alone on
+        // its CU / per workgroup where several share it: 128 x 128 0.95 / 0.75 (1999x2047x1001; 4099x4101x4103), 64 x 64
+        // 0.52 / 0.38 (1024x1023x1024; 1999x2047x1001, 2999x3001x3003); filling and storing cost three and five k-tiles.
+        if (any_addr) {
+            const double alone = t.bp == 64 ? 0.52 : 0.95, shared = t.bp == 64 ? 0.38 : 0.75;
+            cost = (rounds == 1 ? alone : rounds * shared) * (kt + (t.bp == 64 ? 5.0 : 3.0));
+        }
         if (best < 0 || cost < best_cost) { best = i; best_cost = cost; }
     }
     best = env_int("AGH_GEMM_CFG", best);
-    if (best < 0 || best >= kNumCfgs || (any_scalar && !kCfgs[best].scalar_ok))
+    const bool any = any_addr && (best == 3 || best == 4);  // (a forced skinny tile keeps the element-wise loaders)
+    if (any) { lp = lp_any; lq = lq_any; }
+    if (best < 0 || best >= kNumCfgs || (any_scalar && !any && !kCfgs[best].scalar_ok))
         return fail(AGH_ERANGE, "%s: no tile configuration for this shape", name);
     const TileCfg &t = kCfgs[best];
     g.tiles_p = (g.NP + t.bp - 1) / t.bp;
@@ -370,7 +413,7 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
 
     // bf16 with both operands vector-loadable takes the
     // direct-to-LDS kernel (AGH_GEMM_DIRECT=0 forces the register-staged one)
-    const bool direct = direct_ok;
+    const bool direct = direct_ok && (!any_scalar || any);
 
     if (splits > 1) {
         void *ws = nullptr;
@@ -378,7 +421,7 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
         if (int rc = fixed_scratch ? static_workspace(bytes, &ws) : workspace(bytes, &ws)) return rc;
         g.ws = (float *)ws;
         g.store_mode = ST_SPLITK;
-        if (int rc = launch_cfg<T>(best, g, splits, lp, lq, direct)) return rc;
+        if (int rc = launch_cfg<T>(best, g, splits, lp, lq, direct, any)) return rc;
         const size_t total = (size_t)g.NQ * g.NP;
         int lanes = 1;  // threads per output element: about eight partials each
         while (lanes < 16 && lanes * 16 <= splits) lanes *= 2;
@@ -400,7 +443,9 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
     if (direct && best <= 4 && vec_store && beta == 0.0f && g.NP % 8 == 0 && (g.dq % 8 == 0 || g.NQ == 1) &&
         aligned(C, 16) && (batch == 1 || g.batch_d % 8 == 0))
         g.store_mode = ST_STAGED;
-    return launch_cfg<T>(best, g, 1, lp, lq, direct);
+    else if (direct && best <= 4 && g.dp == 1 && beta == 0.0f)
+        g.store_mode = ST_STAGED_ANY;  // the same transposition, 16-byte stores to any element address
+    return launch_cfg<T>(best, g, 1, lp, lq, direct, any);
 }
 
 }  // namespace gemm

@@ -51,7 +51,8 @@ __device__ __forceinline__ void static_for(F &&f) {
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
 enum { LD_K = 0, LD_R = 1, LD_S = 2 };
-enum { ST_SCALAR = 0, ST_VEC = 1, ST_SPLITK = 2, ST_STAGED = 3 };  // ST_STAGED: direct-to-LDS bf16 kernel only
+// ST_STAGED, ST_STAGED_ANY: direct-to-LDS bf16 kernels only
+enum { ST_SCALAR = 0, ST_VEC = 1, ST_SPLITK = 2, ST_STAGED = 3, ST_STAGED_ANY = 4 };
 
 struct Args {
     const void *P;

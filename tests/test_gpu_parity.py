@@ -849,6 +849,54 @@ def test_gemm_bf16_seeded_shapes_in_every_tile_configuration(ag, monkeypatch):
     assert ran[None] == 120 and min(ran.values()) >= 40, ran
 
 
+@pytest.mark.parametrize("k", [8, 9, 15, 63, 64, 65, 127, 128, 129, 191, 257, 321, 389])
+def test_gemm_bf16_operands_at_any_address(ag, monkeypatch, k):
+    """bf16 products whose rows start anywhere (odd k, odd row counts, views shifted by one element), in the chooser's tile and
+    forced into 128 x 128 and 64 x 64: edges of tiles and of k-tiles, fewer rows than a 16-byte chunk, all four layouts, C
+    with odd rows inside a larger buffer.  The tiles agree bit for bit (one f32 sum per output in k order, rounded once),
+    and nothing outside the view of C is written."""
+    rng = np.random.default_rng(k)
+    for m, n in ((1, 1), (5, 131), (63, 65), (130, 7), (129, 257)):
+        for ta, tb in ((False, False), (True, False), (False, True), (True, True)):
+            shift = int(rng.integers(0, 2))
+            ash, bsh = (k, m) if ta else (m, k), (n, k) if tb else (k, n)
+            a = to_dtype(rng.uniform(-1, 1, ash), "bf16")
+            b = to_dtype(rng.uniform(-1, 1, bsh), "bf16")
+            poison = np.uint16(0x7FC0)  # NaN in front of and behind each operand must not reach a result
+            A, B = (ag.Tensor(ag.Tensor.from_array(np.concatenate([np.full(shift, poison), x.ravel(), np.full(3, poison)])).buffer,
+                              x.shape, (x.shape[1], 1), shift, "bf16") for x in (a, b))
+            bias = to_dtype(rng.uniform(-1, 1, n), "bf16")
+            av, bv = (a.T if ta else a), (b.T if tb else b)
+            want = orc.gemm_bf16_f32acc(av, bv, 1.0, 0.0, np.zeros((m, n), np.uint16))
+            seen = []
+            for cfg in (None, "3", "4"):
+                if cfg is None:
+                    monkeypatch.delenv("AGH_GEMM_CFG", raising=False)
+                else:
+                    monkeypatch.setenv("AGH_GEMM_CFG", cfg)
+                big = np.full((m + 2, n + 3), 0x1234, np.uint16)
+                buf = ag.Tensor.from_array(big)
+                C = ag.Tensor(buf.buffer, (m, n), (n + 3, 1), n + 3 + 1, "bf16")
+                try:
+                    ag.gemm(1.0, A.t() if ta else A, B.t() if tb else B, 0.0, C)
+                except ag.AghError as e:  # k-rows closer than 8 elements: element-wise loaders, no 128 x 128 tile
+                    assert cfg == "3" and e.code == -4 and min(m, n) < 8
+                    continue
+                out = buf.into_array()
+                got = out[1:m + 1, 1:n + 1].copy()
+                out[1:m + 1, 1:n + 1] = 0x1234
+                assert np.array_equal(out, big), (m, n, ta, tb, cfg)
+                assert_bf16_gemm_close(got, want, av, bv)
+                seen.append(got)
+                ag.gemm(1.0, A.t() if ta else A, B.t() if tb else B, 0.0, C, bias=ag.Tensor.from_array(bias), relu=True)
+                biased = buf.into_array()[1:m + 1, 1:n + 1]
+                s = orc.f32_to_bf16(orc.bf16_to_f32(got) + orc.bf16_to_f32(bias)[None, :])
+                assert np.array_equal(biased, np.where(orc.bf16_to_f32(s) >= 0, s, np.uint16(0))), (m, n, ta, tb, cfg)
+            if min(m, n) >= 8:
+                assert len(seen) == 3 and all(np.array_equal(seen[0], x) for x in seen[1:]), (m, n, ta, tb)
+    monkeypatch.delenv("AGH_GEMM_CFG", raising=False)
+
+
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
 def test_dense_full_size_bias_relu(ag, dtype):
     """The Dense-shaped GEMM of the benchmark list at full size: M = 16384 (batch), K = 4096, N = 4096 with the
