@@ -414,12 +414,18 @@ struct Col2imRingParams {
     int fh, fw, ph, pw, sh, sw, dh, dw;
     int ktot, cc, nchunk, nband, band_rows;
     int ngroup;  // images * bands
-    int rows;    // patch rows per step (unit-stride kernel)
+    int rows;    // patch rows per step (kernel of strides 1 and 2)
     int lw;     // 32-bit words per patch segment (cc*fh*fw elements)
     int pitch;  // LDS pitch of a staged segment (elements); an odd number of words
     int rh;     // ring rows
     FastDiv div_nchunk, div_nband, div_iw, div_lw, div_sw, div_rh;
 };
+
+// all-zero segments on either side of a staged patch row (strides S, filter width F): a tap of a pixel column, also one
+// that lies just behind the filter row, is never further out
+__host__ __device__ constexpr int col2im_pad_segments(int F, int S, int pw) {
+    return S == 1 ? (F - 1 > pw ? F - 1 - pw : 0) : (F > pw ? (F - pw + S - 1) / S : 0);
+}
 
 constexpr int kCol2imPrefetch = 32;  // 32-bit words a thread holds for the next step
 
@@ -527,17 +533,20 @@ __global__ __launch_bounds__(kThreads) void col2im_ring_kernel(const T *__restri
     }
 }
 
-// Unit stride and dilation, square filter known at compile time: the streaming form with everything
-// the general kernel computes per tap hoisted or folded.  The stage carries FW-1-pw all-zero segments
+// Unit dilation, stride S (1 or 2, the same both ways) and square filter known at compile time: the streaming form with
+// everything the general kernel computes per tap hoisted or folded.  The stage carries (F-1-pw)/S all-zero segments
 // on either side, so a tap never has to ask whether its patch column exists (adding +0 to a running
 // sum changes nothing: a sum that starts at +0 can never be -0).  The F running sums of a pixel
 // column sit in registers and move down one place per step, the finished one leaving for memory.
 // Per thread and step: eight 16-byte loads, the stage write, and per owned pixel column F*F LDS
-// reads and adds.
+// reads and adds.  At stride 2 a pixel column meets every second tap (which ones depends on its parity, a lane's own
+// offset), the sums move two places, and two rows leave per step; where the parity has one tap less, +0 is added.
+// Against the general kernel, which divides and branches per tap: f32 193 x 64 channels, 43 x 19 patches of 5 x 5,
+// 956 -> 304 us, bf16 991 -> 186 us; bf16 64 x 64 channels, 28 x 28 patches of 3 x 3, 96 -> 28 us.
 // Workgroup ids are dealt round-robin to the 8 XCDs, each with an L2 of its own; the chunks of one
 // (image, band) share cache lines where their segments meet, so they are given ids 8 apart: same
 // XCD, dispatched together.
-template <typename T, int F>
+template <typename T, int F, int S>
 __global__ __launch_bounds__(kThreads) void col2im_ring_unit_kernel(const T *__restrict__ x, T *__restrict__ y,
                                                                      Col2imRingParams p) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -546,7 +555,9 @@ __global__ __launch_bounds__(kThreads) void col2im_ring_unit_kernel(const T *__r
     constexpr int NCOL = 4;                   // pixel columns per thread (cc*iw <= NCOL*kThreads)
     const int tid = threadIdx.x;
     const int ncol = p.cc * p.iw;
-    const int padl = max(0, F - 1 - p.pw);
+    constexpr int NR = F > S ? F : S;         // image rows a step holds sums of
+    constexpr int M = (F + S - 1) / S;        // taps of a filter row that a pixel column meets, at most
+    const int padl = col2im_pad_segments(F, S, p.pw);
     T *stage = (T *)smem_raw;                 // [gw + 2*padl][pitch]
     uint32_t *stage32 = (uint32_t *)stage;
     uint32_t slot8, chunk, b, band;
@@ -557,8 +568,9 @@ __global__ __launch_bounds__(kThreads) void col2im_ring_unit_kernel(const T *__r
     constexpr int ff = F * F;
     const int c0 = chunk * p.cc;
     const int hy0 = band * p.band_rows, hy1 = min(p.ih, hy0 + p.band_rows);
-    const int hi_lo = max(0, hy0 + p.ph - (F - 1));
-    const int hi_hi = min(p.gh - 1, hy1 - 1 + p.ph);
+    // patch rows hi whose image rows [hi*S - ph, hi*S - ph + NR) meet the band
+    const int hi_lo = max(0, hy0 + p.ph - (NR - 1) + S - 1) / S;
+    const int hi_hi = min(p.gh - 1, (hy1 - 1 + p.ph) / S);
     const int ktotw = p.ktot / EPW, pitchw = p.pitch / EPW;
 
     for (int r = 0; r < p.rows; ++r)
@@ -585,19 +597,23 @@ __global__ __launch_bounds__(kThreads) void col2im_ring_unit_kernel(const T *__r
     }
     int tap_base[NCOL];
     T *ycol[NCOL];
-    T acc[NCOL][F];
+    bool short_col[NCOL];  // tap M-1 lies behind the filter row
+    T acc[NCOL][NR];
 #pragma unroll
     for (int j = 0; j < NCOL; ++j) {
         const int col = tid + j * kThreads;
         uint32_t cl, wy;
         p.div_iw.divmod((uint32_t)min(col, ncol - 1), cl, wy);
-        // element offset of tap fj = 0 of filter row 0; tap (fi, fj) is at + fi*F - fj*(pitch-1)
-        tap_base[j] = ((int)wy + p.pw + padl) * p.pitch + (int)cl * ff;
+        // element offset of the column's tap m = 0 (fj = rem) of filter row 0; tap (fi, fj = rem + m*S) is at
+        // + fi*F - m*(pitch-S)
+        const int tw = (int)wy + p.pw, rem = tw % S;
+        tap_base[j] = (tw / S + padl) * p.pitch + (int)cl * ff + rem;
+        short_col[j] = rem + (M - 1) * S >= F;
         ycol[j] = y + (((size_t)b * p.c + c0 + cl) * p.ih) * (size_t)p.iw + wy;
 #pragma unroll
-        for (int fi = 0; fi < F; ++fi) acc[j][fi] = Elem<T>::zero();
+        for (int fi = 0; fi < NR; ++fi) acc[j][fi] = Elem<T>::zero();
     }
-    const int tap_step = p.pitch - 1;
+    const int tap_step = p.pitch - S;
 
     u32x4 reg[PFV];
     auto prefetch = [&](int hi) {
@@ -627,7 +643,7 @@ __global__ __launch_bounds__(kThreads) void col2im_ring_unit_kernel(const T *__r
         for (int r = 0; r < rows && hi0 + r <= hi_hi; ++r) {
             // acc[j][fi] is the running sum of image row start + fi
             const int hi = hi0 + r;
-            const int start = hi - p.ph;
+            const int start = hi * S - p.ph;
             const bool last = hi == hi_hi;
             const T *st = stage + r * nseg * p.pitch;
 #pragma unroll
@@ -639,22 +655,24 @@ __global__ __launch_bounds__(kThreads) void col2im_ring_unit_kernel(const T *__r
                         const int hy = start + fi;
                         if (hy >= hy0 && hy < hy1) {  // wave-uniform
 #pragma unroll
-                            for (int fj = F - 1; fj >= 0; --fj) {
-                                const T v = st[tap_base[j] - fj * tap_step + fi * F];
+                            for (int m = M - 1; m >= 0; --m) {
+                                T v = st[tap_base[j] - m * tap_step + fi * F];
+                                if (m == M - 1 && F % S != 0) v = short_col[j] ? Elem<T>::zero() : v;
                                 acc[j][fi] = Elem<T>::from_f32(Elem<T>::raw(acc[j][fi]) + Elem<T>::raw(v));
                             }
                         }
                     }
-                    // row `start` gets nothing from later patch rows; after the last patch row all rows are final
-                    if (start >= hy0 && start < hy1) ycol[j][(size_t)start * p.iw] = acc[j][0];
+                    // the first S rows get nothing from later patch rows; after the last patch row all rows are final
+#pragma unroll
+                    for (int fi = 0; fi < S; ++fi)
+                        if (start + fi >= hy0 && start + fi < hy1) ycol[j][(size_t)(start + fi) * p.iw] = acc[j][fi];
                     if (last) {
 #pragma unroll
-                        for (int fi = 1; fi < F; ++fi)
+                        for (int fi = S; fi < NR; ++fi)
                             if (start + fi >= hy0 && start + fi < hy1) ycol[j][(size_t)(start + fi) * p.iw] = acc[j][fi];
                     }
 #pragma unroll
-                    for (int fi = 0; fi + 1 < F; ++fi) acc[j][fi] = acc[j][fi + 1];
-                    acc[j][F - 1] = Elem<T>::zero();
+                    for (int fi = 0; fi < NR; ++fi) acc[j][fi] = fi + S < NR ? acc[j][fi + S < NR ? fi + S : fi] : Elem<T>::zero();
                 }
             }
         }
@@ -669,9 +687,9 @@ bool col2im_ring_plan(Col2imRingParams &p, size_t &smem, int64_t &nblocks, bool 
     constexpr int64_t es = sizeof(T), epw = 4 / es;
     const int64_t ff = fh * fw, ktot = c * ff;
     if (((uintptr_t)x & 3) != 0 || ktot % epw != 0) return false;
-    // the unit-stride kernel loads 16-byte vectors and carries zero segments around the stage
+    // the kernel of strides 1 and 2 loads 16-byte vectors and carries zero segments around the stage
     if (unit && (((uintptr_t)x & 15) != 0 || (ktot * es) % 16 != 0)) return false;
-    const int64_t segs = unit ? gw + 2 * std::max<int64_t>(0, fw - 1 - pw) : gw;
+    const int64_t segs = unit ? gw + 2 * col2im_pad_segments((int)fw, (int)sw, (int)pw) : gw;
     const int64_t rh = (fh - 1) * dh + 1;
     constexpr int64_t kLdsBudget = 48 * 1024;
     int64_t cc = 0, lds = 0, pitch = 0, nrows = 1;
@@ -752,18 +770,18 @@ int col2im_launch(const char *name, const void *x, void *y, int64_t bs, int64_t 
         Col2imRingParams rp;
         size_t smem = 0;
         int64_t nblocks = 0;
-        const bool unit_geom = sh == 1 && sw == 1 && dh == 1 && dw == 1 && fh == fw &&
+        const bool unit_geom = sh == sw && sh <= 2 && dh == 1 && dw == 1 && fh == fw &&
                                (fh == 1 || fh == 2 || fh == 3 || fh == 5 || fh == 7);
         auto launch = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3((unsigned)nblocks), dim3(kThreads), smem, stream(), (const T *)x, (T *)y, rp);
         };
         if (unit_geom && col2im_ring_plan<T>(rp, smem, nblocks, true, x, bs, c, ih, iw, oh, ow, fh, fw, ph, pw, sh, sw, dh, dw)) {
-            switch (fh) {
-                case 1: launch(col2im_ring_unit_kernel<T, 1>); break;
-                case 2: launch(col2im_ring_unit_kernel<T, 2>); break;
-                case 3: launch(col2im_ring_unit_kernel<T, 3>); break;
-                case 5: launch(col2im_ring_unit_kernel<T, 5>); break;
-                default: launch(col2im_ring_unit_kernel<T, 7>); break;
+            switch (fh * 2 + sh - 1) {
+#define AGH_C2I(FV) \
+    case FV * 2: launch(col2im_ring_unit_kernel<T, FV, 1>); break; \
+    case FV * 2 + 1: launch(col2im_ring_unit_kernel<T, FV, 2>); break
+                AGH_C2I(1); AGH_C2I(2); AGH_C2I(3); AGH_C2I(5); AGH_C2I(7);
+#undef AGH_C2I
             }
             AGH_LAUNCH_CHECK(name);
             return AGH_OK;

@@ -1003,6 +1003,23 @@ def test_im2col_col2im_seeded(ag, dtype, case, ring, monkeypatch):
     assert np.array_equal(dx, want)  # bit-exact incl. bf16's per-add rounding in host order
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("f", [1, 2, 3, 5, 7])
+@pytest.mark.parametrize("size", [(3, 8, 17, 23), (2, 16, 32, 19), (130, 24, 9, 12)])
+@pytest.mark.parametrize("p", [0, 1, 3, 4])
+def test_col2im_stride2(ag, dtype, f, size, p, monkeypatch):
+    """The streaming col2im at stride 2 against the host's order, bit for bit: odd and even images, filters narrower than the
+    stride, padding beyond the filter, several bands per image."""
+    monkeypatch.setenv("AGH_COL2IM_RING", "1")
+    bs, c, gh, gw = size
+    oh, ow = ((g - 1) * 2 + f - 2 * p for g in (gh, gw))
+    rng = np.random.default_rng(19)
+    g = to_dtype(rng.standard_normal((bs * gh * gw, c * f * f)), dtype)
+    dx = ag.Tensor.from_array(g).col2im_conv2(ag.Col2ImConv2Options((gh, gw), (f, f), (p, p), (2, 2))).into_array()
+    assert dx.shape == (bs, c, oh, ow)
+    assert np.array_equal(dx, orc.col2im_conv2(g, (gh, gw), (f, f), (p, p), (2, 2)))
+
+
 def test_col2im_bf16_rounding_order_case(ag):
     f, p = (1, 3), (0, 1)
     cols = np.zeros((3, 3), dtype=np.float32)
