@@ -33,15 +33,6 @@ struct ConvParams {
     FastDiv div_items, div_pix, div_yw;
 };
 
-template <typename T>
-__device__ __forceinline__ T round_bias_relu(float acc, bool has_bias, T bias, int act) {
-    T r = Elem<T>::from_f32(acc);
-    const T rb = Elem<T>::from_f32(Elem<T>::to_f32(bias) + Elem<T>::to_f32(r));
-    r = has_bias ? rb : r;
-    const bool neg = !(Elem<T>::to_f32(r) >= 0.0f);
-    return (act == AGH_ACT_RELU && neg) ? Elem<T>::zero() : r;
-}
-
 // Fills n LDS slots from global memory with U reads of a thread in flight at a time: `get(e)` reads (it is called
 // with e < n only and must not fault), `put(e, v)` stores.  Written as two unrolled passes because a plain
 // `for (e...) lds[e] = g[...]` loop compiles to one read, one wait and one store per trip, and a workgroup that stages
@@ -1582,6 +1573,13 @@ int conv2_direct_entry(const char *name, const void *x, const void *w, const voi
         if (rc != 1) return rc;
     }
 
+    // the matrix-core kernel of any geometry, where it expects to need less than `limit_us` (1: not taken).  The limits
+    // below are fitted to the times of 100 shapes from 1 x 1 x 27 x 66 to 256 x 64 x 96 x 96, both sides measured.
+    auto taps_kernel = [&](double limit_us) {
+        return pool2x2 ? 1 : conv2_taps_try<T>(name, x, w, bias, y, bs, ic, ih, iw, oc, fh, fw, ph, pw, sh, sw, dh, dw, oh, ow, act, limit_us);
+    };
+    if (const int rc = taps_kernel(0.0); rc != 1) return rc;  // (only when forced)
+
     // up to 16 output channels over enough taps on small images: matrix cores fed from the staged image
     if (sh == 1 && sw == 1 && dh == 1 && dw == 1 && oc <= 16) {
         const char *env = getenv("AGH_CONV_SMALL");  // 0 / 1 forces the choice (measurements)
@@ -1677,6 +1675,11 @@ int conv2_direct_entry(const char *name, const void *x, const void *w, const voi
             q.div_ocpad = FastDiv((uint32_t)q.ocpad);
             q.div_pitch = FastDiv((uint32_t)q.pitch);
             q.div_ihp = FastDiv((uint32_t)q.ihp);
+            // one image per workgroup is a long walk where there are many channels and few images: 1 x 3 x 32 x 109 to 64
+            // channels, 5 x 5, 1007 us here and 14 us on the matrix cores; 64 x 3 x 64 x 64 to 64, 3 x 3, 253 and 27
+            const double walk_us = (double)((imgs * items + 255) / 256) * (1.0 + 0.04 * (double)(taps * oct)) *
+                                   std::max(1.0, (double)((bs + imgs - 1) / imgs) / (2.0 * (double)cus));
+            if (const int rc = taps_kernel(0.7 * walk_us); rc != 1) return rc;
             const int64_t work = imgs * items;
             const int threads = work >= 256 ? 256 : (int)((work + 63) / 64 * 64);
             const int64_t blocks = (bs + imgs - 1) / imgs;
@@ -1720,15 +1723,29 @@ int conv2_direct_entry(const char *name, const void *x, const void *w, const voi
     const int64_t taps = ic * fh * fw;
     const int64_t img_bytes = ic * ih * iw * 4, w_bytes = taps * p.ocpad * 4;
     constexpr int64_t kLds = 64 * 1024;
-    if (w_bytes + img_bytes > kLds || items > ((int64_t)1 << 24))
+    if (w_bytes + img_bytes > kLds || items > ((int64_t)1 << 24)) {
+        // otherwise im2col and a product: the patch matrix written and read (faster while the last-level cache holds it), the
+        // product on whole 16-byte rows or through element-wise loaders, 64 channels at least; 30 us for the calls.
+        // Taken against that: 64 x 3 x 95 x 95 to 64, 7 x 7 stride 2, f32 76 -> 44 us; 64 x 24 x 30 x 30 to 48, 3 x 3, f32
+        // 57 -> 23, bf16 35 -> 23 us.  Not taken: 64 x 64 x 56 x 56 to 128, 3 x 3 stride 2, f32 106 (here 149), bf16 39 (157).
+        const bool whole = taps * (int64_t)sizeof(T) % 16 == 0;
+        const double patch = (double)bs * oh * ow * taps * sizeof(T), flops = 2.0 * bs * oh * ow * taps * ((oc + 63) / 64 * 64);
+        const double chain_us = 6.0 + 2.0 * patch / (patch < 128e6 ? 8e6 : 5e6) +
+                                flops / (sizeof(T) == 4 ? (whole ? 100e6 : 50e6) : (whole ? 450e6 : 65e6));
+        if (const int rc = taps_kernel(0.85 * std::max(30.0, chain_us)); rc != 1) return rc;
         return fail(AGH_ERANGE, "%s: image + filter bank (%lld bytes) do not fit in LDS; use im2col + gemm", name,
                     (long long)(w_bytes + img_bytes));
+    }
     // images per workgroup: aim at ~256 work items, stay inside LDS, keep >= 2 workgroups per CU
     int64_t imgs = items >= 256 ? 1 : 256 / items;
     while (imgs > 1 && w_bytes + imgs * img_bytes > kLds) --imgs;
     const int64_t cus = compute_units() > 0 ? compute_units() : 256;
     while (imgs > 1 && (bs + imgs - 1) / imgs < 2 * cus) --imgs;
     if (imgs > bs) imgs = bs;
+    // (5 x 1 x 108 x 108 to 48, 5 x 5 stride 2: 289 us here, 14 us on the matrix cores)
+    const double walk_us = (double)((imgs * items + 255) / 256) * (1.5 + 0.02 * (double)(taps * oct)) *
+                           std::max(1.0, (double)((bs + imgs - 1) / imgs) / (2.0 * (double)cus));
+    if (const int rc = taps_kernel(0.7 * walk_us); rc != 1) return rc;
     p.imgs = (int)imgs;
     p.items_per_img = (int)items;
     p.div_items = FastDiv((uint32_t)items);

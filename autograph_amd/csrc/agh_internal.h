@@ -27,6 +27,12 @@ int static_workspace(size_t bytes, void **ptr);
 template <typename T>
 int conv2_mfma_try(const char *name, const void *x, const void *w, const void *bias, void *y, int64_t bs, int64_t ic, int64_t ih,
                    int64_t iw, int64_t oc, int64_t fh, int64_t fw, int64_t ph, int64_t pw, int64_t oh, int64_t ow, int act);
+// Conv2 forward for any stride, dilation and channel count on the f32 matrix cores (agh_conv_taps.hip); 1 = not taken:
+// the shape is not its own, or it expects to need more than limit_us
+template <typename T>
+int conv2_taps_try(const char *name, const void *x, const void *w, const void *bias, void *y, int64_t bs, int64_t ic, int64_t ih,
+                   int64_t iw, int64_t oc, int64_t fh, int64_t fw, int64_t ph, int64_t pw, int64_t sh, int64_t sw, int64_t dh,
+                   int64_t dw, int64_t oh, int64_t ow, int act, double limit_us);
 
 #define AGH_API_ENTER()                                           \
     std::lock_guard<std::recursive_mutex> _agh_lock(agh::api_mutex()); \
@@ -106,5 +112,15 @@ template <> struct Elem<uint16_t> {
     static __device__ __forceinline__ uint16_t from_f32(float v) { return f32_to_bf16(v); }
     static __device__ __forceinline__ uint16_t zero() { return 0; }
 };
+
+// a convolution's epilogue, in the order of the separate layers: round to T, add the bias in T, ReLU
+template <typename T>
+__device__ __forceinline__ T round_bias_relu(float acc, bool has_bias, T bias, int act) {
+    T r = Elem<T>::from_f32(acc);
+    const T rb = Elem<T>::from_f32(Elem<T>::to_f32(bias) + Elem<T>::to_f32(r));
+    r = has_bias ? rb : r;
+    const bool neg = !(Elem<T>::to_f32(r) >= 0.0f);
+    return (act == AGH_ACT_RELU && neg) ? Elem<T>::zero() : r;
+}
 
 }  // namespace agh

@@ -36,7 +36,7 @@ def conv2_im2col_forward(x, weight, padding=(0, 0), stride=(1, 1), dilation=(1, 
 
 def conv2_direct_forward(x, weight, padding=(0, 0), stride=(1, 1), dilation=(1, 1), bias=None, relu=False, pool2x2=False):
     """Direct convolution out of LDS (agh_conv2_direct_*), optionally with the following Relu and
-    2x2/2 MaxPool2 fused.  Raises AghError(AGH_ERANGE) when the layer does not fit in LDS."""
+    2x2/2 MaxPool2 fused.  Raises AghError(AGH_ERANGE) when the layer does not fit in LDS and no matrix-core kernel takes it."""
     x = x.as_standard_layout()
     bs, ic, ih, iw = x.shape
     oc, ic2, fh, fw = weight.shape

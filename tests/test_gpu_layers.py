@@ -103,6 +103,55 @@ def test_conv2_seeded_both_algorithms(ag, dtype, case):
         assert np.array_equal(yb, ref), alg
 
 
+CONV_TAPS = [
+    # bs, ic, ih, iw, oc, filter, padding, stride, dilation: every tile, ragged positions, channels and taps
+    (2, 3, 95, 95, 64, (7, 7), (3, 3), (2, 2), (1, 1)),      # 147 taps: the last chunk of 16 holds three
+    (64, 3, 95, 95, 50, (7, 7), (3, 3), (2, 2), (1, 1)),     # the largest tile; 50 = 3 * 16 + 2 channels
+    (1, 16, 73, 25, 128, (3, 3), (1, 1), (1, 1), (1, 1)),
+    (3, 256, 9, 8, 33, (3, 3), (0, 0), (1, 1), (1, 1)),      # channels staged in several chunks
+    (2, 37, 41, 43, 17, (5, 3), (2, 1), (3, 2), (2, 1)),
+    (2, 6, 77, 77, 96, (1, 1), (0, 0), (2, 2), (1, 1)),      # fewer taps than one chunk
+    (1, 1, 131, 129, 6, (1, 1), (0, 0), (1, 1), (1, 1)),     # a single tap
+    (1, 3, 7, 2500, 16, (3, 1), (1, 0), (1, 1), (1, 1)),     # rows longer than a tile
+    (1, 200, 1, 90, 5, (1, 4), (0, 2), (1, 1), (1, 2)),
+]
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("case", CONV_TAPS)
+def test_conv2_taps_kernel(ag, dtype, case, monkeypatch):
+    """Convolutions that neither fit in LDS whole nor suit the implicit GEMM of unit stride, one value of the input infinite:
+    the outputs it reaches, and no others, are not finite."""
+    monkeypatch.setenv("AGH_CONV_TAPS", "1")
+    bs, ic, ih, iw, oc, f, p, s, d = case
+    rng = np.random.default_rng(31)
+    x = rng.standard_normal((bs, ic, ih, iw)).astype(np.float32)
+    w = to_dtype(rng.standard_normal((oc, ic) + f) * np.sqrt(2.0 / (ic * f[0] * f[1])), dtype)
+    b = to_dtype(rng.standard_normal(oc) * 0.1, dtype)
+    x[bs - 1, ic - 1, ih // 2 // s[0] * s[0], iw // 2 // s[1] * s[1]] = np.inf
+    x = to_dtype(x, dtype)
+    with np.errstate(invalid="ignore"):
+        want = orc.conv2_naive_f64(as_f32(x), as_f32(w), p, s, d)
+    scale = orc.conv2_naive_f64(np.where(np.isfinite(as_f32(x)), np.abs(as_f32(x)), 0).astype(np.float32), np.abs(as_f32(w)), p, s, d)
+    k = ic * f[0] * f[1]
+    tx, tw, tb = ag.Tensor.from_array(x), ag.Tensor.from_array(w), ag.Tensor.from_array(b)
+    y = ag.conv2_direct_forward(tx, tw, padding=p, stride=s, dilation=d).into_array()
+    got = as_f32(y).astype(np.float64)
+    fin = np.isfinite(want)
+    assert np.array_equal(np.isfinite(got), fin) and not fin.all()
+    got, want, scale = got[fin], want[fin], scale[fin]
+    if dtype == "f32":  # an f32 sum of k products: k roundings at most, sqrt(k) as they fall
+        assert np.all(np.abs(got - want) <= 1e-5 * np.sqrt(k) * scale + 1e-30)
+    else:               # and one rounding to bf16
+        ulp = 2.0 ** (np.floor(np.log2(np.maximum(np.abs(want), 2.0**-126))) - 7)
+        assert np.all(np.abs(got - want) <= ulp + 8 * np.sqrt(k) * 2.0**-24 * scale)
+    yb = as_f32(ag.conv2_direct_forward(tx, tw, padding=p, stride=s, dilation=d, bias=tb, relu=True).into_array())
+    n, c, h, wd = y.shape
+    flat = np.ascontiguousarray(y.transpose(0, 2, 3, 1).reshape(-1, c))
+    ref = as_f32(orc.relu(orc.bias_add_rows(flat, b)).reshape(n, h, wd, c).transpose(0, 3, 1, 2))
+    assert np.array_equal(yb, ref, equal_nan=True)
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 def test_conv2_direct_fused_relu_pool(ag, dtype):
     """conv -> Relu -> MaxPool2(2x2) in one launch equals the three layers applied to the conv result."""
