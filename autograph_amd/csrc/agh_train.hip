@@ -255,8 +255,9 @@ __global__ __launch_bounds__(kThreads) void sgd_momentum_kernel(T *__restrict__ 
 // read, already widened to f32); the other eight waves keep two chunks of 256 rows in flight and store them to LDS,
 // column-major with a pitch of 260 words, so that 16 lanes of either side meet 16 different bank groups.  A bf16 step is
 // two dependent instructions, the addition and v_cvt_pk_bf16_f32 of (0, sum), whose result is the rounded sum as f32.
-// 4096 x 1000: bf16 27.9 us = 6.8 ns a row, two dependent instructions of about eight cycles; f32 22.6 us.  One thread per
-// column that loads and adds by itself (sum_axis0_short_kernel) pays a memory round trip every eight rows: 251 and 174 us.
+// 4096 x 1000: bf16 27.5 us, f32 21.6 us; 8192 x 1000: 51.7 and 40.2 us, that is 5.9 and 4.5 ns a row (two dependent
+// instructions of about seven cycles; one of eleven) behind about 4 us of starting.  One thread per column that loads and adds
+// by itself (sum_axis0_short_kernel) pays a memory round trip every eight rows: 4096 x 1000 f32 172 us.
 constexpr int kSumCols = 64, kSumRows = 256, kSumLoaders = 8, kSumPitch = kSumRows + 4;
 constexpr int kSumRPW = kSumRows / kSumLoaders;  // rows of a chunk that one loading wave moves
 constexpr size_t kSumLds = 2 * (size_t)kSumCols * kSumPitch * sizeof(float);
@@ -355,9 +356,18 @@ __global__ __launch_bounds__(64 * (1 + kSumLoaders)) void sum_axis0_kernel(const
     }
 }
 
-// The same sums with one thread per column, for at most kSumShortRows rows: 64 x 1000 f32 3.2 us against 6.5 us of the
-// kernel above, whose nine waves and 130 KB of LDS take longer to start; at 42 ns a row it is behind from about 130 rows on.
-constexpr int64_t kSumShortRows = 128;
+// The same sums with one thread per column: all columns at once, bound by a memory round trip every eight rows (16 to 18 ns a
+// row out of the caches) and, where the columns fill the chip several times over, by memory itself.
+// The kernel above has one workgroup of 64 columns on a CU (130 KB of LDS), so it pays its 5.5 us of starting, filling and
+// draining once for every round of CUs * 64 columns.  Both measured over 64 to 32768 rows of 64 to 4194304 columns, one
+// thread / staged in us: 224 x 4096 f32 5.3 / 5.6, 256 x 4096 5.9 / 5.7; 320 x 32768 (two rounds) f32 14.3 / 14.0, bf16
+// 8.1 / 11.7; 512 x 40000 (three) 24.9 / 20.4, 25.7 / 18.2; 768 x 65536 (four) 38.1 / 43.4, 33.7 / 38.2; 1024 x 65536 51.7 / 48.4,
+// 45.1 / 40.0; from eight rounds on one thread per column reaches the memory's rate too: 256 x 262144 38.6 / 86.6,
+// 20.1 / 87.9; 2048 x 131072 181.9 / 192.4, 164.9 / 180.3; 4096 x 131072 365 / 358, 330 / 331.
+__host__ inline bool sum_axis0_staged(int64_t rows, int64_t cols, int64_t cus) {
+    const int64_t per_round = cus * kSumCols, rounds = cols / per_round + (cols % per_round != 0);
+    return rounds < 8 && rows > (rounds < 4 ? 140 + 100 * rounds : 220 * rounds);
+}
 
 template <typename T>
 __global__ __launch_bounds__(kThreads) void sum_axis0_short_kernel(const T *__restrict__ x, T *__restrict__ y, int64_t rows, int64_t cols) {
@@ -568,7 +578,8 @@ int sum_axis0_launch(const char *name, const void *x, void *y, int64_t rows, int
     if (rows < 0 || cols < 0) return fail(AGH_EINVAL, "%s: negative shape", name);
     if (cols == 0) return AGH_OK;
     if (!y || (!x && rows > 0)) return fail(AGH_ENULL, "%s: null buffer", name);
-    const bool brief = rows <= kSumShortRows;
+    const char *env = getenv("AGH_SUM_STAGED");  // 0 / 1 forces the choice (measurements, tests)
+    const bool brief = env && *env ? atoi(env) == 0 : !sum_axis0_staged(rows, cols, compute_units() > 0 ? compute_units() : 256);
     const int64_t per_block = brief ? kThreads : kSumCols, blocks = (cols + per_block - 1) / per_block;
     if (blocks > 0x7FFFFFFFll) return fail(AGH_ERANGE, "%s: too many columns", name);
     if (brief) {

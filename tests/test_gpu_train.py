@@ -2,6 +2,7 @@
 scaled_add, SGD, axis-0 sum, cross-entropy) and of one whole LeNet5 training step
 (benches/neural-network-benches/src/autograph_backend.rs:70-86) against the CPU oracle."""
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -102,14 +103,40 @@ def test_scaled_add_sgd_sum_axis0_bit_exact(ag, dtype):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("rows", [0, 1, 9, 128, 129, 255, 256, 257, 511, 512, 513, 769, 1025])
-def test_sum_axis0_chunk_and_column_edges(ag, dtype, rows):
-    # up to 128 rows one thread adds a column, beyond that rows go through LDS in chunks of 256 (two in flight), 64 columns
-    # a workgroup: bit for bit the serial sum either way
+def test_sum_axis0_chunk_and_column_edges(ag, dtype, rows, monkeypatch):
+    # one thread adds a column, or rows go through LDS in chunks of 256 (two in flight), 64 columns a workgroup: bit for bit
+    # the serial sum in either form, and in the one chosen by size
     rng = np.random.default_rng(rows)
     for cols in (1, 63, 64, 65, 130):
         a = to_dtype(rng.standard_normal((rows, cols)) * 4, dtype)
-        assert np.array_equal(ag.Tensor.from_array(a).sum_axis0().into_array(), orc.sum_axis0(a)), cols
+        t, want = ag.Tensor.from_array(a), orc.sum_axis0(a)
+        for staged in ("", "0", "1"):
+            monkeypatch.setenv("AGH_SUM_STAGED", staged)
+            assert np.array_equal(t.sum_axis0().into_array(), want), (cols, staged)
 
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_sum_axis0_form_chosen_by_rows_and_columns(ag, dtype, monkeypatch):
+    """The form chosen by size is the faster one, to within a half: few rows of many columns (one thread per column 3 to 5
+    times as fast), many rows of few columns (the staged form 2 to 8 times as fast)."""
+    for rows, cols in ((129, 262144), (200, 65536), (1024, 64), (4096, 1000)):
+        x = ag.Tensor.zeros((rows, cols), dtype)
+        y = ag.Tensor.uninit((cols,), dtype)
+        f = getattr(ag.lib, f"agh_sum_axis0_{dtype}")
+        us = {}
+        for staged in ("0", "1", ""):
+            monkeypatch.setenv("AGH_SUM_STAGED", staged)
+            best = float("inf")
+            for _ in range(6):
+                ag.lib.agh_sync()
+                t0 = time.perf_counter()
+                for _ in range(100):
+                    assert f(x._data_ptr(), y._data_ptr(), rows, cols) == 0
+                ag.lib.agh_sync()
+                best = min(best, time.perf_counter() - t0)
+            us[staged] = best * 1e4
+        assert us[""] <= 1.5 * min(us["0"], us["1"]), (rows, cols, us)
 
 
 def _view_of(ag, t, a, base):
