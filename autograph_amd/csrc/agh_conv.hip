@@ -1547,6 +1547,126 @@ int launch_oct(int oct, dim3 grid, dim3 block, size_t smem, const T *x, const T 
     return AGH_OK;
 }
 
+// What conv2_direct_entry chooses by, with the 2x2 pool fused or without.
+struct ConvShape {
+    int64_t bs, ic, ih, iw, oc, fh, fw, ph, pw, sh, sw, dh, dw, oh, ow;
+    bool unit() const { return sh == 1 && sw == 1 && dh == 1 && dw == 1; }
+};
+constexpr int64_t kConvLds = 64 * 1024;
+inline int64_t conv_cus() { return compute_units() > 0 ? compute_units() : 256; }
+
+// up to 16 output channels over enough taps on small images: matrix cores fed from the staged image
+bool conv2_small_plan(const ConvShape &c, bool pool, SmallMfmaParams &q, int64_t &fixed_bytes, int64_t &img_bytes) {
+    if (!c.unit() || c.oc > 16) return false;
+    const char *env = getenv("AGH_CONV_SMALL");  // 0 / 1 forces the choice (measurements)
+    const int64_t taps = c.ic * c.fh * c.fw;
+    const bool want = env ? atoi(env) != 0 : (c.oc >= 8 && taps >= 32);
+    q.bs = (int)c.bs; q.ic = (int)c.ic; q.ih = (int)c.ih; q.iw = (int)c.iw; q.oc = (int)c.oc; q.oh = (int)c.oh; q.ow = (int)c.ow;
+    q.fh = (int)c.fh; q.fw = (int)c.fw; q.ph = (int)c.ph; q.pw = (int)c.pw;
+    q.ihp = (int)(c.ih + 2 * c.ph);
+    q.pitch = (int)(c.iw + 2 * c.pw);
+    q.ktot = (int)taps;
+    q.ksteps = (int)((taps + 31) / 32 * 8);
+    const int64_t yh = pool ? c.oh / 2 : c.oh, yw = pool ? c.ow / 2 : c.ow;
+    fixed_bytes = (int64_t)q.ksteps * 4 * 17 * 4;
+    img_bytes = c.ic * (int64_t)q.ihp * q.pitch * 4;
+    return want && taps <= 2048 && fixed_bytes + img_bytes <= kConvLds && yh * yw <= ((int64_t)1 << 20);
+}
+
+// stride 1, dilation 1, filter width 3 or 5: row-tiled kernel.  walk_us: what its work items are expected to take.
+struct LdsPlan {
+    int oct;
+    int64_t items, imgs, w_bytes, img_bytes;
+    double walk_us;
+};
+bool conv2_rowtile_plan(const ConvShape &c, bool pool, RowTileParams &q, LdsPlan &l) {
+    if (!c.unit() || (c.fw != 3 && c.fw != 5)) return false;
+    q.bs = c.bs; q.ic = c.ic; q.ih = c.ih; q.iw = c.iw; q.oc = c.oc; q.oh = c.oh; q.ow = c.ow; q.fh = c.fh; q.ph = c.ph; q.pw = c.pw;
+    // two output channels per work item unless that leaves fewer than ~4 waves per CU in flight
+    const int64_t rows0 = pool ? c.oh / 2 : c.oh, wbs0 = (c.ow + 7) / 8;
+    l.oct = (c.oc <= 1 || c.bs * rows0 * wbs0 * ((c.oc + 1) / 2) < conv_cus() * 4 * 64) ? 1 : 2;
+    q.ngroups = (c.oc + l.oct - 1) / l.oct;
+    q.ocpad = q.ngroups * l.oct;
+    q.nwb = (c.ow + 7) / 8;
+    q.ihp = c.ih + 2 * c.ph;
+    int64_t pitch = c.iw + 2 * c.pw;
+    if (pitch < q.nwb * 8 + c.fw - 1) pitch = q.nwb * 8 + c.fw - 1;
+    // whole 16-byte reads of WT + FW - 1 floats starting at a multiple of 8
+    const int64_t xw4 = ((8 + c.fw - 1 + 3) / 4) * 4;
+    if (pitch < (q.nwb - 1) * 8 + xw4) pitch = (q.nwb - 1) * 8 + xw4;
+    q.pitch = (int)((pitch + 3) & ~(int64_t)3);
+    q.yh = pool ? c.oh / 2 : c.oh;
+    q.yw = pool ? c.ow / 2 : c.ow;
+    q.nrows = q.yh;
+    const int64_t taps = c.ic * c.fh * c.fw;
+    l.items = (int64_t)q.nrows * q.nwb * q.ngroups;
+    l.w_bytes = ((taps * q.ocpad + 3) & ~(int64_t)3) * 4;
+    l.img_bytes = (int64_t)c.ic * q.ihp * q.pitch * 4;
+    if (l.w_bytes + l.img_bytes > kConvLds || l.items > ((int64_t)1 << 24)) return false;
+    l.imgs = l.items >= 256 ? 1 : 256 / l.items;
+    while (l.imgs > 1 && l.w_bytes + l.imgs * l.img_bytes > kConvLds) --l.imgs;
+    while (l.imgs > 1 && (c.bs + l.imgs - 1) / l.imgs < conv_cus()) --l.imgs;
+    if (l.imgs > c.bs) l.imgs = c.bs;
+    // one image per workgroup is a long walk where there are many channels and few images
+    l.walk_us = (double)((l.imgs * l.items + 255) / 256) * (1.0 + 0.04 * (double)(taps * l.oct)) *
+                std::max(1.0, (double)((c.bs + l.imgs - 1) / l.imgs) / (2.0 * (double)conv_cus()));
+    return true;
+}
+
+// any geometry whose image and filter bank fit in LDS
+bool conv2_lds_plan(const ConvShape &c, bool pool, ConvParams &p, LdsPlan &l) {
+    p.bs = c.bs; p.ic = c.ic; p.ih = c.ih; p.iw = c.iw; p.oc = c.oc; p.oh = c.oh; p.ow = c.ow;
+    p.fh = c.fh; p.fw = c.fw; p.ph = c.ph; p.pw = c.pw; p.sh = c.sh; p.sw = c.sw; p.dh = c.dh; p.dw = c.dw;
+    p.yh = pool ? c.oh / 2 : c.oh;
+    p.yw = pool ? c.ow / 2 : c.ow;
+    // output channels per work item: the whole bank when it is small, else groups of 8
+    l.oct = 8;
+    for (int o : {1, 2, 4, 6, 8})
+        if (c.oc <= o) { l.oct = o; break; }
+    p.ngroups = (c.oc + l.oct - 1) / l.oct;
+    p.ocpad = p.ngroups * l.oct;
+    const int64_t taps = c.ic * c.fh * c.fw;
+    l.items = (int64_t)p.yh * p.yw * p.ngroups;
+    l.img_bytes = c.ic * c.ih * c.iw * 4;
+    l.w_bytes = taps * p.ocpad * 4;
+    if (l.w_bytes + l.img_bytes > kConvLds || l.items > ((int64_t)1 << 24)) return false;
+    // images per workgroup: aim at ~256 work items, stay inside LDS, keep >= 2 workgroups per CU
+    l.imgs = l.items >= 256 ? 1 : 256 / l.items;
+    while (l.imgs > 1 && l.w_bytes + l.imgs * l.img_bytes > kConvLds) --l.imgs;
+    while (l.imgs > 1 && (c.bs + l.imgs - 1) / l.imgs < 2 * conv_cus()) --l.imgs;
+    if (l.imgs > c.bs) l.imgs = c.bs;
+    l.walk_us = (double)((l.imgs * l.items + 255) / 256) * (1.5 + 0.02 * (double)(taps * l.oct)) *
+                std::max(1.0, (double)((c.bs + l.imgs - 1) / l.imgs) / (2.0 * (double)conv_cus()));
+    return true;
+}
+
+// The time below which the matrix-core kernel of any geometry (agh_conv_taps.hip) is taken for the convolution without the
+// pool, against what would run in its place.
+template <typename T>
+double conv2_taps_limit(const ConvShape &c) {
+    SmallMfmaParams sq;
+    RowTileParams rq;
+    ConvParams p;
+    LdsPlan l;
+    int64_t fixed_bytes, img_bytes;
+    if (conv2_small_plan(c, false, sq, fixed_bytes, img_bytes)) return 0.0;
+    // 1 x 3 x 32 x 109 to 64 channels, 5 x 5, 1007 us on row tiles and 14 us on the matrix cores; 64 x 3 x 64 x 64 to 64,
+    // 3 x 3, 253 and 27
+    if (conv2_rowtile_plan(c, false, rq, l)) return 0.7 * l.walk_us;
+    // 5 x 1 x 108 x 108 to 48, 5 x 5 stride 2: 289 and 14 us
+    if (conv2_lds_plan(c, false, p, l)) return 0.7 * l.walk_us;
+    // otherwise im2col and a product: the patch matrix written and read (faster while the last-level cache holds it), the
+    // product on whole 16-byte rows or through element-wise loaders, 64 channels at least; 30 us for the calls.
+    // Taken against that: 64 x 3 x 95 x 95 to 64, 7 x 7 stride 2, f32 76 -> 44 us; 64 x 24 x 30 x 30 to 48, 3 x 3, f32
+    // 57 -> 23, bf16 35 -> 23 us.  Not taken: 64 x 64 x 56 x 56 to 128, 3 x 3 stride 2, f32 106 (here 149), bf16 39 (157).
+    const int64_t taps = c.ic * c.fh * c.fw;
+    const bool whole = taps * (int64_t)sizeof(T) % 16 == 0;
+    const double patch = (double)c.bs * c.oh * c.ow * taps * sizeof(T), flops = 2.0 * c.bs * c.oh * c.ow * taps * ((c.oc + 63) / 64 * 64);
+    const double chain_us = 6.0 + 2.0 * patch / (patch < 128e6 ? 8e6 : 5e6) +
+                            flops / (sizeof(T) == 4 ? (whole ? 100e6 : 50e6) : (whole ? 450e6 : 65e6));
+    return 0.85 * std::max(30.0, chain_us);
+}
+
 template <typename T>
 int conv2_direct_entry(const char *name, const void *x, const void *w, const void *bias, void *y, int64_t bs,
                        int64_t ic, int64_t ih, int64_t iw, int64_t oc, int64_t fh, int64_t fw, int64_t ph, int64_t pw,
@@ -1568,49 +1688,44 @@ int conv2_direct_entry(const char *name, const void *x, const void *w, const voi
     if (!x || !w || !y) return fail(AGH_ENULL, "%s: null buffer", name);
 
     // enough channels: implicit GEMM on the matrix cores (returns 1 when the geometry is not its own)
-    if (sh == 1 && sw == 1 && dh == 1 && dw == 1 && !pool2x2) {
+    const char *env = getenv("AGH_CONV_TAPS");  // 0 / 1 forces the choice of the kernel of any geometry (measurements, tests)
+    const int taps_forced = env && *env ? (atoi(env) != 0 ? 1 : 0) : -1;
+    const ConvShape shape = {bs, ic, ih, iw, oc, fh, fw, ph, pw, sh, sw, dh, dw, oh, ow};
+    const bool mfma_geometry = shape.unit() && conv2_mfma_takes<T>(x, w, bs, ic, ih, iw, oc, fh, fw, pw, oh, ow);
+    if (mfma_geometry && !pool2x2 && taps_forced != 1) {
         const int rc = conv2_mfma_try<T>(name, x, w, bias, y, bs, ic, ih, iw, oc, fh, fw, ph, pw, oh, ow, act);
         if (rc != 1) return rc;
     }
 
-    // the matrix-core kernel of any geometry, where it expects to need less than `limit_us` (1: not taken).  The limits
-    // below are fitted to the times of 100 shapes from 1 x 1 x 27 x 66 to 256 x 64 x 96 x 96, both sides measured.
-    auto taps_kernel = [&](double limit_us) {
-        return pool2x2 ? 1 : conv2_taps_try<T>(name, x, w, bias, y, bs, ic, ih, iw, oc, fh, fw, ph, pw, sh, sw, dh, dw, oh, ow, act, limit_us);
-    };
-    if (const int rc = taps_kernel(0.0); rc != 1) return rc;  // (only when forced)
+    // the matrix-core kernel of any geometry, where it expects to need less time than what would run in its place; with the
+    // pool, where the convolution alone would run on it (the fused call returns the same bits as the separate layers)
+    if (taps_forced == 1 || (taps_forced != 0 && !(mfma_geometry && pool2x2))) {
+        const int rc = conv2_taps_try<T>(name, x, w, bias, y, bs, ic, ih, iw, oc, fh, fw, ph, pw, sh, sw, dh, dw, oh, ow, act, pool2x2 != 0,
+                                         taps_forced == 1, conv2_taps_limit<T>(shape));
+        if (rc != 1) return rc;
+        if (taps_forced == 1) return fail(AGH_ERANGE, "%s: AGH_CONV_TAPS=1, and that kernel does not take this shape", name);
+    }
 
-    // up to 16 output channels over enough taps on small images: matrix cores fed from the staged image
-    if (sh == 1 && sw == 1 && dh == 1 && dw == 1 && oc <= 16) {
-        const char *env = getenv("AGH_CONV_SMALL");  // 0 / 1 forces the choice (measurements)
-        const int64_t taps = ic * fh * fw;
-        const bool want = env ? atoi(env) != 0 : (oc >= 8 && taps >= 32);
-        SmallMfmaParams q;
-        q.bs = (int)bs; q.ic = (int)ic; q.ih = (int)ih; q.iw = (int)iw; q.oc = (int)oc; q.oh = (int)oh; q.ow = (int)ow;
-        q.fh = (int)fh; q.fw = (int)fw; q.ph = (int)ph; q.pw = (int)pw;
+    SmallMfmaParams sq;
+    int64_t fixed_bytes = 0, small_img_bytes = 0;
+    if (conv2_small_plan(shape, pool2x2 != 0, sq, fixed_bytes, small_img_bytes)) {
+        SmallMfmaParams &q = sq;
+        const int64_t img_bytes = small_img_bytes, yh = pool2x2 ? oh / 2 : oh, yw = pool2x2 ? ow / 2 : ow;
         q.act = act; q.has_bias = bias != nullptr;
-        q.ihp = (int)(ih + 2 * ph);
-        q.pitch = (int)(iw + 2 * pw);
-        q.ktot = (int)taps;
-        q.ksteps = (int)((taps + 31) / 32 * 8);
-        const int64_t yh = pool2x2 ? oh / 2 : oh, yw = pool2x2 ? ow / 2 : ow;
         q.nout = (int)(yh * yw);
         q.yw = (int)yw;
         q.mtiles = (int)(pool2x2 ? (yh * yw + 3) / 4 : (yh * yw + 15) / 16);
         const int tg = q.mtiles >= 8 ? 4 : 2;
         q.units_per_img = (q.mtiles + tg - 1) / tg;
-        const int64_t kpad = (int64_t)q.ksteps * 4;
-        const int64_t fixed_bytes = kpad * 17 * 4, img_bytes = ic * (int64_t)q.ihp * q.pitch * 4;
-        constexpr int64_t kLds = 64 * 1024;
-        if (want && taps <= 2048 && fixed_bytes + img_bytes <= kLds && yh * yw <= ((int64_t)1 << 20)) {
-            const int64_t cus = compute_units() > 0 ? compute_units() : 256;
+        {
+            const int64_t cus = conv_cus();
             // a workgroup's four waves want a unit each; more images per workgroup only while the grid still
             // covers the chip twice
             int64_t imgs = std::max<int64_t>(1, 4 / q.units_per_img);
-            while (fixed_bytes + (imgs + 1) * img_bytes <= kLds && (imgs + 1) * q.units_per_img <= 8 &&
+            while (fixed_bytes + (imgs + 1) * img_bytes <= kConvLds && (imgs + 1) * q.units_per_img <= 8 &&
                    (bs + imgs) / (imgs + 1) >= 2 * cus)
                 ++imgs;
-            while (imgs > 1 && fixed_bytes + imgs * img_bytes > kLds) --imgs;
+            while (imgs > 1 && fixed_bytes + imgs * img_bytes > kConvLds) --imgs;
             if (imgs > bs) imgs = bs;
             q.imgs = (int)imgs;
             q.div_pitch = FastDiv((uint32_t)q.pitch);
@@ -1636,37 +1751,13 @@ int conv2_direct_entry(const char *name, const void *x, const void *w, const voi
     }
 
     // stride 1, dilation 1, filter width 3 or 5: row-tiled kernel
-    if (sh == 1 && sw == 1 && dh == 1 && dw == 1 && (fw == 3 || fw == 5)) {
+    LdsPlan l;
+    {
         RowTileParams q;
-        q.bs = bs; q.ic = ic; q.ih = ih; q.iw = iw; q.oc = oc; q.oh = oh; q.ow = ow; q.fh = fh; q.ph = ph; q.pw = pw;
-        q.act = act; q.has_bias = bias != nullptr;
-        // two output channels per work item unless that leaves fewer than ~4 waves per CU in flight
-        const int64_t cus0 = compute_units() > 0 ? compute_units() : 256;
-        const int64_t rows0 = pool2x2 ? oh / 2 : oh, wbs0 = (ow + 7) / 8;
-        const int oct = (oc <= 1 || bs * rows0 * wbs0 * ((oc + 1) / 2) < cus0 * 4 * 64) ? 1 : 2;
-        q.ngroups = (oc + oct - 1) / oct;
-        q.ocpad = q.ngroups * oct;
-        q.nwb = (ow + 7) / 8;
-        q.ihp = ih + 2 * ph;
-        int64_t pitch = iw + 2 * pw;
-        if (pitch < q.nwb * 8 + fw - 1) pitch = q.nwb * 8 + fw - 1;
-        // whole 16-byte reads of WT + FW - 1 floats starting at a multiple of 8
-        const int64_t xw4 = ((8 + fw - 1 + 3) / 4) * 4;
-        if (pitch < (q.nwb - 1) * 8 + xw4) pitch = (q.nwb - 1) * 8 + xw4;
-        q.pitch = (int)((pitch + 3) & ~(int64_t)3);
-        q.yh = pool2x2 ? oh / 2 : oh;
-        q.yw = pool2x2 ? ow / 2 : ow;
-        q.nrows = q.yh;
-        const int64_t items = (int64_t)q.nrows * q.nwb * q.ngroups;
-        const int64_t taps = ic * fh * fw;
-        const int64_t w_bytes = ((taps * q.ocpad + 3) & ~(int64_t)3) * 4, img_bytes = (int64_t)ic * q.ihp * q.pitch * 4;
-        constexpr int64_t kLds = 64 * 1024;
-        if (w_bytes + img_bytes <= kLds && items <= ((int64_t)1 << 24)) {
-            const int64_t cus = compute_units() > 0 ? compute_units() : 256;
-            int64_t imgs = items >= 256 ? 1 : 256 / items;
-            while (imgs > 1 && w_bytes + imgs * img_bytes > kLds) --imgs;
-            while (imgs > 1 && (bs + imgs - 1) / imgs < cus) --imgs;
-            if (imgs > bs) imgs = bs;
+        if (conv2_rowtile_plan(shape, pool2x2 != 0, q, l)) {
+            const int oct = l.oct;
+            const int64_t items = l.items, imgs = l.imgs;
+            q.act = act; q.has_bias = bias != nullptr;
             q.imgs = (int)imgs;
             q.items_per_img = (int)items;
             q.div_items = FastDiv((uint32_t)items);
@@ -1675,16 +1766,11 @@ int conv2_direct_entry(const char *name, const void *x, const void *w, const voi
             q.div_ocpad = FastDiv((uint32_t)q.ocpad);
             q.div_pitch = FastDiv((uint32_t)q.pitch);
             q.div_ihp = FastDiv((uint32_t)q.ihp);
-            // one image per workgroup is a long walk where there are many channels and few images: 1 x 3 x 32 x 109 to 64
-            // channels, 5 x 5, 1007 us here and 14 us on the matrix cores; 64 x 3 x 64 x 64 to 64, 3 x 3, 253 and 27
-            const double walk_us = (double)((imgs * items + 255) / 256) * (1.0 + 0.04 * (double)(taps * oct)) *
-                                   std::max(1.0, (double)((bs + imgs - 1) / imgs) / (2.0 * (double)cus));
-            if (const int rc = taps_kernel(0.7 * walk_us); rc != 1) return rc;
             const int64_t work = imgs * items;
             const int threads = work >= 256 ? 256 : (int)((work + 63) / 64 * 64);
             const int64_t blocks = (bs + imgs - 1) / imgs;
             if (blocks > 0x7FFFFFFF) return fail(AGH_ERANGE, "%s: too many workgroups", name);
-            const size_t smem = (size_t)(w_bytes + imgs * img_bytes);
+            const size_t smem = (size_t)(l.w_bytes + imgs * l.img_bytes);
             const dim3 grid((unsigned)blocks), block(threads);
             const T *xp = (const T *)x, *wp = (const T *)w, *bp = (const T *)bias;
             T *yp = (T *)y;
@@ -1707,45 +1793,12 @@ int conv2_direct_entry(const char *name, const void *x, const void *w, const voi
     }
 
     ConvParams p;
-    p.bs = bs; p.ic = ic; p.ih = ih; p.iw = iw; p.oc = oc; p.oh = oh; p.ow = ow;
-    p.fh = fh; p.fw = fw; p.ph = ph; p.pw = pw; p.sh = sh; p.sw = sw; p.dh = dh; p.dw = dw;
-    p.act = act; p.has_bias = bias != nullptr;
-    p.yh = pool2x2 ? oh / 2 : oh;
-    p.yw = pool2x2 ? ow / 2 : ow;
-    // output channels per work item: the whole bank when it is small, else groups of 8
-    int oct = 8;
-    for (int c : {1, 2, 4, 6, 8})
-        if (oc <= c) { oct = c; break; }
-    p.ngroups = (oc + oct - 1) / oct;
-    p.ocpad = p.ngroups * oct;
-    const int64_t pix = (int64_t)p.yh * p.yw;
-    const int64_t items = pix * p.ngroups;
-    const int64_t taps = ic * fh * fw;
-    const int64_t img_bytes = ic * ih * iw * 4, w_bytes = taps * p.ocpad * 4;
-    constexpr int64_t kLds = 64 * 1024;
-    if (w_bytes + img_bytes > kLds || items > ((int64_t)1 << 24)) {
-        // otherwise im2col and a product: the patch matrix written and read (faster while the last-level cache holds it), the
-        // product on whole 16-byte rows or through element-wise loaders, 64 channels at least; 30 us for the calls.
-        // Taken against that: 64 x 3 x 95 x 95 to 64, 7 x 7 stride 2, f32 76 -> 44 us; 64 x 24 x 30 x 30 to 48, 3 x 3, f32
-        // 57 -> 23, bf16 35 -> 23 us.  Not taken: 64 x 64 x 56 x 56 to 128, 3 x 3 stride 2, f32 106 (here 149), bf16 39 (157).
-        const bool whole = taps * (int64_t)sizeof(T) % 16 == 0;
-        const double patch = (double)bs * oh * ow * taps * sizeof(T), flops = 2.0 * bs * oh * ow * taps * ((oc + 63) / 64 * 64);
-        const double chain_us = 6.0 + 2.0 * patch / (patch < 128e6 ? 8e6 : 5e6) +
-                                flops / (sizeof(T) == 4 ? (whole ? 100e6 : 50e6) : (whole ? 450e6 : 65e6));
-        if (const int rc = taps_kernel(0.85 * std::max(30.0, chain_us)); rc != 1) return rc;
+    if (!conv2_lds_plan(shape, pool2x2 != 0, p, l))
         return fail(AGH_ERANGE, "%s: image + filter bank (%lld bytes) do not fit in LDS; use im2col + gemm", name,
-                    (long long)(w_bytes + img_bytes));
-    }
-    // images per workgroup: aim at ~256 work items, stay inside LDS, keep >= 2 workgroups per CU
-    int64_t imgs = items >= 256 ? 1 : 256 / items;
-    while (imgs > 1 && w_bytes + imgs * img_bytes > kLds) --imgs;
-    const int64_t cus = compute_units() > 0 ? compute_units() : 256;
-    while (imgs > 1 && (bs + imgs - 1) / imgs < 2 * cus) --imgs;
-    if (imgs > bs) imgs = bs;
-    // (5 x 1 x 108 x 108 to 48, 5 x 5 stride 2: 289 us here, 14 us on the matrix cores)
-    const double walk_us = (double)((imgs * items + 255) / 256) * (1.5 + 0.02 * (double)(taps * oct)) *
-                           std::max(1.0, (double)((bs + imgs - 1) / imgs) / (2.0 * (double)cus));
-    if (const int rc = taps_kernel(0.7 * walk_us); rc != 1) return rc;
+                    (long long)(l.w_bytes + l.img_bytes));
+    const int oct = l.oct;
+    const int64_t items = l.items, imgs = l.imgs, pix = (int64_t)p.yh * p.yw;
+    p.act = act; p.has_bias = bias != nullptr;
     p.imgs = (int)imgs;
     p.items_per_img = (int)items;
     p.div_items = FastDiv((uint32_t)items);
@@ -1755,7 +1808,7 @@ int conv2_direct_entry(const char *name, const void *x, const void *w, const voi
     int threads = work >= 256 ? 256 : (int)((work + 63) / 64 * 64);
     const int64_t blocks = (bs + imgs - 1) / imgs;
     if (blocks > 0x7FFFFFFF) return fail(AGH_ERANGE, "%s: too many workgroups", name);
-    const size_t smem = (size_t)(w_bytes + imgs * img_bytes);
+    const size_t smem = (size_t)(l.w_bytes + imgs * l.img_bytes);
     if (pool2x2)
         launch_oct<T, true>(oct, dim3((unsigned)blocks), dim3(threads), smem, (const T *)x, (const T *)w, (const T *)bias,
                             (T *)y, p);

@@ -380,27 +380,43 @@ namespace agh {
 
 // Returns 1 when the geometry is not one this kernel takes (the caller goes on to its other paths),
 // otherwise a status code.  The API lock is held by the caller.
+struct MfmaPlan {
+    int64_t icc, smem, tiles, octiles, blocks, lds_limit;  // icc: input channels per pass
+};
+
+// whether the kernel takes these shapes
+template <typename T, int kTilePos, int kWgs>
+static bool conv2_mfma_plan(const void *x, const void *w, int64_t bs, int64_t ic, int64_t ih, int64_t iw, int64_t oc, int64_t fh, int64_t fw,
+                            int64_t pw, int64_t oh, int64_t ow, MfmaPlan &m) {
+    constexpr int ES = Geo<T>::ES, CPC = Geo<T>::CPC;
+    const int64_t npos = oh * ow;
+    if (ic < 2 * CPC || ic % (2 * CPC) != 0 || ic > 8192 || oc % 64 != 0 || iw % CPC != 0 || npos % CPC != 0 || fh * fw > 64) return false;
+    if ((((uintptr_t)x | (uintptr_t)w) & 15) != 0) return false;
+    // little work per output: the LDS-resident scalar kernels do better on small problems
+    if (ic * fh * fw < 128 || npos < 256) return false;
+    const int64_t lcols = iw + 2 * pw;
+    const int64_t rows_out = std::min<int64_t>(oh, (kTilePos - 1) / ow + 2);
+    // kWgs workgroups per CU (160 KB of LDS): the largest power-of-two channel count whose rows fit in a share
+    m.lds_limit = 160 * 1024 / kWgs;
+    m.icc = ic & -ic;  // channels per pass: a power of two that divides ic
+    while (m.icc > 2 * CPC && (rows_out + fh - 1) * lcols * (m.icc * ES + 16) > m.lds_limit) m.icc >>= 1;
+    const int64_t tile_bytes = (rows_out + fh - 1) * lcols * (m.icc * ES + 16);  // staged pixels are padded by 16 bytes
+    m.smem = std::max<int64_t>(tile_bytes, 4 * 32 * Geo<T>::EPITCH);
+    if (m.smem > m.lds_limit) return false;
+    m.tiles = (npos + kTilePos - 1) / kTilePos;
+    m.octiles = (oc + kTileOc - 1) / kTileOc;
+    m.blocks = bs * m.tiles * m.octiles;
+    return m.blocks <= 0x7FFFFFFFll && bs * ic * ih * iw <= ((int64_t)1 << 40);
+}
+
 template <typename T, int kTilePos, int kWgs, int kBRing>
 static int conv2_mfma_launch(const char *name, const void *x, const void *w, const void *bias, void *y, int64_t bs, int64_t ic, int64_t ih,
                    int64_t iw, int64_t oc, int64_t fh, int64_t fw, int64_t ph, int64_t pw, int64_t oh, int64_t ow, int act) {
     constexpr int ES = Geo<T>::ES, CPC = Geo<T>::CPC;
-    const int64_t npos = oh * ow;
-    if (ic < 2 * CPC || ic % (2 * CPC) != 0 || ic > 8192 || oc % 64 != 0 || iw % CPC != 0 || npos % CPC != 0 || fh * fw > 64) return 1;
-    if ((((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) != 0) return 1;
-    // little work per output: the LDS-resident scalar kernels do better on small problems
-    if (ic * fh * fw < 128 || npos < 256) return 1;
-    const int64_t lcols = iw + 2 * pw;
-    const int64_t rows_out = std::min<int64_t>(oh, (kTilePos - 1) / ow + 2);
-    // kWgs workgroups per CU (160 KB of LDS): the largest power-of-two channel count whose rows fit in a share
-    const int64_t lds_limit = 160 * 1024 / kWgs;
-    int64_t icc = ic & -ic;  // channels per pass: a power of two that divides ic
-    while (icc > 2 * CPC && (rows_out + fh - 1) * lcols * (icc * ES + 16) > lds_limit) icc >>= 1;
-    const int64_t tile_bytes = (rows_out + fh - 1) * lcols * (icc * ES + 16);  // staged pixels are padded by 16 bytes
-    const int64_t smem = std::max<int64_t>(tile_bytes, 4 * 32 * Geo<T>::EPITCH);
-    if (smem > lds_limit) return 1;
-    const int64_t tiles = (npos + kTilePos - 1) / kTilePos, octiles = (oc + kTileOc - 1) / kTileOc;
-    const int64_t blocks = bs * tiles * octiles;
-    if (blocks > 0x7FFFFFFFll || bs * ic * ih * iw > ((int64_t)1 << 40)) return 1;
+    const int64_t npos = oh * ow, lcols = iw + 2 * pw;
+    MfmaPlan m;
+    if (((uintptr_t)y & 15) != 0 || !conv2_mfma_plan<T, kTilePos, kWgs>(x, w, bs, ic, ih, iw, oc, fh, fw, pw, oh, ow, m)) return 1;
+    const int64_t icc = m.icc, smem = m.smem, tiles = m.tiles, octiles = m.octiles, blocks = m.blocks, lds_limit = m.lds_limit;
 
     void *wperm = nullptr;
     const size_t wtotal = (size_t)(oc * ic * fh * fw);
@@ -443,20 +459,35 @@ static int conv2_mfma_launch(const char *name, const void *x, const void *w, con
     return AGH_OK;
 }
 
+// f32: 128 positions per workgroup and three workgroups per CU; while one stages its rows or writes its outputs
+// (memory latency), two others keep the matrix pipes fed (measured 132 against 124 TFLOP/s at the 256 x 64 x 56 x 56
+// layer).  bf16, whose k loop is eight times shorter per byte staged: 256 positions and two per CU (halo rows are
+// a smaller share; 878 against 796 TFLOP/s).  AGH_CONV_TILE=128|256 overrides.
+template <typename T>
+static int conv2_mfma_tile() {
+    const char *e = getenv("AGH_CONV_TILE");
+    return e && *e ? atoi(e) : (sizeof(T) == 4 ? 128 : 256);
+}
+
 template <typename T>
 int conv2_mfma_try(const char *name, const void *x, const void *w, const void *bias, void *y, int64_t bs, int64_t ic, int64_t ih,
                    int64_t iw, int64_t oc, int64_t fh, int64_t fw, int64_t ph, int64_t pw, int64_t oh, int64_t ow, int act) {
-    // f32: 128 positions per workgroup and three workgroups per CU; while one stages its rows or writes its outputs
-    // (memory latency), two others keep the matrix pipes fed (measured 132 against 124 TFLOP/s at the 256 x 64 x 56 x 56
-    // layer).  bf16, whose k loop is eight times shorter per byte staged: 256 positions and two per CU (halo rows are
-    // a smaller share; 878 against 796 TFLOP/s).  AGH_CONV_TILE=128|256 overrides.
-    const char *e = getenv("AGH_CONV_TILE");
-    const int tile = e && *e ? atoi(e) : (sizeof(T) == 4 ? 128 : 256);
-    if (tile == 128)
+    if (conv2_mfma_tile<T>() == 128)
         return conv2_mfma_launch<T, 128, 3, 8>(name, x, w, bias, y, bs, ic, ih, iw, oc, fh, fw, ph, pw, oh, ow, act);
     return conv2_mfma_launch<T, 256, 2, 8>(name, x, w, bias, y, bs, ic, ih, iw, oc, fh, fw, ph, pw, oh, ow, act);
 }
 
+template <typename T>
+bool conv2_mfma_takes(const void *x, const void *w, int64_t bs, int64_t ic, int64_t ih, int64_t iw, int64_t oc, int64_t fh, int64_t fw,
+                      int64_t pw, int64_t oh, int64_t ow) {
+    MfmaPlan m;
+    return conv2_mfma_tile<T>() == 128 ? conv2_mfma_plan<T, 128, 3>(x, w, bs, ic, ih, iw, oc, fh, fw, pw, oh, ow, m)
+                                       : conv2_mfma_plan<T, 256, 2>(x, w, bs, ic, ih, iw, oc, fh, fw, pw, oh, ow, m);
+}
+template bool conv2_mfma_takes<uint16_t>(const void *, const void *, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t,
+                                         int64_t, int64_t);
+template bool conv2_mfma_takes<float>(const void *, const void *, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t,
+                                      int64_t, int64_t);
 template int conv2_mfma_try<uint16_t>(const char *, const void *, const void *, const void *, void *, int64_t, int64_t, int64_t, int64_t,
                                       int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int);
 template int conv2_mfma_try<float>(const char *, const void *, const void *, const void *, void *, int64_t, int64_t, int64_t, int64_t,

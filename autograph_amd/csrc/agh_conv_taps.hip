@@ -21,14 +21,14 @@ using namespace agh;
 namespace {
 
 struct TapsParams {
-    int ic, ih, iw, oc, ow, ph, pw, sh, sw, dh, dw;
+    int ic, ih, iw, oc, ph, pw, sh, sw, dh, dw;
     int act, has_bias;
-    int npos;         // output positions per image
+    int npos;         // output positions per image; with the pool, the 4 positions of every window
     int ptiles;       // workgroups per image and channel group
     int chunk;        // input channels staged at a time
     int rows, pitch;  // staged rows per channel and their pitch (floats, a multiple of 4)
     int fhfw, ktot;
-    FastDiv div_ptiles, div_pitch4, div_rows, div_ow, div_fw, div_fhfw;
+    FastDiv div_ptiles, div_pitch4, div_rows, div_yw, div_fw, div_fhfw;  // yw: the result's row, of positions or windows
 };
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -38,7 +38,11 @@ template <typename T> struct Four;
 template <> struct Four<float> { typedef float type __attribute__((ext_vector_type(4), aligned(4))); };
 template <> struct Four<uint16_t> { typedef uint16_t type __attribute__((ext_vector_type(4), aligned(2))); };
 
-template <typename T, int TG, int NT>
+// With the pool, positions are numbered window by window, the four of a window in row order: the accumulator layout then
+// leaves each lane whole 2 x 2 windows of one channel, and bias, ReLU and the first-strict-maximum pooling happen in
+// registers.  A position's taps are staged and added in the same order either way, so the result is, bit for bit, the
+// pool of what the call without it returns.
+template <typename T, int TG, int NT, bool POOL>
 __global__ __launch_bounds__(256, 2) void conv2_taps_kernel(const T *__restrict__ x, const T *__restrict__ w,
                                                             const T *__restrict__ bias, T *__restrict__ y, TapsParams p) {
     using V4 = typename Four<T>::type;
@@ -50,8 +54,15 @@ __global__ __launch_bounds__(256, 2) void conv2_taps_kernel(const T *__restrict_
     uint32_t b, tile;
     p.div_ptiles.divmod(blockIdx.x, b, tile);
     const int p0 = (int)tile * (64 * TG), oc0 = (int)blockIdx.y * (16 * NT);
+    auto output_at = [&](uint32_t pos, uint32_t &oy, uint32_t &ox) {
+        if constexpr (POOL) {
+            p.div_yw.divmod(pos >> 2, oy, ox);
+            oy = 2 * oy + ((pos >> 1) & 1);
+            ox = 2 * ox + (pos & 1);
+        } else p.div_yw.divmod(pos, oy, ox);
+    };
     uint32_t oy0, ox0;
-    p.div_ow.divmod((uint32_t)p0, oy0, ox0);
+    output_at((uint32_t)p0, oy0, ox0);
     const int h0 = (int)oy0 * p.sh - p.ph;  // the image row that staged row 0 holds
     const T *xb = x + (size_t)b * p.ic * p.ih * p.iw;
 
@@ -67,7 +78,7 @@ __global__ __launch_bounds__(256, 2) void conv2_taps_kernel(const T *__restrict_
 #pragma unroll
     for (int t = 0; t < TG; ++t) {
         uint32_t oy, ox;
-        p.div_ow.divmod((uint32_t)min(wp0 + t * 16 + i, p.npos - 1), oy, ox);
+        output_at((uint32_t)min(wp0 + t * 16 + i, p.npos - 1), oy, ox);
         abase[t] = (const char *)(xs + (int)(oy - oy0) * p.sh * p.pitch + (int)ox * p.sw);
     }
     uint32_t wrow[NT];  // elements, below 2^28; a channel behind the last repeats it
@@ -210,20 +221,30 @@ __global__ __launch_bounds__(256, 2) void conv2_taps_kernel(const T *__restrict_
         for (int n = 0; n < NT; ++n) wrow[n] += klen;
     }
 
-    // lane (g, i) holds positions 4g .. 4g+3 of channel i of every tile
+    // lane (g, i) holds positions 4g .. 4g+3 of channel i of every tile: with the pool, one window
+    const int nout = POOL ? p.npos >> 2 : p.npos;
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
         const int ch = oc0 + 16 * n + i;
         if (ch >= p.oc) continue;
         const T bv = p.has_bias ? bias[ch] : Elem<T>::zero();
-        T *yc = y + ((size_t)b * p.oc + ch) * p.npos;
+        T *yc = y + ((size_t)b * p.oc + ch) * nout;
 #pragma unroll
         for (int t = 0; t < TG; ++t) {
             const int pos = wp0 + t * 16 + 4 * g;
             V4 o;
 #pragma unroll
             for (int r = 0; r < 4; ++r) o[r] = round_bias_relu<T>(total[t][n][r] + acc[t][n][r], p.has_bias != 0, bv, p.act);
-            if (pos + 3 < p.npos) {
+            if constexpr (POOL) {
+                T m = o[0];
+                float mf = Elem<T>::to_f32(m);
+#pragma unroll
+                for (int r = 1; r < 4; ++r) {
+                    const float f = Elem<T>::to_f32(o[r]);
+                    if (f > mf) { m = o[r]; mf = f; }
+                }
+                if (pos < p.npos) yc[pos >> 2] = m;
+            } else if (pos + 3 < p.npos) {
                 *(V4 *)(yc + pos) = o;
             } else {
 #pragma unroll
@@ -234,7 +255,8 @@ __global__ __launch_bounds__(256, 2) void conv2_taps_kernel(const T *__restrict_
     }
 }
 
-constexpr int64_t kTapsLds = 48 * 1024;  // three workgroups per CU
+constexpr int64_t kTapsLds = 48 * 1024;      // three workgroups per CU
+constexpr int64_t kTapsPoolLds = 80 * 1024;  // two: whole windows meet up to twice the rows of as many positions in a line
 
 // rows and channels that a workgroup of 64 * tg positions stages; false where not even one channel fits
 bool taps_stage(int tg, int64_t ic, int64_t oh, int64_t ow, int64_t fh, int64_t fw, int64_t sh, int64_t dh, int64_t pitch, int64_t &rows,
@@ -253,14 +275,21 @@ bool taps_stage(int tg, int64_t ic, int64_t oh, int64_t ow, int64_t fh, int64_t 
 
 namespace agh {
 
+template <typename T, int TG, int NT, bool POOL>
+static int taps_launch(const char *name, const void *x, const void *w, const void *bias, void *y, dim3 grid, size_t smem, const TapsParams &q) {
+    if (smem > 64 * 1024)
+        AGH_HIP(hipFuncSetAttribute((const void *)(conv2_taps_kernel<T, TG, NT, POOL>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+    hipLaunchKernelGGL((conv2_taps_kernel<T, TG, NT, POOL>), grid, dim3(256), smem, stream(), (const T *)x, (const T *)w, (const T *)bias, (T *)y, q);
+    AGH_LAUNCH_CHECK(name);
+    return AGH_OK;
+}
+
 template <typename T>
 int conv2_taps_try(const char *name, const void *x, const void *w, const void *bias, void *y, int64_t bs, int64_t ic, int64_t ih,
                    int64_t iw, int64_t oc, int64_t fh, int64_t fw, int64_t ph, int64_t pw, int64_t sh, int64_t sw, int64_t dh,
-                   int64_t dw, int64_t oh, int64_t ow, int act, double limit_us) {
-    const char *env = getenv("AGH_CONV_TAPS");  // 0 / 1 forces the choice (measurements)
-    const bool forced = env && *env && atoi(env) != 0, want = forced || !(env && *env);
+                   int64_t dw, int64_t oh, int64_t ow, int act, bool pool, bool forced, double limit_us) {
     const int64_t npos = oh * ow, ktot = ic * fh * fw, pitch = ((ow - 1) * sw + (fw - 1) * dw + 4) & ~(int64_t)3;
-    if (!want || npos > ((int64_t)1 << 24) || ktot > ((int64_t)1 << 24) || oc * ktot > ((int64_t)1 << 28)) return 1;
+    if (npos > ((int64_t)1 << 24) || ktot > ((int64_t)1 << 24) || oc * ktot > ((int64_t)1 << 28)) return 1;
     // tile: rounds of workgroups times the matrix cycles of one (16 positions x 16 channels x 4 taps = 32 cycles, each wave
     // on a SIMD of its own; a lone wave waits about 500 cycles for the operands of 16 taps), and its staging (batches of 8
     // groups of four cells a thread, a memory round trip each), which later rounds hide in part
@@ -279,39 +308,46 @@ int conv2_taps_try(const char *name, const void *x, const void *w, const void *b
             const double cost = (double)rounds * mfma + stage * (0.6 + 0.4 * (double)rounds);
             if (!tg || cost < best) {
                 best = cost; tg = t; nt = n; rows = r; chunk = c;
-                us = 5.0 + 1.4 * (double)rounds * (mfma + stage) / 2100.0;  // on the safe side of what 100 shapes measured
+                us = 5.0 + 1.4 * (double)rounds * (mfma + stage) / 2100.0;  // on the safe side of what was measured
             }
         }
     }
     if (!tg || (!forced && us > limit_us)) return 1;
+    // the pool is fused where the convolution alone would run here, and stages as many channels at a time (the order of the
+    // sums); only the tile's positions are fewer where its rows, less than three times as many, take too much of the LDS
+    const int64_t ntab = (chunk * fh * fw + 15) & ~(int64_t)15, yh = pool ? oh / 2 : oh, yw = pool ? ow / 2 : ow;
+    const int64_t nall = pool ? yh * yw * 4 : npos;
+    auto lds_bytes = [&]() { return (ntab + chunk * rows * pitch) * 4; };
+    if (pool) {
+        auto pool_rows = [&]() { rows = (2 * std::min(yh - 1, (16 * tg - 1 + yw - 1) / yw) + 1) * sh + (fh - 1) * dh + 1; };
+        for (pool_rows(); tg > 1 && lds_bytes() > kTapsPoolLds; pool_rows()) tg /= 2;
+        if (lds_bytes() > 160 * 1024) return 1;
+    }
     TapsParams q;
-    q.ic = (int)ic; q.ih = (int)ih; q.iw = (int)iw; q.oc = (int)oc; q.ow = (int)ow; q.ph = (int)ph; q.pw = (int)pw;
+    q.ic = (int)ic; q.ih = (int)ih; q.iw = (int)iw; q.oc = (int)oc; q.ph = (int)ph; q.pw = (int)pw;
     q.sh = (int)sh; q.sw = (int)sw; q.dh = (int)dh; q.dw = (int)dw; q.act = act; q.has_bias = bias != nullptr;
-    q.npos = (int)npos;
-    q.ptiles = (int)((npos + 64 * tg - 1) / (64 * tg));
+    q.npos = (int)nall;
+    q.ptiles = (int)((nall + 64 * tg - 1) / (64 * tg));
     q.chunk = (int)chunk; q.rows = (int)rows; q.pitch = (int)pitch; q.fhfw = (int)(fh * fw); q.ktot = (int)ktot;
     q.div_ptiles = FastDiv((uint32_t)q.ptiles); q.div_pitch4 = FastDiv((uint32_t)(pitch / 4)); q.div_rows = FastDiv((uint32_t)rows);
-    q.div_ow = FastDiv((uint32_t)ow); q.div_fw = FastDiv((uint32_t)fw); q.div_fhfw = FastDiv((uint32_t)q.fhfw);
+    q.div_yw = FastDiv((uint32_t)yw); q.div_fw = FastDiv((uint32_t)fw); q.div_fhfw = FastDiv((uint32_t)q.fhfw);
     const int64_t gx = bs * q.ptiles, gy = (n16 + nt - 1) / nt;
     if (gx > 0x7FFFFFFF || gy > 65535) return 1;
-    const size_t smem = (size_t)(((chunk * fh * fw + 15) & ~(int64_t)15) + chunk * rows * pitch) * 4;
-    const dim3 grid((unsigned)gx, (unsigned)gy), block(256);
+    const dim3 grid((unsigned)gx, (unsigned)gy);
 #define AGH_TAPS(TGV, NTV) \
     case TGV * 8 + NTV: \
-        hipLaunchKernelGGL((conv2_taps_kernel<T, TGV, NTV>), grid, block, smem, stream(), (const T *)x, (const T *)w, (const T *)bias, \
-                           (T *)y, q); \
-        break
+        return pool ? taps_launch<T, TGV, NTV, true>(name, x, w, bias, y, grid, (size_t)lds_bytes(), q) \
+                    : taps_launch<T, TGV, NTV, false>(name, x, w, bias, y, grid, (size_t)lds_bytes(), q)
 #define AGH_TAPS4(TGV) AGH_TAPS(TGV, 1); AGH_TAPS(TGV, 2); AGH_TAPS(TGV, 3); AGH_TAPS(TGV, 4)
     switch (tg * 8 + nt) { AGH_TAPS4(4); AGH_TAPS4(2); AGH_TAPS4(1); }
 #undef AGH_TAPS4
 #undef AGH_TAPS
-    AGH_LAUNCH_CHECK(name);
-    return AGH_OK;
+    return 1;
 }
 
 template int conv2_taps_try<float>(const char *, const void *, const void *, const void *, void *, int64_t, int64_t, int64_t, int64_t,
-                                   int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int, double);
+                                   int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int, bool, bool, double);
 template int conv2_taps_try<uint16_t>(const char *, const void *, const void *, const void *, void *, int64_t, int64_t, int64_t, int64_t,
-                                      int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int, double);
+                                      int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int, bool, bool, double);
 
 }  // namespace agh

@@ -27,12 +27,17 @@ int static_workspace(size_t bytes, void **ptr);
 template <typename T>
 int conv2_mfma_try(const char *name, const void *x, const void *w, const void *bias, void *y, int64_t bs, int64_t ic, int64_t ih,
                    int64_t iw, int64_t oc, int64_t fh, int64_t fw, int64_t ph, int64_t pw, int64_t oh, int64_t ow, int act);
-// Conv2 forward for any stride, dilation and channel count on the f32 matrix cores (agh_conv_taps.hip); 1 = not taken:
-// the shape is not its own, or it expects to need more than limit_us
+// whether it takes these shapes (any 16-byte aligned output)
+template <typename T>
+bool conv2_mfma_takes(const void *x, const void *w, int64_t bs, int64_t ic, int64_t ih, int64_t iw, int64_t oc, int64_t fh, int64_t fw,
+                      int64_t pw, int64_t oh, int64_t ow);
+// Conv2 forward for any stride, dilation and channel count on the f32 matrix cores (agh_conv_taps.hip), followed by the
+// 2x2 pool where `pool`; 1 = not taken: the shape is not its own, or the convolution is expected to need more than
+// limit_us there (and is not forced)
 template <typename T>
 int conv2_taps_try(const char *name, const void *x, const void *w, const void *bias, void *y, int64_t bs, int64_t ic, int64_t ih,
                    int64_t iw, int64_t oc, int64_t fh, int64_t fw, int64_t ph, int64_t pw, int64_t sh, int64_t sw, int64_t dh,
-                   int64_t dw, int64_t oh, int64_t ow, int act, double limit_us);
+                   int64_t dw, int64_t oh, int64_t ow, int act, bool pool, bool forced, double limit_us);
 
 #define AGH_API_ENTER()                                           \
     std::lock_guard<std::recursive_mutex> _agh_lock(agh::api_mutex()); \

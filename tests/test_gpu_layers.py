@@ -165,6 +165,33 @@ def test_conv2_direct_fused_relu_pool(ag, dtype):
         assert np.array_equal(fused, orc.max_pool2(orc.relu(conv), (2, 2)))
 
 
+CONV_TAPS_POOL = [
+    # bs, ic, ih, iw, oc, filter, padding, stride: the convolution alone runs out of staged rows
+    (64, 3, 64, 64, 64, (3, 3), (1, 1), (1, 1)),
+    (64, 24, 30, 30, 48, (3, 3), (1, 1), (1, 1)),      # too large for LDS: im2col and a product in its place
+    (16, 3, 95, 95, 64, (7, 7), (3, 3), (2, 2)),       # 48 x 48 windows' cells, 24 x 24 windows
+    (1, 3, 32, 109, 64, (5, 5), (0, 0), (1, 1)),       # odd width: the last column belongs to no window
+    (5, 1, 108, 108, 48, (5, 5), (2, 2), (2, 2)),
+    (4, 40, 61, 33, 50, (3, 5), (1, 2), (1, 1)),       # several stages of channels, odd height
+]
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("case", CONV_TAPS_POOL)
+def test_conv2_fused_pool_out_of_staged_rows_equals_the_layers(ag, dtype, case):
+    """Conv2 with the pool fused, chosen by size as a program has it, returns the bits of Conv2, Relu and MaxPool2."""
+    bs, ic, ih, iw, oc, f, p, s = case
+    rng = np.random.default_rng(33)
+    x = ag.Tensor.from_array(to_dtype(rng.standard_normal((bs, ic, ih, iw)), dtype))
+    w = ag.Tensor.from_array(to_dtype(rng.standard_normal((oc, ic) + f) * np.sqrt(2.0 / (ic * f[0] * f[1])), dtype))
+    b = ag.Tensor.from_array(to_dtype(rng.standard_normal(oc) * 0.1, dtype))
+    for bias, relu in ((None, False), (b, True)):
+        conv = ag.Conv2(w, bias, p, s)
+        want = ag.MaxPool2((2, 2)).forward(conv.forward(x, relu=relu)).into_array()
+        got = conv.forward(x, relu=relu, pool2x2=True).into_array()
+        assert np.array_equal(got, want), (relu, np.mean(got != want))
+
+
 CONV_MFMA = [
     # bs, ic, ih, iw, oc, filter, padding: shapes the implicit-GEMM (matrix core) convolution takes
     (2, 64, 56, 56, 128, (3, 3), (1, 1)),    # config-3 layer, small batch
