@@ -219,6 +219,21 @@ inline int pick_loader_any(int64_t rs, int64_t ks, int K) {
     return LD_S;
 }
 
+// Products that the any-address kernel's two tiles serve worse than the element-wise loaders' 32 x 128 and 128 x 32: one or two
+// k-tiles, so that a workgroup is all filling and storing, few rows or columns, so that half as many workgroups cover C, and
+// more of them than CUs.  Few columns (P, C's unit-stride axis) are the worse for it: C's rows are stored element by element.
+// Element-wise / 64 x 64 in us over the forms of 270 such products: 30 of 29767x11x4 31.7 / 100, 1x115707x13x2 7.3 / 13.5,
+// 44 of 81771x8x2 115 / 239; 51 of 12x9x164388 405 / 574; two k-tiles: 4 of 89307x81x1 26 / 40, but 6 of 111328x121x10 63 / 55.
+// On the other side of the line: 26 of 34426x103x15 101 / 92, 1x13x117x40505 9.9 / 7.7, up to 256 tiles 1.2 times the time.
+inline bool short_and_narrow(const Args &g, int64_t batch, int64_t cus, int lp) {
+    if (g.K > 128 || (g.NP > 32 && g.NQ > 16)) return false;
+    const int64_t tiles = (int64_t)((g.NP + 63) / 64) * ((g.NQ + 63) / 64) * batch;
+    const bool one = g.K <= 64, many = tiles > 4 * cus;
+    if (tiles <= cus) return false;
+    if (g.NP <= 16 ? one || many : g.NP <= 32 && one && many) return true;
+    return g.NQ <= 16 && one && many && (lp == LD_K || tiles > 20 * cus);
+}
+
 // Optional override for experiments: AGH_GEMM_CFG=<config id>, AGH_GEMM_SPLITS=<n>.
 inline int env_int(const char *name, int dflt) {
     const char *s = getenv(name);
@@ -291,7 +306,9 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
         lp_any = pick_loader_any(g.ps, g.pk, g.K);
         lq_any = pick_loader_any(g.qs, g.qk, g.K);
     }
-    const bool any_addr = lp_any != LD_S && lq_any != LD_S;
+    const int cus = compute_units() > 0 ? compute_units() : 256;
+    const int forced_cfg = env_int("AGH_GEMM_CFG", -1);
+    const bool any_addr = lp_any != LD_S && lq_any != LD_S && (forced_cfg >= 0 || !short_and_narrow(g, batch, cus, lp_any));
     const bool any_scalar = (lp == LD_S || lq == LD_S);
     const bool vec_store = g.dp == 1 && g.NP % 4 == 0 && (g.dq % 4 == 0 || g.NQ == 1) && aligned(C, 4 * sizeof(T)) &&
                            (batch == 1 || g.batch_d % 4 == 0);
@@ -304,14 +321,14 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
 #endif
 
     // ---- tile shape: minimise (rounds of workgroups) x (tile area) / efficiency ----
-    const int cus = compute_units() > 0 ? compute_units() : 256;
     // (any k: a last k-tile shorter than 64 is loaded with zeros behind k = K)
     const bool direct_ok = sizeof(T) == 2 && (!any_scalar || any_addr) && g.K > 0 && env_int("AGH_GEMM_DIRECT", 1) != 0;
     int best = -1;
     double best_cost = 0;
     for (int i = 0; i < kNumCfgs; ++i) {
         const TileCfg &t = kCfgs[i];
-        if (any_addr ? i != 3 && i != 4 : any_scalar && !t.scalar_ok) continue;
+        // (any address: of a 128 x 128 tile over at most 64 rows or columns, half would be padding)
+        if (any_addr ? i != 4 && (i != 3 || g.NP <= 64 || g.NQ <= 64) : any_scalar && !t.scalar_ok) continue;
         const int64_t tiles = (int64_t)((g.NP + t.bp - 1) / t.bp) * ((g.NQ + t.bq - 1) / t.bq) * batch;
         if (tiles > 0x7FFFFFFF) continue;
         // a CU works through ceil(tiles / CUs) tiles; co-resident workgroups share its MFMA rate
@@ -373,14 +390,15 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
         }
         // Operands at any element address: bound by the L1s, whatever the clock.  Microseconds a k-tile, a workgroup alone on
         // its CU / per workgroup where several share it: 128 x 128 0.95 / 0.75 (1999x2047x1001; 4099x4101x4103), 64 x 64
-        // 0.52 / 0.38 (1024x1023x1024; 1999x2047x1001, 2999x3001x3003); filling and storing cost three and five k-tiles.
-        if (any_addr) {
-            const double alone = t.bp == 64 ? 0.52 : 0.95, shared = t.bp == 64 ? 0.38 : 0.75;
-            cost = (rounds == 1 ? alone : rounds * shared) * (kt + (t.bp == 64 ? 5.0 : 3.0));
-        }
+        // 0.52 / 0.38 (1024x1023x1024; 1999x2047x1001, 2999x3001x3003).  Filling and storing cost a workgroup alone three and
+        // five k-tiles; of several, one multiplies while another fills, and it is two (1532x25x1126 on 128 x 128 / 64 x 64
+        // tiles 7.4 / 5.8 us, 25 of 239x19x204 7.3 / 5.9; over 223 such products the choice is within 0.5 % of the better
+        // tile, with three and five it was 6 %).
+        if (any_addr)
+            cost = rounds == 1 ? (t.bp == 64 ? 0.52 * (kt + 5.0) : 0.95 * (kt + 3.0)) : (double)rounds * (t.bp == 64 ? 0.38 : 0.75) * (kt + 2.0);
         if (best < 0 || cost < best_cost) { best = i; best_cost = cost; }
     }
-    best = env_int("AGH_GEMM_CFG", best);
+    if (forced_cfg >= 0) best = forced_cfg;
     const bool any = any_addr && (best == 3 || best == 4);  // (a forced skinny tile keeps the element-wise loaders)
     if (any) { lp = lp_any; lq = lq_any; }
     if (best < 0 || best >= kNumCfgs || (any_scalar && !any && !kCfgs[best].scalar_ok))

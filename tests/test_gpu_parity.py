@@ -6,6 +6,7 @@ Bars: im2col / col2im / pooling / relu bit-exact; f32 gemm within 1e-5*sqrt(K) r
 bf16 gemm within 1 bf16 ulp + 1e-2 relative of an f32-accumulated reference.
 """
 import ctypes as C  # noqa: F401
+import time
 
 import numpy as np
 import pytest
@@ -895,6 +896,47 @@ def test_gemm_bf16_operands_at_any_address(ag, monkeypatch, k):
             if min(m, n) >= 8:
                 assert len(seen) == 3 and all(np.array_equal(seen[0], x) for x in seen[1:]), (m, n, ta, tb)
     monkeypatch.delenv("AGH_GEMM_CFG", raising=False)
+
+
+def test_gemm_bf16_form_of_short_and_narrow_ragged_products(ag, monkeypatch):
+    """Ragged products of one or two k-tiles: the form and tile chosen by size is the faster one, to within a half (few columns:
+    element-wise loaders, 3 times as fast; a grid of 64 x 64 tiles where one of 128 x 128 is mostly filling and storing), and
+    the forms agree bit for bit on both sides of the rule's lines."""
+    rng = np.random.default_rng(34)
+    for batch, m, k, n, ta, tb in ((30, 29767, 11, 4, False, True), (1, 148274, 11, 1, True, False), (1, 1532, 25, 1126, True, True),
+                                   (26, 34426, 103, 15, True, True)):
+        a, b, c = (ag.Tensor.zeros((s,), "bf16") for s in (batch * m * k, batch * k * n, batch * m * n))
+        f = ag.lib.agh_gemm_bf16_batched
+        args = (batch, m, k, n, 1.0, a._data_ptr(), 0, *((1, m) if ta else (k, 1)), m * k, b._data_ptr(), 0, *((1, k) if tb else (n, 1)), k * n,
+                0.0, c._data_ptr(), 0, n, 1, m * n, None, 0, 0, 0)
+        us = {}
+        for form, env in (("chosen", {}), ("element-wise", {"AGH_GEMM_DIRECT": "0"}), ("64 x 64", {"AGH_GEMM_CFG": "4"})):
+            with monkeypatch.context() as mp:
+                for var, value in env.items():
+                    mp.setenv(var, value)
+                best = float("inf")
+                for _ in range(6):
+                    ag.lib.agh_sync()
+                    t0 = time.perf_counter()
+                    for _ in range(50):
+                        assert f(*args) == 0
+                    ag.lib.agh_sync()
+                    best = min(best, time.perf_counter() - t0)
+                us[form] = best * 2e4
+        assert us["chosen"] <= 1.5 * min(us.values()), (batch, m, k, n, us)
+    # tiles of 64 x 64 around one and four per CU, 16 | 17 and 32 | 33 columns or rows, one | two | three k-tiles
+    cus = ag.Device(0).info()["compute_units"]
+    for long in (64 * cus, 64 * cus + 1, 256 * cus + 1):
+        for narrow, k in ((1, 63), (7, 9), (16, 64), (17, 64), (33, 33), (15, 65), (16, 127), (8, 129)):
+            for m, n in ((long, narrow), (narrow, long)):
+                for ta, tb in ((False, False), (True, True)):
+                    ash, bsh = (k, m) if ta else (m, k), (n, k) if tb else (k, n)
+                    # whole numbers: every form's sums are exact, so one comparison serves all
+                    av, bv = rng.integers(-3, 4, ash).astype(np.float32), rng.integers(-3, 4, bsh).astype(np.float32)
+                    A, B = (ag.Tensor.from_array(to_dtype(v, "bf16")) for v in (av, bv))
+                    got = (A.t() if ta else A).dot(B.t() if tb else B).into_array()
+                    want = (av.T if ta else av) @ (bv.T if tb else bv)
+                    assert np.array_equal(got, to_dtype(want, "bf16")), (m, k, n, ta, tb)
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "f32"])
