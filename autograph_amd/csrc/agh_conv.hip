@@ -1655,15 +1655,19 @@ double conv2_taps_limit(const ConvShape &c) {
     if (conv2_rowtile_plan(c, false, rq, l)) return 0.7 * l.walk_us;
     // 5 x 1 x 108 x 108 to 48, 5 x 5 stride 2: 289 and 14 us
     if (conv2_lds_plan(c, false, p, l)) return 0.7 * l.walk_us;
-    // otherwise im2col and a product: the patch matrix written and read (faster while the last-level cache holds it), the
-    // product on whole 16-byte rows or through element-wise loaders, 64 channels at least; 30 us for the calls.
-    // Taken against that: 64 x 3 x 95 x 95 to 64, 7 x 7 stride 2, f32 76 -> 44 us; 64 x 24 x 30 x 30 to 48, 3 x 3, f32
-    // 57 -> 23, bf16 35 -> 23 us.  Not taken: 64 x 64 x 56 x 56 to 128, 3 x 3 stride 2, f32 106 (here 149), bf16 39 (157).
+    // otherwise im2col and a product: the patch matrix written and read (faster while the last-level cache holds it; bf16 rows
+    // of no whole 16 bytes go through the any-address kernel), 64 channels at least; 30 us for the calls, as a Python program
+    // makes them (a captured graph or a C++ program waits for the device alone, where one in five of the shapes taken is slower, the
+    // worst 2.2 times).  Fitted to 2600 shapes; of 1000 others three run more than 3 % behind the route not taken (the worst
+    // 22 %), all of them together 1.76 times as fast as without this kernel.
+    // Taken: 64 x 3 x 95 x 95 to 64, 7 x 7 stride 2, f32 76 -> 42 us; 64 x 24 x 30 x 30 to 48, 3 x 3, f32 57 -> 23, bf16 35 -> 25.
+    // Not taken: 64 x 64 x 56 x 56 to 128, 3 x 3 stride 2, f32 106 (here 149), bf16 39 (157); 205 x 3 x 50 x 50 to 128, 7 x 7,
+    // bf16 153 (here 265).
     const int64_t taps = c.ic * c.fh * c.fw;
-    const bool whole = taps * (int64_t)sizeof(T) % 16 == 0;
+    const bool whole = taps * (int64_t)sizeof(T) % 16 == 0, ragged_bf16 = sizeof(T) == 2 && !whole;
     const double patch = (double)c.bs * c.oh * c.ow * taps * sizeof(T), flops = 2.0 * c.bs * c.oh * c.ow * taps * ((c.oc + 63) / 64 * 64);
-    const double chain_us = 6.0 + 2.0 * patch / (patch < 128e6 ? 8e6 : 5e6) +
-                            flops / (sizeof(T) == 4 ? (whole ? 100e6 : 50e6) : (whole ? 450e6 : 65e6));
+    const double chain_us = 6.0 + 2.0 * patch / (ragged_bf16 ? 3e6 : patch < 128e6 ? 8e6 : 5e6) +
+                            flops / (sizeof(T) == 4 ? (whole ? 100e6 : 50e6) : (whole ? 450e6 : 200e6));
     return 0.85 * std::max(30.0, chain_us);
 }
 

@@ -256,7 +256,7 @@ int agh_conv2_backward_input_bf16(const void *dy, const void *w, void *dx, int64
  * bank fit in LDS, and, on the matrix cores as an implicit GEMM, for unit stride and dilation with
  * input channels a multiple of 16 (bf16) or 8 (f32), output channels a multiple of 64 and rows of
  * whole 16-byte vectors (not with the pool), or for any geometry where that is expected to be faster than im2col +
- * gemm (returns AGH_ERANGE otherwise: use those).  Same result as the
+ * gemm as two calls of 30 us in all, or longer (returns AGH_ERANGE otherwise: use those).  Same result as the
  * conv2_im2col chain (src/learn/neural_network/layer.rs:950-1005) up to f32 summation order;
  * the reference's host has the analogous conv_direct path (layer/conv_direct.rs:23-83).
  * x: [bs,ic,ih,iw], w: [oc,ic,fh,fw], bias: null or [oc], added PER OUTPUT CHANNEL (bias[o] to every

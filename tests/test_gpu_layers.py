@@ -5,6 +5,7 @@ Mirrors conv2_im2col_<T>_<opts> (tests/integration_tests.rs:986-993, body :1182-
 checks the chain against the naive 7-deep loop on x, w = (1..=10).cycle() data.
 """
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -190,6 +191,28 @@ def test_conv2_fused_pool_out_of_staged_rows_equals_the_layers(ag, dtype, case):
         want = ag.MaxPool2((2, 2)).forward(conv.forward(x, relu=relu)).into_array()
         got = conv.forward(x, relu=relu, pool2x2=True).into_array()
         assert np.array_equal(got, want), (relu, np.mean(got != want))
+
+
+def test_conv2_route_is_the_faster_one(ag, monkeypatch):
+    """Conv2 out of staged rows or by im2col and a product, as chosen by size: within a quarter of the faster."""
+    for bs, ic, h, oc, f, p, s, dtype in ((205, 3, 50, 128, 7, 3, 1, "bf16"), (4, 128, 81, 16, 7, 0, 1, "bf16"), (64, 3, 95, 64, 7, 3, 2, "f32"),
+                                          (64, 24, 30, 48, 3, 1, 1, "f32"), (64, 64, 56, 128, 3, 1, 2, "bf16")):
+        rng = np.random.default_rng(35)
+        x = ag.Tensor.from_array(to_dtype(rng.standard_normal((bs, ic, h, h)), dtype))
+        conv = ag.Conv2(ag.Tensor.from_array(to_dtype(rng.standard_normal((oc, ic, f, f)), dtype)), None, (p, p), (s, s))
+        us = {}
+        for taps in ("", "0", "1"):
+            monkeypatch.setenv("AGH_CONV_TAPS", taps)
+            best = float("inf")
+            for _ in range(6):
+                ag.lib.agh_sync()
+                t0 = time.perf_counter()
+                for _ in range(30):
+                    conv.forward(x)
+                ag.lib.agh_sync()
+                best = min(best, time.perf_counter() - t0)
+            us[taps] = best / 30 * 1e6
+        assert us[""] <= 1.25 * min(us["0"], us["1"]), (bs, ic, h, oc, f, us)
 
 
 CONV_MFMA = [
