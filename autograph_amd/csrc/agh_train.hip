@@ -364,9 +364,14 @@ __global__ __launch_bounds__(64 * (1 + kSumLoaders)) void sum_axis0_kernel(const
 // 8.1 / 11.7; 512 x 40000 (three) 24.9 / 20.4, 25.7 / 18.2; 768 x 65536 (four) 38.1 / 43.4, 33.7 / 38.2; 1024 x 65536 51.7 / 48.4,
 // 45.1 / 40.0; from eight rounds on one thread per column reaches the memory's rate too: 256 x 262144 38.6 / 86.6,
 // 20.1 / 87.9; 2048 x 131072 181.9 / 192.4, 164.9 / 180.3; 4096 x 131072 365 / 358, 330 / 331.
-__host__ inline bool sum_axis0_staged(int64_t rows, int64_t cols, int64_t cus) {
+// Rows that do not start on 64 bytes cost the staged form more (its waves read 128 or 256 bytes of a row): 600 x 49011 f32
+// 29.3 / 37.2, bf16 28.8 / 33.6; 1050 x 65395 f32 64.2 / 71.5.  Of 616 sizes of one to seven rounds the rule misses the faster form by
+// more than a tenth at 9, by 18 % at most.
+__host__ inline bool sum_axis0_staged(int64_t rows, int64_t cols, int64_t cus, int64_t bytes) {
     const int64_t per_round = cus * kSumCols, rounds = cols / per_round + (cols % per_round != 0);
-    return rounds < 8 && rows > (rounds < 4 ? 140 + 100 * rounds : 220 * rounds);
+    const bool lines = cols % 64 * bytes % 64 == 0;
+    if (rounds < 3 || (rounds == 3 && lines)) return rows > 140 + 100 * rounds;
+    return rounds < 8 && rows > (!lines ? 280 * rounds : bytes == 4 ? 175 * rounds : rounds == 7 ? 1320 : 220 * rounds);
 }
 
 template <typename T>
@@ -579,7 +584,7 @@ int sum_axis0_launch(const char *name, const void *x, void *y, int64_t rows, int
     if (cols == 0) return AGH_OK;
     if (!y || (!x && rows > 0)) return fail(AGH_ENULL, "%s: null buffer", name);
     const char *env = getenv("AGH_SUM_STAGED");  // 0 / 1 forces the choice (measurements, tests)
-    const bool brief = env && *env ? atoi(env) == 0 : !sum_axis0_staged(rows, cols, compute_units() > 0 ? compute_units() : 256);
+    const bool brief = env && *env ? atoi(env) == 0 : !sum_axis0_staged(rows, cols, compute_units() > 0 ? compute_units() : 256, (int64_t)sizeof(T));
     const int64_t per_block = brief ? kThreads : kSumCols, blocks = (cols + per_block - 1) / per_block;
     if (blocks > 0x7FFFFFFFll) return fail(AGH_ERANGE, "%s: too many columns", name);
     if (brief) {

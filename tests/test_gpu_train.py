@@ -119,8 +119,9 @@ def test_sum_axis0_chunk_and_column_edges(ag, dtype, rows, monkeypatch):
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 def test_sum_axis0_form_chosen_by_rows_and_columns(ag, dtype, monkeypatch):
     """The form chosen by size is the faster one, to within a half: few rows of many columns (one thread per column 3 to 5
-    times as fast), many rows of few columns (the staged form 2 to 8 times as fast)."""
-    for rows, cols in ((129, 262144), (200, 65536), (1024, 64), (4096, 1000)):
+    times as fast), many rows of few columns (the staged form 2 to 8 times as fast); to within a fifth where rows that start
+    anywhere tell (one thread per column a quarter faster)."""
+    for rows, cols, bound in ((129, 262144, 1.5), (200, 65536, 1.5), (1024, 64, 1.5), (4096, 1000, 1.5), (900, 65395, 1.2), (1250, 81779, 1.2)):
         x = ag.Tensor.zeros((rows, cols), dtype)
         y = ag.Tensor.uninit((cols,), dtype)
         f = getattr(ag.lib, f"agh_sum_axis0_{dtype}")
@@ -136,7 +137,7 @@ def test_sum_axis0_form_chosen_by_rows_and_columns(ag, dtype, monkeypatch):
                 ag.lib.agh_sync()
                 best = min(best, time.perf_counter() - t0)
             us[staged] = best * 1e4
-        assert us[""] <= 1.5 * min(us["0"], us["1"]), (rows, cols, us)
+        assert us[""] <= bound * min(us["0"], us["1"]), (rows, cols, us)
 
 
 def _view_of(ag, t, a, base):
