@@ -292,7 +292,10 @@ int conv2_taps_try(const char *name, const void *x, const void *w, const void *b
     if (npos > ((int64_t)1 << 24) || ktot > ((int64_t)1 << 24) || oc * ktot > ((int64_t)1 << 28)) return 1;
     // tile: rounds of workgroups times the matrix cycles of one (16 positions x 16 channels x 4 taps = 32 cycles, each wave
     // on a SIMD of its own; a lone wave waits about 500 cycles for the operands of 16 taps), and its staging (batches of 8
-    // groups of four cells a thread, a memory round trip each), which later rounds hide in part
+    // groups of four cells a thread, a memory round trip each), which later rounds hide in part.  AGH_CONV_TAPS_TILE = 10 TG + NT
+    // forces a tile (tests).
+    const char *env = getenv("AGH_CONV_TAPS_TILE");
+    const int tile = env && *env ? atoi(env) : 0;
     const int64_t cus = compute_units() > 0 ? compute_units() : 256, n16 = (oc + 15) / 16;
     int tg = 0, nt = 0;
     int64_t rows = 0, chunk = 0;
@@ -301,7 +304,8 @@ int conv2_taps_try(const char *name, const void *x, const void *w, const void *b
         int64_t r, c;
         if (!taps_stage(t, ic, oh, ow, fh, fw, sh, dh, pitch, r, c)) continue;
         const int64_t stages = (ic + c - 1) / c, batches = (c * r * (pitch / 4) + 8 * 256 - 1) / (8 * 256);
-        for (int n = 1; n <= 4 && n <= n16; ++n) {
+        for (int n = 1; n <= 4 && (n <= n16 || tile); ++n) {
+            if (tile && tile != 10 * t + n) continue;
             const int64_t blocks = bs * ((npos + 64 * t - 1) / (64 * t)) * ((n16 + n - 1) / n), rounds = (blocks + cus - 1) / cus;
             const double mfma = (double)(ktot + 15) / 16.0 * std::max(t * n * 128.0, rounds == 1 ? 500.0 : 0.0);
             const double stage = (double)stages * (1500.0 * (double)batches + 1500.0) + 2500.0;
