@@ -804,8 +804,9 @@ def test_gemm_bf16_seeded_shapes_in_every_tile_configuration(ag, monkeypatch):
     are vector-loadable), m and n mostly multiples of 8, all four layouts, beta 0 or 1, each in the chooser's tile
     configuration and forced into the 256 x 256, 128 x 256, 256 x 128, 128 x 128 and 64 x 64 ones (two, three, three, two or
     four and four LDS stages; a forced large configuration that has no kernel for the operands' loaders is refused, not
-    miscomputed; the 64 x 64 one then takes the register-staged kernel).  The forced configurations must agree bit for
-    bit wherever they take the direct-to-LDS kernel: one f32 sum per output in k order, rounded once."""
+    miscomputed; the 128 x 128 and 64 x 64 ones then take the form for operands at any address, or the 64 x 64 one the
+    register-staged kernel).  The forced configurations must agree bit for bit wherever they take the direct-to-LDS kernel
+    or that form of it: one f32 sum per output in k order, rounded once."""
     rng = np.random.default_rng(321)
     ran = {None: 0, "0": 0, "1": 0, "2": 0, "3": 0, "4": 0}
     for _ in range(120):
@@ -896,6 +897,50 @@ def test_gemm_bf16_operands_at_any_address(ag, monkeypatch, k):
             if min(m, n) >= 8:
                 assert len(seen) == 3 and all(np.array_equal(seen[0], x) for x in seen[1:]), (m, n, ta, tb)
     monkeypatch.delenv("AGH_GEMM_CFG", raising=False)
+
+
+@pytest.mark.parametrize("k", [321, 1001, 2049])
+def test_gemm_bf16_operands_at_any_address_in_splits(ag, monkeypatch, k):
+    """The same form with k split over workgroups: the last split one short k-tile (321 in six splits of 64 and 1), or several with
+    a short one behind them, every layout, both tiles, NaN around the operands, alpha and beta; whole numbers exactly, so a chunk
+    read twice or not at all shows, and random values against the f32-accumulated reference, with the same bits in both tiles."""
+    rng = np.random.default_rng(k + 1)
+    for m, n in ((63, 65), (130, 37), (9, 129)):
+        for ta, tb in ((False, False), (True, False), (False, True), (True, True)):
+            shift = int(rng.integers(0, 2))
+            ash, bsh = (k, m) if ta else (m, k), (n, k) if tb else (k, n)
+
+            def operands(a, b):
+                return (ag.Tensor(ag.Tensor.from_array(np.concatenate([np.full(shift, np.uint16(0x7FC0)), v.ravel(),
+                                                                       np.full(3, np.uint16(0x7FC0))])).buffer,
+                                  v.shape, (v.shape[1], 1), shift, "bf16") for v in (a, b))
+
+            ai, bi = rng.integers(-2, 3, ash).astype(np.float32), rng.integers(-2, 3, bsh).astype(np.float32)
+            exact = to_dtype((ai.T if ta else ai) @ (bi.T if tb else bi), "bf16")
+            a, b = to_dtype(rng.uniform(-1, 1, ash), "bf16"), to_dtype(rng.uniform(-1, 1, bsh), "bf16")
+            c0 = to_dtype(rng.uniform(-1, 1, (m, n)), "bf16")
+            av, bv = (a.T if ta else a), (b.T if tb else b)
+            want, want_beta = orc.gemm_bf16_f32acc(av, bv, 1.0, 0.0, c0), orc.gemm_bf16_f32acc(av, bv, 0.5, 1.0, c0)
+            floor = 0.5 * 8 * np.sqrt(k) * 2.0**-24 * (np.abs(as_f32(av)) @ np.abs(as_f32(bv)))  # another order of the f32 sums
+            AI, BI = operands(to_dtype(ai, "bf16"), to_dtype(bi, "bf16"))
+            A, B = operands(a, b)
+            for splits in (2, 3, (k + 63) // 64):
+                monkeypatch.setenv("AGH_GEMM_SPLITS", str(splits))
+                seen = []
+                for cfg in ("3", "4"):
+                    monkeypatch.setenv("AGH_GEMM_CFG", cfg)
+                    C = ag.Tensor.from_array(np.full((m, n), 0x7FC0, np.uint16))
+                    ag.gemm(1.0, AI.t() if ta else AI, BI.t() if tb else BI, 0.0, C)
+                    assert np.array_equal(C.into_array(), exact), (m, n, ta, tb, splits, cfg)
+                    ag.gemm(1.0, A.t() if ta else A, B.t() if tb else B, 0.0, C)
+                    got = C.into_array()
+                    assert_bf16_gemm_close(got, want, av, bv)
+                    seen.append(got)
+                    C = ag.Tensor.from_array(c0)
+                    ag.gemm(0.5, A.t() if ta else A, B.t() if tb else B, 1.0, C)
+                    gf, wf = as_f32(C.into_array()).astype(np.float64), as_f32(want_beta).astype(np.float64)
+                    assert np.all(np.abs(gf - wf) <= np.maximum(bf16_ulp(gf), bf16_ulp(wf)) + floor), (m, n, ta, tb, splits, cfg)
+                assert np.array_equal(*seen), (m, n, ta, tb, splits)
 
 
 def test_gemm_bf16_form_of_short_and_narrow_ragged_products(ag, monkeypatch):
