@@ -534,10 +534,10 @@ __global__ __launch_bounds__(kThreads) void col2im_ring_kernel(const T *__restri
 }
 
 // Unit dilation, stride S (1 or 2, the same both ways) and square filter known at compile time: the streaming form with
-// everything the general kernel computes per tap hoisted or folded.  The stage carries (F-1-pw)/S all-zero segments
-// on either side, so a tap never has to ask whether its patch column exists (adding +0 to a running
-// sum changes nothing: a sum that starts at +0 can never be -0).  The F running sums of a pixel
-// column sit in registers and move down one place per step, the finished one leaving for memory.
+// everything the general kernel computes per tap hoisted or folded.  The stage carries all-zero segments on either side
+// (F-1-pw at stride 1, (F-pw)/2 rounded up at stride 2: col2im_pad_segments), so a tap never has to ask whether its patch
+// column exists (adding +0 to a running sum changes nothing: a sum that starts at +0 can never be -0).  The F running sums
+// of a pixel column sit in registers and move down one place per step, the finished one leaving for memory.
 // Per thread and step: eight 16-byte loads, the stage write, and per owned pixel column F*F LDS
 // reads and adds.  At stride 2 a pixel column meets every second tap (which ones depends on its parity, a lane's own
 // offset), the sums move two places, and two rows leave per step; where the parity has one tap less, +0 is added.
