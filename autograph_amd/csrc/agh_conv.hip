@@ -1695,15 +1695,15 @@ int conv2_direct_entry(const char *name, const void *x, const void *w, const voi
     const char *env = getenv("AGH_CONV_TAPS");  // 0 / 1 forces the choice of the kernel of any geometry (measurements, tests)
     const int taps_forced = env && *env ? (atoi(env) != 0 ? 1 : 0) : -1;
     const ConvShape shape = {bs, ic, ih, iw, oc, fh, fw, ph, pw, sh, sw, dh, dw, oh, ow};
-    const bool mfma_geometry = shape.unit() && conv2_mfma_takes<T>(x, w, bs, ic, ih, iw, oc, fh, fw, pw, oh, ow);
-    if (mfma_geometry && !pool2x2 && taps_forced != 1) {
+    if (shape.unit() && !pool2x2 && taps_forced != 1) {
         const int rc = conv2_mfma_try<T>(name, x, w, bias, y, bs, ic, ih, iw, oc, fh, fw, ph, pw, oh, ow, act);
         if (rc != 1) return rc;
     }
 
     // the matrix-core kernel of any geometry, where it expects to need less time than what would run in its place; with the
     // pool, where the convolution alone would run on it (the fused call returns the same bits as the separate layers)
-    if (taps_forced == 1 || (taps_forced != 0 && !(mfma_geometry && pool2x2))) {
+    const bool other = pool2x2 && shape.unit() && conv2_mfma_takes<T>(x, w, bs, ic, ih, iw, oc, fh, fw, pw, oh, ow);
+    if (taps_forced == 1 || (taps_forced != 0 && !other)) {
         const int rc = conv2_taps_try<T>(name, x, w, bias, y, bs, ic, ih, iw, oc, fh, fw, ph, pw, sh, sw, dh, dw, oh, ow, act, pool2x2 != 0,
                                          taps_forced == 1, conv2_taps_limit<T>(shape));
         if (rc != 1) return rc;
