@@ -195,11 +195,11 @@ struct FragRead {
 // DEPTH > 0: the form for operands that the direct loads cannot take (rows that do not start on 16-byte boundaries, k or a
 // row count that is no multiple of 8).  Same tiles, LDS layout, fragments and sums; the operand chunks travel through
 // registers instead: 16-byte loads from element addresses, DEPTH k-tiles in flight in as many register sets, each set
-// written to the LDS stage (two of them) one k-tile before it is multiplied.  What bounds it is the rate at
-// which a CU's L1 serves 16-byte loads that cross cache lines, about 60 cycles an instruction (16 when aligned).  The last k-tile is the only one in which a 16-byte chunk can pass the end of a row or of the
-// operand: its addresses are moved back by the overhang.  Against
-// the element-wise loaders: 1999x2047x1001 99 -> 25.8 us, 4099x4101x4103 1344 -> 238, 1058x4544x699 111 -> 24.1,
-// 8191x333x127 (transposed) 15.9 -> 6.5.
+// written to the LDS stage (two of them) one k-tile before it is multiplied.  What bounds it is the CU's L1: a 16-byte load of
+// 64 lanes that starts anywhere costs 56 accesses, and 0.9 of one access a cycle is made over the whole launch
+// (4099x4101x4103).  The last k-tile is the only one in which a 16-byte chunk can pass the end of a row or of the operand: its
+// addresses are moved back by the overhang.  Against the element-wise loaders: 1999x2047x1001 99 -> 26.8 us,
+// 4099x4101x4103 1344 -> 239, 1058x4544x699 111 -> 24.1, 8191x333x127 (transposed) 15.9 -> 6.5.
 template <int BP, int BQ, int WGP, int WGQ, int LP, int LQ, bool STAGED, int NS = 2, int DEPTH = 0>
 __global__ __launch_bounds__(WGP *WGQ * 64, DEPTH > 0 ? 2 : 1) void gemm_bf16_dl_kernel(Args g) {
     typedef uint16_t T;
