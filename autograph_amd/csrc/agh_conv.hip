@@ -1550,6 +1550,7 @@ int launch_oct(int oct, dim3 grid, dim3 block, size_t smem, const T *x, const T 
 // What conv2_direct_entry chooses by, with the 2x2 pool fused or without.
 struct ConvShape {
     int64_t bs, ic, ih, iw, oc, fh, fw, ph, pw, sh, sw, dh, dw, oh, ow;
+    int small_forced;  // AGH_CONV_SMALL: 0 / 1 forces the choice of conv2_small_mfma_kernel (measurements), -1 by size
     bool unit() const { return sh == 1 && sw == 1 && dh == 1 && dw == 1; }
 };
 constexpr int64_t kConvLds = 64 * 1024;
@@ -1558,9 +1559,8 @@ inline int64_t conv_cus() { return compute_units() > 0 ? compute_units() : 256; 
 // up to 16 output channels over enough taps on small images: matrix cores fed from the staged image
 bool conv2_small_plan(const ConvShape &c, bool pool, SmallMfmaParams &q, int64_t &fixed_bytes, int64_t &img_bytes) {
     if (!c.unit() || c.oc > 16) return false;
-    const char *env = getenv("AGH_CONV_SMALL");  // 0 / 1 forces the choice (measurements)
     const int64_t taps = c.ic * c.fh * c.fw;
-    const bool want = env ? atoi(env) != 0 : (c.oc >= 8 && taps >= 32);
+    const bool want = c.small_forced >= 0 ? c.small_forced != 0 : (c.oc >= 8 && taps >= 32);
     q.bs = (int)c.bs; q.ic = (int)c.ic; q.ih = (int)c.ih; q.iw = (int)c.iw; q.oc = (int)c.oc; q.oh = (int)c.oh; q.ow = (int)c.ow;
     q.fh = (int)c.fh; q.fw = (int)c.fw; q.ph = (int)c.ph; q.pw = (int)c.pw;
     q.ihp = (int)(c.ih + 2 * c.ph);
@@ -1694,7 +1694,8 @@ int conv2_direct_entry(const char *name, const void *x, const void *w, const voi
     // enough channels: implicit GEMM on the matrix cores (returns 1 when the geometry is not its own)
     const char *env = getenv("AGH_CONV_TAPS");  // 0 / 1 forces the choice of the kernel of any geometry (measurements, tests)
     const int taps_forced = env && *env ? (atoi(env) != 0 ? 1 : 0) : -1;
-    const ConvShape shape = {bs, ic, ih, iw, oc, fh, fw, ph, pw, sh, sw, dh, dw, oh, ow};
+    const char *small_env = oc <= 16 ? getenv("AGH_CONV_SMALL") : nullptr;
+    const ConvShape shape = {bs, ic, ih, iw, oc, fh, fw, ph, pw, sh, sw, dh, dw, oh, ow, small_env ? atoi(small_env) != 0 : -1};
     if (shape.unit() && !pool2x2 && taps_forced != 1) {
         const int rc = conv2_mfma_try<T>(name, x, w, bias, y, bs, ic, ih, iw, oc, fh, fw, ph, pw, oh, ow, act);
         if (rc != 1) return rc;
@@ -1702,10 +1703,11 @@ int conv2_direct_entry(const char *name, const void *x, const void *w, const voi
 
     // the matrix-core kernel of any geometry, where it expects to need less time than what would run in its place; with the
     // pool, where the convolution alone would run on it (the fused call returns the same bits as the separate layers)
-    const bool other = pool2x2 && shape.unit() && conv2_mfma_takes<T>(x, w, bs, ic, ih, iw, oc, fh, fw, pw, oh, ow);
-    if (taps_forced == 1 || (taps_forced != 0 && !other)) {
+    const double taps_limit = taps_forced != 0 ? conv2_taps_limit<T>(shape) : 0.0;
+    if (taps_forced == 1 || (taps_limit >= kTapsLeastUs && !(pool2x2 && shape.unit() &&
+                                                            conv2_mfma_takes<T>(x, w, bs, ic, ih, iw, oc, fh, fw, pw, oh, ow)))) {
         const int rc = conv2_taps_try<T>(name, x, w, bias, y, bs, ic, ih, iw, oc, fh, fw, ph, pw, sh, sw, dh, dw, oh, ow, act, pool2x2 != 0,
-                                         taps_forced == 1, conv2_taps_limit<T>(shape));
+                                         taps_forced == 1, taps_limit);
         if (rc != 1) return rc;
         if (taps_forced == 1) return fail(AGH_ERANGE, "%s: AGH_CONV_TAPS=1, and that kernel does not take this shape", name);
     }

@@ -289,8 +289,6 @@ int conv2_taps_try(const char *name, const void *x, const void *w, const void *b
                    int64_t iw, int64_t oc, int64_t fh, int64_t fw, int64_t ph, int64_t pw, int64_t sh, int64_t sw, int64_t dh,
                    int64_t dw, int64_t oh, int64_t ow, int act, bool pool, bool forced, double limit_us) {
     const int64_t npos = oh * ow, ktot = ic * fh * fw, pitch = ((ow - 1) * sw + (fw - 1) * dw + 4) & ~(int64_t)3;
-    constexpr double kLeastUs = 4.4;  // below what any shape is expected to need: small layers decide without the search
-    if (!forced && limit_us < kLeastUs) return 1;
     if (npos > ((int64_t)1 << 24) || ktot > ((int64_t)1 << 24) || oc * ktot > ((int64_t)1 << 28)) return 1;
     // tile: rounds of workgroups times the matrix cycles of one (16 positions x 16 channels x 4 taps = 32 cycles, each wave
     // on a SIMD of its own; a lone wave waits about 500 cycles for the operands of 16 taps), and its staging (batches of 8
@@ -318,7 +316,7 @@ int conv2_taps_try(const char *name, const void *x, const void *w, const void *b
                 // cycles or, up to three workgroups of a CU together, the waits for operands come to, the stages, of which
                 // later rounds hide a quarter, and the bytes that no cache holds
                 const double chunks = (double)(ktot + 15) / 16.0;
-                us = kLeastUs + (std::max(1.375 * (double)rounds * chunks * t * n * 128.0, 0.9 * chunks * 500.0 * (double)((rounds + 2) / 3)) +
+                us = kTapsLeastUs + (std::max(1.375 * (double)rounds * chunks * t * n * 128.0, 0.9 * chunks * 500.0 * (double)((rounds + 2) / 3)) +
                             (double)stages * (2200.0 * (double)batches + 3300.0) * (0.25 + 0.75 * (double)rounds)) / 2100.0 +
                      0.11e-6 * (double)sizeof(T) * (double)bs * ((double)ic * ih * iw + (double)oc * npos);
             }

@@ -31,6 +31,7 @@ int conv2_mfma_try(const char *name, const void *x, const void *w, const void *b
 template <typename T>
 bool conv2_mfma_takes(const void *x, const void *w, int64_t bs, int64_t ic, int64_t ih, int64_t iw, int64_t oc, int64_t fh, int64_t fw,
                       int64_t pw, int64_t oh, int64_t ow);
+constexpr double kTapsLeastUs = 4.4;  // what no shape is expected to need less than in the kernel below
 // Conv2 forward for any stride, dilation and channel count on the f32 matrix cores (agh_conv_taps.hip), followed by the
 // 2x2 pool where `pool`; 1 = not taken: the shape is not its own, or the convolution is expected to need more than
 // limit_us there (and is not forced)
