@@ -251,16 +251,27 @@ __global__ __launch_bounds__(kThreads) void sgd_momentum_kernel(T *__restrict__ 
 // ------------------------------------------------------------- sum axis 0 ----
 // Rows are added one at a time in the element type, in row order, starting from zero: per column one serial chain of
 // `rows` dependent additions (and roundings), which is what bounds the launch; nothing of it can be split.  A workgroup
-// owns 64 columns.  Its first wave does nothing but the chain, one column per lane, out of LDS (four rows per 16-byte
-// read, already widened to f32); the other eight waves keep two chunks of 256 rows in flight and store them to LDS,
+// owns COLS columns.  Its first wave does nothing but the chain, one column per lane, out of LDS (four rows per 16-byte
+// read, already widened to f32); the LOADERS other waves keep two chunks of 256 rows in flight and store them to LDS,
 // column-major with a pitch of 260 words, so that 16 lanes of either side meet 16 different bank groups.  A bf16 step is
 // two dependent instructions, the addition and v_cvt_pk_bf16_f32 of (0, sum), whose result is the rounded sum as f32.
-// 4096 x 1000: bf16 27.5 us, f32 21.6 us; 8192 x 1000: 51.7 and 40.2 us, that is 5.9 and 4.5 ns a row (two dependent
-// instructions of about seven cycles; one of eleven) behind about 4 us of starting.  One thread per column that loads and adds
-// by itself (sum_axis0_short_kernel) pays a memory round trip every eight rows: 4096 x 1000 f32 172 us.
-constexpr int kSumCols = 64, kSumRows = 256, kSumLoaders = 8, kSumPitch = kSumRows + 4;
-constexpr int kSumRPW = kSumRows / kSumLoaders;  // rows of a chunk that one loading wave moves
-constexpr size_t kSumLds = 2 * (size_t)kSumCols * kSumPitch * sizeof(float);
+// A wave issues an instruction every four cycles at best, so everything in the chain's wave that is not the chain counts:
+// one wait per 32 rows (the compiler's own waits, one per LDS read, are three times as many instructions as the reads), a whole chunk
+// unrolled with constant offsets, and few distinct columns per wave, which makes the LDS reads shorter (16 columns: the
+// lanes behind them read the same words).  8192 x 1000, 64 columns with the compiler's waits / 64 / 32 / 16 columns in us: bf16 52.2 /
+// 45.9 / 40.0 / 38.4, f32 38.7 / 37.9 / 28.3 / 26.2; out of memory instead of the caches 59.9 / 56.3 / 47.1 / 42.4 and 59.7 /
+// 59.6 / 40.7 / 30.4 (few columns a workgroup also means more CUs that load).  A bare chain of these instructions takes 3.55 ns
+// (bf16) and 1.88 ns (f32) a row, the kernel 4.4 and 2.9.  One thread per column that loads and adds by itself
+// (sum_axis0_short_kernel) pays a memory round trip every eight rows: 4096 x 1000 f32 172 us.
+// Neighbouring groups of columns share cache lines: each XCD takes a contiguous run of them (4096 x 4096 f32 in 16 columns 25.9 us
+// without, 17.7 with).
+constexpr int kSumRows = 256, kSumPitch = kSumRows + 4;
+template <int COLS>
+struct SumGeo {
+    static constexpr int LOADERS = COLS == 64 ? 8 : 4;
+    static constexpr int RPL = kSumRows * COLS / (LOADERS * 64);  // consecutive rows of a chunk that one lane moves
+    static constexpr size_t LDS = 2 * (size_t)COLS * kSumPitch * sizeof(float);
+};
 
 template <typename T>
 __device__ __forceinline__ float add_rounded(float acc, float v) {
@@ -269,109 +280,135 @@ __device__ __forceinline__ float add_rounded(float acc, float v) {
     else return s;
 }
 
-template <typename T>
-__global__ __launch_bounds__(64 * (1 + kSumLoaders)) void sum_axis0_kernel(const T *__restrict__ x, T *__restrict__ y, int64_t rows,
-                                                                            int64_t cols) {
+// 256 rows of cols columns are addressed by 32-bit byte offsets (checked by the host)
+template <typename T, int COLS>
+__global__ __launch_bounds__(64 * (1 + SumGeo<COLS>::LOADERS)) void sum_axis0_kernel(const T *__restrict__ x, T *__restrict__ y,
+                                                                                   int64_t rows, int64_t cols) {
+    constexpr int RPL = SumGeo<COLS>::RPL, BLOCK = 32;
     extern __shared__ __align__(16) float sum_lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t j0 = (int64_t)blockIdx.x * kSumCols, j = j0 + lane;
+    // workgroup b runs on XCD b % 8; the grid is a multiple of eight
+    const int64_t group = (int64_t)(blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    const int64_t j0 = group * COLS;
+    if (j0 >= cols) return;
     const int64_t trips = (rows + 2 * kSumRows - 1) / (2 * kSumRows) * 2;  // chunks of rows, rounded up to an even number
-    float *const buf0 = sum_lds + lane * kSumPitch, *const buf1 = buf0 + kSumCols * kSumPitch;
     if (wave == 0) {
+        const int col = lane & (COLS - 1);
+        const float *const buf0 = sum_lds + col * kSumPitch;
         float acc = 0.0f;
+        auto landed = [] {  // every LDS read has: the compiler adds no wait of its own behind this one
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto fetch = [](float4 (&v)[BLOCK / 4], const float *src) {
+#pragma unroll
+            for (int u = 0; u < BLOCK / 4; ++u) v[u] = *(const float4 *)(src + u * 4);
+        };
+        auto add = [&](const float4 (&v)[BLOCK / 4]) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < BLOCK / 4; ++u) {
+                acc = add_rounded<T>(acc, v[u].x);
+                acc = add_rounded<T>(acc, v[u].y);
+                acc = add_rounded<T>(acc, v[u].z);
+                acc = add_rounded<T>(acc, v[u].w);
+            }
+        };
         auto add_chunk = [&](const float *buf, int64_t left) {
-            // whole blocks of 32 rows: the rows behind the last one are zeros in LDS, and adding +0 to a sum that is
-            // never -0 is exact
-            const int blocks = (int)min((left + 31) >> 5, (int64_t)(kSumRows / 32));  // none in a chunk behind the last row
-            float4 v[2][8];
+            if (left <= 0) return;
+            float4 v[2][BLOCK / 4];
+            fetch(v[0], buf);
+            landed();
+            if (left >= kSumRows) {
 #pragma unroll
-            for (int u = 0; u < 8; ++u) v[0][u] = *(const float4 *)(buf + u * 4);
-            auto block = [&](const float4 (&cur)[8], float4 (&nxt)[8], int b) {
-                const float *src = buf + min(b + 1, kSumRows / 32 - 1) * 32;  // the next block is read while this one is added
-#pragma unroll
-                for (int u = 0; u < 8; ++u) nxt[u] = *(const float4 *)(src + u * 4);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    acc = add_rounded<T>(acc, cur[u].x);
-                    acc = add_rounded<T>(acc, cur[u].y);
-                    acc = add_rounded<T>(acc, cur[u].z);
-                    acc = add_rounded<T>(acc, cur[u].w);
+                for (int b = 0; b < kSumRows / BLOCK; ++b) {  // the next block is read while this one is added
+                    if (b + 1 < kSumRows / BLOCK) fetch(v[(b + 1) & 1], buf + (b + 1) * BLOCK);
+                    add(v[b & 1]);
+                    if (b + 1 < kSumRows / BLOCK) landed();
                 }
-            };
-            for (int b = 0; b < blocks; b += 2) {
-                block(v[0], v[1], b);
-                if (b + 1 < blocks) block(v[1], v[0], b + 1);
+            } else {
+                // whole blocks of 32 rows: the rows behind the last one are zeros in LDS, and adding +0 to a sum that is
+                // never -0 is exact
+                const int blocks = (int)((left + BLOCK - 1) / BLOCK);
+                for (int b = 0; b < blocks; b += 2) {
+                    fetch(v[1], buf + min(b + 1, kSumRows / BLOCK - 1) * BLOCK);
+                    add(v[0]);
+                    landed();
+                    if (b + 1 >= blocks) break;
+                    fetch(v[0], buf + min(b + 2, kSumRows / BLOCK - 1) * BLOCK);
+                    add(v[1]);
+                    landed();
+                }
             }
         };
         __syncthreads();
         for (int64_t c = 0; c < trips; ++c) {
-            add_chunk(c & 1 ? buf1 : buf0, rows - c * kSumRows);
+            add_chunk(buf0 + (c & 1 ? COLS * kSumPitch : 0), rows - c * kSumRows);
             __syncthreads();
         }
-        if (j < cols) {
-            if constexpr (sizeof(T) == 2) y[j] = (T)(__float_as_uint(acc) >> 16);
-            else y[j] = acc;
+        if (lane < COLS && j0 + col < cols) {
+            if constexpr (sizeof(T) == 2) y[j0 + col] = (T)(__float_as_uint(acc) >> 16);
+            else y[j0 + col] = acc;
         }
     } else {
-        const int r0 = (wave - 1) * kSumRPW;  // first row of this wave within a chunk
-        const T *const xs = x + j0;
-        const uint32_t jb = (uint32_t)min((int64_t)lane, cols - 1 - j0) * (uint32_t)sizeof(T);
-        T reg0[kSumRPW], reg1[kSumRPW];
-        auto load = [&](T (&reg)[kSumRPW], int64_t c) {
-            const int64_t r = c * kSumRows + r0;
-            // buffer loads: a row behind the last one has no bytes in range and reads as zeros, without a branch (left to
-            // pointers, the compiler puts one around every load, and each then waits for all loads in flight)
-            const T *p = xs + r * cols;
-            // rows of this wave's that exist (readfirstlane: compared on the scalar side below)
-            const int have = __builtin_amdgcn_readfirstlane((int)min(max(rows - r, (int64_t)0), (int64_t)kSumRPW));
+        // consecutive lanes take consecutive columns; 64 / COLS groups of RPL rows a wave
+        const int t = (wave - 1) * 64 + lane, col = t & (COLS - 1), r0 = t / COLS * RPL;
+        const uint32_t row_bytes = (uint32_t)cols * (uint32_t)sizeof(T);
+        const uint32_t first = (uint32_t)r0 * row_bytes + (uint32_t)min(j0 + col, cols - 1) * (uint32_t)sizeof(T);
+        T reg0[RPL], reg1[RPL];
+        auto load = [&](T (&reg)[RPL], int64_t c) {
+            // buffer loads: a row behind the last one is out of range and reads as zeros, without a branch (left to pointers, the
+            // compiler puts one around every load, and each then waits for all loads in flight)
+            const int64_t r = c * kSumRows, left = max(rows - r, (int64_t)0);
+            const int64_t bytes = min(left, (int64_t)kSumRows) * cols * (int64_t)sizeof(T);
+            const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(x + (left > 0 ? r : 0) * cols), 0, (uint32_t)bytes, 0x00020000);
 #pragma unroll
-            for (int u = 0; u < kSumRPW; ++u, p += cols) {
-                const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, u < have ? kSumCols * (int)sizeof(T) : 0, 0x00020000);
-                if constexpr (sizeof(T) == 2) reg[u] = (T)__builtin_amdgcn_raw_buffer_load_b16(rsrc, jb, 0, 0);
-                else reg[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, jb, 0, 0));
+            for (int u = 0; u < RPL; ++u) {
+                if constexpr (sizeof(T) == 2) reg[u] = (T)__builtin_amdgcn_raw_buffer_load_b16(rsrc, first + u * row_bytes, 0, 0);
+                else reg[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, first + u * row_bytes, 0, 0));
             }
             __builtin_amdgcn_sched_barrier(0);
         };
-        auto store = [&](const T (&reg)[kSumRPW], float *buf) {
+        auto store = [&](const T (&reg)[RPL], int buf) {
+            float *dst = sum_lds + (buf * COLS + col) * kSumPitch + r0;
 #pragma unroll
-            for (int u = 0; u < kSumRPW; u += 4)
-                *(float4 *)(buf + r0 + u) = make_float4(Elem<T>::raw(reg[u]), Elem<T>::raw(reg[u + 1]), Elem<T>::raw(reg[u + 2]), Elem<T>::raw(reg[u + 3]));
+            for (int u = 0; u < RPL; u += 4)
+                *(float4 *)(dst + u) = make_float4(Elem<T>::raw(reg[u]), Elem<T>::raw(reg[u + 1]), Elem<T>::raw(reg[u + 2]), Elem<T>::raw(reg[u + 3]));
             __builtin_amdgcn_sched_barrier(0);
         };
         load(reg0, 0);
         load(reg1, 1);
-        store(reg0, buf0);
+        store(reg0, 0);
         load(reg0, 2);
         __syncthreads();
         // trip c: chunk c is being added out of its buffer, chunk c + 1 goes into the other, chunk c + 3 is requested
         for (int64_t c = 0; c < trips; c += 2) {
-            store(reg1, buf1);
+            store(reg1, 1);
             load(reg1, c + 3);
             __syncthreads();
-            store(reg0, buf0);
+            store(reg0, 0);
             load(reg0, c + 4);
             __syncthreads();
         }
     }
 }
 
-// The same sums with one thread per column: all columns at once, bound by a memory round trip every eight rows (16 to 18 ns a
+// The same sums with one thread per column (0): all columns at once, bound by a memory round trip every eight rows (about 25 ns a
 // row out of the caches) and, where the columns fill the chip several times over, by memory itself.
-// The kernel above has one workgroup of 64 columns on a CU (130 KB of LDS), so it pays its 5.5 us of starting, filling and
-// draining once for every round of CUs * 64 columns.  Both measured over 64 to 32768 rows of 64 to 4194304 columns, one
-// thread / staged in us: 224 x 4096 f32 5.3 / 5.6, 256 x 4096 5.9 / 5.7; 320 x 32768 (two rounds) f32 14.3 / 14.0, bf16
-// 8.1 / 11.7; 512 x 40000 (three) 24.9 / 20.4, 25.7 / 18.2; 768 x 65536 (four) 38.1 / 43.4, 33.7 / 38.2; 1024 x 65536 51.7 / 48.4,
-// 45.1 / 40.0; from eight rounds on one thread per column reaches the memory's rate too: 256 x 262144 38.6 / 86.6,
-// 20.1 / 87.9; 2048 x 131072 181.9 / 192.4, 164.9 / 180.3; 4096 x 131072 365 / 358, 330 / 331.
-// Rows that do not start on 64 bytes cost the staged form more (its waves read 128 or 256 bytes of a row): 600 x 49011 f32
-// 29.3 / 37.2, bf16 28.8 / 33.6; 1050 x 65395 f32 64.2 / 71.5.  Of 616 sizes of one to seven rounds the rule misses the faster form by
-// more than a tenth at 9, by 18 % at most.
-__host__ inline bool sum_axis0_staged(int64_t rows, int64_t cols, int64_t cus, int64_t bytes) {
-    const int64_t per_round = cus * kSumCols, rounds = cols / per_round + (cols % per_round != 0);
-    const bool lines = cols % 64 * bytes % 64 == 0;
-    if (rounds < 3 || (rounds == 3 && lines)) return rows > 140 + 100 * rounds;
-    return rounds < 8 && rows > (!lines ? 280 * rounds : bytes == 4 ? 175 * rounds : rounds == 7 ? 1320 : 220 * rounds);
+// Staged, a round of 16, 32 or 64 columns on every CU takes 2.2 to 4.5 us of starting and 2.9 to 5 ns a row: as few columns a
+// workgroup as one round allows, and for a last round that is at most half full two workgroups of 32 side by side on a CU instead of
+// one of 64.  Measured over 1192 sizes of 32 to 16384 rows and 10 to 400000 columns, one thread / 16 / 32 / 64 columns in us:
+// 71 x 8128 f32 4.2 / 3.7 / 3.8 / 4.6, 92 x 7184 3.7 / 3.5 / 3.6 / 4.6, 2293 x 3056 99 / 9.4 / 10.9 / 12.3; bf16 142 x 14496 5.2 / 8.3 /
+// 5.5 / 5.3, 1252 x 14196 60.7 / 26.3 / 13.0 / 11.3; two rounds: bf16 244 x 23824 7.2 / 12.5 / 8.6 / 9.9, 677 x 16624 30.9 / 17.0 / 12.5 /
+// 14.3, f32 160 x 32736 4.7 / 10.8 / 9.9 / 8.1, 257 x 18291 11.7 / 8.3 / 7.1 / 8.2; four: bf16 724 x 58496 37.3 / 50.9 / 33.8 / 31.7;
+// from eight rounds on one thread per column reaches the memory's rate too (256 x 262144 f32 38.6 / 64 columns 86.6; 4096 x 131072 365 /
+// 358).  Of the 1192 sizes 17 are more than a tenth behind the best form, all together 0.6 %.
+__host__ inline int sum_axis0_columns(int64_t rows, int64_t cols, int64_t cus, int64_t bytes, bool always) {
+    const int64_t per_round = cus * 64, rounds = cols / per_round + (cols % per_round != 0), last = cols % per_round;
+    const int64_t least = cols <= cus * 32 ? 90 : rounds == 1 ? 160 : rounds <= 3 ? (bytes == 4 ? 190 : 260) : 140 * rounds - 200;
+    if (!always && (rounds >= 8 || rows <= least)) return 0;
+    return cols <= cus * 16 ? 16 : cols <= cus * 32 || (rounds > 1 && last > 0 && last <= per_round / 2) ? 32 : 64;
 }
 
 template <typename T>
@@ -577,28 +614,41 @@ int sgd_momentum_launch(const char *name, void *w, const void *dw, float lr, flo
     return AGH_OK;
 }
 
+template <typename T, int COLS>
+int sum_axis0_staged_launch(const char *name, const void *x, void *y, int64_t rows, int64_t cols) {
+    const int64_t blocks = ((cols + COLS - 1) / COLS + 7) / 8 * 8;
+    static bool attr_done = false;
+    if (!attr_done) {
+        AGH_HIP(hipFuncSetAttribute((const void *)sum_axis0_kernel<T, COLS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)SumGeo<COLS>::LDS));
+        attr_done = true;
+    }
+    hipLaunchKernelGGL((sum_axis0_kernel<T, COLS>), dim3((unsigned)blocks), dim3(64 * (1 + SumGeo<COLS>::LOADERS)), SumGeo<COLS>::LDS, stream(),
+                       (const T *)x, (T *)y, rows, cols);
+    AGH_LAUNCH_CHECK(name);
+    return AGH_OK;
+}
+
 template <typename T>
 int sum_axis0_launch(const char *name, const void *x, void *y, int64_t rows, int64_t cols) {
     AGH_API_ENTER();
     if (rows < 0 || cols < 0) return fail(AGH_EINVAL, "%s: negative shape", name);
     if (cols == 0) return AGH_OK;
     if (!y || (!x && rows > 0)) return fail(AGH_ENULL, "%s: null buffer", name);
-    const char *env = getenv("AGH_SUM_STAGED");  // 0 / 1 forces the choice (measurements, tests)
-    const bool brief = env && *env ? atoi(env) == 0 : !sum_axis0_staged(rows, cols, compute_units() > 0 ? compute_units() : 256, (int64_t)sizeof(T));
-    const int64_t per_block = brief ? kThreads : kSumCols, blocks = (cols + per_block - 1) / per_block;
+    // 0: one thread a column, 1: staged, 16 / 32 / 64: staged with that many columns a workgroup (measurements, tests)
+    const char *env = getenv("AGH_SUM_STAGED");
+    const int forced = env && *env ? atoi(env) : -1;
+    const int64_t cus = compute_units() > 0 ? compute_units() : 256;
+    const bool fits = cols <= (int64_t)1 << 20;  // 256 rows within 32-bit offsets
+    const int staged = !fits || forced == 0 ? 0 : forced > 1 ? forced : sum_axis0_columns(rows, cols, cus, (int64_t)sizeof(T), forced == 1);
+    switch (staged) {
+        case 16: return sum_axis0_staged_launch<T, 16>(name, x, y, rows, cols);
+        case 32: return sum_axis0_staged_launch<T, 32>(name, x, y, rows, cols);
+        case 64: return sum_axis0_staged_launch<T, 64>(name, x, y, rows, cols);
+        default: break;
+    }
+    const int64_t blocks = (cols + kThreads - 1) / kThreads;
     if (blocks > 0x7FFFFFFFll) return fail(AGH_ERANGE, "%s: too many columns", name);
-    if (brief) {
-        hipLaunchKernelGGL(sum_axis0_short_kernel<T>, dim3((unsigned)blocks), dim3(kThreads), 0, stream(), (const T *)x, (T *)y, rows, cols);
-        AGH_LAUNCH_CHECK(name);
-        return AGH_OK;
-    }
-    static bool attr_done = false;
-    if (!attr_done) {
-        AGH_HIP(hipFuncSetAttribute((const void *)sum_axis0_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSumLds));
-        attr_done = true;
-    }
-    hipLaunchKernelGGL(sum_axis0_kernel<T>, dim3((unsigned)blocks), dim3(64 * (1 + kSumLoaders)), kSumLds, stream(),
-                       (const T *)x, (T *)y, rows, cols);
+    hipLaunchKernelGGL(sum_axis0_short_kernel<T>, dim3((unsigned)blocks), dim3(kThreads), 0, stream(), (const T *)x, (T *)y, rows, cols);
     AGH_LAUNCH_CHECK(name);
     return AGH_OK;
 }

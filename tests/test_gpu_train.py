@@ -140,6 +140,22 @@ def test_sum_axis0_form_chosen_by_rows_and_columns(ag, dtype, monkeypatch):
         assert us[""] <= bound * min(us["0"], us["1"]), (rows, cols, us)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("columns", [16, 32, 64])
+def test_sum_axis0_columns_of_a_workgroup(ag, dtype, columns, monkeypatch):
+    """16, 32 or 64 columns a workgroup: bit for bit the serial sum at the edges of a workgroup's columns, of its chunks of 256
+    rows and its blocks of 32, with more groups than one XCD's share and a grid that is no multiple of eight; infinities and
+    NaN stay in their column."""
+    monkeypatch.setenv("AGH_SUM_STAGED", str(columns))
+    rng = np.random.default_rng(columns)
+    for rows, cols in ((1, 15), (31, 16), (32, 17), (33, 33), (255, 64), (256, 65), (288, 143), (512, 1000), (544, 31), (1023, 9 * columns + 1)):
+        a = to_dtype(rng.standard_normal((rows, cols)) * 4, dtype)
+        special = to_dtype(np.array([np.inf, -np.inf, np.nan], np.float32), dtype)
+        a[rows // 2, 0], a[rows - 1, cols - 1], a[rows // 3, cols // 2] = special
+        assert np.array_equal(ag.Tensor.from_array(a).sum_axis0().into_array(), orc.sum_axis0(a), equal_nan=dtype == "f32"), (rows, cols)
+
+
 def _view_of(ag, t, a, base):
     """The device Tensor that shows the same elements of `t` (uploaded from `base`) as the numpy view `a` of `base`."""
     es = base.itemsize
