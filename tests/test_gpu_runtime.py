@@ -311,3 +311,26 @@ def test_calibration_launches(ag):
     assert lib.calib_mfma_dma(st, tsrc._ptr(), 65536, sink._ptr(), 4, 65536, 8, 4) == -4
     assert lib.calib_mix(st, tsrc._ptr(), tdst._ptr(), 4 * n + 4, 2, 8) == -1
     assert lib.calib_copy(st, tsrc._ptr(), tdst._ptr(), 4 * n, 0) == -1
+
+
+@pytest.mark.parametrize("extra", [0, 1, 15, 16, 4097, -1])
+def test_large_copies_between_device_blocks(ag, extra):
+    """Copies from 112 MB on between blocks of the allocator are a launch of their own: every byte arrives and none behind the
+    last, at any length; offsets that are no whole vectors and overlapping ranges that are the same take the runtime's copy."""
+    least = 112 << 20
+    n = least + extra
+    rng = np.random.default_rng(7)
+    host = rng.integers(0, 256, n + 64, dtype=np.uint8)
+    check = ag._ffi.check
+    src, dst = ag.Buffer(n + 64), ag.Buffer(n + 64)
+    check(ag.lib.agh_memcpy_h2d(src.ptr, host.ctypes.data, n + 64))
+    for so, do in ((0, 0), (16, 32), (3, 0), (0, 8)):
+        check(ag.lib.agh_memset(dst.ptr, 0xA5, n + 64))
+        check(ag.lib.agh_memcpy_d2d(dst.ptr + do, src.ptr + so, n))
+        got = np.empty(n + 64, np.uint8)
+        check(ag.lib.agh_memcpy_d2h(got.ctypes.data, dst.ptr, n + 64))
+        assert np.array_equal(got[do:do + n], host[so:so + n]) and (got[:do] == 0xA5).all() and (got[do + n:] == 0xA5).all(), (so, do)
+    check(ag.lib.agh_memcpy_d2d(src.ptr, src.ptr, n))
+    got = np.empty(n, np.uint8)
+    check(ag.lib.agh_memcpy_d2h(got.ctypes.data, src.ptr, n))
+    assert np.array_equal(got, host[:n])
