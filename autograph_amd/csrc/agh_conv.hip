@@ -1692,9 +1692,9 @@ int conv2_direct_entry(const char *name, const void *x, const void *w, const voi
     if (!x || !w || !y) return fail(AGH_ENULL, "%s: null buffer", name);
 
     // enough channels: implicit GEMM on the matrix cores (returns 1 when the geometry is not its own)
-    const char *env = getenv("AGH_CONV_TAPS");  // 0 / 1 forces the choice of the kernel of any geometry (measurements, tests)
+    const char *env = setting("AGH_CONV_TAPS");  // 0 / 1 forces the choice of the kernel of any geometry (measurements, tests)
     const int taps_forced = env && *env ? (atoi(env) != 0 ? 1 : 0) : -1;
-    const char *small_env = oc <= 16 ? getenv("AGH_CONV_SMALL") : nullptr;
+    const char *small_env = oc <= 16 ? setting("AGH_CONV_SMALL") : nullptr;
     const ConvShape shape = {bs, ic, ih, iw, oc, fh, fw, ph, pw, sh, sw, dh, dw, oh, ow, small_env ? atoi(small_env) != 0 : -1};
     if (shape.unit() && !pool2x2 && taps_forced != 1) {
         const int rc = conv2_mfma_try<T>(name, x, w, bias, y, bs, ic, ih, iw, oc, fh, fw, ph, pw, oh, ow, act);

@@ -435,12 +435,12 @@ static int conv2_mfma_launch(const char *name, const void *x, const void *w, con
     p.K = fh * fw * ic;
     p.per_xcd = blocks % 8 == 0 ? (int)(blocks / 8) : 0;
     {
-        const char *e = getenv("AGH_CONV_REMAP");
+        const char *e = setting("AGH_CONV_REMAP");
         p.remap = e && *e ? atoi(e) : 1;
         // An output that could not stay in the 256 MB last-level cache next to the input anyway is stored with the
         // streaming hint, which leaves that cache to the input rows neighbouring tiles share (config 3 in bf16: 0.135 ->
         // 0.124 ms); a smaller one is stored plainly, for the layer that reads it next.  AGH_CONV_NT=0|1 overrides.
-        const char *nt = getenv("AGH_CONV_NT");
+        const char *nt = setting("AGH_CONV_NT");
         const size_t out_bytes = (size_t)bs * oc * npos * sizeof(T);
         p.nt_store = nt && *nt ? atoi(nt) : out_bytes > ((size_t)64 << 20);
     }
@@ -465,7 +465,7 @@ static int conv2_mfma_launch(const char *name, const void *x, const void *w, con
 // a smaller share; 878 against 796 TFLOP/s).  AGH_CONV_TILE=128|256 overrides.
 template <typename T>
 static int conv2_mfma_tile() {
-    const char *e = getenv("AGH_CONV_TILE");
+    const char *e = setting("AGH_CONV_TILE");
     return e && *e ? atoi(e) : (sizeof(T) == 4 ? 128 : 256);
 }
 

@@ -294,7 +294,7 @@ int conv2_taps_try(const char *name, const void *x, const void *w, const void *b
     // on a SIMD of its own; a lone wave waits about 500 cycles for the operands of 16 taps), and its staging (batches of 8
     // groups of four cells a thread, a memory round trip each), which later rounds hide in part.  AGH_CONV_TAPS_TILE = 10 TG + NT
     // forces a tile where the kernel is forced (tests).
-    const char *env = forced ? getenv("AGH_CONV_TAPS_TILE") : nullptr;
+    const char *env = forced ? setting("AGH_CONV_TAPS_TILE") : nullptr;
     const int tile = env && *env ? atoi(env) : 0;
     const int64_t cus = compute_units() > 0 ? compute_units() : 256, n16 = (oc + 15) / 16;
     int tg = 0, nt = 0;

@@ -108,8 +108,8 @@ inline int gemm_f32_small_try(Args &g, int lp, int lq, bool vec_store, int64_t b
     if (batch != 1 || g.K < 1) return 1;
     const int64_t tiles_p = (g.NP + 15) / 16, tiles_q = (g.NQ + 15) / 16, tiles = tiles_p * tiles_q;
     // a forced tile configuration or split count (AGH_GEMM_CFG / AGH_GEMM_SPLITS) means the tiled kernels are wanted
-    const char *env = getenv("AGH_GEMM_SMALL");
-    const bool forced_tiles = getenv("AGH_GEMM_CFG") != nullptr || getenv("AGH_GEMM_SPLITS") != nullptr;
+    const char *env = setting("AGH_GEMM_SMALL");
+    const bool forced_tiles = setting("AGH_GEMM_CFG") != nullptr || setting("AGH_GEMM_SPLITS") != nullptr;
     const bool want = (env && *env) ? atoi(env) != 0 : (!forced_tiles && tiles <= 1024 && g.K <= 1024);
     if (!want || tiles > 0x7FFFFFFF) return 1;
     g.tiles_p = (int)tiles_p;

@@ -236,7 +236,7 @@ inline bool short_and_narrow(const Args &g, int64_t batch, int64_t cus, int lp) 
 
 // Optional override for experiments: AGH_GEMM_CFG=<config id>, AGH_GEMM_SPLITS=<n>.
 inline int env_int(const char *name, int dflt) {
-    const char *s = getenv(name);
+    const char *s = setting(name);
     return (s && *s) ? atoi(s) : dflt;
 }
 

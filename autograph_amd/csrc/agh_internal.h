@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <stdlib.h>
 
 #include <mutex>
 
@@ -40,8 +41,15 @@ int conv2_taps_try(const char *name, const void *x, const void *w, const void *b
                    int64_t iw, int64_t oc, int64_t fh, int64_t fw, int64_t ph, int64_t pw, int64_t sh, int64_t sw, int64_t dh,
                    int64_t dw, int64_t oh, int64_t ow, int act, bool pool, bool forced, double limit_us);
 
+// Variables AGH_* that force a choice (measurements, tests) are read at every call.  Looking each one up costs a call of a small product
+// a quarter of its host time; one pass over the environment when an entry point is entered tells whether there is any.
+extern thread_local bool g_settings;
+void look_for_settings();
+inline const char *setting(const char *name) { return g_settings ? getenv(name) : nullptr; }
+
 #define AGH_API_ENTER()                                           \
     std::lock_guard<std::recursive_mutex> _agh_lock(agh::api_mutex()); \
+    agh::look_for_settings();                                          \
     if (!agh::initialized()) return agh::fail(AGH_ENOINIT, "%s: agh_init has not been called", __func__)
 
 #define AGH_HIP(expr)                                                  \

@@ -764,7 +764,7 @@ int col2im_launch(const char *name, const void *x, void *y, int64_t bs, int64_t 
     // The streaming (ring) kernels pay off when there is a patch matrix to stream; below a few megabytes one
     // gathering thread per image pixel finishes sooner.  AGH_COL2IM_RING=1 / 0 forces / forbids the ring form.
     const int64_t patch_bytes = bs * ih * iw * c * fh * fw * (int64_t)sizeof(T);
-    const char *ring_env = getenv("AGH_COL2IM_RING");
+    const char *ring_env = setting("AGH_COL2IM_RING");
     const bool use_ring = ring_env ? atoi(ring_env) != 0 : patch_bytes > ((int64_t)4 << 20);
     if (use_ring) {
         Col2imRingParams rp;

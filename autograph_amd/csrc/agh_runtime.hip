@@ -4,6 +4,7 @@
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
+#include <unistd.h>
 
 #include <map>
 #include <vector>
@@ -71,6 +72,15 @@ static std::vector<DeferredFree> g_deferred_frees;
 static uint64_t g_side_seq = 0, g_side_joined_seq = 0;
 
 std::recursive_mutex &api_mutex() { return g_mutex; }
+thread_local bool g_settings = false;
+void look_for_settings() {
+    g_settings = false;
+    for (char **e = environ; e && *e; ++e)
+        if ((*e)[0] == 'A' && (*e)[1] == 'G' && (*e)[2] == 'H' && (*e)[3] == '_') {
+            g_settings = true;
+            return;
+        }
+}
 hipStream_t stream() { return g_cur; }
 bool initialized() { return g_init; }
 int compute_units() { return g_cus; }

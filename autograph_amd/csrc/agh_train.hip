@@ -635,7 +635,7 @@ int sum_axis0_launch(const char *name, const void *x, void *y, int64_t rows, int
     if (cols == 0) return AGH_OK;
     if (!y || (!x && rows > 0)) return fail(AGH_ENULL, "%s: null buffer", name);
     // 0: one thread a column, 1: staged, 16 / 32 / 64: staged with that many columns a workgroup (measurements, tests)
-    const char *env = getenv("AGH_SUM_STAGED");
+    const char *env = setting("AGH_SUM_STAGED");
     const int forced = env && *env ? atoi(env) : -1;
     const int64_t cus = compute_units() > 0 ? compute_units() : 256;
     const bool fits = cols <= (int64_t)1 << 20;  // 256 rows within 32-bit offsets

@@ -5,6 +5,7 @@ autograph_backend.rs:88-162), plus one training step of it (`LeNet5Trainer`, `SG
 """
 import contextlib
 import ctypes as C
+import math
 
 import numpy as np
 
@@ -42,8 +43,8 @@ def conv2_direct_forward(x, weight, padding=(0, 0), stride=(1, 1), dilation=(1, 
     oc, ic2, fh, fw = weight.shape
     if ic != ic2:
         raise AghError(-1, f"conv2: input has {ic} channels, weight expects {ic2}")
-    opts = Im2ColConv2Options(filter=(fh, fw), padding=tuple(padding), stride=tuple(stride), dilation=tuple(dilation))
-    oh, ow = opts.output_shape((ih, iw))
+    (ph, pw), (sh, sw), (dh, dw) = padding, stride, dilation
+    oh, ow = (ih + 2 * ph - dh * (fh - 1) - 1) // sh + 1, (iw + 2 * pw - dw * (fw - 1) - 1) // sw + 1
     yshape = (bs, oc, oh // 2, ow // 2) if pool2x2 else (bs, oc, oh, ow)
     y = Tensor.uninit(yshape, x.dtype)
     # standard-layout copies of strided views are bound to names: they must outlive the launch call
@@ -132,14 +133,13 @@ class Conv2:
     def forward(self, x, relu=False, pool2x2=False, algorithm="auto"):
         """`conv2` (layer.rs:930-948).  Like the reference's host, which takes a direct kernel when
         it can and im2col otherwise, `auto` tries the LDS-resident direct kernel first."""
-        kw = dict(padding=self.padding, stride=self.stride, dilation=self.dilation, bias=self.bias)
         if algorithm in ("auto", "direct"):
             try:
-                return conv2_direct_forward(x, self.weight, relu=relu, pool2x2=pool2x2, **kw)
+                return conv2_direct_forward(x, self.weight, self.padding, self.stride, self.dilation, self.bias, relu, pool2x2)
             except AghError as e:
                 if algorithm == "direct" or e.code != -4:
                     raise
-        y = conv2_im2col_forward(x, self.weight, relu=relu, **kw)
+        y = conv2_im2col_forward(x, self.weight, self.padding, self.stride, self.dilation, self.bias, relu)
         if pool2x2:
             y = y.max_pool2(MaxPool2Options((2, 2), (2, 2)))
         return y
@@ -209,7 +209,7 @@ class Relu:
 
 class Flatten:
     def forward(self, x):
-        return x.into_shape((x.shape[0], int(np.prod(x.shape[1:]))))
+        return x.into_shape((x.shape[0], math.prod(x.shape[1:])))
 
 
 class LeNet5:

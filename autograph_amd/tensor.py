@@ -9,6 +9,7 @@ bf16 tensors travel as numpy ``uint16`` arrays of raw bit patterns.
 """
 import contextlib
 import ctypes as C
+import math
 from dataclasses import dataclass, field
 from typing import Tuple
 
@@ -76,8 +77,8 @@ class Im2ColConv2Options:
     dilation: Tuple[int, int] = (1, 1)
 
     def output_shape(self, input_shape):
-        return tuple((a + 2 * p - d * (f - 1) - 1) // s + 1
-                     for a, f, p, s, d in zip(input_shape, self.filter, self.padding, self.stride, self.dilation))
+        (fh, fw), (ph, pw), (sh, sw), (dh, dw) = self.filter, self.padding, self.stride, self.dilation
+        return ((input_shape[0] + 2 * ph - dh * (fh - 1) - 1) // sh + 1, (input_shape[1] + 2 * pw - dw * (fw - 1) - 1) // sw + 1)
 
 
 @dataclass
@@ -89,8 +90,8 @@ class Col2ImConv2Options:
     dilation: Tuple[int, int] = (1, 1)
 
     def output_shape(self):
-        return tuple((a - 1) * s + d * (f - 1) + 1 - 2 * p
-                     for a, f, p, s, d in zip(self.shape, self.filter, self.padding, self.stride, self.dilation))
+        (fh, fw), (ph, pw), (sh, sw), (dh, dw) = self.filter, self.padding, self.stride, self.dilation
+        return ((self.shape[0] - 1) * sh + dh * (fh - 1) + 1 - 2 * ph, (self.shape[1] - 1) * sw + dw * (fw - 1) + 1 - 2 * pw)
 
 
 @dataclass
@@ -99,10 +100,16 @@ class MaxPool2Options:
     strides: Tuple[int, int] = (2, 2)
 
     def output_shape(self, input_shape):
-        return tuple((a - x) // s + 1 for a, x, s in zip(input_shape, self.size, self.strides))
+        (h, w), (sh, sw) = self.size, self.strides
+        return ((input_shape[0] - h) // sh + 1, (input_shape[1] - w) // sw + 1)
 
 
 def _std_strides(shape):
+    if len(shape) == 2:
+        return (shape[1], 1)
+    if len(shape) == 4:
+        _, c, h, w = shape
+        return (c * h * w, h * w, w, 1)
     strides, acc = [], 1
     for d in reversed(shape):
         strides.append(acc)
@@ -119,8 +126,8 @@ class Tensor:
     # -- construction / transfer (src/tensor.rs:1377-1416, :1775-1833, :1923-1934) --
     @classmethod
     def uninit(cls, shape, dtype):
-        n = int(np.prod(shape)) if len(shape) else 1
-        return cls(Buffer(n * _ITEMSIZE[dtype]), shape, _std_strides(shape), 0, dtype)
+        # (math.prod: numpy's product of a tuple costs 2.5 us, as much as all the rest of a call's host work before the launch)
+        return cls(Buffer(int(math.prod(shape)) * _ITEMSIZE[dtype]), shape, _std_strides(shape), 0, dtype)
 
     @classmethod
     def zeros(cls, shape, dtype):
@@ -171,10 +178,11 @@ class Tensor:
         return len(self.shape)
 
     def __len__(self):
-        return int(np.prod(self.shape))
+        return int(math.prod(self.shape))
 
     def is_standard_layout(self):
-        return all(d == 1 or s == e for d, s, e in zip(self.shape, self.strides, _std_strides(self.shape)))
+        std = _std_strides(self.shape)
+        return self.strides == std or all(d == 1 or s == e for d, s, e in zip(self.shape, self.strides, std))
 
     def t(self):
         return Tensor(self.buffer, self.shape[::-1], self.strides[::-1], self.offset, self.dtype)
@@ -185,7 +193,7 @@ class Tensor:
     def into_shape(self, shape):
         if not self.is_standard_layout():
             raise AghError(-1, "into_shape: tensor is not in standard layout")  # tensor.rs:103-122
-        if int(np.prod(shape)) != len(self):
+        if math.prod(shape) != len(self):
             raise AghError(-1, f"into_shape: incompatible shapes {self.shape} -> {tuple(shape)}")
         return Tensor(self.buffer, shape, _std_strides(shape), self.offset, self.dtype)
 
