@@ -221,10 +221,9 @@ __global__ __launch_bounds__(WGP *WGQ * 64, DEPTH > 0 ? 2 : 1) void gemm_bf16_dl
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wp = wave % WGP, wq = wave / WGP;
-    int tp, tq;
-    tile_coords(blockIdx.x, g.tiles_p, g.tiles_q, tp, tq);
+    int tp, tq, split;
+    tile_coords(g, tp, tq, split);
     const int p0 = tp * BP, q0 = tq * BQ;
-    const int split = blockIdx.y;
     const int kbeg = split * g.k_per_split;
     const int kend = min(g.K, kbeg + g.k_per_split);
     // whole k-tiles; depth of a shorter last one (the last split's only).  DEPTH > 0: all k-tiles, the last one of all

@@ -84,10 +84,9 @@ __global__ __launch_bounds__(256 * KS) void gemm_f32_dl_kernel(Args g) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wp = wave & 1, wq = (wave >> 1) & 1;
     const int kh = wave >> 2;  // which half of every k-tile's substeps (KS == 2)
-    int tp, tq;
-    tile_coords(blockIdx.x, g.tiles_p, g.tiles_q, tp, tq);
+    int tp, tq, split;
+    tile_coords(g, tp, tq, split);
     const int p0 = tp * BP, q0 = tq * BQ;
-    const int split = blockIdx.y;
     const int kbeg = split * g.k_per_split;
     const int kend = min(g.K, kbeg + g.k_per_split);
     const int KT = kend > kbeg ? (kend - kbeg) / BK : 0;   // whole k-tiles

@@ -282,10 +282,7 @@ template <> struct Mma<float> {
 // Workgroups are dealt round-robin to the 8 XCDs, each with its own L2.  Give every XCD a
 // contiguous run of tile ids, and walk tiles in panels of GROUP_P tile rows so that tiles
 // running together on an XCD share operand panels.
-__device__ __forceinline__ void tile_coords(int bid, int tiles_p, int tiles_q, int &tp, int &tq) {
-    const int nb = tiles_p * tiles_q;
-    int id = bid;
-    if ((nb & 7) == 0) id = (bid & 7) * (nb >> 3) + (bid >> 3);
+__device__ __forceinline__ void tile_walk(int id, int tiles_p, int tiles_q, int &tp, int &tq) {
     constexpr int GROUP_P = 8;
     const int per_group = GROUP_P * tiles_q;
     const int group = id / per_group;
@@ -294,6 +291,25 @@ __device__ __forceinline__ void tile_coords(int bid, int tiles_p, int tiles_q, i
     const int in_group = id - group * per_group;
     tp = first_p + in_group % gsz;
     tq = in_group / gsz;
+}
+// In split-K the run goes through the tiles of one split before the next split's: the tiles that an XCD works on together then
+// read the same k range, so a panel enters its L2 once (dense backward bf16 4096x2048x1000 72.3 -> 70.3 us; f32 128x50176x576 in 14 splits 77.5 ->
+// 75.4).
+__device__ __forceinline__ void tile_coords(const Args &g, int &tp, int &tq, int &split) {
+    const int tiles = g.tiles_p * g.tiles_q;
+    int id = blockIdx.x;
+    split = blockIdx.y;
+    if (gridDim.y > 1) {
+        const int n = tiles * (int)gridDim.y;
+        id += split * tiles;
+        const int xcd = id & 7;
+        id = xcd * (n >> 3) + min(xcd, n & 7) + (id >> 3);
+        split = id / tiles;
+        id -= split * tiles;
+    } else if ((tiles & 7) == 0) {
+        id = (id & 7) * (tiles >> 3) + (id >> 3);
+    }
+    tile_walk(id, g.tiles_p, g.tiles_q, tp, tq);
 }
 
 // ------------------------------------------------------------ epilogue ----
@@ -409,10 +425,9 @@ __global__ __launch_bounds__(WGP *WGQ * 64) void gemm_kernel(Args g) {
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int wp = wave % WGP, wq = wave / WGP;
-    int tp, tq;
-    tile_coords(blockIdx.x, g.tiles_p, g.tiles_q, tp, tq);
+    int tp, tq, split;
+    tile_coords(g, tp, tq, split);
     const int p0 = tp * BP, q0 = tq * BQ;
-    const int split = blockIdx.y;
     const int kbeg = split * g.k_per_split;
     const int kend = min(g.K, kbeg + g.k_per_split);
     const int KT = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
