@@ -3,6 +3,7 @@
 #define AGH_GEMM_WITH_F32_SMALL
 #include "agh_gemm_f32_dl.h"
 #include "agh_gemm_f32_small.h"
+#include "agh_gemm_f32_stream.h"
 #include "agh_gemm_host.h"
 
 extern "C" {

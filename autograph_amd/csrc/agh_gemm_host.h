@@ -118,6 +118,23 @@ int launch_f32_dl(const Args &g, int splits) {
 }
 #endif
 
+#ifdef AGH_GEMM_WITH_F32_DIRECT
+// two workgroups per CU over all tiles (agh_gemm_f32_stream.h)
+template <int LP, int LQ>
+int launch_f32_stream(const Args &g, int cus) {
+    auto kern = gemm_f32_stream_kernel<LP, LQ>;
+    constexpr size_t smem = F32StreamGeo<LP, LQ>::SMEM_BYTES;
+    static bool attr_done = false;
+    if (!attr_done) {
+        AGH_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+        attr_done = true;
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)((cus + 7) / 8 * 8 * kStreamPerCu)), dim3(512), smem, stream(), g);
+    AGH_LAUNCH_CHECK("gemm (f32 stream) kernel launch");
+    return AGH_OK;
+}
+#endif
+
 template <typename T, int BP, int BQ, int WGP, int WGQ, bool SCALAR_OK>
 int launch_loaders(const Args &g, int splits, int lp, int lq, bool direct, bool any) {
 #ifdef AGH_GEMM_WITH_F32_DIRECT
@@ -317,6 +334,31 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
     if constexpr (sizeof(T) == 4) {
         const int rc = gemm_f32_small_try(g, lp, lq, vec_store, batch);
         if (rc != 1) return rc;
+    }
+#endif
+
+#ifdef AGH_GEMM_WITH_F32_DIRECT
+    if constexpr (sizeof(T) == 4) {
+        // Short k and a tile for every CU at least: two workgroups per CU over all tiles.  Over 400 products of 64 to 120000 x 8 to 1200 x 16 to
+        // 8192, of those the rule takes 4 are more than 3 % behind the kernels of one tile a workgroup, 6 % at most (49690 x 256 x 112
+        // 40.7 / 43.3 us), all together 1.2 times as fast (3883 x 300 x 3092 92.9 / 73.3; 4758 x 32 x 416 11.1 / 8.0).  From k = 320 on a tile's
+        // own k-tiles hide most of what is gained (384 to 512: 0.95 to 1.14); up to 32 columns of C the 32 x 128 tile has less padding (94418 x
+        // 196 x 16 20.5 / 41.7).  AGH_GEMM_STREAM=0|1 overrides.
+        const int64_t tiles_p = (g.NP + kStreamBP - 1) / kStreamBP, tiles_q = (g.NQ + kStreamBQ - 1) / kStreamBQ;
+        const bool can = batch == 1 && !any_scalar && g.K > 0 && beta == 0.0f && !bias && act == AGH_ACT_NONE && g.dp == 1 && g.dq > 0 &&
+                         g.dq < (1 << 24) && tiles_p * tiles_q * ((g.K + 31) / 32) < 0x7FFFFFFF && env_int("AGH_GEMM_DIRECT", 1) != 0;
+        const bool suits = g.K <= 256 && g.NP > 32 && g.NQ > 64 && tiles_p * tiles_q >= cus && forced_cfg < 0 && !setting("AGH_GEMM_SPLITS");
+        if (can && env_int("AGH_GEMM_STREAM", suits) != 0) {
+            g.tiles_p = (int)tiles_p;
+            g.tiles_q = (int)tiles_q;
+            switch (lp * 3 + lq) {
+                case LD_K * 3 + LD_K: return launch_f32_stream<LD_K, LD_K>(g, cus);
+                case LD_K * 3 + LD_R: return launch_f32_stream<LD_K, LD_R>(g, cus);
+                case LD_R * 3 + LD_K: return launch_f32_stream<LD_R, LD_K>(g, cus);
+                case LD_R * 3 + LD_R: return launch_f32_stream<LD_R, LD_R>(g, cus);
+                default: break;
+            }
+        }
     }
 #endif
 

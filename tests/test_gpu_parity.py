@@ -1314,3 +1314,40 @@ def test_relu_reference_cases(ag, dtype):
     sp = to_dtype(np.array([[-0.0, np.nan, np.inf, -np.inf, 1e-30, -1e-30]], dtype=np.float32), dtype)
     got = ag.Tensor.from_array(sp).relu().into_array()
     assert np.array_equal(got.view(np.uint8), orc.relu(sp).view(np.uint8))
+
+
+@pytest.mark.parametrize("ta", [False, True])
+@pytest.mark.parametrize("tb", [False, True])
+def test_gemm_f32_stream_over_tiles(ag, monkeypatch, ta, tb):
+    """f32 products of short k and many tiles in two workgroups per CU (agh_gemm_f32_stream.h): edges of the 64 x 128 tile, one to
+    many tiles a workgroup, fewer tiles than workgroups, k-tiles of 1 to 32, k of one to nine k-tiles, row pitches of C beyond its
+    columns (nothing else is written), alpha; NaN behind the operands' ends.  Against float64 within the bound of a sum of k
+    products in any order, gamma_k |A||B| (k <= 288: 288 x 2^-24 = 1.8e-5), and bit for bit the kernel of one tile a workgroup
+    where both add k in order."""
+    rng = np.random.default_rng(11)
+    for m, k, n, pad in ((1, 4, 4, 0), (128, 32, 64, 0), (129, 36, 68, 4), (127, 8, 60, 3), (1000, 128, 576, 0), (4100, 64, 132, 1), (300, 288, 260, 0),
+                         (40000, 32, 64, 0), (2500, 260, 700, 5), (8320, 4, 1088, 0)):
+        if ta and m % 4 or not ta and k % 4:
+            m = -(-m // 4) * 4
+        pad_a = rng.standard_normal((k, m) if ta else (m, k)).astype(np.float32)
+        pad_b = rng.standard_normal((n, k) if tb else (k, n)).astype(np.float32)
+        a, b = [ag.Tensor.from_array(np.concatenate([x.reshape(-1), np.full(64, np.nan, np.float32)])) for x in (pad_a, pad_b)]
+        a = ag.Tensor(a.buffer, pad_a.shape, ag.tensor._std_strides(pad_a.shape), 0, "f32")
+        b = ag.Tensor(b.buffer, pad_b.shape, ag.tensor._std_strides(pad_b.shape), 0, "f32")
+        a, b = a.t() if ta else a, b.t() if tb else b
+        ha, hb = (pad_a.T if ta else pad_a).astype(np.float64), (pad_b.T if tb else pad_b).astype(np.float64)
+        got = {}
+        for stream in ("1", "0"):
+            monkeypatch.setenv("AGH_GEMM_STREAM", stream)
+            monkeypatch.setenv("AGH_GEMM_SMALL", "0")
+            monkeypatch.setenv("AGH_GEMM_KSPLIT", "0")
+            monkeypatch.setenv("AGH_GEMM_SPLITS", "1")
+            c = ag.Tensor.from_array(np.full((m, n + pad), 7.0, np.float32))
+            ag.gemm(0.5, a, b, 0.0, ag.Tensor(c.buffer, (m, n), (n + pad, 1), 0, "f32"))
+            out = c.into_array()
+            assert (out[:, n:] == 7.0).all(), (m, k, n)
+            got[stream] = out[:, :n]
+        err = np.abs(got["1"] - 0.5 * (ha @ hb))
+        assert (err <= k * 2.0 ** -24 * (0.5 * (np.abs(ha) @ np.abs(hb))) + 2.0 ** -24 * np.abs(ha @ hb)).all(), (m, k, n)
+        if not pad:
+            assert np.array_equal(got["1"], got["0"]), (m, k, n)
