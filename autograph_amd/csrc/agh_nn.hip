@@ -428,6 +428,7 @@ __host__ __device__ constexpr int col2im_pad_segments(int F, int S, int pw) {
 }
 
 constexpr int kCol2imPrefetch = 32;  // 32-bit words a thread holds for the next step
+constexpr int kCol2imPrefetchWide = 64;  // where a patch row is more than 256 threads hold in those
 
 template <typename T>
 __global__ __launch_bounds__(kThreads) void col2im_ring_kernel(const T *__restrict__ x, T *__restrict__ y,
@@ -546,11 +547,18 @@ __global__ __launch_bounds__(kThreads) void col2im_ring_kernel(const T *__restri
 // Workgroup ids are dealt round-robin to the 8 XCDs, each with an L2 of its own; the chunks of one
 // (image, band) share cache lines where their segments meet, so they are given ids 8 apart: same
 // XCD, dispatched together.
-template <typename T, int F, int S>
+//
+// WORDS: words a thread holds for the next step.  The least number of channels whose segments are whole 16-byte vectors (8 in bf16, 4 in
+// f32) of 5x5 patches fills 32 words a thread at 81 patches a row, of 7x7 at 41; wider rows have a form with 64 (two workgroups a CU
+// for their LDS), up to 163 and 83.  The general kernel there / this one in us: bf16 93 x 64 channels, 36 x 83 patches of 5x5 877 / 468,
+// 40 x 64, 60 x 60 of 7x7 660 / 333, 20 x 16, 50 x 50 of 7x7 at stride 2 130 / 71, f32 25 x 64, 60 x 60 of 7x7 864 / 415, 30 x 64, 48 x 83 of
+// 5x5 at stride 2 766 / 320, 20 x 32, 100 x 100 of 5x5 351 / 350; f32 16 x 64, 50 x 112 of 5x5 248 / 262, so f32 5x5 rows of more than
+// 102 patches at stride 1 stay with the general kernel.
+template <typename T, int F, int S, int WORDS>
 __global__ __launch_bounds__(kThreads) void col2im_ring_unit_kernel(const T *__restrict__ x, T *__restrict__ y,
                                                                      Col2imRingParams p) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    constexpr int PFV = kCol2imPrefetch / 4;  // 16-byte vectors a thread holds for the next step
+    constexpr int PFV = WORDS / 4;  // 16-byte vectors a thread holds for the next step
     constexpr int EPW = 4 / (int)sizeof(T);
     constexpr int NCOL = 4;                   // pixel columns per thread (cc*iw <= NCOL*kThreads)
     const int tid = threadIdx.x;
@@ -681,7 +689,7 @@ __global__ __launch_bounds__(kThreads) void col2im_ring_unit_kernel(const T *__r
 
 // Picks the chunk/band split of the streaming kernel; false when the geometry does not fit.
 template <typename T>
-bool col2im_ring_plan(Col2imRingParams &p, size_t &smem, int64_t &nblocks, bool unit, const void *x, int64_t bs, int64_t c,
+bool col2im_ring_plan(Col2imRingParams &p, size_t &smem, int64_t &nblocks, bool unit, int words, const void *x, int64_t bs, int64_t c,
                       int64_t gh, int64_t gw, int64_t ih, int64_t iw, int64_t fh, int64_t fw, int64_t ph, int64_t pw,
                       int64_t sh, int64_t sw, int64_t dh, int64_t dw) {
     constexpr int64_t es = sizeof(T), epw = 4 / es;
@@ -691,23 +699,23 @@ bool col2im_ring_plan(Col2imRingParams &p, size_t &smem, int64_t &nblocks, bool 
     if (unit && (((uintptr_t)x & 15) != 0 || (ktot * es) % 16 != 0)) return false;
     const int64_t segs = unit ? gw + 2 * col2im_pad_segments((int)fw, (int)sw, (int)pw) : gw;
     const int64_t rh = (fh - 1) * dh + 1;
-    constexpr int64_t kLdsBudget = 48 * 1024;
+    const int64_t budget = words > kCol2imPrefetch ? 76 * 1024 : 48 * 1024;
     int64_t cc = 0, lds = 0, pitch = 0, nrows = 1;
     for (int64_t d = c; d >= 1; --d) {
         if (c % d != 0 || (d * ff) % epw != 0) continue;
         if (unit && ((d * ff * es) % 16 != 0 || d * iw > 4 * kThreads)) continue;
         const int64_t lw = d * ff / epw;
-        if (gw * lw > (int64_t)kThreads * kCol2imPrefetch) continue;
+        if (gw * lw > (int64_t)kThreads * words) continue;
         const int64_t pitchw = lw | 1;  // odd: threads of a wave walk patches, i.e. whole pitches
         int64_t need = rh * d * iw * 4 + segs * pitchw * 4;
         if (unit) {
             // as many patch rows per step as the prefetch registers and 40 KB of LDS hold
             const int64_t per_row = (gw * (lw / 4) + kThreads - 1) / kThreads;
-            nrows = std::max<int64_t>(1, std::min<int64_t>({(int64_t)(kCol2imPrefetch / 4) / per_row, gh,
+            nrows = std::max<int64_t>(1, std::min<int64_t>({(int64_t)(words / 4) / per_row, gh,
                                                              (40 * 1024) / (segs * pitchw * 4)}));
             need = nrows * segs * pitchw * 4;
         }
-        if (need > kLdsBudget) continue;
+        if (need > budget) continue;
         cc = d; lds = need; pitch = pitchw * epw;
         break;
     }
@@ -743,6 +751,19 @@ bool col2im_ring_plan(Col2imRingParams &p, size_t &smem, int64_t &nblocks, bool 
     return true;
 }
 
+template <typename T, int F, int S>
+int col2im_wide_launch(const char *name, size_t smem, int64_t nblocks, const void *x, void *y, const Col2imRingParams &rp) {
+    auto kernel = col2im_ring_unit_kernel<T, F, S, kCol2imPrefetchWide>;
+    static bool attr_done = false;
+    if (!attr_done) {
+        AGH_HIP(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 76 * 1024));
+        attr_done = true;
+    }
+    hipLaunchKernelGGL(kernel, dim3((unsigned)nblocks), dim3(kThreads), smem, stream(), (const T *)x, (T *)y, rp);
+    AGH_LAUNCH_CHECK(name);
+    return AGH_OK;
+}
+
 template <typename T>
 int col2im_launch(const char *name, const void *x, void *y, int64_t bs, int64_t c, int64_t ih, int64_t iw,
                   int64_t fh, int64_t fw, int64_t ph, int64_t pw, int64_t sh, int64_t sw, int64_t dh, int64_t dw) {
@@ -775,18 +796,27 @@ int col2im_launch(const char *name, const void *x, void *y, int64_t bs, int64_t 
         auto launch = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3((unsigned)nblocks), dim3(kThreads), smem, stream(), (const T *)x, (T *)y, rp);
         };
-        if (unit_geom && col2im_ring_plan<T>(rp, smem, nblocks, true, x, bs, c, ih, iw, oh, ow, fh, fw, ph, pw, sh, sw, dh, dw)) {
+        if (unit_geom && col2im_ring_plan<T>(rp, smem, nblocks, true, kCol2imPrefetch, x, bs, c, ih, iw, oh, ow, fh, fw, ph, pw, sh, sw, dh, dw)) {
             switch (fh * 2 + sh - 1) {
 #define AGH_C2I(FV) \
-    case FV * 2: launch(col2im_ring_unit_kernel<T, FV, 1>); break; \
-    case FV * 2 + 1: launch(col2im_ring_unit_kernel<T, FV, 2>); break
+    case FV * 2: launch(col2im_ring_unit_kernel<T, FV, 1, kCol2imPrefetch>); break; \
+    case FV * 2 + 1: launch(col2im_ring_unit_kernel<T, FV, 2, kCol2imPrefetch>); break
                 AGH_C2I(1); AGH_C2I(2); AGH_C2I(3); AGH_C2I(5); AGH_C2I(7);
 #undef AGH_C2I
             }
             AGH_LAUNCH_CHECK(name);
             return AGH_OK;
         }
-        if (col2im_ring_plan<T>(rp, smem, nblocks, false, x, bs, c, ih, iw, oh, ow, fh, fw, ph, pw, sh, sw, dh, dw)) {
+        if (unit_geom && fh >= 5 && !(sizeof(T) == 4 && fh == 5 && sh == 1 && iw > 102) &&
+            col2im_ring_plan<T>(rp, smem, nblocks, true, kCol2imPrefetchWide, x, bs, c, ih, iw, oh, ow, fh, fw, ph, pw, sh, sw, dh, dw)) {
+            switch (fh * 2 + sh - 1) {
+                case 10: return col2im_wide_launch<T, 5, 1>(name, smem, nblocks, x, y, rp);
+                case 11: return col2im_wide_launch<T, 5, 2>(name, smem, nblocks, x, y, rp);
+                case 14: return col2im_wide_launch<T, 7, 1>(name, smem, nblocks, x, y, rp);
+                default: return col2im_wide_launch<T, 7, 2>(name, smem, nblocks, x, y, rp);
+            }
+        }
+        if (col2im_ring_plan<T>(rp, smem, nblocks, false, kCol2imPrefetch, x, bs, c, ih, iw, oh, ow, fh, fw, ph, pw, sh, sw, dh, dw)) {
             launch(col2im_ring_kernel<T>);
             AGH_LAUNCH_CHECK(name);
             return AGH_OK;

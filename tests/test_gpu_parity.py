@@ -1351,3 +1351,18 @@ def test_gemm_f32_stream_over_tiles(ag, monkeypatch, ta, tb):
         assert (err <= k * 2.0 ** -24 * (0.5 * (np.abs(ha) @ np.abs(hb))) + 2.0 ** -24 * np.abs(ha @ hb)).all(), (m, k, n)
         if not pad:
             assert np.array_equal(got["1"], got["0"]), (m, k, n)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("c,gh,gw,f,s,p", [(8, 3, 82, 5, 1, 2), (16, 7, 83, 5, 1, 0), (8, 4, 102, 5, 1, 1), (8, 4, 103, 5, 1, 2), (8, 5, 128, 5, 1, 4),
+                                           (8, 9, 42, 7, 1, 3), (16, 4, 60, 7, 1, 0), (8, 9, 83, 7, 1, 6), (8, 3, 84, 7, 1, 3), (8, 6, 64, 5, 2, 2),
+                                           (8, 5, 62, 7, 2, 3), (4, 6, 110, 5, 2, 1)])
+def test_col2im_rows_wider_than_a_step(ag, monkeypatch, dtype, c, gh, gw, f, s, p):
+    """Patch rows that fill more than 32 words a thread: 5x5 from 82 patches a row on, 7x7 from 42, up to the end of the 64-word form and one
+    beyond, stride 2, padding up to f - 1: bit for bit the oracle (the order of additions is the same in every form)."""
+    monkeypatch.setenv("AGH_COL2IM_RING", "1")
+    rng = np.random.default_rng(gw)
+    x = to_dtype(rng.standard_normal((2 * gh * gw, c * f * f)), dtype)
+    opts = ag.Col2ImConv2Options(shape=(gh, gw), filter=(f, f), padding=(p, p), stride=(s, s))
+    got = ag.Tensor.from_array(x).col2im_conv2(opts).into_array()
+    assert np.array_equal(got, orc.col2im_conv2(x, (gh, gw), (f, f), (p, p), (s, s), (1, 1)))
