@@ -222,7 +222,7 @@ __global__ __launch_bounds__(WGP *WGQ * 64, DEPTH > 0 ? 2 : 1) void gemm_bf16_dl
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wp = wave % WGP, wq = wave / WGP;
     int tp, tq, split;
-    tile_coords(g, tp, tq, split);
+    tile_coords<DEPTH == 0>(g, tp, tq, split);
     const int p0 = tp * BP, q0 = tq * BQ;
     const int kbeg = split * g.k_per_split;
     const int kend = min(g.K, kbeg + g.k_per_split);

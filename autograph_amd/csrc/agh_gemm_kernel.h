@@ -295,11 +295,13 @@ __device__ __forceinline__ void tile_walk(int id, int tiles_p, int tiles_q, int 
 // In split-K the run goes through the tiles of one split before the next split's: the tiles that an XCD works on together then
 // read the same k range, so a panel enters its L2 once (dense backward bf16 4096x2048x1000 72.3 -> 70.3 us; f32 128x50176x576 in 14 splits 77.5 ->
 // 75.4).
+// (RUNS false: not for the any-address kernel, whose unsplit launches it would cost 0.7 %.)
+template <bool RUNS = true>
 __device__ __forceinline__ void tile_coords(const Args &g, int &tp, int &tq, int &split) {
     const int tiles = g.tiles_p * g.tiles_q;
     int id = blockIdx.x;
     split = blockIdx.y;
-    if (gridDim.y > 1) {
+    if (RUNS && g.store_mode == ST_SPLITK) {
         const int n = tiles * (int)gridDim.y;
         id += split * tiles;
         const int xcd = id & 7;
