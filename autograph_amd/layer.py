@@ -356,7 +356,7 @@ class LeNet5Trainer:
         # in place of nine; the weight gradients are the same GEMMs either way
         self.fused_backward = fused_backward
         # overlap: issue the weight gradients on the second stream beside the input-gradient chain.  Default: only for the
-        # layer-by-layer backward pass; with the one-launch forms a step is six kernels, and the fork and join of a second
+        # layer-by-layer backward pass; with the one-launch forms a step is five kernels, and the fork and join of a second
         # stream cost more (about 10 us) than the one launch they would hide
         if overlap is None:
             overlap = not fused_backward
@@ -504,17 +504,20 @@ class LeNet5Trainer:
                 self.logits._ptr(), target.ptr, 1.0, self.c1._ptr(), self.c2._ptr(), self.d1._ptr(), self.d2._ptr(),
                 w2._data_ptr(), wd1._data_ptr(), wd2._data_ptr(), wd3._data_ptr(), self.g_logits._ptr(), self.g_d2._ptr(),
                 self.g_d1._ptr(), self.gm2._ptr(), self.gm1._ptr(), bs))
-            # everything below only waits for that launch: the dense layers' weight gradients, the bias gradient and the
-            # loss are one launch on the second stream, the convolutions' weight gradients (formed without patch
-            # matrices) two on the first
-            with self._branch():
-                check(self._fn("agh_lenet5_dense_weight_grads")(
-                    self.a2._ptr(), self.a1._ptr(), f._data_ptr(), self.g_logits._ptr(), self.g_d2._ptr(), self.g_d1._ptr(),
-                    dwd3._data_ptr(), dwd2._data_ptr(), dwd1._data_ptr(), db3._data_ptr(), self.logits._ptr(), target.ptr,
-                    self._loss_host, bs))
-            check(self._fn("agh_lenet5_conv_weight_grads")(x._data_ptr(), self.p1._ptr(), self.gm1._ptr(), self.gm2._ptr(),
-                                                           dw1._data_ptr(), dw2._data_ptr(), bs))
-            join()
+            # everything below only waits for that launch: the dense layers' weight gradients, the bias gradient, the loss and the
+            # images' shares of the convolutions' weight gradients (formed without patch matrices) are one launch, the sum of those
+            # shares another; with `overlap` the first part goes to the second stream
+            dense = (self.a2._ptr(), self.a1._ptr(), f._data_ptr(), self.g_logits._ptr(), self.g_d2._ptr(), self.g_d1._ptr(),
+                     dwd3._data_ptr(), dwd2._data_ptr(), dwd1._data_ptr(), db3._data_ptr(), self.logits._ptr(), target.ptr,
+                     self._loss_host)
+            conv = (x._data_ptr(), self.p1._ptr(), self.gm1._ptr(), self.gm2._ptr(), dw1._data_ptr(), dw2._data_ptr())
+            if self._branch is branch:
+                with branch():
+                    check(self._fn("agh_lenet5_dense_weight_grads")(*dense, bs))
+                check(self._fn("agh_lenet5_conv_weight_grads")(*conv, bs))
+                join()
+            else:
+                check(self._fn("agh_lenet5_weight_grads")(*dense, *conv, bs))
         else:
             check(self._fn("agh_cross_entropy_backward")(self.logits._ptr(), target.ptr, 1.0, self.g_logits._ptr(), bs, 10))
             gemm(1.0, self.g_logits, wd3.t(), 0.0, self.g_a2)

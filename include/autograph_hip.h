@@ -339,6 +339,16 @@ int agh_lenet5_conv_weight_grads_f32(const void *x, const void *p1, const void *
 int agh_lenet5_conv_weight_grads_bf16(const void *x, const void *p1, const void *gm1, const void *gm2, void *dw1, void *dw2,
                                       int64_t bs);
 
+/* Both of the above (same values, same bits) with the dense layers' gradients and the images' partial sums in one launch. */
+int agh_lenet5_weight_grads_f32(const void *a2, const void *a1, const void *f, const void *g_logits, const void *g_d2,
+                                const void *g_d1, void *dwd3, void *dwd2, void *dwd1, void *db3, const void *logits,
+                                const void *target, void *loss, const void *x, const void *p1, const void *gm1, const void *gm2,
+                                void *dw1, void *dw2, int64_t bs);
+int agh_lenet5_weight_grads_bf16(const void *a2, const void *a1, const void *f, const void *g_logits, const void *g_d2,
+                                 const void *g_d1, void *dwd3, void *dwd2, void *dwd1, void *db3, const void *logits,
+                                 const void *target, void *loss, const void *x, const void *p1, const void *gm1, const void *gm2,
+                                 void *dw1, void *dw2, int64_t bs);
+
 /* ---------------------------------------------------------------- max pool ---- */
 
 /* MaxPool2 device branch (src/tensor/ops.rs:1117-1133; rule from the host impl

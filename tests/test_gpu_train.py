@@ -392,6 +392,25 @@ def test_lenet5_backward_one_launch_against_the_separate_launches(ag, dtype):
             assert np.abs(g - w).max() <= 2.0**-6 * scale and np.abs(g - w).mean() <= 2.0**-11 * scale, name
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("bs", [1, 3, 100, 128, 129, 257])
+def test_lenet5_weight_grads_in_one_launch(ag, dtype, bs):
+    """agh_lenet5_weight_grads_<T> against the two entries it joins: every gradient and the loss bit for bit, at batches around the
+    128 rows of a pass and the 200 of the bias gradient's."""
+    rng = np.random.default_rng(bs)
+    params = [to_dtype(p, dtype) for p in lenet_params(rng)]
+    x = to_dtype(rng.uniform(0, 1, (bs, 1, 28, 28)), dtype)
+    tx, tt = ag.Tensor.from_array(x), labels(ag, rng.integers(0, 10, bs).astype(np.uint8))
+    out = {}
+    for overlap in (False, True):  # one launch / the dense layers' entry beside the convolutions'
+        tr = ag.LeNet5Trainer(ag.LeNet5.from_arrays(*params), bs, optimizer=ag.SGD(None), overlap=overlap)
+        tr.step(tx, tt)
+        ag._ffi.check(ag.lib.agh_sync())
+        out[overlap] = [g.into_array() for g in tr.grads] + [np.float32(tr.loss())]
+    for a, b in zip(out[False], out[True]):
+        assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("fused_backward", [True, False])
 @pytest.mark.parametrize("fused_forward", [True, False])
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
