@@ -104,6 +104,11 @@ class MaxPool2Options:
         return ((input_shape[0] - h) // sh + 1, (input_shape[1] - w) // sw + 1)
 
 
+def _dims(shape):
+    """The dimensions as Python integers: products of them must not wrap, as those of 8-, 16- or 32-bit numpy integers do."""
+    return tuple(map(int, shape))
+
+
 def _std_strides(shape):
     if len(shape) == 2:
         return (shape[1], 1)
@@ -121,13 +126,14 @@ class Tensor:
     """`TensorBase` = {dim, strides, buffer, offset} (src/tensor.rs:327-332) on the device."""
 
     def __init__(self, buffer, shape, strides, offset, dtype):
-        self.buffer, self.shape, self.strides, self.offset, self.dtype = buffer, tuple(shape), tuple(strides), offset, dtype
+        self.buffer, self.shape, self.strides, self.offset, self.dtype = buffer, _dims(shape), tuple(strides), offset, dtype
 
     # -- construction / transfer (src/tensor.rs:1377-1416, :1775-1833, :1923-1934) --
     @classmethod
     def uninit(cls, shape, dtype):
         # (math.prod: numpy's product of a tuple costs 2.5 us, as much as all the rest of a call's host work before the launch)
-        return cls(Buffer(int(math.prod(shape)) * _ITEMSIZE[dtype]), shape, _std_strides(shape), 0, dtype)
+        shape = _dims(shape)
+        return cls(Buffer(math.prod(shape) * _ITEMSIZE[dtype]), shape, _std_strides(shape), 0, dtype)
 
     @classmethod
     def zeros(cls, shape, dtype):
@@ -178,7 +184,7 @@ class Tensor:
         return len(self.shape)
 
     def __len__(self):
-        return int(math.prod(self.shape))
+        return math.prod(self.shape)
 
     def is_standard_layout(self):
         std = _std_strides(self.shape)
@@ -193,8 +199,9 @@ class Tensor:
     def into_shape(self, shape):
         if not self.is_standard_layout():
             raise AghError(-1, "into_shape: tensor is not in standard layout")  # tensor.rs:103-122
+        shape = _dims(shape)
         if math.prod(shape) != len(self):
-            raise AghError(-1, f"into_shape: incompatible shapes {self.shape} -> {tuple(shape)}")
+            raise AghError(-1, f"into_shape: incompatible shapes {self.shape} -> {shape}")
         return Tensor(self.buffer, shape, _std_strides(shape), self.offset, self.dtype)
 
     def slice_rows(self, start, stop, step=1):

@@ -3,6 +3,10 @@ header declares, and argument errors come back as status codes without a GPU."""
 import ctypes as C
 import os
 import re
+import types
+
+import numpy as np
+import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -43,6 +47,28 @@ def test_option_shape_formulas():
     c = Col2ImConv2Options(shape=(5, 6), filter=(3, 5), padding=(1, 0), stride=(2, 1), dilation=(1, 2))
     assert c.output_shape() == (orc.col2im_out(5, 3, 1, 2, 1), orc.col2im_out(6, 5, 0, 1, 2))
     assert MaxPool2Options((2, 3), (2, 2)).output_shape((9, 8)) == (orc.pool_out(9, 2, 2), orc.pool_out(8, 3, 2))
+
+
+@pytest.mark.parametrize("shape", [(np.int16(300), np.int16(300)), (np.uint8(28), np.uint8(28)), (100, np.int16(1000)),
+                                   (np.int32(802816), np.int32(3200)), (np.int8(100),) * 3, (np.int16(100),) * 4, np.array([200, 200], np.uint8)])
+def test_narrow_integers_as_dimensions(monkeypatch, shape):
+    """8-, 16- and 32-bit numpy integers as dimensions: allocated size, length, strides and reshapes are those of the same Python integers
+    (products of such numbers wrap; no device: the allocation is only recorded)."""
+    from autograph_amd import tensor
+    sizes = []
+    monkeypatch.setattr(tensor, "Buffer", lambda nbytes: sizes.append(nbytes) or types.SimpleNamespace(ptr=0, nbytes=nbytes))
+    dims = tuple(int(d) for d in shape)
+    want = 1
+    for d in dims:
+        want *= d
+    for dtype, size in (("f32", 4), ("bf16", 2)):
+        t = tensor.Tensor.uninit(shape, dtype)
+        assert sizes.pop() == size * want and t.shape == dims and all(type(d) is int for d in t.shape)
+        assert len(t) == want and t.strides == tensor._std_strides(dims) and t.is_standard_layout()
+        assert t.into_shape((want,)).into_shape(shape).strides == t.strides
+        assert len(tensor.Tensor(t.buffer, shape, t.strides, 0, dtype)) == want
+    with pytest.raises(tensor.AghError):
+        t.into_shape((want + 1,))
 
 
 _C_TO_RUST = {"int": "c_int", "int64_t": "i64", "float": "f32", "size_t": "usize", "char": "c_char", "void": "c_void"}
