@@ -41,15 +41,16 @@ int conv2_taps_try(const char *name, const void *x, const void *w, const void *b
                    int64_t iw, int64_t oc, int64_t fh, int64_t fw, int64_t ph, int64_t pw, int64_t sh, int64_t sw, int64_t dh,
                    int64_t dw, int64_t oh, int64_t ow, int act, bool pool, bool forced, double limit_us);
 
-// Variables AGH_* that force a choice (measurements, tests) are read at every call.  Looking each one up costs a call of a small product
-// a quarter of its host time; one pass over the environment when an entry point is entered tells whether there is any.
-extern thread_local bool g_settings;
-void look_for_settings();
-inline const char *setting(const char *name) { return g_settings ? getenv(name) : nullptr; }
+// Variables AGH_* that force a choice (measurements, tests) are read at every call; looked up one by one they cost a call of a small
+// product a quarter of its host time.  The first one that a call asks for walks the environment once and notes the few entries that begin
+// with AGH_; the others are looked up among those.  Calls that ask for none (allocation, copies) pay nothing, and variables that
+// calls do not read (AGH_CACHE_LIMIT_MB) one comparison each.  Read and written under the API lock.
+extern bool g_settings_known;  // false: the environment has not been looked at since the entry point was entered
+const char *setting(const char *name);
 
 #define AGH_API_ENTER()                                           \
     std::lock_guard<std::recursive_mutex> _agh_lock(agh::api_mutex()); \
-    agh::look_for_settings();                                          \
+    agh::g_settings_known = false;                                     \
     if (!agh::initialized()) return agh::fail(AGH_ENOINIT, "%s: agh_init has not been called", __func__)
 
 #define AGH_HIP(expr)                                                  \

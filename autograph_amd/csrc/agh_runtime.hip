@@ -72,14 +72,23 @@ static std::vector<DeferredFree> g_deferred_frees;
 static uint64_t g_side_seq = 0, g_side_joined_seq = 0;
 
 std::recursive_mutex &api_mutex() { return g_mutex; }
-thread_local bool g_settings = false;
-void look_for_settings() {
-    g_settings = false;
-    for (char **e = environ; e && *e; ++e)
-        if ((*e)[0] == 'A' && (*e)[1] == 'G' && (*e)[2] == 'H' && (*e)[3] == '_') {
-            g_settings = true;
-            return;
-        }
+bool g_settings_known = false;
+static const char *g_settings[32];  // "AGH_NAME=value", as they stand in the environment
+static int g_setting_count = 0;     // how many there are; more than the array holds: not noted
+const char *setting(const char *name) {
+    constexpr int kHeld = (int)(sizeof(g_settings) / sizeof(g_settings[0]));
+    if (!g_settings_known) {
+        g_setting_count = 0;
+        for (char **e = environ; e && *e; ++e)
+            if (strncmp(*e, "AGH_", 4) == 0 && g_setting_count++ < kHeld) g_settings[g_setting_count - 1] = *e;
+        g_settings_known = true;
+    }
+    if (g_setting_count > kHeld) return getenv(name);
+    for (int i = 0; i < g_setting_count; ++i) {
+        const size_t n = strlen(name);
+        if (strncmp(g_settings[i], name, n) == 0 && g_settings[i][n] == '=') return g_settings[i] + n + 1;
+    }
+    return nullptr;
 }
 hipStream_t stream() { return g_cur; }
 bool initialized() { return g_init; }

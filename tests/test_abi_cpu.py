@@ -3,6 +3,7 @@ header declares, and argument errors come back as status codes without a GPU."""
 import ctypes as C
 import os
 import re
+import time
 import types
 
 import numpy as np
@@ -37,6 +38,25 @@ def test_calls_before_init_fail_with_status_not_crash():
     assert rc == -2  # AGH_ENOINIT
     assert b"agh_init" in _ffi.lib.agh_last_error_string()
     assert _ffi.lib.agh_gemm_f32(1, 1, 1, 1.0, None, 0, 1, 1, None, 0, 1, 1, 0.0, None, 0, 1, 1) == -2
+
+
+def test_calls_that_read_no_variable_do_not_walk_the_environment(monkeypatch):
+    """An entry point that no AGH_* variable concerns costs the same whatever the environment's size (a walk through 8000 variables
+    takes over 10 us, the call itself under 1)."""
+    from autograph_amd import _ffi
+
+    def us():
+        best = float("inf")
+        for _ in range(20):
+            t0 = time.perf_counter()
+            for _ in range(50):
+                _ffi.lib.agh_branch_join()
+            best = min(best, time.perf_counter() - t0)
+        return best / 50 * 1e6
+    few = us()
+    for i in range(8000):
+        monkeypatch.setenv(f"FILLER_{i}", "1")
+    assert us() < 2 * few + 2
 
 
 def test_option_shape_formulas():

@@ -2,6 +2,7 @@
 (the reference allocates one output per op, src/tensor.rs:1377-1389), the library's workspace under live
 graphs, and the branch stream's bookkeeping around waits and copies."""
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -334,3 +335,42 @@ def test_large_copies_between_device_blocks(ag, extra):
     got = np.empty(n, np.uint8)
     check(ag.lib.agh_memcpy_d2h(got.ctypes.data, src.ptr, n))
     assert np.array_equal(got, host[:n])
+
+
+def test_variables_that_calls_do_not_read_cost_them_nothing(ag, monkeypatch):
+    """A call reads the environment once however many of its choices could be forced, with or without an AGH_* variable set
+    (AGH_CACHE_LIMIT_MB, which only agh_init reads); 4000 other variables make each further walk show."""
+    a = ag.Tensor.zeros((16, 16), "f32")
+    c = ag.Tensor.zeros((16, 16), "f32")
+
+    def us():
+        best = float("inf")
+        for _ in range(10):
+            ag._ffi.check(ag.lib.agh_sync())
+            t0 = time.perf_counter()
+            for _ in range(30):
+                ag.gemm(1.0, a, a, 0.0, c)
+            best = min(best, time.perf_counter() - t0)
+        return best / 30 * 1e6
+    for i in range(4000):
+        monkeypatch.setenv(f"FILLER_{i}", "1")
+    without = us()
+    monkeypatch.setenv("AGH_CACHE_LIMIT_MB", "4096")
+    assert us() < 1.5 * without
+
+
+def test_forced_choices_are_read_among_many_variables(ag, monkeypatch):
+    """A variable is found among more AGH_* variables than are noted, its prefix is not taken for it, and it no longer counts once it
+    is gone.  (A forced tile configuration that does not exist is refused.)"""
+    a, c = ag.Tensor.zeros((128, 128), "f32"), ag.Tensor.zeros((128, 128), "f32")
+    for fillers in (0, 31, 32, 40):
+        for i in range(fillers):
+            monkeypatch.setenv(f"AGH_FILLER_{i}", "1")
+        monkeypatch.setenv("AGH_GEMM_CFGS", "99")
+        monkeypatch.delenv("AGH_GEMM_CFG", raising=False)
+        ag.gemm(1.0, a, a, 0.0, c)
+        monkeypatch.setenv("AGH_GEMM_CFG", "99")
+        with pytest.raises(ag.AghError):
+            ag.gemm(1.0, a, a, 0.0, c)
+        monkeypatch.delenv("AGH_GEMM_CFG")
+        ag.gemm(1.0, a, a, 0.0, c)
