@@ -42,7 +42,7 @@ def test_calls_before_init_fail_with_status_not_crash():
 
 def test_calls_that_read_no_variable_do_not_walk_the_environment(monkeypatch):
     """An entry point that no AGH_* variable concerns costs the same whatever the environment's size (a walk through 8000 variables
-    takes over 10 us, the call itself under 1)."""
+    takes about 5 us, the call itself 0.3)."""
     from autograph_amd import _ffi
 
     def us():
