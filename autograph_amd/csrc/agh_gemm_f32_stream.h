@@ -8,9 +8,10 @@
 // order).  One of a CU's two workgroups has a higher priority, so that one stores while the other multiplies (without: 75.5 against
 // 73.4 us below).
 //
-// Tile 64 (p) x 128 (q), eight waves in a 2 x 4 grid, one 32 x 32 accumulator a wave, three stages of 24 KB.  LDS images, fragments and
-// order of sums as in agh_gemm_f32_dl.h with one wave per tile position.  The operands change places in the MFMA: lane l
-// holds D[8 (r / 4) + 4 (l / 32) + r % 4][l % 32] as (q, p), so a store instruction writes whole 128-byte lines of two rows of C.
+// Tile 64 (p) x 128 (q), eight waves in a 2 x 4 grid, one 32 x 32 tile a wave, three stages of 24 KB.  LDS images, fragments and
+// order of sums as in agh_gemm_f32_dl.h: KS = 1 one accumulator, as with one wave per tile position there, KS = 2 one for either half of
+// every k-tile, added at the tile's end, as with two (agh_gemm_host.h says where; 109 to 111 and 125 to 127 of 128 registers).  The operands
+// change places in the MFMA: lane l holds D[8 (r / 4) + 4 (l / 32) + r % 4][l % 32] as (q, p), so a store instruction writes whole 128-byte lines of two rows of C.
 //
 // 50176 x 128 x 576 97 -> 73 us, 802816 x 64 x 576 950 -> 647, 16384 x 64 x 8192 250 -> 190, 12012 x 128 x 6400 216 -> 183, 100000 x 128 x 64
 // 49 -> 25.  What bounds it at k = 128: 61 us a multiple of the 52 that the matrix pipes need, and 4 TB/s of stores in between.
@@ -40,8 +41,9 @@ __device__ __forceinline__ void store_counted(const float *uniform_base, uint32_
     asm volatile("global_store_dword %0, %1, %2" ::"v"(byte_off), "v"(v), "s"(uniform_base) : "memory");
 }
 
-template <int LP, int LQ>
+template <int LP, int LQ, int KS>
 __global__ __launch_bounds__(512, 2 * kStreamPerCu) void gemm_f32_stream_kernel(Args g) {
+    static_assert(KS == 1 || KS == 2, "one chain of additions over k, or one for each half of the k-tiles");
     typedef F32StreamGeo<LP, LQ> Geo_;
     typedef typename Geo_::OpP OpP;
     typedef typename Geo_::OpQ OpQ;
@@ -150,9 +152,14 @@ __global__ __launch_bounds__(512, 2 * kStreamPerCu) void gemm_f32_stream_kernel(
         qf = frag_read(std::common_type<OpQ>{}, std::integral_constant<int, LQ>{}, stage + OpP::BYTES, fq, sc);
     };
 
-    f32x16 acc;
+    f32x16 acc[KS];
+    auto clear = [&] {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+        for (int h = 0; h < KS; ++h)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[h][r] = 0.0f;
+    };
+    clear();
     uint4 pa, qa, pb, qb;
     aim_tile(first);
     for (int t = 0; t < AHEAD; ++t) static_for<NL>([&](auto lc) { request(t, lc); });
@@ -162,10 +169,10 @@ __global__ __launch_bounds__(512, 2 * kStreamPerCu) void gemm_f32_stream_kernel(
     read_frags(pa, qa, smem, std::integral_constant<int, 0>{});
 
     // a substep's four MFMAs out of one fragment set; the next substep's fragments are read in front of the first
-    auto substep = [&](const uint4 &xp, const uint4 &xq, uint4 &yp, uint4 &yq, const unsigned char *stage, auto sc, auto &&extra) {
+    auto substep = [&](f32x16 &sum, const uint4 &xp, const uint4 &xq, uint4 &yp, uint4 &yq, const unsigned char *stage, auto sc, auto &&extra) {
         read_frags(yp, yq, stage, sc);
         static_for<4>([&](auto mc) {
-            Mma<float>::template part<decltype(mc)::value>(acc, xq, xp);
+            Mma<float>::template part<decltype(mc)::value>(sum, xq, xp);
             extra(mc);
             __builtin_amdgcn_sched_barrier(0);
         });
@@ -176,22 +183,26 @@ __global__ __launch_bounds__(512, 2 * kStreamPerCu) void gemm_f32_stream_kernel(
     for (int s = 0; s < steps; ++s) {
         const int nslot = slot + 1 == NS ? 0 : slot + 1, free_slot = slot == 0 ? NS - 1 : slot - 1;  // left in the last step
         const unsigned char *cur = smem + slot * STAGE_BYTES, *nxt = smem + nslot * STAGE_BYTES;
-        substep(pa, qa, pb, qb, cur, std::integral_constant<int, 1>{}, [&](auto mc) {
+        substep(acc[0], pa, qa, pb, qb, cur, std::integral_constant<int, 1>{}, [&](auto mc) {
             constexpr int m = decltype(mc)::value;
             if constexpr (m < NL) request(free_slot, mc);
         });
-        substep(pb, qb, pa, qa, cur, std::integral_constant<int, 2>{}, nothing);
-        substep(pa, qa, pb, qb, cur, std::integral_constant<int, 3>{}, nothing);
+        substep(acc[0], pb, qb, pa, qa, cur, std::integral_constant<int, 2>{}, nothing);
+        substep(acc[KS - 1], pa, qa, pb, qb, cur, std::integral_constant<int, 3>{}, nothing);
         // The next k-tile becomes visible.  Its loads went out in the last step; issued since: those of the k-tile behind it, and the
         // stores of a whole tile that ended with that step (other stores are not counted: waiting for more than needed is safe).
         if (stored) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(INFLIGHT + STORES) : "memory");
         else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(INFLIGHT) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        substep(pb, qb, pa, qa, nxt, std::integral_constant<int, 0>{}, nothing);
+        substep(acc[KS - 1], pb, qb, pa, qa, nxt, std::integral_constant<int, 0>{}, nothing);
         slot = nslot;
         stored = false;
         if (++kt < KT) continue;
+        if constexpr (KS == 2) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[0][r] += acc[1][r];
+        }
         // ---- the tile is complete: element r = D[p][q] with p = p0 + l % 32, q = q0 + 8 (r / 4) + 4 (l / 32) + r % 4 ----
         kt = 0;
         const int tq = tile / g.tiles_p, tp = tile - tq * g.tiles_p;
@@ -202,17 +213,16 @@ __global__ __launch_bounds__(512, 2 * kStreamPerCu) void gemm_f32_stream_kernel(
             // sixteen stores, counted above
             const uint32_t off = (lg * 4u * (uint32_t)g.dq + lrow) * 4u;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) store_counted(row + (int64_t)(8 * (r >> 2) + (r & 3)) * g.dq, off, g.alpha * acc[r]);
+            for (int r = 0; r < 16; ++r) store_counted(row + (int64_t)(8 * (r >> 2) + (r & 3)) * g.dq, off, g.alpha * acc[0][r]);
             stored = true;
         } else {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int q = (int)lg * 4 + 8 * (r >> 2) + (r & 3);
-                if (p0 + (int)lrow < g.NP && q0 + q < g.NQ) row[(int64_t)q * g.dq + lrow] = finish_plain<float>(acc[r], g.alpha);
+                if (p0 + (int)lrow < g.NP && q0 + q < g.NQ) row[(int64_t)q * g.dq + lrow] = finish_plain<float>(acc[0][r], g.alpha);
             }
         }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+        clear();
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the requests past the last k-tile still write LDS
 }

@@ -120,9 +120,11 @@ int launch_f32_dl(const Args &g, int splits) {
 
 #ifdef AGH_GEMM_WITH_F32_DIRECT
 // two workgroups per CU over all tiles (agh_gemm_f32_stream.h)
-template <int LP, int LQ>
-int launch_f32_stream(const Args &g, int cus) {
-    auto kern = gemm_f32_stream_kernel<LP, LQ>;
+template <int LP, int LQ, int KS = 1>
+int launch_f32_stream(const Args &g, int cus, bool halves) {
+    if constexpr (KS == 1)
+        if (halves) return launch_f32_stream<LP, LQ, 2>(g, cus, true);
+    auto kern = gemm_f32_stream_kernel<LP, LQ, KS>;
     constexpr size_t smem = F32StreamGeo<LP, LQ>::SMEM_BYTES;
     static bool attr_done = false;
     if (!attr_done) {
@@ -337,31 +339,6 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
     }
 #endif
 
-#ifdef AGH_GEMM_WITH_F32_DIRECT
-    if constexpr (sizeof(T) == 4) {
-        // Short k and a tile for every CU at least: two workgroups per CU over all tiles.  Over 400 products of 64 to 120000 x 8 to 1200 x 16 to
-        // 8192, of those the rule takes 4 are more than 3 % behind the kernels of one tile a workgroup, 6 % at most (49690 x 256 x 112
-        // 40.7 / 43.3 us), all together 1.2 times as fast (3883 x 300 x 3092 92.9 / 73.3; 4758 x 32 x 416 11.1 / 8.0).  From k = 320 on a tile's
-        // own k-tiles hide most of what is gained (384 to 512: 0.95 to 1.14); up to 32 columns of C the 32 x 128 tile has less padding (94418 x
-        // 196 x 16 20.5 / 41.7).  AGH_GEMM_STREAM=0|1 overrides.
-        const int64_t tiles_p = (g.NP + kStreamBP - 1) / kStreamBP, tiles_q = (g.NQ + kStreamBQ - 1) / kStreamBQ;
-        const bool can = batch == 1 && !any_scalar && g.K > 0 && beta == 0.0f && !bias && act == AGH_ACT_NONE && g.dp == 1 && g.dq > 0 &&
-                         g.dq < (1 << 24) && tiles_p * tiles_q * ((g.K + 31) / 32) < 0x7FFFFFFF && env_int("AGH_GEMM_DIRECT", 1) != 0;
-        const bool suits = g.K <= 256 && g.NP > 32 && g.NQ > 64 && tiles_p * tiles_q >= cus && forced_cfg < 0 && !setting("AGH_GEMM_SPLITS");
-        if (can && env_int("AGH_GEMM_STREAM", suits) != 0) {
-            g.tiles_p = (int)tiles_p;
-            g.tiles_q = (int)tiles_q;
-            switch (lp * 3 + lq) {
-                case LD_K * 3 + LD_K: return launch_f32_stream<LD_K, LD_K>(g, cus);
-                case LD_K * 3 + LD_R: return launch_f32_stream<LD_K, LD_R>(g, cus);
-                case LD_R * 3 + LD_K: return launch_f32_stream<LD_R, LD_K>(g, cus);
-                case LD_R * 3 + LD_R: return launch_f32_stream<LD_R, LD_R>(g, cus);
-                default: break;
-            }
-        }
-    }
-#endif
-
     // ---- tile shape: minimise (rounds of workgroups) x (tile area) / efficiency ----
     // (any k: a last k-tile shorter than 64 is loaded with zeros behind k = K)
     const bool direct_ok = sizeof(T) == 2 && (!any_scalar || any_addr) && g.K > 0 && env_int("AGH_GEMM_DIRECT", 1) != 0;
@@ -441,6 +418,42 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
         if (best < 0 || cost < best_cost) { best = i; best_cost = cost; }
     }
     if (forced_cfg >= 0) best = forced_cfg;
+
+#ifdef AGH_GEMM_WITH_F32_DIRECT
+    if constexpr (sizeof(T) == 4) {
+        // Short k and a tile for every CU at least: two workgroups per CU over all tiles.  Over 400 products of 64 to 120000 x 8 to 1200 x 16 to
+        // 8192, of those the rule takes 4 are more than 3 % behind the kernels of one tile a workgroup, 6 % at most (49690 x 256 x 112
+        // 40.7 / 43.3 us), all together 1.2 times as fast (3883 x 300 x 3092 92.9 / 73.3; 4758 x 32 x 416 11.1 / 8.0).  From k = 320 on a tile's
+        // own k-tiles hide most of what is gained (384 to 512: 0.95 to 1.14); up to 32 columns of C the 32 x 128 tile has less padding (94418 x
+        // 196 x 16 20.5 / 41.7).  AGH_GEMM_STREAM=0|1 overrides.
+        const int64_t tiles_p = (g.NP + kStreamBP - 1) / kStreamBP, tiles_q = (g.NQ + kStreamBQ - 1) / kStreamBQ;
+        const bool can = batch == 1 && !any_scalar && g.K > 0 && beta == 0.0f && !bias && act == AGH_ACT_NONE && g.dp == 1 && g.dq > 0 &&
+                         g.dq < (1 << 24) && tiles_p * tiles_q * ((g.K + 31) / 32) < 0x7FFFFFFF && env_int("AGH_GEMM_DIRECT", 1) != 0;
+        const int ksplit = env_int("AGH_GEMM_KSPLIT", -1);
+        const bool suits = g.K <= 256 && g.NP > 32 && g.NQ > 64 && tiles_p * tiles_q >= cus && forced_cfg < 0 && !setting("AGH_GEMM_SPLITS");
+        // Where its tiles leave a CU one workgroup at most, launch_f32_dl adds the two halves of every k-tile in sums of their own, which rounds
+        // less (relative error against 64 bits at k = 128, halves / one chain: 1.47e-7 / 2.03e-7 on normal values, 0.87e-7 / 1.58e-7 on uniform ones
+        // from 0 to 1).  So does this kernel for those products, with the same bits; it costs 0.9 % over 179 of them, 1.31 times as fast
+        // as there (4273 x 244 x 564 27.6 / 24.6 us, the least gain).
+        bool halves = ksplit > 0;
+        if (ksplit < 0 && (best == 3 || best == 4)) {
+            const TileCfg &t = kCfgs[best];
+            halves = (int64_t)((g.NP + t.bp - 1) / t.bp) * ((g.NQ + t.bq - 1) / t.bq) <= cus;
+        }
+        if (can && env_int("AGH_GEMM_STREAM", suits) != 0) {
+            g.tiles_p = (int)tiles_p;
+            g.tiles_q = (int)tiles_q;
+            switch (lp * 3 + lq) {
+                case LD_K * 3 + LD_K: return launch_f32_stream<LD_K, LD_K>(g, cus, halves);
+                case LD_K * 3 + LD_R: return launch_f32_stream<LD_K, LD_R>(g, cus, halves);
+                case LD_R * 3 + LD_K: return launch_f32_stream<LD_R, LD_K>(g, cus, halves);
+                case LD_R * 3 + LD_R: return launch_f32_stream<LD_R, LD_R>(g, cus, halves);
+                default: break;
+            }
+        }
+    }
+#endif
+
     const bool any = any_addr && (best == 3 || best == 4);  // (a forced skinny tile keeps the element-wise loaders)
     if (any) { lp = lp_any; lq = lq_any; }
     if (best < 0 || best >= kNumCfgs || (any_scalar && !any && !kCfgs[best].scalar_ok))

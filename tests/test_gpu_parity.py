@@ -1353,6 +1353,42 @@ def test_gemm_f32_stream_over_tiles(ag, monkeypatch, ta, tb):
             assert np.array_equal(got["1"], got["0"]), (m, k, n)
 
 
+def _stream_operands(ag, rng, m, k, n, ta, tb):
+    """Operands of an f32 product and their values, with NaN behind the last element of either."""
+    pad_a, pad_b = [rng.standard_normal(s[::-1] if t else s).astype(np.float32) for s, t in (((m, k), ta), ((k, n), tb))]
+    out = []
+    for x, t in ((pad_a, ta), (pad_b, tb)):
+        d = ag.Tensor.from_array(np.concatenate([x.reshape(-1), np.full(64, np.nan, np.float32)]))
+        d = ag.Tensor(d.buffer, x.shape, ag.tensor._std_strides(x.shape), 0, "f32")
+        out.append((d.t() if t else d, (x.T if t else x).astype(np.float64)))
+    return out[0][0], out[1][0], out[0][1], out[1][1]
+
+
+@pytest.mark.parametrize("ta", [False, True])
+@pytest.mark.parametrize("tb", [False, True])
+@pytest.mark.parametrize("m,k,n", [(2048, 256, 2048), (2048, 128, 2048), (2048, 36, 2048), (4096, 128, 1000), (4096, 8, 1000), (1500, 200, 2400),
+                                   (16384, 64, 256), (1996, 100, 2044), (8192, 128, 1024), (4100, 48, 2052)])
+def test_gemm_f32_stream_sums_as_one_tile_a_workgroup_does(ag, monkeypatch, m, k, n, ta, tb):
+    """Products that leave a CU one workgroup of 128 x 128 at most add each half of the k-tiles by itself, which rounds less than one chain;
+    so do they where two workgroups per CU stream over the tiles: default route bit for bit that of one tile a workgroup, inside that
+    class of sizes and outside (the last two).  Also with rows of C further apart than its columns."""
+    rng = np.random.default_rng(k)
+    a, b, ha, hb = _stream_operands(ag, rng, m, k, n, ta, tb)
+    got = {}
+    for stream in ("", "0"):
+        for pad in (0, 3):
+            monkeypatch.setenv("AGH_GEMM_STREAM", stream)
+            c = ag.Tensor.from_array(np.full((m, n + pad), 7.0, np.float32))
+            ag.gemm(1.0, a, b, 0.0, ag.Tensor(c.buffer, (m, n), (n + pad, 1), 0, "f32"))
+            out = c.into_array()
+            assert (out[:, n:] == 7.0).all()
+            got[stream, pad] = out[:, :n]
+    for key in (("", 3), ("0", 0), ("0", 3)):
+        assert np.array_equal(got["", 0], got[key]), key
+    # gamma_k |A||B| of a sum of k products in any order
+    assert (np.abs(got["", 0] - ha @ hb) <= (k + 1) * 2.0 ** -24 * (np.abs(ha) @ np.abs(hb))).all()
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("c,gh,gw,f,s,p", [(8, 3, 82, 5, 1, 2), (16, 7, 83, 5, 1, 0), (8, 4, 102, 5, 1, 1), (8, 4, 103, 5, 1, 2), (8, 5, 128, 5, 1, 4),
                                            (8, 9, 42, 7, 1, 3), (16, 4, 60, 7, 1, 0), (8, 9, 83, 7, 1, 6), (8, 3, 84, 7, 1, 3), (8, 6, 64, 5, 2, 2),
