@@ -430,7 +430,9 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
         const bool can = batch == 1 && !any_scalar && g.K > 0 && beta == 0.0f && !bias && act == AGH_ACT_NONE && g.dp == 1 && g.dq > 0 &&
                          g.dq < (1 << 24) && tiles_p * tiles_q * ((g.K + 31) / 32) < 0x7FFFFFFF && env_int("AGH_GEMM_DIRECT", 1) != 0;
         const int ksplit = env_int("AGH_GEMM_KSPLIT", -1);
-        const bool suits = g.K <= 256 && g.NP > 32 && g.NQ > 64 && tiles_p * tiles_q >= cus && forced_cfg < 0 && !setting("AGH_GEMM_SPLITS");
+        // (a forced tile configuration, split count or eight-wave form means the kernels of one tile a workgroup are wanted)
+        const bool suits = g.K <= 256 && g.NP > 32 && g.NQ > 64 && tiles_p * tiles_q >= cus && forced_cfg < 0 && !setting("AGH_GEMM_SPLITS") &&
+                           ksplit <= 0;
         // Where its tiles leave a CU one workgroup at most, launch_f32_dl adds the two halves of every k-tile in sums of their own, which rounds
         // less (relative error against 64 bits at k = 128, halves / one chain: 1.47e-7 / 2.03e-7 on normal values, 0.87e-7 / 1.58e-7 on uniform ones
         // from 0 to 1).  So does this kernel for those products, with the same bits; it costs 0.9 % over 179 of them, 1.31 times as fast

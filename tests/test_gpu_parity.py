@@ -1389,6 +1389,28 @@ def test_gemm_f32_stream_sums_as_one_tile_a_workgroup_does(ag, monkeypatch, m, k
     assert (np.abs(got["", 0] - ha @ hb) <= (k + 1) * 2.0 ** -24 * (np.abs(ha) @ np.abs(hb))).all()
 
 
+def test_gemm_f32_ksplit_names_the_kernel_that_runs(ag, monkeypatch):
+    """AGH_GEMM_KSPLIT=1 forces the eight-wave form of one tile a workgroup also where two workgroups per CU would stream over the
+    tiles (100000 x 128 x 64 takes half the time there), and AGH_GEMM_STREAM=1 wins over it."""
+    a, b, c = (ag.Tensor.zeros(s, "f32") for s in ((100000, 128), (128, 64), (100000, 64)))
+
+    def us():
+        best = float("inf")
+        for _ in range(8):
+            ag._ffi.check(ag.lib.agh_sync())
+            t0 = time.perf_counter()
+            for _ in range(40):
+                ag.gemm(1.0, a, b, 0.0, c)
+            ag._ffi.check(ag.lib.agh_sync())
+            best = min(best, time.perf_counter() - t0)
+        return best / 40 * 1e6
+    chosen = us()
+    monkeypatch.setenv("AGH_GEMM_KSPLIT", "1")
+    forced = us()
+    monkeypatch.setenv("AGH_GEMM_STREAM", "1")
+    assert forced > 1.3 * chosen and us() < 1.15 * chosen, (chosen, forced)
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("c,gh,gw,f,s,p", [(8, 3, 82, 5, 1, 2), (16, 7, 83, 5, 1, 0), (8, 4, 102, 5, 1, 1), (8, 4, 103, 5, 1, 2), (8, 5, 128, 5, 1, 4),
                                            (8, 9, 42, 7, 1, 3), (16, 4, 60, 7, 1, 0), (8, 9, 83, 7, 1, 6), (8, 3, 84, 7, 1, 3), (8, 6, 64, 5, 2, 2),
