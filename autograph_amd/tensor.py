@@ -106,7 +106,11 @@ class MaxPool2Options:
 
 def _dims(shape):
     """The dimensions as Python integers: products of them must not wrap, as those of 8-, 16- or 32-bit numpy integers do."""
-    return tuple(map(int, shape))
+    shape = tuple(shape)
+    dims = tuple(map(int, shape))
+    if dims != shape:  # int() cuts fractions off and reads strings
+        raise AghError(-1, f"dimensions {shape} are not whole numbers")
+    return dims
 
 
 def _std_strides(shape):

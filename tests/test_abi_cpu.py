@@ -91,6 +91,19 @@ def test_narrow_integers_as_dimensions(monkeypatch, shape):
         t.into_shape((want + 1,))
 
 
+@pytest.mark.parametrize("shape", [(2.5, 4), ("2", 4), ("24"), (np.float32(2.5), 4)])
+def test_dimensions_that_are_no_whole_numbers_are_refused(monkeypatch, shape):
+    """Not cut down to whole ones: 2.5 x 4 is no shape of the eight elements of 2 x 4.  (Whole floats count as the integers they are.)"""
+    from autograph_amd import tensor
+    monkeypatch.setattr(tensor, "Buffer", lambda nbytes: types.SimpleNamespace(ptr=0, nbytes=nbytes))
+    t = tensor.Tensor.uninit((2, 4), "f32")
+    with pytest.raises(tensor.AghError):
+        t.into_shape(shape)
+    with pytest.raises(tensor.AghError):
+        tensor.Tensor.uninit(shape, "f32")
+    assert t.into_shape((4.0, np.int8(2))).shape == (4, 2)
+
+
 _C_TO_RUST = {"int": "c_int", "int64_t": "i64", "float": "f32", "size_t": "usize", "char": "c_char", "void": "c_void"}
 
 
