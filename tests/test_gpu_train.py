@@ -102,15 +102,15 @@ def test_scaled_add_sgd_sum_axis0_bit_exact(ag, dtype):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
-@pytest.mark.parametrize("rows", [0, 1, 9, 128, 129, 255, 256, 257, 511, 512, 513, 769, 1025])
+@pytest.mark.parametrize("rows", [0, 1, 9, 128, 129, 255, 256, 257, 511, 512, 513, 769, 1025, 1537, 2305])
 def test_sum_axis0_chunk_and_column_edges(ag, dtype, rows, monkeypatch):
-    # one thread adds a column, or rows go through LDS in chunks of 256 (two in flight), 64 columns a workgroup: bit for bit
-    # the serial sum in either form, and in the one chosen by size
+    # one thread adds a column, or rows go through LDS in chunks of 256 (two in flight, from the fifth on in registers and buffers
+    # that held earlier ones), 16, 32 or 64 columns a workgroup: bit for bit the serial sum in every form, and in the one chosen by size
     rng = np.random.default_rng(rows)
     for cols in (1, 63, 64, 65, 130):
         a = to_dtype(rng.standard_normal((rows, cols)) * 4, dtype)
         t, want = ag.Tensor.from_array(a), orc.sum_axis0(a)
-        for staged in ("", "0", "1"):
+        for staged in ("", "0", "1", "16", "32", "64"):
             monkeypatch.setenv("AGH_SUM_STAGED", staged)
             assert np.array_equal(t.sum_axis0().into_array(), want), (cols, staged)
 
