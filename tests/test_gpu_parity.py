@@ -1320,7 +1320,7 @@ def test_relu_reference_cases(ag, dtype):
 @pytest.mark.parametrize("tb", [False, True])
 def test_gemm_f32_stream_over_tiles(ag, monkeypatch, ta, tb):
     """f32 products of short k and many tiles in two workgroups per CU (agh_gemm_f32_stream.h): edges of the 64 x 128 tile, one to
-    many tiles a workgroup, fewer tiles than workgroups, k-tiles of 1 to 32, k of one to nine k-tiles, row pitches of C beyond its
+    many tiles a workgroup, fewer tiles than workgroups, last k-tiles of 4 to 32 (test_gemm_f32_stream_any_k: of 1 to 32), k of one to ten k-tiles, row pitches of C beyond its
     columns (nothing else is written), alpha; NaN behind the operands' ends.  Against float64 within the bound of a sum of k
     products in any order, gamma_k |A||B| (k <= 288: 288 x 2^-24 = 1.8e-5), and bit for bit the kernel of one tile a workgroup
     where both add k in order."""
@@ -1353,9 +1353,10 @@ def test_gemm_f32_stream_over_tiles(ag, monkeypatch, ta, tb):
             assert np.array_equal(got["1"], got["0"]), (m, k, n)
 
 
-def _stream_operands(ag, rng, m, k, n, ta, tb):
-    """Operands of an f32 product and their values, with NaN behind the last element of either."""
-    pad_a, pad_b = [rng.standard_normal(s[::-1] if t else s).astype(np.float32) for s, t in (((m, k), ta), ((k, n), tb))]
+def _stream_operands(ag, rng, m, k, n, ta, tb, whole=False):
+    """Operands of an f32 product (whole numbers from -8 to 8 if asked for) and their values, with NaN behind the last element of either."""
+    values = (lambda s: rng.integers(-8, 9, s)) if whole else rng.standard_normal
+    pad_a, pad_b = [values(s[::-1] if t else s).astype(np.float32) for s, t in (((m, k), ta), ((k, n), tb))]
     out = []
     for x, t in ((pad_a, ta), (pad_b, tb)):
         d = ag.Tensor.from_array(np.concatenate([x.reshape(-1), np.full(64, np.nan, np.float32)]))
@@ -1387,6 +1388,24 @@ def test_gemm_f32_stream_sums_as_one_tile_a_workgroup_does(ag, monkeypatch, m, k
         assert np.array_equal(got["", 0], got[key]), key
     # gamma_k |A||B| of a sum of k products in any order
     assert (np.abs(got["", 0] - ha @ hb) <= (k + 1) * 2.0 ** -24 * (np.abs(ha) @ np.abs(hb))).all()
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 5, 27, 31, 33, 63, 75, 77, 147, 255])
+def test_gemm_f32_stream_any_k(ag, monkeypatch, k):
+    """Left operand transposed and right one not: both are k-major, any k is accepted, and the rows of a load behind k = K are zeros one by
+    one (NaN stands behind the operands' ends).  Whole numbers, whose sums are exact in any order, so that a row too few or too many shows;
+    forced in one chain and in two, and sizes that the default rule takes."""
+    rng = np.random.default_rng(k)
+    for m, n, env in ((132, 260, {"AGH_GEMM_STREAM": "1", "AGH_GEMM_KSPLIT": "0"}), (132, 260, {"AGH_GEMM_STREAM": "1", "AGH_GEMM_KSPLIT": "1"}),
+                      (4096, 1000, {}), (8192, 1024, {})):
+        a, b, ha, hb = _stream_operands(ag, rng, m, k, n, True, False, whole=True)
+        for name in ("AGH_GEMM_STREAM", "AGH_GEMM_KSPLIT"):
+            monkeypatch.delenv(name, raising=False)
+        for name, value in {"AGH_GEMM_SMALL": "0", **env}.items():
+            monkeypatch.setenv(name, value)
+        c = ag.Tensor.from_array(np.full((m, n), 7.0, np.float32))
+        ag.gemm(1.0, a, b, 0.0, c)
+        assert np.array_equal(c.into_array(), (ha @ hb).astype(np.float32)), (m, n, env)
 
 
 def test_gemm_f32_ksplit_names_the_kernel_that_runs(ag, monkeypatch):
