@@ -550,7 +550,9 @@ __global__ __launch_bounds__(kThreads) void col2im_ring_kernel(const T *__restri
 //
 // WORDS: words a thread holds for the next step.  The least number of channels whose segments are whole 16-byte vectors (8 in bf16, 4 in
 // f32) of 5x5 patches fills 32 words a thread at 81 patches a row, of 7x7 at 41; wider rows have a form with 64 (two workgroups a CU
-// for their LDS), up to 163 and 83.  The general kernel there / this one in us: bf16 93 x 64 channels, 36 x 83 patches of 5x5 877 / 468,
+// for their LDS), up to 163 and 83 where the image is no wider than the 4 x 256 pixel columns of these channels (128 in bf16, 256 in f32): in
+// bf16 5x5 ends at 124 patches a row plus twice the padding, 7x7 at stride 2 at 61 plus the padding, in f32 5x5 at stride 2 at 126 plus
+// the padding.  The general kernel there / this one in us: bf16 93 x 64 channels, 36 x 83 patches of 5x5 877 / 468,
 // 40 x 64, 60 x 60 of 7x7 660 / 333, 20 x 16, 50 x 50 of 7x7 at stride 2 130 / 71, f32 25 x 64, 60 x 60 of 7x7 864 / 415, 30 x 64, 48 x 83 of
 // 5x5 at stride 2 766 / 320, 20 x 32, 100 x 100 of 5x5 351 / 350; f32 16 x 64, 50 x 112 of 5x5 248 / 262, so f32 5x5 rows of more than
 // 102 patches at stride 1 stay with the general kernel.
@@ -807,14 +809,16 @@ int col2im_launch(const char *name, const void *x, void *y, int64_t bs, int64_t 
             AGH_LAUNCH_CHECK(name);
             return AGH_OK;
         }
-        if (unit_geom && fh >= 5 && !(sizeof(T) == 4 && fh == 5 && sh == 1 && iw > 102) &&
+        // (bf16 5x5 at stride 2: the 1024 pixel columns of 8 channels end at 62 patches a row plus the padding, in front of the 82 that are too
+        // many for 32 words; f32 at stride 1: measured above)
+        const bool wide = fh == 7 || (fh == 5 && (sizeof(T) == 2 ? sh == 1 : sh == 2 || iw <= 102));
+        if (unit_geom && wide &&
             col2im_ring_plan<T>(rp, smem, nblocks, true, kCol2imPrefetchWide, x, bs, c, ih, iw, oh, ow, fh, fw, ph, pw, sh, sw, dh, dw)) {
-            switch (fh * 2 + sh - 1) {
-                case 10: return col2im_wide_launch<T, 5, 1>(name, smem, nblocks, x, y, rp);
-                case 11: return col2im_wide_launch<T, 5, 2>(name, smem, nblocks, x, y, rp);
-                case 14: return col2im_wide_launch<T, 7, 1>(name, smem, nblocks, x, y, rp);
-                default: return col2im_wide_launch<T, 7, 2>(name, smem, nblocks, x, y, rp);
-            }
+            if (fh == 7 && sh == 1) return col2im_wide_launch<T, 7, 1>(name, smem, nblocks, x, y, rp);
+            if (fh == 7) return col2im_wide_launch<T, 7, 2>(name, smem, nblocks, x, y, rp);
+            if constexpr (sizeof(T) == 4)
+                if (sh == 2) return col2im_wide_launch<T, 5, 2>(name, smem, nblocks, x, y, rp);
+            return col2im_wide_launch<T, 5, 1>(name, smem, nblocks, x, y, rp);
         }
         if (col2im_ring_plan<T>(rp, smem, nblocks, false, kCol2imPrefetch, x, bs, c, ih, iw, oh, ow, fh, fw, ph, pw, sh, sw, dh, dw)) {
             launch(col2im_ring_kernel<T>);

@@ -1433,10 +1433,10 @@ def test_gemm_f32_ksplit_names_the_kernel_that_runs(ag, monkeypatch):
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("c,gh,gw,f,s,p", [(8, 3, 82, 5, 1, 2), (16, 7, 83, 5, 1, 0), (8, 4, 102, 5, 1, 1), (8, 4, 103, 5, 1, 2), (8, 5, 128, 5, 1, 4),
                                            (8, 9, 42, 7, 1, 3), (16, 4, 60, 7, 1, 0), (8, 9, 83, 7, 1, 6), (8, 3, 84, 7, 1, 3), (8, 6, 64, 5, 2, 2),
-                                           (8, 5, 62, 7, 2, 3), (4, 6, 110, 5, 2, 1)])
+                                           (8, 5, 62, 7, 2, 3), (4, 6, 110, 5, 2, 1), (8, 30, 84, 5, 2, 22), (4, 6, 130, 5, 2, 4)])
 def test_col2im_rows_wider_than_a_step(ag, monkeypatch, dtype, c, gh, gw, f, s, p):
     """Patch rows that fill more than 32 words a thread: 5x5 from 82 patches a row on, 7x7 from 42, up to the end of the 64-word form and one
-    beyond, stride 2, padding up to f - 1: bit for bit the oracle (the order of additions is the same in every form)."""
+    beyond, stride 2, padding up to f - 1 and, where rows end up narrow again, beyond: bit for bit the oracle (the order of additions is the same in every form)."""
     monkeypatch.setenv("AGH_COL2IM_RING", "1")
     rng = np.random.default_rng(gw)
     x = to_dtype(rng.standard_normal((2 * gh * gw, c * f * f)), dtype)
