@@ -203,9 +203,9 @@ static int release_cached_blocks() {
 }
 
 // ---- large copies between blocks of this allocator ----
-// From kCopyStream bytes on source and destination do not fit in the 256 MB last-level cache together: one launch with the streaming hint
-// on both sides leaves that cache to what runs before and after, and lacks the barriers that the runtime's copy puts between the launches
-// around it.  MaxPool2 forward, copy of its input, MaxPool2 backward on the copy, f32, the runtime's copy / this one in us for inputs of
+// From kCopyStream bytes on: one launch with the streaming hint on both sides leaves the last-level cache to what runs before and after, and
+// lacks the barriers that the runtime's copy puts between the launches around it.  Where the line lies is measured, between 103 and 120
+// MB.  MaxPool2 forward, copy of its input, MaxPool2 backward on the copy, f32, the runtime's copy / this one in us for inputs of
 // 206 / 160 / 120 MB: 208 / 177, 152 / 135, 104 / 94.  Below, the runtime's copy stays: at 103 MB 71.3 / with the hint 81.7, plain 72.6;
 // at 77 MB 55.8, plain 56.6; at 51 MB 39.5, plain 40.0.
 constexpr size_t kCopyStream = (size_t)112 << 20;

@@ -337,6 +337,27 @@ def test_large_copies_between_device_blocks(ag, extra):
     assert np.array_equal(got, host[:n])
 
 
+@pytest.mark.parametrize("shift", [16, 4096, (112 << 20) - 16, 112 << 20])
+@pytest.mark.parametrize("forward", [True, False])
+def test_large_copies_of_ranges_that_overlap(ag, shift, forward):
+    """112 MB within one block to a place that overlaps or just touches the source, in either direction.  The bytes repeat every 16, so the
+    result is the same in whatever order they are moved; what the source does not cover held others before."""
+    n, end = 112 << 20, 64
+    rng = np.random.default_rng(shift)
+    period = rng.integers(0, 128, 16, dtype=np.uint8)
+    want = np.full(n + shift + end, 0xA5, np.uint8)
+    src, dst = (0, shift) if forward else (shift, 0)
+    want[src:src + n] = np.resize(period, n)
+    check = ag._ffi.check
+    block = ag.Buffer(want.size)
+    check(ag.lib.agh_memcpy_h2d(block.ptr, want.ctypes.data, want.size))
+    check(ag.lib.agh_memcpy_d2d(block.ptr + dst, block.ptr + src, n))
+    want[:n + shift] = np.resize(period, n + shift)
+    got = np.empty(want.size, np.uint8)
+    check(ag.lib.agh_memcpy_d2h(got.ctypes.data, block.ptr, want.size))
+    assert np.array_equal(got, want)
+
+
 def test_variables_that_calls_do_not_read_cost_them_nothing(ag, monkeypatch):
     """A call reads the environment once however many of its choices could be forced, with or without an AGH_* variable set
     (AGH_CACHE_LIMIT_MB, which only agh_init reads); 4000 other variables make each further walk show."""
