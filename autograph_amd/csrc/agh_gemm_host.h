@@ -422,10 +422,11 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
 #ifdef AGH_GEMM_WITH_F32_DIRECT
     if constexpr (sizeof(T) == 4) {
         // Short k and a tile for every CU at least: two workgroups per CU over all tiles.  Over 400 products of 64 to 120000 x 8 to 1200 x 16 to
-        // 8192, of those the rule takes 4 are more than 3 % behind the kernels of one tile a workgroup, 6 % at most (49690 x 256 x 112
-        // 40.7 / 43.3 us), all together 1.2 times as fast (3883 x 300 x 3092 92.9 / 73.3; 4758 x 32 x 416 11.1 / 8.0).  From k = 320 on a tile's
-        // own k-tiles hide most of what is gained (384 to 512: 0.95 to 1.14); up to 32 columns of C the 32 x 128 tile has less padding (94418 x
-        // 196 x 16 20.5 / 41.7).  AGH_GEMM_STREAM=0|1 overrides.
+        // 8192, of those the rule takes 4 are more than 3 % behind the kernels of one tile a workgroup, 6 % at most, all together they are 1.2
+        // times as fast (4758 x 32 x 416 10.4 / 7.0 us, 23193 x 256 x 220 40.3 / 31.7; the least 53765 x 256 x 68 40.2 / 40.5; at k = 64 / 128 / 192 /
+        // 256 1.39 / 1.23 / 1.13 / 1.09 times).  Beyond the rule, k of 260 to 320 is 0.98 to 1.54 times as fast here, 1.12 over 99 products (3883 x
+        // 300 x 3092 92.4 / 71.5); at 352 and 384 it is 1.01 and 1.06 (1076 x 352 x 1800 16.9 / 28.1).  Up to 32 columns of C the 32 x 128
+        // tile has less padding (94418 x 196 x 16 20.5 / 41.7).  AGH_GEMM_STREAM=0|1 overrides.
         const int64_t tiles_p = (g.NP + kStreamBP - 1) / kStreamBP, tiles_q = (g.NQ + kStreamBQ - 1) / kStreamBQ;
         const bool can = batch == 1 && !any_scalar && g.K > 0 && beta == 0.0f && !bias && act == AGH_ACT_NONE && g.dp == 1 && g.dq > 0 &&
                          g.dq < (1 << 24) && tiles_p * tiles_q * ((g.K + 31) / 32) < 0x7FFFFFFF && env_int("AGH_GEMM_DIRECT", 1) != 0;
