@@ -107,6 +107,8 @@ class MaxPool2Options:
 def _dims(shape):
     """The dimensions as Python integers: products of them must not wrap, as those of 8-, 16- or 32-bit numpy integers do."""
     shape = tuple(shape)
+    if type(math.prod(shape)) is int:  # then so is every dimension; converting them anyway costs a call 0.2 us a tensor
+        return shape
     dims = tuple(map(int, shape))
     if dims != shape:  # int() cuts fractions off and reads strings
         raise AghError(-1, f"dimensions {shape} are not whole numbers")
@@ -126,6 +128,17 @@ def _std_strides(shape):
     return tuple(reversed(strides))
 
 
+def _tensor(buffer, shape, strides, offset, dtype):
+    """A Tensor whose dimensions and strides are tuples, the former of Python integers: nothing to look at."""
+    t = object.__new__(Tensor)
+    t.buffer = buffer
+    t.shape = shape
+    t.strides = strides
+    t.offset = offset
+    t.dtype = dtype
+    return t
+
+
 class Tensor:
     """`TensorBase` = {dim, strides, buffer, offset} (src/tensor.rs:327-332) on the device."""
 
@@ -136,8 +149,13 @@ class Tensor:
     @classmethod
     def uninit(cls, shape, dtype):
         # (math.prod: numpy's product of a tuple costs 2.5 us, as much as all the rest of a call's host work before the launch)
-        shape = _dims(shape)
-        return cls(Buffer(math.prod(shape) * _ITEMSIZE[dtype]), shape, _std_strides(shape), 0, dtype)
+        shape = tuple(shape)
+        n = math.prod(shape)
+        if type(n) is not int:  # nor are all the dimensions
+            shape = _dims(shape)
+            n = math.prod(shape)
+        args = Buffer(n * _ITEMSIZE[dtype]), shape, _std_strides(shape), 0, dtype
+        return _tensor(*args) if cls is Tensor else cls(*args)
 
     @classmethod
     def zeros(cls, shape, dtype):
@@ -195,7 +213,7 @@ class Tensor:
         return self.strides == std or all(d == 1 or s == e for d, s, e in zip(self.shape, self.strides, std))
 
     def t(self):
-        return Tensor(self.buffer, self.shape[::-1], self.strides[::-1], self.offset, self.dtype)
+        return _tensor(self.buffer, self.shape[::-1], self.strides[::-1], self.offset, self.dtype)
 
     def permuted_axes(self, axes):
         return Tensor(self.buffer, [self.shape[a] for a in axes], [self.strides[a] for a in axes], self.offset, self.dtype)
@@ -206,7 +224,7 @@ class Tensor:
         shape = _dims(shape)
         if math.prod(shape) != len(self):
             raise AghError(-1, f"into_shape: incompatible shapes {self.shape} -> {shape}")
-        return Tensor(self.buffer, shape, _std_strides(shape), self.offset, self.dtype)
+        return _tensor(self.buffer, shape, _std_strides(shape), self.offset, self.dtype)
 
     def slice_rows(self, start, stop, step=1):
         """Row slice of a 2-D tensor; a negative step gives the negative-stride views ndarray allows."""

@@ -91,7 +91,7 @@ def test_narrow_integers_as_dimensions(monkeypatch, shape):
         t.into_shape((want + 1,))
 
 
-@pytest.mark.parametrize("shape", [(2.5, 4), ("2", 4), ("24"), (np.float32(2.5), 4)])
+@pytest.mark.parametrize("shape", [(2.5, 4), ("2", 4), ("24",), (np.float32(2.5), 4)])
 def test_dimensions_that_are_no_whole_numbers_are_refused(monkeypatch, shape):
     """Not cut down to whole ones: 2.5 x 4 is no shape of the eight elements of 2 x 4.  (Whole floats count as the integers they are.)"""
     from autograph_amd import tensor
