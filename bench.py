@@ -105,7 +105,7 @@ def main():
     args = ap.parse_args()
     sections = set(args.sections.split(","))
     if args.gpus != 1:
-        sys.exit("bench.py: this build measures one GPU only (--gpus 1); nothing here runs across GPUs")
+        sys.exit("bench.py: this benchmark measures one GPU only (--gpus 1); nothing here runs across GPUs")
 
     import autograph_amd as ag
     import autograph_amd._ffi  # noqa: F401

@@ -431,7 +431,7 @@ void orc_gemm_f32_host(i64 m, i64 k, i64 n, float alpha, const float *a, i64 off
 
 /* The 7-deep loop the reference's own tests use as the convolution definition
  * (tests/integration_tests.rs:1127-1174), accumulating in f64 here so it can serve as
- * the checker for both f32 and (after widening) bf16 inputs. */
+ * the oracle for both f32 and (after widening) bf16 inputs. */
 void orc_conv2_naive_f64(const float *x, const float *w, double *y, i64 bs, i64 ic, i64 ih, i64 iw, i64 oc,
                          i64 fh, i64 fw, i64 ph, i64 pw, i64 sh, i64 sw, i64 dh, i64 dw) {
     const i64 oh = orc_conv_out(ih, fh, ph, sh, dh), ow = orc_conv_out(iw, fw, pw, sw, dw);
