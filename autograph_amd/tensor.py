@@ -107,7 +107,10 @@ class MaxPool2Options:
 def _dims(shape):
     """The dimensions as Python integers: products of them must not wrap, as those of 8-, 16- or 32-bit numpy integers do."""
     shape = tuple(shape)
-    if type(math.prod(shape)) is int:  # then so is every dimension; converting them anyway costs a call 0.2 us a tensor
+    for d in shape:
+        if type(d) is not int:
+            break
+    else:  # converting them anyway costs a call 0.2 us a tensor
         return shape
     dims = tuple(map(int, shape))
     if dims != shape:  # int() cuts fractions off and reads strings
@@ -139,6 +142,11 @@ def _tensor(buffer, shape, strides, offset, dtype):
     return t
 
 
+def _uninit(shape, dtype):
+    """Tensor.uninit where every dimension is one of another tensor's."""
+    return _tensor(Buffer(math.prod(shape) * _ITEMSIZE[dtype]), shape, _std_strides(shape), 0, dtype)
+
+
 class Tensor:
     """`TensorBase` = {dim, strides, buffer, offset} (src/tensor.rs:327-332) on the device."""
 
@@ -149,13 +157,9 @@ class Tensor:
     @classmethod
     def uninit(cls, shape, dtype):
         # (math.prod: numpy's product of a tuple costs 2.5 us, as much as all the rest of a call's host work before the launch)
-        shape = tuple(shape)
-        n = math.prod(shape)
-        if type(n) is not int:  # nor are all the dimensions
-            shape = _dims(shape)
-            n = math.prod(shape)
-        args = Buffer(n * _ITEMSIZE[dtype]), shape, _std_strides(shape), 0, dtype
-        return _tensor(*args) if cls is Tensor else cls(*args)
+        shape = _dims(shape)
+        make = _tensor if cls is Tensor else cls
+        return make(Buffer(math.prod(shape) * _ITEMSIZE[dtype]), shape, _std_strides(shape), 0, dtype)
 
     @classmethod
     def zeros(cls, shape, dtype):
@@ -216,7 +220,7 @@ class Tensor:
         return _tensor(self.buffer, self.shape[::-1], self.strides[::-1], self.offset, self.dtype)
 
     def permuted_axes(self, axes):
-        return Tensor(self.buffer, [self.shape[a] for a in axes], [self.strides[a] for a in axes], self.offset, self.dtype)
+        return _tensor(self.buffer, tuple([self.shape[a] for a in axes]), tuple([self.strides[a] for a in axes]), self.offset, self.dtype)
 
     def into_shape(self, shape):
         if not self.is_standard_layout():
@@ -231,7 +235,7 @@ class Tensor:
         assert self.ndim == 2
         idx = range(self.shape[0])[start:stop:step]
         off = self.offset + (idx.start if len(idx) else 0) * self.strides[0]
-        return Tensor(self.buffer, (len(idx), self.shape[1]), (self.strides[0] * step, self.strides[1]), off, self.dtype)
+        return _tensor(self.buffer, (len(idx), self.shape[1]), (self.strides[0] * step, self.strides[1]), off, self.dtype)
 
     def _ptr(self):
         return self.buffer.ptr
@@ -250,7 +254,7 @@ class Tensor:
         k2, n = rhs.shape
         if k != k2:
             raise AghError(-1, f"a_cols != b_rows, {k} != {k2}")  # linalg.rs:274-276
-        out = Tensor.uninit((m, n), self.dtype)
+        out = _uninit((m, n), self.dtype)
         gemm(1.0, self, rhs, 0.0, out, bias=bias, relu=relu)
         return out
 
@@ -298,13 +302,13 @@ class Tensor:
     # -- relu, layer.rs:1269-1510 --
     def relu(self):
         x = self.as_standard_layout()
-        y = Tensor.uninit(x.shape, x.dtype)
+        y = _uninit(x.shape, x.dtype)
         check(self._fn("agh_relu")(x._data_ptr(), y._ptr(), len(x)))
         return y
 
     def relu_backward(self, output_grad):
         x, dy = self.as_standard_layout(), output_grad.as_standard_layout()
-        dx = Tensor.uninit(x.shape, x.dtype)
+        dx = _uninit(x.shape, x.dtype)
         check(self._fn("agh_relu_backward")(x._data_ptr(), dy._data_ptr(), dx._ptr(), len(x)))
         return dx
 
@@ -314,7 +318,7 @@ class Tensor:
 
     def clone(self):
         assert self.is_standard_layout()
-        out = Tensor.uninit(self.shape, self.dtype)
+        out = _uninit(self.shape, self.dtype)
         check(lib.agh_memcpy_d2d(out._ptr(), self._data_ptr(), len(self) * _ITEMSIZE[self.dtype]))
         return out
 
@@ -328,7 +332,7 @@ class Tensor:
         """Strided copy into a fresh standard-layout tensor (`assign`, src/tensor/ops.rs:257-318)."""
         if self.ndim > 4:
             raise AghError(-1, "to_standard_layout: more than 4 dimensions")
-        out = Tensor.uninit(self.shape, self.dtype)
+        out = _uninit(self.shape, self.dtype)
         pad = 4 - self.ndim
         dims = [1] * pad + list(self.shape)
         sx = [0] * pad + list(self.strides)
@@ -391,7 +395,7 @@ class Tensor:
     def sum_axis0(self):
         x = self.as_standard_layout()
         rows, cols = x.shape
-        y = Tensor.uninit((cols,), self.dtype)
+        y = _uninit((cols,), self.dtype)
         check(self._fn("agh_sum_axis0")(x._data_ptr(), y._ptr(), rows, cols))
         return y
 
@@ -412,7 +416,7 @@ class Tensor:
     def cross_entropy_loss_backward(self, target, dy=1.0):
         x = self.as_standard_layout()
         bs, classes = x.shape
-        dx = Tensor.uninit(x.shape, x.dtype)
+        dx = _uninit(x.shape, x.dtype)
         check(self._fn("agh_cross_entropy_backward")(x._data_ptr(), target.ptr, dy, dx._ptr(), bs, classes))
         return dx
 
