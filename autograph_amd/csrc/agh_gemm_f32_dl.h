@@ -30,6 +30,13 @@
 // 16-byte aligned, unit stride along k (LD_K: k a multiple of 4) or along rows (LD_R) with the other stride a
 // multiple of 4 elements, rows a multiple of 4 for LD_R.  A last k-tile shorter than 32 is multiplied after the
 // pipelined loop, its lanes reading zeros behind k = K.
+//
+// W = 1 is the form for operands at any element address, k and row counts of any size (unit stride along k or along rows
+// is all that is asked): the direct loads take 4 bytes a lane instead of 16, four of them a 1 KB image, and put every element where
+// the 16-byte load would have.  The matrix pipes bound it like the form above (a 64 x 64 k-tile is 1024 matrix cycles and 64
+// loads of 256 bytes), where the element-wise loaders of agh_gemm_kernel.h spend as long on addresses, conditions and LDS
+// writes: 4099x4101x4103 2011 -> 1470 us, 1999x2047x1001 131 -> 89, 133x7001x3003 249 -> 112, 2632x323x6065 179 -> 138.  What is left
+// to the aligned form (1190, 73, 97, 104 us) are the loads: 256 a k-tile of 128 x 128 through the CU's one address path.
 #pragma once
 #include "agh_gemm_bf16_dl.h"
 
@@ -60,9 +67,18 @@ struct F32DlGeo {
 // what the lanes of a shorter last k-tile read in place of elements at k >= K
 __device__ __align__(16) static const uint32_t kZeroChunkF32[4] = {0u, 0u, 0u, 0u};
 
-template <int TP, int TQ, int NS, int LP, int LQ, int KS = 1>
+// 4-byte direct load: lane L's element lands at LDS address lds_base + 4*L
+__device__ __forceinline__ void direct_load4(const void *gptr, uint32_t lds_addr_uniform) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
+                 :
+                 : "v"(gptr), "s"(lds_addr_uniform)
+                 : "memory", "m0");
+}
+
+template <int TP, int TQ, int NS, int LP, int LQ, int KS = 1, int W = 4>
 __global__ __launch_bounds__(256 * KS) void gemm_f32_dl_kernel(Args g) {
     typedef float T;
+    static_assert(W == 4 || W == 1, "16 or 4 bytes a lane");
     static_assert((LP == LD_K || LP == LD_R) && (LQ == LD_K || LQ == LD_R), "vector layouts only");
     static_assert(KS == 1 || KS == 2, "a k-tile goes to one wave or is split between two");
     constexpr int SPW = 4 / KS;  // substeps of a k-tile per wave
@@ -71,7 +87,8 @@ __global__ __launch_bounds__(256 * KS) void gemm_f32_dl_kernel(Args g) {
     typedef typename Geo_::OpQ OpQ;
     constexpr int BP = Geo_::BP, BQ = Geo_::BQ, BK = 32;
     constexpr int STAGE_BYTES = Geo_::STAGE_BYTES;
-    constexpr int LPWP = OpP::LOADS / (4 * KS), LPWQ = OpQ::LOADS / (4 * KS), LPW = LPWP + LPWQ;  // direct loads per wave and k-tile
+    constexpr int LPI = 4 / W;  // direct loads per 1 KB image
+    constexpr int LPWP = OpP::LOADS / (4 * KS) * LPI, LPWQ = OpQ::LOADS / (4 * KS) * LPI, LPW = LPWP + LPWQ;  // per wave and k-tile
     static_assert(LPWP >= 1 && LPWQ >= 1, "every wave issues loads of both operands");
     static_assert(NS >= 2 && (NS - 1) * LPW <= 63, "the loads in flight must fit the counter");
     constexpr bool EARLY = NS >= 3;                  // requests in the first substep (see above)
@@ -96,15 +113,31 @@ __global__ __launch_bounds__(256 * KS) void gemm_f32_dl_kernel(Args g) {
     // per-lane global address for k-tile 0, LDS offset of the load's image inside the operand, bytes per k-tile
     const unsigned char *gp[LPWP], *gq[LPWQ];
     uint32_t lp[LPWP], lq[LPWQ];
+    // W == 1: the tile row and k of the element that belongs at this lane's place of load `n` of an operand
+    auto element_of = [&](auto opc, auto modec, int n, int &row, int &k) {
+        typedef typename decltype(opc)::type Op;
+        if constexpr (decltype(modec)::value == LD_K) {
+            row = n * 2 + (lane >> 5);
+            k = (((lane & 31) >> 2) ^ (int)swz((uint32_t)row)) * 4 + (lane & 3);
+        } else {
+            constexpr int BR = 256 / Op::KRPI;  // rows of a k-row
+            row = (n * 64 + lane) % BR;
+            k = (n * 64 + lane) / BR;
+        }
+    };
     auto setup = [&](auto opc, auto modec, auto nc, const void *base, int64_t rs, int64_t ks, int64_t batch_off, int r0,
                      int NR, auto &gptr, auto &loff, int64_t &kstep) {
         typedef typename decltype(opc)::type Op;
         constexpr int MODE = decltype(modec)::value, N = decltype(nc)::value;
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-            const int inst = wave * N + i;
+            const int inst = (wave * N + i) / LPI;
             int64_t off;
-            if constexpr (MODE == LD_K) {
+            if constexpr (W == 1) {
+                int row, k;
+                element_of(opc, modec, wave * N + i, row, k);
+                off = (int64_t)min(r0 + row, NR - 1) * rs + (int64_t)(kbeg + k) * ks;
+            } else if constexpr (MODE == LD_K) {
                 const int row = inst * 8 + (lane >> 3);
                 const int c = (lane & 7) ^ (int)swz((uint32_t)row);
                 const int rowg = min(r0 + row, NR - 1);
@@ -116,7 +149,7 @@ __global__ __launch_bounds__(256 * KS) void gemm_f32_dl_kernel(Args g) {
                 if (rowg >= NR) rowg = NR - 4;  // NR is a multiple of 4 on this path
                 off = (int64_t)(kbeg + kr) * ks + rowg;
             }
-            loff[i] = (uint32_t)inst * Op::IMG;
+            loff[i] = (uint32_t)(inst * Op::IMG + (wave * N + i) % LPI * 256);
             gptr[i] = (const unsigned char *)base + (off + batch_off) * 4;
         }
         kstep = (MODE == LD_K ? (int64_t)BK : (int64_t)BK * ks) * 4;
@@ -127,13 +160,17 @@ __global__ __launch_bounds__(256 * KS) void gemm_f32_dl_kernel(Args g) {
     setup(std::common_type<OpQ>{}, std::integral_constant<int, LQ>{}, std::integral_constant<int, LPWQ>{}, g.Q, g.qs, g.qk,
           (int64_t)blockIdx.z * g.batch_q, q0, g.NQ, gq, lq, stepQ);
     const uint32_t smem_addr = __builtin_amdgcn_readfirstlane(lds_address(smem));
+    auto direct = [&](const void *gptr, uint32_t lds_addr) __attribute__((always_inline)) {
+        if constexpr (W == 4) direct_load16(gptr, lds_addr);
+        else direct_load4(gptr, lds_addr);
+    };
     // load l of this wave's LPW for k-tile t (clamped to the last k-tile: that image is then never read)
     auto request_one = [&](int t, auto lc) {
         constexpr int l = decltype(lc)::value;
         const int tc = min(t, KT - 1);
         const uint32_t st = smem_addr + (uint32_t)(t % NS) * STAGE_BYTES;
-        if constexpr (l < LPWP) direct_load16(gp[l] + (int64_t)tc * stepP, st + lp[l]);
-        else direct_load16(gq[l - LPWP] + (int64_t)tc * stepQ, st + OpP::BYTES + lq[l - LPWP]);
+        if constexpr (l < LPWP) direct(gp[l] + (int64_t)tc * stepP, st + lp[l]);
+        else direct(gq[l - LPWP] + (int64_t)tc * stepQ, st + OpP::BYTES + lq[l - LPWP]);
     };
 
     // ---- fragment reads: lane l supplies row l % 32, k = 8 s + 4 (l / 32) + e ----
@@ -238,7 +275,11 @@ __global__ __launch_bounds__(256 * KS) void gemm_f32_dl_kernel(Args g) {
         asm volatile("" ::: "memory");
         auto below = [&](auto opc, auto modec, int inst) {
             typedef typename decltype(opc)::type Op;
-            if constexpr (decltype(modec)::value == LD_K) {
+            if constexpr (W == 1) {
+                int row, k;
+                element_of(opc, modec, inst, row, k);
+                return k < rem;
+            } else if constexpr (decltype(modec)::value == LD_K) {
                 const int row = inst * 8 + (lane >> 3);
                 return (((lane & 7) ^ (int)swz((uint32_t)row)) * 4) < rem;
             } else {
@@ -249,11 +290,11 @@ __global__ __launch_bounds__(256 * KS) void gemm_f32_dl_kernel(Args g) {
             constexpr int l = decltype(lc)::value;
             if constexpr (l < LPWP) {
                 const bool in = below(std::common_type<OpP>{}, std::integral_constant<int, LP>{}, wave * LPWP + l);
-                direct_load16(in ? (const void *)(gp[l] + (int64_t)KT * stepP) : (const void *)kZeroChunkF32, smem_addr + lp[l]);
+                direct(in ? (const void *)(gp[l] + (int64_t)KT * stepP) : (const void *)kZeroChunkF32, smem_addr + lp[l]);
             } else {
                 const bool in = below(std::common_type<OpQ>{}, std::integral_constant<int, LQ>{}, wave * LPWQ + (l - LPWP));
-                direct_load16(in ? (const void *)(gq[l - LPWP] + (int64_t)KT * stepQ) : (const void *)kZeroChunkF32,
-                              smem_addr + OpP::BYTES + lq[l - LPWP]);
+                direct(in ? (const void *)(gq[l - LPWP] + (int64_t)KT * stepQ) : (const void *)kZeroChunkF32,
+                       smem_addr + OpP::BYTES + lq[l - LPWP]);
             }
         });
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

@@ -93,14 +93,17 @@ int launch_dl_ring(const Args &g, int splits) {
 #endif
 
 #ifdef AGH_GEMM_WITH_F32_DIRECT
+// its form for operands at any element address (agh_gemm_f32_any.hip)
+template <int TP, int TQ, int NS, int LP, int LQ>
+int launch_one_f32_any(const Args &g, int splits);
 // direct-to-LDS f32 kernel for 64 x 64 tiles (agh_gemm_f32_dl.h)
 template <int TP, int TQ, int NS, int LP, int LQ, int KS = 1>
 int launch_f32_dl(const Args &g, int splits) {
     if constexpr (KS == 1 && TP * TQ <= 4) {
-        // a grid that gives a CU one workgroup at most: eight waves, every k-tile split between two (AGH_GEMM_KSPLIT=0|1
-        // forbids / forces it)
+        // a grid that gives a CU one workgroup at most, or a product that would on larger tiles: eight waves, every k-tile
+        // split between two (AGH_GEMM_KSPLIT=0|1 forbids / forces it)
         const int64_t wgs = (int64_t)g.tiles_p * g.tiles_q * splits * g.batch;
-        const int ks = env_int("AGH_GEMM_KSPLIT", wgs <= (compute_units() > 0 ? compute_units() : 256) ? 1 : 0);
+        const int ks = env_int("AGH_GEMM_KSPLIT", g.two_sums || wgs <= (compute_units() > 0 ? compute_units() : 256) ? 1 : 0);
         if (ks) return launch_f32_dl<TP, TQ, NS, LP, LQ, 2>(g, splits);
     }
     auto kern = gemm_f32_dl_kernel<TP, TQ, NS, LP, LQ, KS>;
@@ -146,6 +149,17 @@ int launch_loaders(const Args &g, int splits, int lp, int lq, bool direct, bool 
         // workgroups per CU; 128 x 128: two stages (a k-tile is four times as long), two workgroups per CU; the
         // larger tiles: two stages, one workgroup per CU.
         constexpr int TPW = BP / 64, TQW = BQ / 64, NS = BP == 64 ? 4 : 2;
+        if constexpr (BP == BQ && BP <= 128) {
+            if (any) {
+                switch (lp * 3 + lq) {
+                    case LD_K * 3 + LD_K: return launch_one_f32_any<TPW, TQW, NS, LD_K, LD_K>(g, splits);
+                    case LD_K * 3 + LD_R: return launch_one_f32_any<TPW, TQW, NS, LD_K, LD_R>(g, splits);
+                    case LD_R * 3 + LD_K: return launch_one_f32_any<TPW, TQW, NS, LD_R, LD_K>(g, splits);
+                    case LD_R * 3 + LD_R: return launch_one_f32_any<TPW, TQW, NS, LD_R, LD_R>(g, splits);
+                    default: break;
+                }
+            }
+        }
         if (lp != LD_S && lq != LD_S && g.K > 0 && env_int("AGH_GEMM_DIRECT", 1) != 0) {
             switch (lp * 3 + lq) {
                 case LD_K * 3 + LD_K: return launch_f32_dl<TPW, TQW, NS, LD_K, LD_K>(g, splits);
@@ -230,8 +244,10 @@ int pick_loader(const void *base, int64_t rs, int64_t ks, int NR, int K) {
 // The same for the bf16 kernel that reads 16 bytes from any element address: no multiple of anything is needed, but
 // k >= 8 (a last chunk is read from up to 7 elements further down its row), and for rows as the unit-stride axis k-rows
 // that follow each other upwards at least 8 elements apart (a chunk that runs past the last row of a k-row stays inside the
-// operand's memory).
-inline int pick_loader_any(int64_t rs, int64_t ks, int K) {
+// operand's memory).  The f32 kernel's form loads elements: a unit stride is enough.
+template <typename T>
+int pick_loader_any(int64_t rs, int64_t ks, int K) {
+    if (sizeof(T) == 4) return ks == 1 ? LD_K : rs == 1 ? LD_R : LD_S;
     if (K < 8) return LD_S;
     if (ks == 1) return LD_K;
     if (rs == 1 && ks >= 8) return LD_R;
@@ -257,6 +273,30 @@ inline bool short_and_narrow(const Args &g, int64_t batch, int64_t cus, int lp) 
 inline int env_int(const char *name, int dflt) {
     const char *s = setting(name);
     return (s && *s) ? atoi(s) : dflt;
+}
+
+// k-tiles a split and splits of a product: one split where the tile grid fills half the chip or k is short
+inline int plan_splits(int64_t tiles, int ktiles, int64_t cus, int kmin) {
+    if (tiles * 2 > cus || ktiles < 32) return 1;
+    return (int)std::max<int64_t>(1, std::min(std::min(cus / tiles, (int64_t)(ktiles / kmin)), (int64_t)256));
+}
+
+// Time in us of an f32 product on the direct-to-LDS kernels' 64 x 64 or 128 x 128 tiles, fitted to 450 products of 16 to 60000 x 16 to
+// 8192 x 16 to 8192 outside the small kernel's range (mean error 4 % with whole vectors, 6 % at any address): a launch, rounds of
+// workgroups of so many k-tiles and a store each, the bytes of C, and for split k the second launch and its partial sums.
+struct F32TileTime { double launch, ktile, store, c_mb, reduce, part_mb; };
+inline double f32_tile_us(int edge, bool any, int64_t np, int64_t nq, int64_t k, int64_t batch, int64_t cus, int *splits) {
+    static const F32TileTime kTimes[2][2] = {{{3.54, 0.54, 0.33, 0.27, 2.81, 0.31}, {7.12, 1.96, 0.42, 0.17, 0.22, 0.56}},
+                                             {{3.28, 0.68, 1.67, 0.06, 3.16, 0.25}, {4.50, 2.30, 4.35, 0.12, 0.00, 0.41}}};
+    const F32TileTime &t = kTimes[any][edge == 128];
+    const int64_t tiles = ((np + edge - 1) / edge) * ((nq + edge - 1) / edge) * batch;
+    const int ktiles = (int)((k + 31) / 32);
+    int s = batch == 1 ? plan_splits(tiles, ktiles, cus, 4) : 1;
+    const int per_split = (ktiles + s - 1) / s;
+    s = (ktiles + per_split - 1) / per_split;
+    *splits = s;
+    const double rounds = (double)((tiles * s + cus - 1) / cus), mb = (double)np * nq * batch * 4e-6;
+    return t.launch + rounds * (t.ktile * per_split + t.store) + (s > 1 ? t.reduce + t.part_mb * s * mb : t.c_mb * mb);
 }
 
 template <typename T>
@@ -318,16 +358,20 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
     // every matrix of a batch must satisfy the same alignment as the first
     const bool batch_aligned = batch == 1 || (g.batch_p % EPC == 0 && g.batch_q % EPC == 0);
     if (!batch_aligned) lp = lq = LD_S;
-    // bf16 operands that are no whole 16-byte vectors but have a unit-stride axis each take the direct-to-LDS kernel's form
+    // operands that are no whole 16-byte vectors but have a unit-stride axis each take the direct-to-LDS kernels' forms
     // for any element address (tiles 128 x 128 and 64 x 64); what is left has the element-wise loader
     int lp_any = LD_S, lq_any = LD_S;
-    if (sizeof(T) == 2 && (lp == LD_S || lq == LD_S) && k > 0 && env_int("AGH_GEMM_DIRECT", 1) != 0) {
-        lp_any = pick_loader_any(g.ps, g.pk, g.K);
-        lq_any = pick_loader_any(g.qs, g.qk, g.K);
+    if ((lp == LD_S || lq == LD_S) && k > 0 && env_int("AGH_GEMM_DIRECT", 1) != 0) {
+        lp_any = pick_loader_any<T>(g.ps, g.pk, g.K);
+        lq_any = pick_loader_any<T>(g.qs, g.qk, g.K);
     }
     const int cus = compute_units() > 0 ? compute_units() : 256;
     const int forced_cfg = env_int("AGH_GEMM_CFG", -1);
-    const bool any_addr = lp_any != LD_S && lq_any != LD_S && (forced_cfg >= 0 || !short_and_narrow(g, batch, cus, lp_any));
+    // f32 up to k = 64 keeps the element-wise loaders: two k-tiles are all filling, and those read only what there is (3889x18x648
+    // 7.9 / 10.7 us, 37905x32x448 28.6 / 37.9, 3460x57x1352 15.2 / 18.5; 584x107x2002 16.4 / 13.3, 5088x95x642 21.8 / 20.2)
+    const bool any_addr = lp_any != LD_S && lq_any != LD_S &&
+                          (forced_cfg >= 0 || (sizeof(T) == 4 ? g.K > 64 : !short_and_narrow(g, batch, cus, lp_any)));
+    const bool skinny = g.NP <= 32 || g.NQ <= 32;  // where the 32 x 128 and 128 x 32 tiles pad less
     const bool any_scalar = (lp == LD_S || lq == LD_S);
     const bool vec_store = g.dp == 1 && g.NP % 4 == 0 && (g.dq % 4 == 0 || g.NQ == 1) && aligned(C, 4 * sizeof(T)) &&
                            (batch == 1 || g.batch_d % 4 == 0);
@@ -347,7 +391,8 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
     for (int i = 0; i < kNumCfgs; ++i) {
         const TileCfg &t = kCfgs[i];
         // (any address: of a 128 x 128 tile over at most 64 rows or columns, half would be padding)
-        if (any_addr ? i != 4 && (i != 3 || g.NP <= 64 || g.NQ <= 64) : any_scalar && !t.scalar_ok) continue;
+        if (any_addr && sizeof(T) == 2 ? i != 4 && (i != 3 || g.NP <= 64 || g.NQ <= 64) : any_scalar && !t.scalar_ok && !(any_addr && i == 3)) continue;
+        if (any_addr && sizeof(T) == 4 && !skinny && i != 3 && i != 4) continue;
         const int64_t tiles = (int64_t)((g.NP + t.bp - 1) / t.bp) * ((g.NQ + t.bq - 1) / t.bq) * batch;
         if (tiles > 0x7FFFFFFF) continue;
         // a CU works through ceil(tiles / CUs) tiles; co-resident workgroups share its MFMA rate
@@ -360,9 +405,10 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
         // the 64 x 64 direct tile is measured at 0.8 of the 256 x 256 tile's rate per CU (3072^3: 118 TFLOP/s, where
         // 144 tiles of 256 x 256 leave 112 CUs idle)
         // f32: the 64 x 64 and 128 x 128 tiles have direct-to-LDS kernels (agh_gemm_f32_dl.h)
-        const bool f32_dl_ok = sizeof(T) == 4 && !any_scalar && g.K > 0 && env_int("AGH_GEMM_DIRECT", 1) != 0;
+        const bool f32_dl_ok = sizeof(T) == 4 && (!any_scalar || any_addr) && g.K > 0 && env_int("AGH_GEMM_DIRECT", 1) != 0;
         const bool f32_direct = f32_dl_ok && t.bp == 64 && t.bq == 64;
-        if (f32_direct) eff = 0.80;
+        // (at any address, against the skinny element-wise tiles alone: 47921 x 2701 x 31 242 / 202 us, 25048 x 751 x 24 41 / 38)
+        if (f32_direct) eff = any_addr ? 0.48 : 0.80;
         if (f32_dl_ok && t.bp == 128 && t.bq == 128) eff = 0.95;  // 4096^3: 135 TFLOP/s, the 256 x 256 tile's rate
         // a tile's prologue and epilogue cost about four k-tiles of time when the CU holds one workgroup, next
         // to nothing when a second workgroup multiplies meanwhile: decides short-k shapes (conv GEMM, k = 576).
@@ -413,7 +459,7 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
         // five k-tiles; of several, one multiplies while another fills, and it is two (1532x25x1126 on 128 x 128 / 64 x 64
         // tiles 7.4 / 5.8 us, 25 of 239x19x204 7.3 / 5.9; over 223 such products the choice is within 0.5 % of the better
         // tile, with three and five it was 6 %).
-        if (any_addr)
+        if (any_addr && sizeof(T) == 2)
             cost = rounds == 1 ? (t.bp == 64 ? 0.52 * (kt + 5.0) : 0.95 * (kt + 3.0)) : (double)rounds * (t.bp == 64 ? 0.38 : 0.75) * (kt + 2.0);
         if (best < 0 || cost < best_cost) { best = i; best_cost = cost; }
     }
@@ -421,6 +467,24 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
 
 #ifdef AGH_GEMM_WITH_F32_DIRECT
     if constexpr (sizeof(T) == 4) {
+        // 64 x 64 or 128 x 128: by fitted times.  The cost above counts a round of 144 to 256 tiles of 128 x 128 like a full one, and those
+        // tiles as if they always shared a CU: 1132x272x3944 44 -> 32 us on 64 x 64, 3632x1008x64 21 -> 12; 133x7001x3003 123 -> 97 on
+        // 128 x 128.  No product's sums get longer by it: where 128 x 128 would be two sums (one workgroup per CU) or more splits of k,
+        // 64 x 64 is taken with two sums, or not at all.
+        const bool f32_direct = (any_addr || !any_scalar) && g.K > 0 && env_int("AGH_GEMM_DIRECT", 1) != 0;
+        if (f32_direct && forced_cfg < 0 && (best == 3 || best == 4) && !(any_addr && skinny) && !setting("AGH_GEMM_SPLITS") &&
+            !setting("AGH_GEMM_KSPLIT")) {
+            int s64, s128;
+            const double us64 = f32_tile_us(64, any_addr, g.NP, g.NQ, g.K, batch, cus, &s64);
+            const double us128 = f32_tile_us(128, any_addr, g.NP, g.NQ, g.K, batch, cus, &s128);
+            const int64_t tiles128 = (int64_t)((g.NP + 127) / 128) * ((g.NQ + 127) / 128) * batch;
+            if (any_addr) best = us128 < us64 ? 3 : 4;
+            else if (best == 4 && us128 < 0.97 * us64) best = 3;
+            else if (best == 3 && us64 < 0.97 * us128 && s64 >= s128) {
+                best = 4;
+                g.two_sums = tiles128 * s128 <= cus;
+            }
+        }
         // Short k and a tile for every CU at least: two workgroups per CU over all tiles.  Over 400 products of 64 to 120000 x 8 to 1200 x 16 to
         // 8192, of those the rule takes 4 are more than 3 % behind the kernels of one tile a workgroup, 6 % at most, all together they are 1.2
         // times as fast (4758 x 32 x 416 10.4 / 7.0 us, 23193 x 256 x 220 40.3 / 31.7; the least 53765 x 256 x 68 40.2 / 40.5; at k = 64 / 128 / 192 /
@@ -441,7 +505,7 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
         bool halves = ksplit > 0;
         if (ksplit < 0 && (best == 3 || best == 4)) {
             const TileCfg &t = kCfgs[best];
-            halves = (int64_t)((g.NP + t.bp - 1) / t.bp) * ((g.NQ + t.bq - 1) / t.bq) <= cus;
+            halves = g.two_sums || (int64_t)((g.NP + t.bp - 1) / t.bp) * ((g.NQ + t.bq - 1) / t.bq) <= cus;
         }
         if (can && env_int("AGH_GEMM_STREAM", suits) != 0) {
             g.tiles_p = (int)tiles_p;
@@ -457,7 +521,7 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
     }
 #endif
 
-    const bool any = any_addr && (best == 3 || best == 4);  // (a forced skinny tile keeps the element-wise loaders)
+    const bool any = any_addr && (best == 3 || best == 4);  // (a skinny tile keeps the element-wise loaders)
     if (any) { lp = lp_any; lq = lq_any; }
     if (best < 0 || best >= kNumCfgs || (any_scalar && !any && !kCfgs[best].scalar_ok))
         return fail(AGH_ERANGE, "%s: no tile configuration for this shape", name);
@@ -467,18 +531,10 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
 
     // ---- split-K when the tile grid cannot fill the chip and k is long ----
     const int64_t tiles = (int64_t)g.tiles_p * g.tiles_q * batch;
-    const int64_t slots = (int64_t)cus;
-    int splits = 1;
     const int ktiles = (g.K + BK - 1) / BK;
-    if (tiles * 2 <= slots && ktiles >= 32 && batch == 1) {
-        int64_t s = slots / tiles;
-        // at least four k-tiles a split; twelve for the bf16 128 x 128 direct tile, whose four-stage ring makes fewer,
-        // longer splits the better trade (128x4096x4096: 17.0-17.2 us in 4 to 6 splits, 19.5 in 8)
-        const int kmin = direct_ok && best == 3 ? 12 : 4;
-        if (s > ktiles / kmin) s = ktiles / kmin;
-        if (s > 256) s = 256;
-        if (s > 1) splits = (int)s;
-    }
+    // at least four k-tiles a split; twelve for the bf16 128 x 128 direct tile, whose four-stage ring makes fewer,
+    // longer splits the better trade (128x4096x4096: 17.0-17.2 us in 4 to 6 splits, 19.5 in 8)
+    int splits = batch == 1 ? plan_splits(tiles, ktiles, cus, direct_ok && best == 3 ? 12 : 4) : 1;
     if (batch == 1) splits = env_int("AGH_GEMM_SPLITS", splits);
     if (splits < 1) splits = 1;
     if (splits > ktiles && ktiles > 0) splits = ktiles;
@@ -514,6 +570,20 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
         return AGH_OK;
     }
     g.store_mode = vec_store ? ST_VEC : ST_SCALAR;
+    if (sizeof(T) == 4 && any && !vec_store && g.dp == 1) {
+        // Rows of C that no 16-byte store fits: P and Q change places, so that a store instruction's lanes lie along C's unit-stride
+        // axis (the products commute and their order over k stays, so the bits do too): whole lines of C instead of 4 bytes in each of 64.
+        std::swap(g.P, g.Q);
+        std::swap(g.ps, g.qs);
+        std::swap(g.pk, g.qk);
+        std::swap(g.NP, g.NQ);
+        std::swap(g.dp, g.dq);
+        std::swap(g.batch_p, g.batch_q);
+        std::swap(g.tiles_p, g.tiles_q);
+        std::swap(lp, lq);
+        g.NPpad = (g.NP + 3) & ~3;
+        g.bias_on_p = !g.bias_on_p;
+    }
     // the direct-to-LDS kernel can transpose its output tile through LDS and store full 16-byte
     // chunks when nothing has to be read back from C
     if (direct && best <= 4 && vec_store && beta == 0.0f && g.NP % 8 == 0 && (g.dq % 8 == 0 || g.NQ == 1) &&

@@ -68,6 +68,7 @@ struct Args {
     float alpha, beta;
     int bias_on_p, has_bias, act;
     int store_mode;
+    int two_sums;  // f32 direct kernels: every k-tile split between two waves whatever the grid
 };
 
 template <typename T> struct Geo;

@@ -1443,3 +1443,38 @@ def test_col2im_rows_wider_than_a_step(ag, monkeypatch, dtype, c, gh, gw, f, s, 
     opts = ag.Col2ImConv2Options(shape=(gh, gw), filter=(f, f), padding=(p, p), stride=(s, s))
     got = ag.Tensor.from_array(x).col2im_conv2(opts).into_array()
     assert np.array_equal(got, orc.col2im_conv2(x, (gh, gw), (f, f), (p, p), (s, s), (1, 1)))
+
+
+@pytest.mark.parametrize("m,k,n", [(33, 65, 33), (127, 96, 129), (65, 97, 255), (201, 131, 67), (130, 1027, 61)])
+def test_gemm_f32_operands_at_any_address(ag, monkeypatch, m, k, n):
+    """The direct-to-LDS f32 kernels' form for rows that are no whole 16-byte vectors: edges of both tiles, k on both sides of a k-tile's
+    end, all four layouts, an odd element offset into every buffer, both tiles and split-K forced.  Whole numbers exactly, with infinities
+    around the views (read, they would show), alpha and beta, the fused bias and relu with the bits of the separate operations."""
+    rng = np.random.default_rng(m)
+
+    def view(values, transposed):
+        h = np.ascontiguousarray(values.T if transposed else values)
+        flat = np.full(h.size + 8, np.inf, np.float32)
+        flat[3:3 + h.size] = h.ravel()
+        t = ag.Tensor.from_array(flat)
+        t = ag.Tensor(t.buffer, h.shape, (h.shape[1], 1), 3, "f32")
+        return t.t() if transposed else t
+    ai, bi = rng.integers(-8, 9, (m, k)).astype(np.float32), rng.integers(-8, 9, (k, n)).astype(np.float32)
+    ar, br, c0 = (rng.uniform(-1, 1, s).astype(np.float32) for s in ((m, k), (k, n), (m, n)))
+    bias = rng.uniform(-1, 1, n).astype(np.float32)
+    for cfg, splits in ((None, None), ("3", None), ("4", None), ("3", "3"), ("4", "3")):
+        for name, value in (("AGH_GEMM_CFG", cfg), ("AGH_GEMM_SPLITS", splits), ("AGH_GEMM_SMALL", "0")):
+            monkeypatch.delenv(name, raising=False)
+            if value is not None:
+                monkeypatch.setenv(name, value)
+        for ta in (False, True):
+            for tb in (False, True):
+                assert np.array_equal(view(ai, ta).dot(view(bi, tb)).into_array(), ai @ bi), (cfg, splits, ta, tb)
+                plain = view(ar, ta).dot(view(br, tb)).into_array()
+                assert_f32_gemm_close(plain, ar, br)
+                C = ag.Tensor.from_array(c0)
+                ag.gemm(0.5, view(ar, ta), view(br, tb), -2.0, C)
+                want = 0.5 * (ar.astype(np.float64) @ br) - 2.0 * c0
+                assert np.abs(C.into_array() - want).max() <= 1e-5 * np.sqrt(k) * (np.abs(ar) @ np.abs(br)).max()
+                fused = view(ar, ta).dot(view(br, tb), bias=ag.Tensor.from_array(bias), relu=True).into_array()
+                assert np.array_equal(fused, orc.relu(orc.bias_add_rows(plain, bias))), (cfg, splits, ta, tb)
