@@ -656,8 +656,11 @@ int conv2_direct_entry(const char *name, const void *x, const void *w, const voi
     if (!x || !w || !y) return fail(AGH_ENULL, "%s: null buffer", name);
 
     // enough channels: implicit GEMM on the matrix cores (returns 1 when the geometry is not its own)
-    const char *env = setting("AGH_CONV_TAPS");  // 0 / 1 forces the choice of the kernel of any geometry (measurements, tests)
-    const int taps_forced = env && *env ? (atoi(env) != 0 ? 1 : 0) : -1;
+    // 0 forbids the kernels of any geometry, 1 forces the one on the f32 matrix cores, 2 that on the bf16 ones (measurements, tests)
+    const char *env = setting("AGH_CONV_TAPS");
+    const int taps_value = env && *env ? atoi(env) : -1;
+    const bool taps16_forced = sizeof(T) == 2 && taps_value == 2;
+    const int taps_forced = taps_value < 0 ? -1 : taps_value != 0 ? 1 : 0;
     const char *small_env = oc <= 16 ? setting("AGH_CONV_SMALL") : nullptr;
     const ConvShape shape = {bs, ic, ih, iw, oc, fh, fw, ph, pw, sh, sw, dh, dw, oh, ow, small_env ? atoi(small_env) != 0 : -1};
     if (shape.unit() && !pool2x2 && taps_forced != 1) {
@@ -668,8 +671,24 @@ int conv2_direct_entry(const char *name, const void *x, const void *w, const voi
     // the matrix-core kernel of any geometry, where it expects to need less time than what would run in its place; with the
     // pool, where the convolution alone would run on it (the fused call returns the same bits as the separate layers)
     const double taps_limit = taps_forced != 0 ? conv2_taps_limit<T>(shape) : 0.0;
-    if (taps_forced == 1 || (taps_limit >= kTapsLeastUs && !(pool2x2 && shape.unit() &&
-                                                            conv2_mfma_takes<T>(x, w, bs, ic, ih, iw, oc, fh, fw, pw, oh, ow)))) {
+    const bool implicit_gemm_plain = pool2x2 && shape.unit() && conv2_mfma_takes<T>(x, w, bs, ic, ih, iw, oc, fh, fw, pw, oh, ow);
+    if (sizeof(T) == 2 && (taps16_forced || (taps_forced < 0 && taps_limit >= kTapsLeastUs && !implicit_gemm_plain))) {
+        double f32_us = 1e30;
+        if (!taps16_forced)
+            conv2_taps_try<T>(name, x, w, bias, y, bs, ic, ih, iw, oc, fh, fw, ph, pw, sh, sw, dh, dw, oh, ow, act, false, false, 0.0, &f32_us);
+        // Where the f32 kernel would be taken otherwise, its second launch (the packed bank, 3 us of a program's time) has to be worth it:
+        // two microseconds and a quarter of a time that is on the safe side (12 x 12 pixels, 32 to 16 channels, 3 x 3: 10.4 us there, 13.7 here).
+        // Over 250 shapes the choice is 6 % behind the best of the three, two are 4 and 6 % slower than before.  Against im2col and a product a
+        // tenth is left for the estimate's error (33 x 128 x 12 x 76 to 256, 3 x 3: 75 us there, 83 here).
+        const double limit = f32_us <= taps_limit ? 0.75 * f32_us - 2.0 : 0.9 * taps_limit;
+        const int rc = !taps16_forced && limit < kTaps16LeastUs
+                           ? 1
+                           : conv2_taps16_try(name, x, w, bias, y, bs, ic, ih, iw, oc, fh, fw, ph, pw, sh, sw, dh, dw, oh, ow, act, pool2x2 != 0,
+                                              taps16_forced, limit);
+        if (rc != 1) return rc;
+        if (taps16_forced) return fail(AGH_ERANGE, "%s: AGH_CONV_TAPS=2, and that kernel does not take this shape", name);
+    }
+    if (taps_forced == 1 || (taps_limit >= kTapsLeastUs && !implicit_gemm_plain)) {
         const int rc = conv2_taps_try<T>(name, x, w, bias, y, bs, ic, ih, iw, oc, fh, fw, ph, pw, sh, sw, dh, dw, oh, ow, act, pool2x2 != 0,
                                          taps_forced == 1, taps_limit);
         if (rc != 1) return rc;

@@ -287,7 +287,7 @@ static int taps_launch(const char *name, const void *x, const void *w, const voi
 template <typename T>
 int conv2_taps_try(const char *name, const void *x, const void *w, const void *bias, void *y, int64_t bs, int64_t ic, int64_t ih,
                    int64_t iw, int64_t oc, int64_t fh, int64_t fw, int64_t ph, int64_t pw, int64_t sh, int64_t sw, int64_t dh,
-                   int64_t dw, int64_t oh, int64_t ow, int act, bool pool, bool forced, double limit_us) {
+                   int64_t dw, int64_t oh, int64_t ow, int act, bool pool, bool forced, double limit_us, double *estimate_us) {
     const int64_t npos = oh * ow, ktot = ic * fh * fw, pitch = ((ow - 1) * sw + (fw - 1) * dw + 4) & ~(int64_t)3;
     if (npos > ((int64_t)1 << 24) || ktot > ((int64_t)1 << 24) || oc * ktot > ((int64_t)1 << 28)) return 1;
     // tile: rounds of workgroups times the matrix cycles of one (16 positions x 16 channels x 4 taps = 32 cycles, each wave
@@ -322,7 +322,8 @@ int conv2_taps_try(const char *name, const void *x, const void *w, const void *b
             }
         }
     }
-    if (!tg || (!forced && us > limit_us)) return 1;
+    if (estimate_us) *estimate_us = tg ? us : 1e30;
+    if (!tg || estimate_us || (!forced && us > limit_us)) return 1;
     // the pool is fused where the convolution alone would run here, and stages as many channels at a time (the order of the
     // sums); only the tile's positions are fewer where its rows, less than three times as many, take too much of the LDS
     const int64_t ntab = (chunk * fh * fw + 15) & ~(int64_t)15, yh = pool ? oh / 2 : oh, yw = pool ? ow / 2 : ow;
@@ -356,8 +357,8 @@ int conv2_taps_try(const char *name, const void *x, const void *w, const void *b
 }
 
 template int conv2_taps_try<float>(const char *, const void *, const void *, const void *, void *, int64_t, int64_t, int64_t, int64_t,
-                                   int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int, bool, bool, double);
+                                   int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int, bool, bool, double, double *);
 template int conv2_taps_try<uint16_t>(const char *, const void *, const void *, const void *, void *, int64_t, int64_t, int64_t, int64_t,
-                                      int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int, bool, bool, double);
+                                      int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int, bool, bool, double, double *);
 
 }  // namespace agh

@@ -21,6 +21,8 @@ int fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));
 int hip_fail(hipError_t e, const char *what);
 // Scratch owned by the library (split-K partials); grows on demand, never shrinks.
 int workspace(size_t bytes, void **ptr);
+// whether workspace() can serve so many bytes now (inside a capture it cannot grow)
+bool workspace_ready(size_t bytes);
 // The fixed scratch buffer of agh_gemm_bf16_noalloc instead: never allocates, fails beyond its size.
 int static_workspace(size_t bytes, void **ptr);
 // Conv2 forward as an implicit GEMM (agh_conv_mfma.hip), T = uint16_t (bf16) or float; 1 = geometry not taken,
@@ -35,11 +37,16 @@ bool conv2_mfma_takes(const void *x, const void *w, int64_t bs, int64_t ic, int6
 constexpr double kTapsLeastUs = 4.4;  // what no shape is expected to need less than in the kernel below
 // Conv2 forward for any stride, dilation and channel count on the f32 matrix cores (agh_conv_taps.hip), followed by the
 // 2x2 pool where `pool`; 1 = not taken: the shape is not its own, or the convolution is expected to need more than
-// limit_us there (and is not forced)
+// limit_us there (and is not forced).  With `estimate_us`, only says there what the convolution is expected to need, and returns 1.
 template <typename T>
 int conv2_taps_try(const char *name, const void *x, const void *w, const void *bias, void *y, int64_t bs, int64_t ic, int64_t ih,
                    int64_t iw, int64_t oc, int64_t fh, int64_t fw, int64_t ph, int64_t pw, int64_t sh, int64_t sw, int64_t dh,
-                   int64_t dw, int64_t oh, int64_t ow, int act, bool pool, bool forced, double limit_us);
+                   int64_t dw, int64_t oh, int64_t ow, int act, bool pool, bool forced, double limit_us, double *estimate_us = nullptr);
+// The same on the bf16 matrix cores (agh_conv_taps_bf16.hip)
+constexpr double kTaps16LeastUs = 6.4;  // what no shape is expected to need less than there
+int conv2_taps16_try(const char *name, const void *x, const void *w, const void *bias, void *y, int64_t bs, int64_t ic, int64_t ih,
+                     int64_t iw, int64_t oc, int64_t fh, int64_t fw, int64_t ph, int64_t pw, int64_t sh, int64_t sw, int64_t dh,
+                     int64_t dw, int64_t oh, int64_t ow, int act, bool pool, bool forced, double limit_us);
 
 // Variables AGH_* that force a choice (measurements, tests) are read at every call; looked up one by one they cost a call of a small
 // product a quarter of its host time.  The first one that a call asks for walks the environment once and notes the few entries that begin

@@ -140,6 +140,11 @@ int workspace(size_t bytes, void **ptr) {
     return AGH_OK;
 }
 
+bool workspace_ready(size_t bytes) {
+    const bool side = g_cur == g_side && g_side != nullptr;
+    return !g_capturing || bytes <= (side ? g_ws_side : g_ws).bytes;
+}
+
 int static_workspace(size_t bytes, void **ptr) {
     if (g_cur != g_stream)
         return fail(AGH_EINVAL, "agh_gemm_bf16_noalloc: called inside a branch, where it would share the fixed scratch "

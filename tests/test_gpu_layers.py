@@ -231,6 +231,82 @@ def test_conv2_taps_kernel_sums_in_parts(ag, ic, f, monkeypatch):
     assert error(got.astype(np.float64)) <= 0.4 * error(chain.astype(np.float64)), (error(got), error(chain))
 
 
+CONV_TAPS16 = CONV_TAPS_TILES + [
+    (2, 1, 21, 17, 6, (7, 7), (3, 3), (2, 2), (1, 1)),       # one channel of a group of eight, 49 units in 13 steps
+    (1, 8, 12, 130, 16, (1, 4), (0, 2), (1, 1), (1, 2)),     # four units: one step exactly
+    (1, 256, 9, 8, 40, (3, 3), (0, 0), (1, 1), (1, 1)),      # a position tile larger than the image
+    (3, 20, 15, 1, 70, (3, 1), (1, 0), (1, 1), (1, 1)),      # rows of one pixel, the last group of channels half empty
+    (1, 128, 30, 101, 64, (5, 5), (2, 2), (2, 2), (1, 1)),   # channels in passes
+]
+
+
+@pytest.mark.parametrize("case", CONV_TAPS16)
+def test_conv2_taps_kernel_on_the_bf16_matrix_cores(ag, case, monkeypatch):
+    """The same in bf16 throughout, every tile forced: whole numbers exactly, random values within a rounding of the f32 sum, an infinite
+    input reaches the outputs it has a tap to and no others (padding and missing channels multiply nothing), the fused pool returns the
+    bits of the separate one."""
+    bs, ic, ih, iw, oc, f, p, s, d = case
+    rng = np.random.default_rng(38)
+    k = ic * f[0] * f[1]
+    xi, wi = rng.integers(-3, 4, (bs, ic, ih, iw)).astype(np.float32), rng.integers(-3, 4, (oc, ic) + f).astype(np.float32)
+    exact = to_dtype(orc.conv2_naive_f64(xi, wi, p, s, d).astype(np.float32), "bf16")
+    x = rng.standard_normal((bs, ic, ih, iw)).astype(np.float32)
+    x[bs - 1, ic - 1, ih // 2 // s[0] * s[0], iw // 2 // s[1] * s[1]] = np.inf
+    x = to_dtype(x, "bf16")
+    w = to_dtype(rng.standard_normal((oc, ic) + f) * np.sqrt(2.0 / k), "bf16")
+    with np.errstate(invalid="ignore"):
+        want = orc.conv2_naive_f64(as_f32(x), as_f32(w), p, s, d)
+    fin = np.isfinite(want)
+    scale = orc.conv2_naive_f64(np.where(np.isfinite(as_f32(x)), np.abs(as_f32(x)), 0).astype(np.float32), np.abs(as_f32(w)), p, s, d)
+    bound = 8 * np.sqrt(k) * 2.0**-24 * scale + 2.0 ** (np.floor(np.log2(np.maximum(np.abs(np.where(fin, want, 0)), 2.0**-126))) - 7)
+    b = ag.Tensor.from_array(to_dtype(rng.standard_normal(oc) * 0.1, "bf16"))
+    tx, tw, txi, twi = (ag.Tensor.from_array(a) for a in (x, w, to_dtype(xi, "bf16"), to_dtype(wi, "bf16")))
+    monkeypatch.setenv("AGH_CONV_TAPS", "2")
+    kw = dict(padding=p, stride=s, dilation=d)
+    for tile in [""] + [str(10 * tg + nt) for tg in (1, 2, 4) for nt in (1, 2, 3, 4)]:
+        monkeypatch.setenv("AGH_CONV_TAPS_TILE", tile)
+        assert np.array_equal(ag.conv2_direct_forward(txi, twi, **kw).into_array(), exact), tile
+        y = as_f32(ag.conv2_direct_forward(tx, tw, **kw).into_array())
+        assert np.array_equal(np.isfinite(y), fin), tile
+        assert np.all(np.abs(y[fin] - want[fin]) <= bound[fin]), tile
+        if y.shape[2] > 1 and y.shape[3] > 1:
+            plain = ag.conv2_direct_forward(txi, twi, bias=b, relu=True, **kw)
+            fused = ag.conv2_direct_forward(txi, twi, bias=b, relu=True, pool2x2=True, **kw).into_array()
+            assert np.array_equal(fused, ag.MaxPool2((2, 2)).forward(plain).into_array()), tile
+
+
+def test_conv2_taps_bf16_captured(ag):
+    """A convolution with a packed filter bank inside a captured graph: on the main stream the bits of the eager call at every replay; in a
+    branch, whose scratch memory may not be there yet and cannot grow, it is captured all the same (on the kernel without a bank)."""
+    rng = np.random.default_rng(39)
+    x = ag.Tensor.from_array(to_dtype(rng.standard_normal((4, 32, 41, 41)), "bf16"))
+    w = ag.Tensor.from_array(to_dtype(rng.standard_normal((48, 32, 5, 5)) * 0.05, "bf16"))
+    y, z = (ag.Tensor.uninit((4, 48, 37, 37), "bf16") for _ in range(2))
+    check, lib = ag._ffi.check, ag.lib
+
+    def call(out):
+        check(lib.agh_conv2_direct_bf16(x._data_ptr(), w._data_ptr(), None, out._ptr(), 4, 32, 41, 41, 48, 5, 5, 0, 0, 1, 1, 1, 1, 0, 0))
+    call(y)
+    want = y.into_array()
+    graph = C.c_void_p()
+    check(lib.agh_graph_begin())
+    check(lib.agh_branch_begin())
+    call(z)
+    check(lib.agh_branch_end())
+    call(y)
+    check(lib.agh_branch_join())
+    check(lib.agh_graph_end(C.byref(graph)))
+    for _ in range(3):
+        for t in (y, z):
+            check(lib.agh_memset(t._ptr(), 0, t.buffer.nbytes))
+        check(lib.agh_graph_launch(graph))
+        check(lib.agh_sync())
+        assert np.array_equal(y.into_array(), want)
+        got, ref = as_f32(z.into_array()), as_f32(want)
+        assert np.all(np.abs(got - ref) <= 2.0**-7 * np.abs(ref) + 1e-4)  # another order of sums of 800 terms below 1, one rounding
+    check(lib.agh_graph_destroy(graph))
+
+
 CONV_TAPS_POOL = [
     # bs, ic, ih, iw, oc, filter, padding, stride: the convolution alone runs out of staged rows
     (64, 3, 64, 64, 64, (3, 3), (1, 1), (1, 1)),
