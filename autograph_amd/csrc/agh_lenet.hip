@@ -1,5 +1,7 @@
 // The LeNet5 of the reference's benchmark (benches/neural-network-benches/src/autograph_backend.rs:70-162): inference in one
 // launch, and the launches of its training step.
+#include <type_traits>
+
 #include "agh_internal.h"
 
 using namespace agh;
@@ -130,24 +132,38 @@ __device__ __forceinline__ uint32_t lds_address_of(const void *p) {
 // conv2's taps split between two waves per pooled row), so that a stage takes a quarter of the time: the launch is a
 // chain of stage latencies, and with four images per workgroup a small batch would leave most of the chip idle while
 // each busy CU walks four images' worth of every stage.
-template <typename T, bool SAVE, int IMGS>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void lenet5_forward_kernel(const T *__restrict__ x, const T *__restrict__ w1,
-                                                              const T *__restrict__ w2, const T *__restrict__ wd1,
-                                                              const T *__restrict__ wd2, const T *__restrict__ wd3,
-                                                              const T *__restrict__ b3, T *__restrict__ out, int bs,
-                                                              LenetSaves<T> sv, int w23_aligned) {
+template <typename T, int IMGS>
+struct LenetForwardLds {
+    __align__(16) float xs[IMGS * 28 * 28];     // input images, pitch 28
+    __align__(16) float w1s[25 * 6];            // [tap][oc]
+    __align__(16) float p1[IMGS * 6 * 12 * 12]; // after conv1 + relu + pool
+    __align__(16) float w2s[160 * 16];          // [ci][fi][fj][oc], ten rows of zeros behind the 150 taps
+    int tap2[160];                              // byte offset of tap k inside an image of p1 (0 behind the taps)
+    __align__(16) float p2[IMGS * 256];         // after conv2 + relu + pool, flattened [c][h][w]
+    __align__(16) float d1[IMGS * 128];
+    __align__(16) float d2[IMGS * 84];
+    __align__(16) float parts[16 * IMGS * 128];  // dense1 partial sums
+    __align__(16) T wd2s[128 * 84];              // dense2 / dense3 weights as they lie in memory
+    __align__(16) T wd3s[1024];                  // (84 * 10, rounded up to whole KB)
+};
+// What the backward half of the same launch reads in place of the saved copies: the dense layers' outputs before the relu and the logits
+struct LenetStepLds {
+    float pre1[128], pre2[84], lg[10];
+};
+
+// `conv_done` runs behind the barrier after which both convolutions' outputs are saved; `step` (one image a workgroup) is filled if not null
+// WHOLE: with one image a workgroup, conv2's sums over all taps in one chain, as four images a workgroup have them (a batch above 256 then
+// gives the same bits either way)
+template <typename T, bool SAVE, int IMGS, bool WHOLE, typename F>
+__device__ __forceinline__ void lenet5_forward_body(LenetForwardLds<T, IMGS> &s, const T *__restrict__ x, const T *__restrict__ w1,
+                                                    const T *__restrict__ w2, const T *__restrict__ wd1, const T *__restrict__ wd2,
+                                                    const T *__restrict__ wd3, const T *__restrict__ b3, T *__restrict__ out, int bs,
+                                                    LenetSaves<T> sv, int w23_aligned, LenetStepLds *step, float4 (&wreg)[16], F &&conv_done) {
     static_assert(IMGS == 1 || IMGS == 4, "one image or four per workgroup");
-    __shared__ __align__(16) float xs[IMGS * 28 * 28];     // input images, pitch 28
-    __shared__ __align__(16) float w1s[25 * 6];            // [tap][oc]
-    __shared__ __align__(16) float p1[IMGS * 6 * 12 * 12]; // after conv1 + relu + pool
-    __shared__ __align__(16) float w2s[160 * 16];          // [ci][fi][fj][oc], ten rows of zeros behind the 150 taps
-    __shared__ int tap2[160];                              // byte offset of tap k inside an image of p1 (0 behind the taps)
-    __shared__ __align__(16) float p2[IMGS * 256];         // after conv2 + relu + pool, flattened [c][h][w]
-    __shared__ __align__(16) float d1[IMGS * 128];
-    __shared__ __align__(16) float d2[IMGS * 84];
-    __shared__ __align__(16) float parts[16 * IMGS * 128];  // dense1 partial sums
-    __shared__ __align__(16) T wd2s[128 * 84];              // dense2 / dense3 weights as they lie in memory
-    __shared__ __align__(16) T wd3s[1024];                  // (84 * 10, rounded up to whole KB)
+    float *const xs = s.xs, *const w1s = s.w1s, *const p1 = s.p1, *const w2s = s.w2s, *const p2 = s.p2, *const d1 = s.d1, *const d2 = s.d2,
+                 *const parts = s.parts;
+    int *const tap2 = s.tap2;
+    T *const wd2s = s.wd2s, *const wd3s = s.wd3s;
     constexpr int NT = 512;  // 8 waves: two per SIMD, so one can wait on LDS while the other multiplies
     constexpr int kD3Off = 4 * IMGS * 84;  // dense3's partial sums in `parts`, behind dense2's
     const int tid = threadIdx.x;
@@ -173,16 +189,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         const T *xb = x + (size_t)b0 * 784;
 #pragma unroll
         for (int u = 0; u < XU; ++u) xv[u] = xb[min(tid + u * NT, nx - 1)];
-        if (tid < 150) w1s[tid] = Elem<T>::to_f32(w1v);
+        // (widened plainly: all of it is only ever multiplied, which quiets a signalling NaN by itself)
+        if (tid < 150) w1s[tid] = Elem<T>::raw(w1v);
 #pragma unroll
         for (int u = 0; u < 5; ++u) {
             const int e = tid + u * NT;
-            w2s[e] = (e >> 4) < 150 ? Elem<T>::to_f32(w2v[u]) : 0.0f;
+            w2s[e] = (e >> 4) < 150 ? Elem<T>::raw(w2v[u]) : 0.0f;
         }
 #pragma unroll
         for (int u = 0; u < XU; ++u) {
             const int e = tid + u * NT;
-            if (e < IMGS * 784) xs[e] = e < nx ? Elem<T>::to_f32(xv[u]) : 0.0f;
+            if (e < IMGS * 784) xs[e] = e < nx ? Elem<T>::raw(xv[u]) : 0.0f;
         }
     }
     if (tid < 160) {
@@ -190,7 +207,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         tap2[tid] = tid < 150 ? (ci * 144 + fi * 12 + fj) * 4 : 0;
     }
     // dense1 weights of this thread (see the dense1 stage below), requested now, used much later
-    float4 wreg[16];
     {
         const int cg = tid & 31, kg = tid >> 5;
 #pragma unroll
@@ -200,8 +216,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 wreg[kk] = *(const float4 *)src;
             } else {
                 const uint2 raw = *(const uint2 *)src;
-                wreg[kk] = make_float4(bf16_to_f32((uint16_t)(raw.x & 0xFFFF)), bf16_to_f32((uint16_t)(raw.x >> 16)),
-                                       bf16_to_f32((uint16_t)(raw.y & 0xFFFF)), bf16_to_f32((uint16_t)(raw.y >> 16)));
+                wreg[kk] = make_float4(__uint_as_float(raw.x << 16), __uint_as_float(raw.x & 0xFFFF0000u), __uint_as_float(raw.y << 16),
+                                       __uint_as_float(raw.y & 0xFFFF0000u));
             }
         }
     }
@@ -289,24 +305,28 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         const char *abase = (const char *)(p1 + (2 * row + ((i >> 1) & 1)) * 12 + 2 * (i >> 2) + (i & 1));
         const char *Bl = (const char *)(w2s + lane) + kh * 20 * 256, *tl = (const char *)(tap2 + g) + kh * 20 * 16;
         f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        float bq[20];
-        int tq[20];
-#pragma unroll
-        for (int q = 0; q < 20; ++q) {
-            bq[q] = *(const float *)(Bl + q * 256);
-            tq[q] = *(const int *)(tl + q * 16);
-        }
-#pragma unroll
-        for (int q = 0; q < 20; ++q) {
-            float a = *(const float *)(abase + tq[q]);
-            if (4 * (kh * 20 + q) + g >= 150) a = 0.0f;  // behind the taps: zero times zero, whatever p1 holds
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a, bq[q], acc, 0, 0, 0);
-        }
         f32x4_t *xch = (f32x4_t *)parts;  // free until dense1
-        if (kh == 1) xch[row * 64 + lane] = acc;
-        __syncthreads();
+#pragma unroll
+        for (int part = 0; part < (WHOLE ? 2 : 1); ++part) {
+            if (WHOLE && kh == 1) break;  // (waves 0 to 3 take the second half too)
+            float bq[20];
+            int tq[20];
+#pragma unroll
+            for (int q = 0; q < 20; ++q) {
+                bq[q] = *(const float *)(Bl + (part * 20 + q) * 256);
+                tq[q] = *(const int *)(tl + (part * 20 + q) * 16);
+            }
+#pragma unroll
+            for (int q = 0; q < 20; ++q) {
+                float a = *(const float *)(abase + tq[q]);
+                if (4 * ((WHOLE ? part : kh) * 20 + q) + g >= 150) a = 0.0f;  // behind the taps: zero times zero, whatever p1 holds
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a, bq[q], acc, 0, 0, 0);
+            }
+        }
+        if (!WHOLE && kh == 1) xch[row * 64 + lane] = acc;
+        if (!WHOLE) __syncthreads();
         if (kh == 0) {
-            acc += xch[row * 64 + lane];
+            if (!WHOLE) acc += xch[row * 64 + lane];
             const T zero = Elem<T>::zero();
             float mf = Elem<T>::to_f32(round_bias_relu<T>(acc[0], false, zero, AGH_ACT_RELU));
 #pragma unroll
@@ -390,6 +410,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
     }
     __syncthreads();
+    conv_done();
 
     // dense1 256 -> 128 + relu.  Thread (cg, kg) owns the weights W1[16kg .. 16kg+15][4cg .. 4cg+3]; they
     // were fetched into registers at the top of the kernel (16 coalesced 16-byte loads per thread, in
@@ -434,6 +455,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int kg = 0; kg < 16; ++kg) a += parts[kg * IMGS * 128 + o];
         const T act = round_bias_relu<T>(a, false, Elem<T>::zero(), AGH_ACT_RELU);
         d1[o] = Elem<T>::to_f32(act);
+        if constexpr (SAVE && IMGS == 1) if (step) step->pre1[o] = Elem<T>::to_f32(Elem<T>::from_f32(a));
         if constexpr (SAVE) {
             if ((o >> 7) < nimg) {
                 sv.d1[(size_t)b0 * 128 + o] = Elem<T>::from_f32(a);
@@ -458,8 +480,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             float4 xk[IMGS];
 #pragma unroll
             for (int r = 0; r < IMGS; ++r) xk[r] = *(const float4 *)(d1 + r * 128 + k);
-            const float w0 = Elem<T>::to_f32(wd2s[k * 84 + c]), w1v = Elem<T>::to_f32(wd2s[(k + 1) * 84 + c]);
-            const float w2v = Elem<T>::to_f32(wd2s[(k + 2) * 84 + c]), w3v = Elem<T>::to_f32(wd2s[(k + 3) * 84 + c]);
+            const float w0 = Elem<T>::raw(wd2s[k * 84 + c]), w1v = Elem<T>::raw(wd2s[(k + 1) * 84 + c]);
+            const float w2v = Elem<T>::raw(wd2s[(k + 2) * 84 + c]), w3v = Elem<T>::raw(wd2s[(k + 3) * 84 + c]);
 #pragma unroll
             for (int r = 0; r < IMGS; ++r) {
                 part[r] = __builtin_fmaf(xk[r].x, w0, part[r]);
@@ -479,6 +501,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int kq = 1; kq < 4; ++kq) a += parts[kq * IMGS * 84 + tid];
         const T act = round_bias_relu<T>(a, false, Elem<T>::zero(), AGH_ACT_RELU);
         d2[tid] = Elem<T>::to_f32(act);
+        if constexpr (SAVE && IMGS == 1) if (step) step->pre2[tid] = Elem<T>::to_f32(Elem<T>::from_f32(a));
         if constexpr (SAVE) {
             if (r < nimg) {
                 sv.d2[(size_t)b0 * 84 + tid] = Elem<T>::from_f32(a);
@@ -496,10 +519,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (int kk = 0; kk < 12; kk += 4) {
             const float4 xk = *(const float4 *)(xr + kk);
             const int k = kp * 12 + kk;
-            a = __builtin_fmaf(xk.x, Elem<T>::to_f32(wd3s[k * 10 + c]), a);
-            a = __builtin_fmaf(xk.y, Elem<T>::to_f32(wd3s[(k + 1) * 10 + c]), a);
-            a = __builtin_fmaf(xk.z, Elem<T>::to_f32(wd3s[(k + 2) * 10 + c]), a);
-            a = __builtin_fmaf(xk.w, Elem<T>::to_f32(wd3s[(k + 3) * 10 + c]), a);
+            a = __builtin_fmaf(xk.x, Elem<T>::raw(wd3s[k * 10 + c]), a);
+            a = __builtin_fmaf(xk.y, Elem<T>::raw(wd3s[(k + 1) * 10 + c]), a);
+            a = __builtin_fmaf(xk.z, Elem<T>::raw(wd3s[(k + 2) * 10 + c]), a);
+            a = __builtin_fmaf(xk.w, Elem<T>::raw(wd3s[(k + 3) * 10 + c]), a);
         }
         parts[kD3Off + tid] = a;  // behind the dense2 partials, which other waves may still be reading
     }
@@ -509,8 +532,21 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         float a = parts[kD3Off + tid];
 #pragma unroll
         for (int kp = 1; kp < 7; ++kp) a += parts[kD3Off + kp * IMGS * 10 + tid];
-        if (r < nimg) out[(size_t)(b0 + r) * 10 + c] = round_bias_relu<T>(a, true, b3[c], AGH_ACT_NONE);
+        const T logit = round_bias_relu<T>(a, true, b3[c], AGH_ACT_NONE);
+        if constexpr (SAVE && IMGS == 1) if (step) step->lg[c] = Elem<T>::to_f32(logit);
+        if (r < nimg) out[(size_t)(b0 + r) * 10 + c] = logit;
     }
+}
+
+template <typename T, bool SAVE, int IMGS>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void lenet5_forward_kernel(const T *__restrict__ x, const T *__restrict__ w1,
+                                                              const T *__restrict__ w2, const T *__restrict__ wd1,
+                                                              const T *__restrict__ wd2, const T *__restrict__ wd3,
+                                                              const T *__restrict__ b3, T *__restrict__ out, int bs,
+                                                              LenetSaves<T> sv, int w23_aligned) {
+    __shared__ LenetForwardLds<T, IMGS> s;
+    float4 wreg[16];
+    lenet5_forward_body<T, SAVE, IMGS, false>(s, x, w1, w2, wd1, wd2, wd3, b3, out, bs, sv, w23_aligned, nullptr, wreg, [] {});
 }
 
 // The input-gradient chain of a LeNet5 training step in one launch, one workgroup per image: cross-entropy backward,
@@ -548,12 +584,74 @@ __device__ __forceinline__ void pool_relu_window_backward(const T (&xv)[4], floa
     for (int k = 0; k < 4; ++k) cell[k] = (am == k && Elem<T>::raw(xv[k]) >= 0.0f) ? g : Elem<T>::zero();
 }
 
+constexpr int kPmPitch = 151;  // odd: the col2im reads of neighbouring pixels fall into different banks
+// The product gm2 [64 positions, 16 channels] . W [16, 150 taps] of conv2's input gradient, every entry rounded to T, by NW waves: forty tiles of
+// 16 positions x 16 taps, four v_mfma_f32_16x16x4_f32 each (as FMAs 5400 cycles of the training step's launch)
+template <typename T, int NW>
+__device__ __forceinline__ void lenet5_pm(const float *gm2s, const float *wl, float *pm) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, i = lane & 15;
+    static_assert(40 % NW == 0, "whole rounds of tiles");
+#pragma unroll
+    for (int n = 0; n < 40 / NW; ++n) {
+        const int unit = wave + NW * n, pt = unit & 3, k = (unit >> 2) * 16 + i;
+        // MFMA q takes channel 4 g + q of lane group g on both sides: one 16-byte read each
+        const f32x4_t va = *(const f32x4_t *)(gm2s + (pt * 16 + i) * 16 + 4 * g), vb = *(const f32x4_t *)(wl + min(k, 149) * 16 + 4 * g);
+        f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(va[q], vb[q], acc, 0, 0, 0);
+        if (k < 150) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) pm[(pt * 16 + 4 * g + r) * kPmPitch + k] = Elem<T>::to_f32(Elem<T>::from_f32(acc[r]));
+        }
+    }
+}
+
+// One row of dense2's input gradient, 84 products: part q of four chains the groups of four q, q + 4, ..., the parts are added (0 + 1) + (2 + 3),
+// the order in which four lanes of lenet5_step_image_kernel share a row
+template <typename G, typename W>
+__device__ __forceinline__ float dense2_row_sum(G &&g, W &&w) {
+    float v[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        v[q] = 0.0f;
+#pragma unroll
+        for (int c = q; c < 21; c += 4)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[q] = __builtin_fmaf(g(4 * c + e), w(4 * c + e), v[q]);
+    }
+    return (v[0] + v[1]) + (v[2] + v[3]);
+}
+
+// One row of dense1's input gradient, 128 products: 32 chains of four neighbouring ones, added pairwise (i with i + 16, then + 8 ... + 1), the order
+// in which the lanes of lenet5_step_image_kernel add them
+template <typename G, typename W>
+__device__ __forceinline__ float dense1_row_sum(G &&g, W &&w) {
+    float v[32];
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+        v[i] = 0.0f;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) v[i] = __builtin_fmaf(g(4 * i + c), w(4 * i + c), v[i]);
+    }
+    // (by constants: an array indexed by the variable of a loop that is not unrolled costs a select per element)
+    auto fold = [&](auto halfc) {
+        constexpr int half = decltype(halfc)::value;
+#pragma unroll
+        for (int i = 0; i < half; ++i) v[i] += v[i + half];
+    };
+    fold(std::integral_constant<int, 16>{});
+    fold(std::integral_constant<int, 8>{});
+    fold(std::integral_constant<int, 4>{});
+    fold(std::integral_constant<int, 2>{});
+    fold(std::integral_constant<int, 1>{});
+    return v[0];
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void lenet5_backward_kernel(LenetBackward<T> a) {
     __shared__ __align__(16) float wl[150 * 16];   // conv2's filter bank, [ci*25 + fi*5 + fj][oc]
     __shared__ __align__(16) float gm2s[64 * 16];  // gradient of conv2's output, [y*8 + x][oc]
     __shared__ float gls[16], gd2s[84], gd1s[128], gfs[256], gp1s[864];
-    constexpr int kPmPitch = 151;                  // odd: the col2im reads of neighbouring pixels fall into different banks
     __shared__ float pm[64 * kPmPitch];            // gm2 . W, every entry rounded to T
     constexpr int NT = 256;
     constexpr int EPV = 16 / (int)sizeof(T);  // elements per 16-byte load
@@ -643,9 +741,7 @@ __global__ __launch_bounds__(256) void lenet5_backward_kernel(LenetBackward<T> a
     __syncthreads();
     // dense2: g_a1 = g_d2 . wd2^T (wd2 [128, 84]), relu backward on dense1's pre-activation
     if (tid < 128) {
-        float d = 0.0f;
-#pragma unroll
-        for (int c = 0; c < 84; ++c) d = __builtin_fmaf(gd2s[c], elem(w2r, c), d);
+        const float d = dense2_row_sum([&](int c) { return gd2s[c]; }, [&](int c) { return elem(w2r, c); });
         const T ga = Elem<T>::from_f32(d);
         const T gd = Elem<T>::raw(d1v) >= 0.0f ? ga : Elem<T>::zero();
         a.g_d1[b * 128 + tid] = gd;
@@ -653,12 +749,7 @@ __global__ __launch_bounds__(256) void lenet5_backward_kernel(LenetBackward<T> a
     }
     __syncthreads();
     // dense1: g_f = g_d1 . wd1^T (wd1 [256, 128])
-    {
-        float d = 0.0f;
-#pragma unroll
-        for (int c = 0; c < 128; ++c) d = __builtin_fmaf(gd1s[c], elem(w1r, c), d);
-        gfs[tid] = Elem<T>::to_f32(Elem<T>::from_f32(d));
-    }
+    gfs[tid] = Elem<T>::to_f32(Elem<T>::from_f32(dense1_row_sum([&](int c) { return gd1s[c]; }, [&](int c) { return elem(w1r, c); })));
     __syncthreads();
     // pooling + relu backward of conv2's output: one window per thread (16 channels x 4 x 4 windows)
     {
@@ -673,36 +764,9 @@ __global__ __launch_bounds__(256) void lenet5_backward_kernel(LenetBackward<T> a
         }
     }
     __syncthreads();
-    // conv2's input gradient in two steps, as the host does it.  First the product gm2 . W, a [64, 150] matrix whose
-    // entries are f32 dots over the 16 output channels (ascending) rounded to T: a thread owns 4 positions x 10 taps and
-    // keeps its four gradient rows in registers, so an entry costs a fraction of the LDS reads a per-pixel walk would need.
-    if (tid < 240) {
-        const int pg = tid / 15, kg = tid - pg * 15;
-        float4 g[4][4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) g[r][q] = *(const float4 *)(gm2s + (pg * 4 + r) * 16 + q * 4);
-#pragma unroll 2
-        for (int kk = 0; kk < 10; ++kk) {
-            const int k = kg * 10 + kk;
-            float4 w[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) w[q] = *(const float4 *)(wl + k * 16 + q * 4);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                float d = 0.0f;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    d = __builtin_fmaf(g[r][q].x, w[q].x, d);
-                    d = __builtin_fmaf(g[r][q].y, w[q].y, d);
-                    d = __builtin_fmaf(g[r][q].z, w[q].z, d);
-                    d = __builtin_fmaf(g[r][q].w, w[q].w, d);
-                }
-                pm[(pg * 4 + r) * kPmPitch + k] = Elem<T>::to_f32(Elem<T>::from_f32(d));
-            }
-        }
-    }
+    // conv2's input gradient in two steps, as the host does it: the product gm2 . W, a [64, 150] matrix whose entries are f32 dots over the 16
+    // output channels rounded to T,
+    lenet5_pm<T, NT / 64>(gm2s, wl, pm);
     __syncthreads();
     // then col2im: per pixel of the [6, 12, 12] map the patch entries that land on it, added in T in the host's order
     // (filter rows and columns descending)
@@ -781,21 +845,51 @@ struct LenetDenseGrads {
     int bs;
 };
 
-// 256 threads of workgroup `wg` (of 184)
+// The update of a training step, applied by whoever finishes a gradient: scaled_add with -lr (no velocities) or SGD with momentum, operation
+// for operation as scaled_add_kernel and sgd_momentum_kernel do it.  Order: conv1, conv2, dense1, dense2, dense3, dense3's bias.
 template <typename T>
-__device__ __forceinline__ void lenet5_dense_grads(const LenetDenseGrads<T> q, int wg) {
+struct LenetUpdate {
+    T *w[6], *v[6];
+    float lr, momentum;
+};
+template <typename T>
+struct LenetOld { T w, v; };  // a parameter and its velocity, requested before the sums
+template <typename T>
+__device__ __forceinline__ LenetOld<T> lenet5_old(const LenetUpdate<T> &u, int which, int i) {
+    return {u.w[which][i], u.v[which] ? u.v[which][i] : Elem<T>::zero()};
+}
+template <typename T>
+__device__ __forceinline__ void lenet5_update(const LenetUpdate<T> &u, int which, int i, const LenetOld<T> &old, T g) {
+    if (u.v[which]) {
+        const float mv = u.momentum * Elem<T>::to_f32(old.v);
+        const float vn = mv + Elem<T>::to_f32(g);
+        const float step = u.lr * vn;
+        u.v[which][i] = Elem<T>::from_f32(vn);
+        u.w[which][i] = Elem<T>::from_f32(Elem<T>::to_f32(old.w) - step);
+    } else {
+        const float a = Elem<T>::to_f32(Elem<T>::from_f32(-u.lr));
+        const T prod = Elem<T>::from_f32(a * Elem<T>::to_f32(g));
+        u.w[which][i] = Elem<T>::from_f32(Elem<T>::to_f32(prod) + Elem<T>::to_f32(old.w));
+    }
+}
+
+// 256 threads of workgroup `wg` (of 184); UPDATE: the parameters too
+template <typename T, bool UPDATE>
+__device__ __forceinline__ void lenet5_dense_grads(const LenetDenseGrads<T> q, int wg, const LenetUpdate<T> &upd) {
     constexpr int RCH = 128;  // batch rows per pass
     __shared__ float as[RCH * 16], gs[RCH * 16];
-    __shared__ float part[256];
+    __shared__ __align__(16) float part[256];
     const int tid = threadIdx.x;
     // tiles: dwd1 16 x 8, dwd2 8 x 6, dwd3 6 x 1, then the bias gradient, then the loss
     const T *A, *G;
     T *D;
-    int K, N, tk, tn;
-    if (wg < 128) { A = q.f; G = q.g_d1; D = q.dwd1; K = 256; N = 128; tk = wg / 8; tn = wg % 8; }
-    else if (wg < 176) { wg -= 128; A = q.a1; G = q.g_d2; D = q.dwd2; K = 128; N = 84; tk = wg / 6; tn = wg % 6; }
-    else if (wg < 182) { wg -= 176; A = q.a2; G = q.g_logits; D = q.dwd3; K = 84; N = 10; tk = wg; tn = 0; }
+    int K, N, tk, tn, which;
+    if (wg < 128) { A = q.f; G = q.g_d1; D = q.dwd1; K = 256; N = 128; tk = wg / 8; tn = wg % 8; which = 2; }
+    else if (wg < 176) { wg -= 128; A = q.a1; G = q.g_d2; D = q.dwd2; K = 128; N = 84; tk = wg / 6; tn = wg % 6; which = 3; }
+    else if (wg < 182) { wg -= 176; A = q.a2; G = q.g_logits; D = q.dwd3; K = 84; N = 10; tk = wg; tn = 0; which = 4; }
     else if (wg == 182) {
+        LenetOld<T> old = {};
+        if (UPDATE && tid < 10) old = lenet5_old(upd, 5, tid);
         // the rows go through LDS, 200 at a time: read straight from memory the hundred dependent additions of a column
         // would each wait for their own load
         T acc = Elem<T>::zero();
@@ -809,10 +903,24 @@ __device__ __forceinline__ void lenet5_dense_grads(const LenetDenseGrads<T> q, i
             for (int u = 0; u < 8; ++u)
                 if (tid + u * 256 < cnt) as[tid + u * 256] = Elem<T>::to_f32(v[u]);
             __syncthreads();
-            if (tid < 10)
-                for (int r = 0; r < cnt / 10; ++r) acc = Elem<T>::from_f32(Elem<T>::raw(acc) + as[r * 10 + tid]);
+            if (tid < 10) {
+                // sixteen rows are read before the first is added (the chain itself is a few cycles a row)
+                const int nr = cnt / 10;
+                int r = 0;
+                for (; r + 16 <= nr; r += 16) {
+                    float h[16];
+#pragma unroll
+                    for (int u = 0; u < 16; ++u) h[u] = as[(r + u) * 10 + tid];
+#pragma unroll
+                    for (int u = 0; u < 16; ++u) acc = Elem<T>::from_f32(Elem<T>::raw(acc) + h[u]);
+                }
+                for (; r < nr; ++r) acc = Elem<T>::from_f32(Elem<T>::raw(acc) + as[r * 10 + tid]);
+            }
         }
-        if (tid < 10) q.db3[tid] = acc;
+        if (tid < 10) {
+            q.db3[tid] = acc;
+            if (UPDATE) lenet5_update(upd, 5, tid, old, acc);
+        }
         return;
     } else {
         if (!q.loss) return;
@@ -832,7 +940,20 @@ __device__ __forceinline__ void lenet5_dense_grads(const LenetDenseGrads<T> q, i
             __syncthreads();
             if (tid == 0) {
                 const int cnt = min(256, q.bs - base);
-                for (int i = 0; i < cnt; ++i) total += part[i];
+                int i = 0;
+                for (; i + 32 <= cnt; i += 32) {
+                    float4 h[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) h[u] = *(const float4 *)(part + i + 4 * u);
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) {
+                        total += h[u].x;
+                        total += h[u].y;
+                        total += h[u].z;
+                        total += h[u].w;
+                    }
+                }
+                for (; i < cnt; ++i) total += part[i];
             }
             __syncthreads();
         }
@@ -841,19 +962,27 @@ __device__ __forceinline__ void lenet5_dense_grads(const LenetDenseGrads<T> q, i
     }
     const int k0 = tk * 16, n0 = tn * 16;
     const int i = tid >> 4, j = tid & 15;
+    const bool mine = k0 + i < K && n0 + j < N;
+    const int at = (k0 + i) * N + n0 + j;
+    LenetOld<T> old = {};
+    if (UPDATE && mine) old = lenet5_old(upd, which, at);
     float acc = 0.0f;
-    for (int r0 = 0; r0 < q.bs; r0 += RCH) {
+    // all 16 elements of a thread are requested before the first is stored (one at a time the staging alone would be a chain of eight
+    // memory latencies), and those of the next pass before this one's products
+    T av[RCH * 16 / 256], gv[RCH * 16 / 256];
+    auto request = [&](int r0) __attribute__((always_inline)) {
         const int rows = min(RCH, q.bs - r0);
-        __syncthreads();
-        // all 16 elements of a thread are requested before the first is stored: one at a time the staging alone would
-        // be a chain of eight memory latencies
-        T av[RCH * 16 / 256], gv[RCH * 16 / 256];
 #pragma unroll
         for (int u = 0; u < RCH * 16 / 256; ++u) {
             const int e = tid + u * 256, r = min(e >> 4, rows - 1), c = e & 15;
             av[u] = A[(size_t)(r0 + r) * K + min(k0 + c, K - 1)];
             gv[u] = G[(size_t)(r0 + r) * N + min(n0 + c, N - 1)];
         }
+    };
+    request(0);
+    for (int r0 = 0; r0 < q.bs; r0 += RCH) {
+        const int rows = min(RCH, q.bs - r0);
+        __syncthreads();
 #pragma unroll
         for (int u = 0; u < RCH * 16 / 256; ++u) {
             const int e = tid + u * 256, r = e >> 4, c = e & 15;
@@ -862,15 +991,20 @@ __device__ __forceinline__ void lenet5_dense_grads(const LenetDenseGrads<T> q, i
             gs[e] = rok && n0 + c < N ? Elem<T>::to_f32(gv[u]) : 0.0f;
         }
         __syncthreads();
-#pragma unroll 8
+        if (r0 + RCH < q.bs) request(r0 + RCH);
+#pragma unroll 16
         for (int r = 0; r < rows; ++r) acc = __builtin_fmaf(as[r * 16 + i], gs[r * 16 + j], acc);
     }
-    if (k0 + i < K && n0 + j < N) D[(size_t)(k0 + i) * N + n0 + j] = Elem<T>::from_f32(acc);
+    if (mine) {
+        const T g = Elem<T>::from_f32(acc);
+        D[at] = g;
+        if (UPDATE) lenet5_update(upd, which, at, old, g);
+    }
 }
 constexpr int kLenetDenseGroups = 184;
 template <typename T>
 __global__ __launch_bounds__(256) void lenet5_dense_grads_kernel(LenetDenseGrads<T> q) {
-    lenet5_dense_grads<T>(q, (int)blockIdx.x);
+    lenet5_dense_grads<T, false>(q, (int)blockIdx.x, {});
 }
 
 template <typename T>
@@ -908,6 +1042,70 @@ int lenet5_dense_grads_entry(const char *name, const void *a2, const void *a1, c
 // partial sums from operands staged in LDS; a second launch adds the partials in image order and rounds once to T, as
 // the split-K GEMM does.
 constexpr int kLenetPartPitch = 2560;  // per image: 2400 entries of dw2, 150 of dw1
+// 512 threads: one image's partial sums out of LDS: g2 [y*8 + x][oc] and g1 [y*24 + x][oc] the gradients of the convolutions' outputs, p1s and
+// xs their inputs; q2 and q1 take the second half of conv2's positions and conv1's eight row groups.  On v_mfma_f32_16x16x4_f32 (lane (g, i):
+// row i of A, column i of B, k = g; accumulator r: row 4 g + r, column i): rows are output channels, columns taps, k positions, both operands
+// gathered with one 4-byte read at a constant offset.  As FMAs with a thread per tap the reads of the gradient rows, 2000 LDS instructions an
+// image, were what it took: 15200 cycles, 6.5 us of the training step's launch.
+__device__ __forceinline__ void lenet5_conv_grads_sums(const float *g2, const float *g1, const float *p1s, const float *xs, float *q2, float *q1,
+                                                       float *__restrict__ out) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, i = lane & 15;
+    // conv2: ten tiles of 16 taps x two halves of the 64 positions are twenty units of 8 MFMAs, unit = 2 tile + half; a wave has up to three
+    f32x4_t acc2[3];
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+        acc2[n] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        const int unit = wave + 8 * n;
+        if (unit >= 20) continue;  // wave-uniform
+        const int half = unit & 1, k = min((unit >> 1) * 16 + i, 149), ci = k / 25, t = k - ci * 25, fi = t / 5, fj = t - fi * 5;
+        const float *A = g2 + half * 512 + g * 16 + i, *B = p1s + ci * 144 + (half * 4 + fi) * 12 + fj + g;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) acc2[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[q * 64], B[(q >> 1) * 12 + (q & 1) * 4], acc2[n], 0, 0, 0);
+        if (half == 1 && (unit >> 1) * 16 + i < 150) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) q2[(4 * g + r) * 150 + k] = acc2[n][r];
+        }
+    }
+    // conv1: a wave takes three of the 24 output rows (72 positions), two tiles of taps; rows behind the six channels repeat the last
+    {
+        const int ta = i, tb = min(16 + i, 24);
+        const float *A = g1 + (wave * 72 + g) * 6 + min(i, 5), *X = xs + wave * 84 + g;
+        const float *Ba = X + (ta / 5) * 28 + ta % 5, *Bb = X + (tb / 5) * 28 + tb % 5;
+        f32x4_t a0 = {0.0f, 0.0f, 0.0f, 0.0f}, a1 = a0;
+#pragma unroll
+        for (int q = 0; q < 18; ++q) {
+            const float v = A[q * 24];
+            const int at = (q / 6) * 28 + (q % 6) * 4;
+            a0 = __builtin_amdgcn_mfma_f32_16x16x4f32(v, Ba[at], a0, 0, 0, 0);
+            a1 = __builtin_amdgcn_mfma_f32_16x16x4f32(v, Bb[at], a1, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int oc = 4 * g + r;
+            if (oc < 6) {
+                q1[wave * 150 + oc * 25 + ta] = a0[r];
+                if (16 + i < 25) q1[wave * 150 + oc * 25 + tb] = a1[r];
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+        const int unit = wave + 8 * n, k = (unit >> 1) * 16 + i;
+        if (unit < 20 && (unit & 1) == 0 && k < 150) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) out[(4 * g + r) * 150 + k] = acc2[n][r] + q2[(4 * g + r) * 150 + k];
+        }
+    }
+    const int k = threadIdx.x - 300;
+    if (k >= 0 && k < 150) {
+        float s = q1[k];
+#pragma unroll
+        for (int rg = 1; rg < 8; ++rg) s += q1[rg * 150 + k];
+        out[2400 + k] = s;
+    }
+}
+
 template <typename T>
 __device__ __forceinline__ void lenet5_conv_grads(const T *__restrict__ x, const T *__restrict__ p1, const T *__restrict__ gm1,
                                                   const T *__restrict__ gm2, float *__restrict__ part, size_t b) {
@@ -940,72 +1138,7 @@ __device__ __forceinline__ void lenet5_conv_grads(const T *__restrict__ x, const
             if (tid + u * NT < 3456) g1[tid + u * NT] = Elem<T>::to_f32(v1[u]);
     }
     __syncthreads();
-    float *out = part + b * kLenetPartPitch;
-    float acc2[16];
-    if (tid < 300) {
-        // conv2: one tap (ci, fi, fj) x 16 output channels over half of the 64 positions (ascending); the gradient row is
-        // a broadcast read
-        const int half = tid / 150, k = tid - half * 150;
-        const int ci = k / 25, t = k - ci * 25, fi = t / 5, fj = t - fi * 5;
-#pragma unroll
-        for (int o = 0; o < 16; ++o) acc2[o] = 0.0f;
-#pragma unroll
-        for (int yy = 0; yy < 4; ++yy) {
-            const int y = half * 4 + yy;
-#pragma unroll
-            for (int xx = 0; xx < 8; ++xx) {
-                const float v = p1s[ci * 144 + (y + fi) * 12 + xx + fj];
-                const float4 *g = (const float4 *)(g2 + (y * 8 + xx) * 16);
-#pragma unroll
-                for (int qd = 0; qd < 4; ++qd) {
-                    const float4 gv = g[qd];
-                    acc2[4 * qd + 0] = __builtin_fmaf(gv.x, v, acc2[4 * qd + 0]);
-                    acc2[4 * qd + 1] = __builtin_fmaf(gv.y, v, acc2[4 * qd + 1]);
-                    acc2[4 * qd + 2] = __builtin_fmaf(gv.z, v, acc2[4 * qd + 2]);
-                    acc2[4 * qd + 3] = __builtin_fmaf(gv.w, v, acc2[4 * qd + 3]);
-                }
-            }
-        }
-        if (half == 1) {
-#pragma unroll
-            for (int o = 0; o < 16; ++o) q2[o * 150 + k] = acc2[o];
-        }
-    } else if (tid < 500) {
-        // conv1: one tap x 6 output channels over three of the 24 output rows
-        const int t = tid - 300, rg = t / 25, tap = t - rg * 25, fi = tap / 5, fj = tap - fi * 5;
-        float acc[6];
-#pragma unroll
-        for (int o = 0; o < 6; ++o) acc[o] = 0.0f;
-#pragma unroll
-        for (int yy = 0; yy < 3; ++yy) {
-            const int y = 3 * rg + yy;
-#pragma unroll 12
-            for (int xx = 0; xx < 24; ++xx) {
-                const float v = xs[(y + fi) * 28 + xx + fj];
-                const float2 *g = (const float2 *)(g1 + (y * 24 + xx) * 6);
-                const float2 ga = g[0], gb = g[1], gc = g[2];
-                acc[0] = __builtin_fmaf(ga.x, v, acc[0]);
-                acc[1] = __builtin_fmaf(ga.y, v, acc[1]);
-                acc[2] = __builtin_fmaf(gb.x, v, acc[2]);
-                acc[3] = __builtin_fmaf(gb.y, v, acc[3]);
-                acc[4] = __builtin_fmaf(gc.x, v, acc[4]);
-                acc[5] = __builtin_fmaf(gc.y, v, acc[5]);
-            }
-        }
-#pragma unroll
-        for (int o = 0; o < 6; ++o) q1[rg * 150 + o * 25 + tap] = acc[o];
-    }
-    __syncthreads();
-    if (tid < 150) {
-#pragma unroll
-        for (int o = 0; o < 16; ++o) out[o * 150 + tid] = acc2[o] + q2[o * 150 + tid];
-    } else if (tid >= 300 && tid < 450) {
-        const int k = tid - 300;
-        float s = q1[k];
-#pragma unroll
-        for (int rg = 1; rg < 8; ++rg) s += q1[rg * 150 + k];
-        out[2400 + k] = s;
-    }
+    lenet5_conv_grads_sums(g2, g1, p1s, xs, q2, q1, part + b * kLenetPartPitch);
 }
 
 template <typename T>
@@ -1026,36 +1159,58 @@ __global__ __launch_bounds__(512) void lenet5_weight_grads_kernel(LenetDenseGrad
         lenet5_conv_grads<T>(x, p1, gm1, gm2, part, blockIdx.x - kLenetDenseGroups);
     } else {
         if (threadIdx.x >= 256) return;  // a barrier waits for the waves that have not ended
-        lenet5_dense_grads<T>(q, (int)blockIdx.x);
+        lenet5_dense_grads<T, false>(q, (int)blockIdx.x, {});
     }
 }
 
-// 64 outputs per workgroup; wave j adds the images of the j-th quarter of the batch (its loads all in flight together),
-// the four sums are then added in a fixed order
+// 64 outputs per workgroup `wg` (of 40) of 256 threads; wave j adds the images of the j-th quarter of the batch in two interleaved sums (sixteen
+// loads in flight), the eight sums are then added in a fixed order
+constexpr int kLenetReduceGroups = 40;
+template <typename T, bool UPDATE>
+__device__ __forceinline__ void lenet5_conv_reduce(const float *__restrict__ part, T *__restrict__ dw1, T *__restrict__ dw2, int bs, int wg,
+                                                   const LenetUpdate<T> &upd) {
+    __shared__ float sums[4][64];
+    const int lane = threadIdx.x & 63, j = threadIdx.x >> 6;
+    const int k = min(wg * 64 + lane, 2549), which = k < 2400 ? 1 : 0, at = k < 2400 ? k : k - 2400;
+    const bool mine = j == 0 && wg * 64 + lane < 2550;
+    LenetOld<T> old = {};
+    if (UPDATE && mine) old = lenet5_old(upd, which, at);
+    const int per = (bs + 3) / 4, b0 = j * per, b1 = min(bs, b0 + per);
+    float s0 = 0.0f, s1 = 0.0f;
+    int b = b0;
+    for (; b + 16 <= b1; b += 16) {
+        float v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = part[(size_t)(b + u) * kLenetPartPitch + k];
+#pragma unroll
+        for (int u = 0; u < 16; u += 2) {
+            s0 += v[u];
+            s1 += v[u + 1];
+        }
+    }
+    if (b < b1) {
+        float v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = part[(size_t)min(b + u, b1 - 1) * kLenetPartPitch + k];
+#pragma unroll
+        for (int u = 0; u < 16; u += 2) {
+            s0 += b + u < b1 ? v[u] : 0.0f;
+            s1 += b + u + 1 < b1 ? v[u + 1] : 0.0f;
+        }
+    }
+    sums[j][lane] = s0 + s1;
+    __syncthreads();
+    if (mine) {
+        const float tot = (sums[0][lane] + sums[1][lane]) + (sums[2][lane] + sums[3][lane]);
+        const T g = Elem<T>::from_f32(tot);
+        (which ? dw2 : dw1)[at] = g;
+        if (UPDATE) lenet5_update(upd, which, at, old, g);
+    }
+}
 template <typename T>
 __global__ __launch_bounds__(256) void lenet5_conv_grads_reduce_kernel(const float *__restrict__ part, T *__restrict__ dw1,
                                                                          T *__restrict__ dw2, int bs) {
-    __shared__ float sums[4][64];
-    const int lane = threadIdx.x & 63, j = threadIdx.x >> 6;
-    const int k = min((int)blockIdx.x * 64 + lane, 2549);
-    const int per = (bs + 3) / 4, b0 = j * per, b1 = min(bs, b0 + per);
-    float s = 0.0f;
-    int b = b0;
-    for (; b + 8 <= b1; b += 8) {
-        float v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = part[(size_t)(b + u) * kLenetPartPitch + k];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) s += v[u];
-    }
-    for (; b < b1; ++b) s += part[(size_t)b * kLenetPartPitch + k];
-    sums[j][lane] = s;
-    __syncthreads();
-    if (j == 0 && (int)blockIdx.x * 64 + lane < 2550) {
-        const float tot = (sums[0][lane] + sums[1][lane]) + (sums[2][lane] + sums[3][lane]);
-        if (k < 2400) dw2[k] = Elem<T>::from_f32(tot);
-        else dw1[k - 2400] = Elem<T>::from_f32(tot);
-    }
+    lenet5_conv_reduce<T, false>(part, dw1, dw2, bs, (int)blockIdx.x, {});
 }
 
 template <typename T>
@@ -1071,7 +1226,7 @@ int lenet5_conv_grads_entry(const char *name, const void *x, const void *p1, con
     hipLaunchKernelGGL(lenet5_conv_grads_kernel<T>, dim3((unsigned)bs), dim3(512), 0, stream(), (const T *)x, (const T *)p1,
                        (const T *)gm1, (const T *)gm2, (float *)ws);
     AGH_LAUNCH_CHECK(name);
-    hipLaunchKernelGGL(lenet5_conv_grads_reduce_kernel<T>, dim3(40), dim3(256), 0, stream(), (const float *)ws, (T *)dw1,
+    hipLaunchKernelGGL(lenet5_conv_grads_reduce_kernel<T>, dim3(kLenetReduceGroups), dim3(256), 0, stream(), (const float *)ws, (T *)dw1,
                        (T *)dw2, (int)bs);
     AGH_LAUNCH_CHECK(name);
     return AGH_OK;
@@ -1094,8 +1249,267 @@ int lenet5_weight_grads_entry(const char *name, const void *a2, const void *a1, 
     hipLaunchKernelGGL(lenet5_weight_grads_kernel<T>, dim3((unsigned)bs + kLenetDenseGroups), dim3(512), 0, stream(), q, (const T *)x,
                        (const T *)p1, (const T *)gm1, (const T *)gm2, (float *)ws);
     AGH_LAUNCH_CHECK(name);
-    hipLaunchKernelGGL(lenet5_conv_grads_reduce_kernel<T>, dim3(40), dim3(256), 0, stream(), (const float *)ws, (T *)dw1,
+    hipLaunchKernelGGL(lenet5_conv_grads_reduce_kernel<T>, dim3(kLenetReduceGroups), dim3(256), 0, stream(), (const float *)ws, (T *)dw1,
                        (T *)dw2, (int)bs);
+    AGH_LAUNCH_CHECK(name);
+    return AGH_OK;
+}
+
+
+// ---- a whole training step in two launches ----
+//
+// The step as five launches (forward, input gradients, weight gradients, the sum of the images' shares, update) is a chain of launches whose
+// work is small: at batch 100 in bf16 10.2 + 14.4 + 9.6 + 4.5 + 4.4 us, of which the backward one waits 6 us for the first touch of a dozen
+// buffers that the launch before it wrote.  Here a workgroup takes ONE image through forward, input gradients and its share of the
+// convolutions' weight gradients with activations, gradients and the small layers' weights in LDS; the second launch forms the dense layers'
+// gradients, adds the shares, and whoever finishes a gradient updates its parameter (nothing else reads the parameters there).  Every value is
+// rounded where the separate launches round it and summed in their order, so gradients, loss and parameters have their bits.  What bounds the
+// first launch is its chain of eighteen stages behind barriers, 40000 cycles in bf16, the longest 7000 (shares of the weight gradients), 4300
+// (staging), 3900 (col2im) and 3800 (conv2); a batch beyond 256 is several rounds of it, one workgroup per CU.  A captured step, bf16 /
+// f32: batch 100 42.3 -> 27.4 us / 42.7 -> 26.0, 400 70.8 -> 48.9 / 82.0 -> 45.5, 1000 109 -> 90 / 135 -> 82.
+template <typename T>
+struct LenetStep {
+    const T *x, *w1, *w2, *wd1, *wd2, *wd3, *b3;
+    const uint8_t *target;
+    T *logits, *g_logits, *g_d2, *g_d1, *gm2, *gm1;
+    float *part;
+    float dy;
+    int bs, w23_aligned;
+};
+
+template <typename T, bool WHOLE>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void lenet5_step_image_kernel(LenetStep<T> a, LenetSaves<T> sv) {
+    __shared__ LenetForwardLds<T, 1> s;
+    __shared__ LenetStepLds st;
+    __shared__ __align__(16) float gm2s[64 * 16];  // gradient of conv2's output, [y*8 + x][oc]
+    __shared__ __align__(8) float g1[576 * 6];     // of conv1's output, [y*24 + x][oc]
+    __shared__ __align__(16) float gd1s[128], gd2s[84];
+    __shared__ float gls[16], gfs[256], gp1s[864];
+    __shared__ float pm[64 * kPmPitch];            // gm2 . W, every entry rounded to T
+    __shared__ float q2[16 * 150], q1[8 * 150];
+    constexpr int NT = 512;
+    const int tid = threadIdx.x;
+    const size_t b = blockIdx.x;
+    const int label = a.target[b];
+    float4 wreg[16];  // dense1's weights [16 kg ..][4 cg ..], for both directions
+    T x2[4], x1[2][4];  // the pooling windows: requested when the convolutions' outputs are saved, used behind the dense layers
+    lenet5_forward_body<T, true, 1, WHOLE>(s, a.x, a.w1, a.w2, a.wd1, a.wd2, a.wd3, a.b3, a.logits, a.bs, sv, a.w23_aligned, &st, wreg, [&]() __attribute__((always_inline)) {
+        {
+            const int t = tid & 255, oc = t >> 4, ho = (t >> 2) & 3, wo = t & 3;
+            const T *xp = sv.c2 + ((b * 16 + oc) * 8 + 2 * ho) * 8 + 2 * wo;
+            x2[0] = xp[0]; x2[1] = xp[1]; x2[2] = xp[8]; x2[3] = xp[9];
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int e = min(tid + u * NT, 863);
+            const int ci = e / 144, r = e - ci * 144, ho = r / 12, wo = r - ho * 12;
+            const T *xp = sv.c1 + ((b * 6 + ci) * 24 + 2 * ho) * 24 + 2 * wo;
+            x1[u][0] = xp[0]; x1[u][1] = xp[1]; x1[u][2] = xp[24]; x1[u][3] = xp[25];
+        }
+    });
+    __syncthreads();
+    // cross-entropy backward (softmax - one-hot, times dy), rounded to T
+    if (tid < 10) {
+        float m = st.lg[0];
+#pragma unroll
+        for (int j = 0; j < 10; ++j) m = fmaxf(m, st.lg[j]);
+        float sum = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 10; ++j) sum += expf(st.lg[j] - m);
+        const float pr = expf(st.lg[tid] - m) / sum;
+        const T g = Elem<T>::from_f32(a.dy * (pr - (tid == label ? 1.0f : 0.0f)));
+        a.g_logits[b * 10 + tid] = g;
+        gls[tid] = Elem<T>::to_f32(g);
+    }
+    __syncthreads();
+    // dense3, dense2 (weights in LDS) and dense1: input gradients, relu backward on the pre-activations
+    if (tid < 84) {
+        float d = 0.0f;
+#pragma unroll
+        for (int c = 0; c < 10; ++c) d = __builtin_fmaf(gls[c], Elem<T>::to_f32(s.wd3s[tid * 10 + c]), d);
+        const T gd = st.pre2[tid] >= 0.0f ? Elem<T>::from_f32(d) : Elem<T>::zero();
+        a.g_d2[b * 84 + tid] = gd;
+        gd2s[tid] = Elem<T>::to_f32(gd);
+    }
+    __syncthreads();
+    {
+        // four lanes share a row of wd2 (dense2_row_sum adds in the same order)
+        const int row = tid >> 2, q = tid & 3;
+        float d = 0.0f;
+#pragma unroll
+        for (int n = 0; n < 6; ++n) {
+            const int c = q + 4 * n;
+            if (c >= 21) break;
+            const float4 g = *(const float4 *)(gd2s + 4 * c);
+            float w[4];
+            if constexpr (sizeof(T) == 4) {
+                const float4 r = *(const float4 *)(s.wd2s + row * 84 + 4 * c);
+                w[0] = r.x; w[1] = r.y; w[2] = r.z; w[3] = r.w;
+            } else {
+                const uint2 r = *(const uint2 *)(s.wd2s + row * 84 + 4 * c);
+                w[0] = __uint_as_float(r.x << 16); w[1] = __uint_as_float(r.x & 0xFFFF0000u);
+                w[2] = __uint_as_float(r.y << 16); w[3] = __uint_as_float(r.y & 0xFFFF0000u);
+            }
+            d = __builtin_fmaf(g.x, w[0], d);
+            d = __builtin_fmaf(g.y, w[1], d);
+            d = __builtin_fmaf(g.z, w[2], d);
+            d = __builtin_fmaf(g.w, w[3], d);
+        }
+        d += __shfl_xor(d, 1);
+        d += __shfl_xor(d, 2);
+        if (q == 0) {
+            const T gd = st.pre1[row] >= 0.0f ? Elem<T>::from_f32(d) : Elem<T>::zero();
+            a.g_d1[b * 128 + row] = gd;
+            gd1s[row] = Elem<T>::to_f32(gd);
+        }
+    }
+    __syncthreads();
+    {
+        // thread (cg, kg): four of the 128 products of 16 rows; the 32 lanes of a half-wave add their parts pairwise, each step halving the rows
+        // a lane goes on with (dense1_row_sum adds in the same order)
+        const int cg = tid & 31, kg = tid >> 5;
+        const float4 g = *(const float4 *)(gd1s + cg * 4);
+        float v[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            v[r] = __builtin_fmaf(g.x, wreg[r].x, 0.0f);
+            v[r] = __builtin_fmaf(g.y, wreg[r].y, v[r]);
+            v[r] = __builtin_fmaf(g.z, wreg[r].z, v[r]);
+            v[r] = __builtin_fmaf(g.w, wreg[r].w, v[r]);
+        }
+        auto fold = [&](auto halfc) {
+            constexpr int half = decltype(halfc)::value;
+            const bool up = (cg & (2 * half)) != 0;
+#pragma unroll
+            for (int r = 0; r < half; ++r) {
+                const float keep = up ? v[r + half] : v[r], send = up ? v[r] : v[r + half];
+                v[r] = keep + __shfl_xor(send, 2 * half);
+            }
+        };
+        fold(std::integral_constant<int, 8>{});
+        fold(std::integral_constant<int, 4>{});
+        fold(std::integral_constant<int, 2>{});
+        fold(std::integral_constant<int, 1>{});
+        const float d = v[0] + __shfl_xor(v[0], 1);
+        if ((cg & 1) == 0) gfs[kg * 16 + (cg >> 1)] = Elem<T>::to_f32(Elem<T>::from_f32(d));
+    }
+    __syncthreads();
+    // pooling + relu backward of conv2's output: one window per thread (16 channels x 4 x 4 windows)
+    if (tid < 256) {
+        const int oc = tid >> 4, ho = (tid >> 2) & 3, wo = tid & 3;
+        T cell[4];
+        pool_relu_window_backward<T>(x2, gfs[tid], cell);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int pos = (2 * ho + (k >> 1)) * 8 + 2 * wo + (k & 1);
+            gm2s[pos * 16 + oc] = Elem<T>::to_f32(cell[k]);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 2; ++u) a.gm2[b * 1024 + tid + u * NT] = Elem<T>::from_f32(gm2s[tid + u * NT]);  // (exact: T values)
+    // conv2's input gradient: the product gm2 . W, then col2im in the host's order, as lenet5_backward_kernel does it; a thread takes two pixels,
+    // whose chains of 25 additions run side by side
+    lenet5_pm<T, NT / 64>(gm2s, s.w2s, pm);
+    __syncthreads();
+    if (tid < 432) {
+        T acc[2] = {Elem<T>::zero(), Elem<T>::zero()};
+        const int ci0 = tid / 144, r0 = tid - ci0 * 144, hy = r0 / 12, wy = r0 - hy * 12;  // pixel e = tid + 432: three channels on
+#pragma unroll
+        for (int fi = 4; fi >= 0; --fi) {
+            const int th = hy - fi;
+            const bool hok = th >= 0 && th < 8;
+            const int thc = min(max(th, 0), 7);
+#pragma unroll
+            for (int fj = 4; fj >= 0; --fj) {
+                const int tw = wy - fj;
+                const bool ok = hok && tw >= 0 && tw < 8;
+                const float *v = pm + (thc * 8 + min(max(tw, 0), 7)) * kPmPitch + ci0 * 25 + fi * 5 + fj;
+#pragma unroll
+                for (int u = 0; u < 2; ++u) acc[u] = Elem<T>::from_f32(Elem<T>::raw(acc[u]) + (ok ? v[75 * u] : 0.0f));
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) gp1s[tid + 432 * u] = Elem<T>::to_f32(acc[u]);
+    }
+    __syncthreads();
+    // pooling + relu backward of conv1's output (6 channels x 12 x 12 windows), as the [576, 6] matrix
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int e = tid + u * NT;
+        if (e < 864) {
+            const int ci = e / 144, r = e - ci * 144, ho = r / 12, wo = r - ho * 12;
+            T cell[4];
+            pool_relu_window_backward<T>(x1[u], gp1s[e], cell);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int pos = (2 * ho + (k >> 1)) * 24 + 2 * wo + (k & 1);
+                g1[pos * 6 + ci] = Elem<T>::to_f32(cell[k]);
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 7; ++u)
+        if (tid + u * NT < 3456) a.gm1[b * 3456 + tid + u * NT] = Elem<T>::from_f32(g1[tid + u * NT]);
+    lenet5_conv_grads_sums(gm2s, g1, s.p1, s.xs, q2, q1, a.part + b * kLenetPartPitch);
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void lenet5_finish_kernel(LenetDenseGrads<T> q, const float *__restrict__ part, T *__restrict__ dw1,
+                                                             T *__restrict__ dw2, LenetUpdate<T> upd) {
+    if (blockIdx.x < kLenetDenseGroups) lenet5_dense_grads<T, true>(q, (int)blockIdx.x, upd);
+    else lenet5_conv_reduce<T, true>(part, dw1, dw2, q.bs, (int)blockIdx.x - kLenetDenseGroups, upd);
+}
+
+template <typename T>
+int lenet5_train_step_entry(const char *name, const void *x, const void *target, void *const *params, void *const *velocities,
+                            void *const *grads, void *const *saves, void *const *input_grads, float dy, float lr, float momentum, void *loss,
+                            int64_t bs) {
+    AGH_API_ENTER();
+    if (bs < 0) return fail(AGH_EINVAL, "%s: negative batch size", name);
+    if (bs == 0) return AGH_OK;
+    if (bs > ((int64_t)1 << 20)) return fail(AGH_ERANGE, "%s: batch too large", name);
+    if (!x || !target || !params || !grads || !saves || !input_grads) return fail(AGH_ENULL, "%s: null buffer", name);
+    for (int i = 0; i < 6; ++i)
+        if (!params[i] || !grads[i] || (velocities && !velocities[i])) return fail(AGH_ENULL, "%s: null parameter, gradient or velocity", name);
+    for (int i = 0; i < 9; ++i)
+        if (!saves[i]) return fail(AGH_ENULL, "%s: null buffer for a saved activation", name);
+    for (int i = 0; i < 5; ++i)
+        if (!input_grads[i]) return fail(AGH_ENULL, "%s: null buffer for an input gradient", name);
+    if (((uintptr_t)params[2] & 15) != 0 || ((uintptr_t)params[3] & 7) != 0)
+        return fail(AGH_EINVAL, "%s: wd1 must be 16-byte and wd2 8-byte aligned", name);
+    LenetDenseGrads<T> q;
+    if (int rc = lenet5_dense_grads_check<T>(name, saves[7], saves[5], saves[3], input_grads[0], input_grads[1], input_grads[2], grads[4], grads[3],
+                                             grads[2], grads[5], saves[8], target, loss, bs, q))
+        return rc;
+    void *ws = nullptr;
+    if (int rc = workspace((size_t)bs * kLenetPartPitch * sizeof(float), &ws)) return rc;
+    LenetStep<T> a;
+    a.x = (const T *)x; a.target = (const uint8_t *)target;
+    a.w1 = (const T *)params[0]; a.w2 = (const T *)params[1]; a.wd1 = (const T *)params[2]; a.wd2 = (const T *)params[3];
+    a.wd3 = (const T *)params[4]; a.b3 = (const T *)params[5];
+    a.logits = (T *)saves[8];
+    a.g_logits = (T *)input_grads[0]; a.g_d2 = (T *)input_grads[1]; a.g_d1 = (T *)input_grads[2];
+    a.gm2 = (T *)input_grads[3]; a.gm1 = (T *)input_grads[4];
+    a.part = (float *)ws;
+    a.dy = dy / (float)bs;  // `dy /= batch_size` first, in f32, as the host does
+    a.bs = (int)bs;
+    a.w23_aligned = (((uintptr_t)params[3] | (uintptr_t)params[4]) & 15) == 0;
+    const LenetSaves<T> sv = {(T *)saves[0], (T *)saves[1], (T *)saves[2], (T *)saves[3], (T *)saves[4], (T *)saves[5], (T *)saves[6], (T *)saves[7]};
+    LenetUpdate<T> upd;
+    for (int i = 0; i < 6; ++i) {
+        upd.w[i] = (T *)params[i];
+        upd.v[i] = velocities ? (T *)velocities[i] : nullptr;
+    }
+    upd.lr = lr;
+    upd.momentum = momentum;
+    // (the forward entries take four images a workgroup above 256)
+    if (bs <= 256) hipLaunchKernelGGL((lenet5_step_image_kernel<T, false>), dim3((unsigned)bs), dim3(512), 0, stream(), a, sv);
+    else hipLaunchKernelGGL((lenet5_step_image_kernel<T, true>), dim3((unsigned)bs), dim3(512), 0, stream(), a, sv);
+    AGH_LAUNCH_CHECK(name);
+    hipLaunchKernelGGL(lenet5_finish_kernel<T>, dim3(kLenetDenseGroups + kLenetReduceGroups), dim3(256), 0, stream(), q, (const float *)a.part,
+                       (T *)grads[0], (T *)grads[1], upd);
     AGH_LAUNCH_CHECK(name);
     return AGH_OK;
 }
@@ -1198,6 +1612,18 @@ int agh_lenet5_conv_weight_grads_f32(const void *x, const void *p1, const void *
 int agh_lenet5_conv_weight_grads_bf16(const void *x, const void *p1, const void *gm1, const void *gm2, void *dw1, void *dw2,
                                       int64_t bs) {
     return lenet5_conv_grads_entry<uint16_t>("agh_lenet5_conv_weight_grads_bf16", x, p1, gm1, gm2, dw1, dw2, bs);
+}
+
+#define AGH_LENET_STEP_ARGS                                                                                                     \
+    const void *x, const void *target, void **params, void **velocities, void **grads, void **saves, void **input_grads, float dy, \
+        float learning_rate, float momentum, void *loss, int64_t bs
+int agh_lenet5_train_step_f32(AGH_LENET_STEP_ARGS) {
+    return lenet5_train_step_entry<float>("agh_lenet5_train_step_f32", x, target, params, velocities, grads, saves, input_grads, dy, learning_rate,
+                                          momentum, loss, bs);
+}
+int agh_lenet5_train_step_bf16(AGH_LENET_STEP_ARGS) {
+    return lenet5_train_step_entry<uint16_t>("agh_lenet5_train_step_bf16", x, target, params, velocities, grads, saves, input_grads, dy,
+                                             learning_rate, momentum, loss, bs);
 }
 
 }  // extern "C"

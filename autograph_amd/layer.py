@@ -356,8 +356,8 @@ class LeNet5Trainer:
         # in place of nine; the weight gradients are the same GEMMs either way
         self.fused_backward = fused_backward
         # overlap: issue the weight gradients on the second stream beside the input-gradient chain.  Default: only for the
-        # layer-by-layer backward pass; with the one-launch forms a step is five kernels, and the fork and join of a second
-        # stream cost more (about 10 us) than the one launch they would hide
+        # layer-by-layer backward pass; with the one-launch forms a step is two kernels on one stream (agh_lenet5_train_step_*),
+        # and the fork and join of a second stream cost about 10 us
         if overlap is None:
             overlap = not fused_backward
         self._branch = branch if overlap else contextlib.nullcontext
@@ -462,6 +462,15 @@ class LeNet5Trainer:
         bs = self.bs
         if not x.is_standard_layout() or x.shape != (bs, 1, 28, 28):
             raise AghError(-1, f"LeNet5Trainer.step: x must be a standard-layout [{bs},1,28,28] tensor")
+        # the one-launch forms on one stream, followed by this module's own update: the whole step is one entry point
+        if self.fused_forward and self.fused_backward and self._branch is not branch and type(self.opt) is SGD:
+            ptrs = lambda tensors: (C.c_void_p * len(tensors))(*[t._data_ptr() for t in tensors])  # noqa: E731
+            momentum = self.opt.momentum
+            check(self._fn("agh_lenet5_train_step")(
+                x._data_ptr(), target.ptr, ptrs(self.params), ptrs(self.velocities) if momentum is not None else None, ptrs(self.grads),
+                ptrs((self.c1, self.p1, self.c2, self.p2, self.d1, self.a1, self.d2, self.a2, self.logits)),
+                ptrs((self.g_logits, self.g_d2, self.g_d1, self.gm2, self.gm1)), 1.0, self.lr, momentum or 0.0, self._loss_host, bs))
+            return
         w1, w2, wd1, wd2, wd3, b3 = self.params
         dw1, dw2, dwd1, dwd2, dwd3, db3 = self.grads
         # forward

@@ -349,6 +349,18 @@ int agh_lenet5_weight_grads_bf16(const void *a2, const void *a1, const void *f, 
                                  const void *target, void *loss, const void *x, const void *p1, const void *gm1, const void *gm2,
                                  void *dw1, void *dw2, int64_t bs);
 
+/* The whole step (autograph_backend.rs:70-86): forward, loss, gradients and the update of all six parameters, two launches up to a batch of
+ * 256 and four beyond.  Same values and bits as the entry points above followed by agh_sgd_momentum_<T> (agh_scaled_add_<T> with
+ * -learning_rate where velocities is null).  Arrays of device pointers, read before the call returns:
+ *   params, velocities, grads   conv1 [6,1,5,5], conv2 [16,6,5,5], dense1 [256,128], dense2 [128,84], dense3 [84,10], its bias [10]
+ *   saves                       c1, p1, c2, p2, d1, a1, d2, a2 as agh_lenet5_forward_train_<T> writes them, logits [bs,10]
+ *   input_grads                 g_logits, g_d2, g_d1, gm2, gm1 as agh_lenet5_backward_<T> writes them
+ * dense1's weight must be 16-byte and dense2's 8-byte aligned.  loss: one f32 in device or pinned host memory, or null. */
+int agh_lenet5_train_step_f32(const void *x, const void *target, void **params, void **velocities, void **grads, void **saves,
+                              void **input_grads, float dy, float learning_rate, float momentum, void *loss, int64_t bs);
+int agh_lenet5_train_step_bf16(const void *x, const void *target, void **params, void **velocities, void **grads, void **saves,
+                               void **input_grads, float dy, float learning_rate, float momentum, void *loss, int64_t bs);
+
 /* ---------------------------------------------------------------- max pool ---- */
 
 /* MaxPool2 device branch (src/tensor/ops.rs:1117-1133; rule from the host impl

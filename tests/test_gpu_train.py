@@ -411,6 +411,37 @@ def test_lenet5_weight_grads_in_one_launch(ag, dtype, bs):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("bs", [1, 100, 256, 257, 513])
+@pytest.mark.parametrize("momentum", [None, 0.9])
+def test_lenet5_train_step_in_two_launches(ag, dtype, bs, momentum):
+    """agh_lenet5_train_step_<T> against the separate entries and the optimizer's own launch, two steps, a batch on either side of the 256 images
+    above which the forward entries take four a workgroup: every saved activation, gradient, parameter and velocity and the loss bit for bit.
+    A missing buffer is an error, never a launch."""
+    rng = np.random.default_rng(bs)
+    params = [to_dtype(p, dtype) for p in lenet_params(rng)]
+    tx = ag.Tensor.from_array(to_dtype(rng.uniform(0, 1, (bs, 1, 28, 28)), dtype))
+    tt = labels(ag, rng.integers(0, 10, bs).astype(np.uint8))
+    out = {}
+    for overlap in (False, True):  # the step entry / the separate ones
+        tr = ag.LeNet5Trainer(ag.LeNet5.from_arrays(*params), bs, optimizer=ag.SGD(momentum), overlap=overlap)
+        for _ in range(2):
+            tr.step(tx, tt)
+        ag._ffi.check(ag.lib.agh_sync())
+        names = ("c1", "p1", "c2", "p2", "d1", "a1", "d2", "a2", "logits", "g_logits", "g_d2", "g_d1", "gm2", "gm1")
+        out[overlap] = [getattr(tr, n).into_array() for n in names] + [t.into_array() for t in tr.params + tr.grads]
+        out[overlap] += [np.float32(tr.loss())] + [v.into_array() for v in tr.velocities if v is not None]
+    for a, b in zip(out[False], out[True]):
+        assert np.array_equal(a, b)
+    ptrs = lambda ts: (C.c_void_p * len(ts))(*[t._data_ptr() for t in ts])  # noqa: E731
+    saves, back = ptrs([getattr(tr, n) for n in names[:9]]), ptrs([getattr(tr, n) for n in names[9:]])
+    for missing in range(5):
+        args = [ptrs(tr.params), ptrs(tr.grads), ptrs(tr.grads), saves, back]
+        args[missing] = (C.c_void_p * 9)(*list(args[missing])[:-1])  # the last pointer is null
+        with pytest.raises(ag.AghError):
+            ag._ffi.check(getattr(ag.lib, f"agh_lenet5_train_step_{dtype}")(tx._ptr(), tt.ptr, *args, 1.0, 0.1, 0.9, None, bs))
+
+
 @pytest.mark.parametrize("fused_backward", [True, False])
 @pytest.mark.parametrize("fused_forward", [True, False])
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
