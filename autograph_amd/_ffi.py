@@ -132,3 +132,15 @@ class AghError(RuntimeError):
 def check(code):
     if code != 0:
         raise AghError(code, lib.agh_last_error_string().decode(errors="replace"))
+
+
+def _through_ctypes(name, args):
+    check(getattr(lib, name)(*args))
+
+
+# The same entry points without ctypes for the calls a program makes often (agh_calls.cpp): they raise by themselves and return None
+try:
+    from . import _calls as calls
+except ImportError as e:
+    raise ImportError(f"autograph_amd._calls: {e}; build it with `make -C {os.path.join(_HERE, 'csrc')}`") from e
+calls.setup(AghError, _through_ctypes)

@@ -9,7 +9,7 @@ import math
 
 import numpy as np
 
-from ._ffi import AghError, check, lib
+from ._ffi import AghError, calls, check, lib
 from .tensor import Im2ColConv2Options, MaxPool2Options, Tensor, _ITEMSIZE, _std_strides, branch, gemm, join
 
 
@@ -29,9 +29,9 @@ def conv2_im2col_forward(x, weight, padding=(0, 0), stride=(1, 1), dilation=(1, 
     L, K = oh * ow, ic * fh * fw
     bp, bo, bst = (bias._ptr(), bias.offset, bias.strides[0]) if bias is not None else (None, 0, 0)
     # A_b = cols[b*L:(b+1)*L, :], B = wm^T (rsb = 1, csb = K), C_b[hw, o] at y + b*oc*L + o*L + hw
-    check(getattr(lib, f"agh_gemm_{x.dtype}_batched")(
+    getattr(calls, f"agh_gemm_{x.dtype}_batched")(
         bs, L, K, oc, 1.0, cols._ptr(), cols.offset, K, 1, L * K, wm._ptr(), wm.offset, 1, K, 0,
-        0.0, y._ptr(), y.offset, 1, L, oc * L, bp, bo, bst, 1 if relu else 0))
+        0.0, y._ptr(), y.offset, 1, L, oc * L, bp, bo, bst, 1 if relu else 0)
     return y
 
 
@@ -50,9 +50,9 @@ def conv2_direct_forward(x, weight, padding=(0, 0), stride=(1, 1), dilation=(1, 
     # standard-layout copies of strided views are bound to names: they must outlive the launch call
     w = weight.as_standard_layout()
     b = bias.as_standard_layout() if bias is not None else None
-    check(getattr(lib, f"agh_conv2_direct_{x.dtype}")(
+    getattr(calls, f"agh_conv2_direct_{x.dtype}")(
         x._data_ptr(), w._data_ptr(), b._data_ptr() if b is not None else None,
-        y._ptr(), bs, ic, ih, iw, oc, fh, fw, *padding, *stride, *dilation, 1 if relu else 0, 1 if pool2x2 else 0))
+        y._ptr(), bs, ic, ih, iw, oc, fh, fw, *padding, *stride, *dilation, 1 if relu else 0, 1 if pool2x2 else 0)
     return y
 
 
@@ -260,7 +260,7 @@ class LeNet5:
         # standard-layout copies of strided views stay referenced by `ws` until the launch call has returned
         ws = [w.as_standard_layout() for w in (self.conv1.weight, self.conv2.weight, self.dense1.weight, self.dense2.weight,
                                                self.dense3.weight, self.dense3.bias)]
-        check(getattr(lib, f"agh_lenet5_forward_{x.dtype}")(x._data_ptr(), *[w._data_ptr() for w in ws], out_ptr, bs))
+        getattr(calls, f"agh_lenet5_forward_{x.dtype}")(x._data_ptr(), *[w._data_ptr() for w in ws], out_ptr, bs)
         return out
 
     # -- graph-captured inference on fixed buffers --
@@ -303,7 +303,7 @@ class LeNet5:
                    b3._ptr(), b3.offset, b3.strides[0], 0))
 
     def replay(self):
-        check(lib.agh_graph_launch(self._graph))
+        calls.agh_graph_launch(self._graph)
 
     def __del__(self):
         g, self._graph = getattr(self, "_graph", None), None
@@ -568,4 +568,4 @@ class LeNet5Trainer:
         self._graph = g
 
     def replay(self):
-        check(lib.agh_graph_launch(self._graph))
+        calls.agh_graph_launch(self._graph)

@@ -15,7 +15,7 @@ from typing import Tuple
 
 import numpy as np
 
-from ._ffi import AghError, check, lib
+from ._ffi import AghError, calls, check, lib
 
 F32 = "f32"
 BF16 = "bf16"
@@ -50,22 +50,8 @@ class Device:
         check(lib.agh_sync())
 
 
-class Buffer:
-    """Owning device allocation (krnl `Buffer`); freed when dropped."""
-
-    def __init__(self, nbytes):
-        p = C.c_void_p()
-        check(lib.agh_malloc(C.byref(p), nbytes))
-        self.ptr = p.value
-        self.nbytes = nbytes
-
-    def __del__(self):
-        ptr, self.ptr = getattr(self, "ptr", None), None
-        if ptr:
-            try:
-                lib.agh_free(ptr)
-            except Exception:
-                pass
+class Buffer(calls.Buffer):
+    """Owning device allocation (krnl `Buffer`), freed when dropped: `Buffer(nbytes)` with `ptr` and `nbytes`."""
 
 
 # ---- option structs, src/ops.rs:9-108 ----
@@ -243,6 +229,10 @@ class Tensor:
     def _fn(self, stem):
         return getattr(lib, f"{stem}_{self.dtype}")
 
+    def _call(self, stem):
+        """The same without ctypes: raises by itself."""
+        return getattr(calls, f"{stem}_{self.dtype}")
+
     # -- Dot, src/tensor/linalg.rs:362-468 --
     def dot(self, rhs, bias=None, relu=False):
         """`self.dot(&rhs)`; with `bias`/`relu` the Dense epilogue is fused into the same launch."""
@@ -265,7 +255,7 @@ class Tensor:
         oh, ow = options.output_shape((ih, iw))
         (fh, fw), (ph, pw), (sh, sw), (dh, dw) = options.filter, options.padding, options.stride, options.dilation
         y = Tensor.uninit((bs * oh * ow, c * fh * fw), self.dtype)
-        check(self._fn("agh_im2col_conv2")(x._data_ptr(), y._ptr(), bs, c, ih, iw, fh, fw, ph, pw, sh, sw, dh, dw))
+        self._call("agh_im2col_conv2")(x._data_ptr(), y._ptr(), bs, c, ih, iw, fh, fw, ph, pw, sh, sw, dh, dw)
         return y
 
     def col2im_conv2(self, options):
@@ -276,7 +266,7 @@ class Tensor:
         bs, c = rows // (ih * iw), cols // (fh * fw)
         oh, ow = options.output_shape()
         y = Tensor.uninit((bs, c, oh, ow), self.dtype)
-        check(self._fn("agh_col2im_conv2")(x._data_ptr(), y._ptr(), bs, c, ih, iw, fh, fw, ph, pw, sh, sw, dh, dw))
+        self._call("agh_col2im_conv2")(x._data_ptr(), y._ptr(), bs, c, ih, iw, fh, fw, ph, pw, sh, sw, dh, dw)
         return y
 
     # -- MaxPool2 / MaxPool2Backward, src/tensor/ops.rs:1106-1141, :1228-1275 --
@@ -285,7 +275,7 @@ class Tensor:
         bs, c, ih, iw = x.shape
         oh, ow = options.output_shape((ih, iw))
         y = Tensor.uninit((bs, c, oh, ow), self.dtype)
-        check(self._fn("agh_max_pool2")(x._data_ptr(), y._ptr(), bs * c, ih, iw, *options.size, *options.strides))
+        self._call("agh_max_pool2")(x._data_ptr(), y._ptr(), bs * c, ih, iw, *options.size, *options.strides)
         return y
 
     def max_pool2_backward(self, output_grad, options):
@@ -296,20 +286,19 @@ class Tensor:
             raise AghError(-1, "max_pool2_backward: input gradient must be in standard layout")
         dy = output_grad.as_standard_layout()
         bs, c, ih, iw = self.shape
-        check(self._fn("agh_max_pool2_backward")(self._data_ptr(), dy._data_ptr(), bs * c, ih, iw,
-                                                 *options.size, *options.strides))
+        self._call("agh_max_pool2_backward")(self._data_ptr(), dy._data_ptr(), bs * c, ih, iw, *options.size, *options.strides)
 
     # -- relu, layer.rs:1269-1510 --
     def relu(self):
         x = self.as_standard_layout()
         y = _uninit(x.shape, x.dtype)
-        check(self._fn("agh_relu")(x._data_ptr(), y._ptr(), len(x)))
+        self._call("agh_relu")(x._data_ptr(), y._ptr(), len(x))
         return y
 
     def relu_backward(self, output_grad):
         x, dy = self.as_standard_layout(), output_grad.as_standard_layout()
         dx = _uninit(x.shape, x.dtype)
-        check(self._fn("agh_relu_backward")(x._data_ptr(), dy._data_ptr(), dx._ptr(), len(x)))
+        self._call("agh_relu_backward")(x._data_ptr(), dy._data_ptr(), dx._ptr(), len(x))
         return dx
 
     # -- helpers --
@@ -319,7 +308,7 @@ class Tensor:
     def clone(self):
         assert self.is_standard_layout()
         out = _uninit(self.shape, self.dtype)
-        check(lib.agh_memcpy_d2d(out._ptr(), self._data_ptr(), len(self) * _ITEMSIZE[self.dtype]))
+        calls.agh_memcpy_d2d(out._ptr(), self._data_ptr(), len(self) * _ITEMSIZE[self.dtype])
         return out
 
     def as_standard_layout(self):
@@ -337,7 +326,7 @@ class Tensor:
         dims = [1] * pad + list(self.shape)
         sx = [0] * pad + list(self.strides)
         sy = [0] * pad + list(out.strides)
-        check(self._fn("agh_assign")(self._ptr(), self.offset, *sx, out._ptr(), 0, *sy, *dims))
+        self._call("agh_assign")(self._ptr(), self.offset, *sx, out._ptr(), 0, *sy, *dims)
         return out
 
     def broadcast(self, shape):
@@ -367,7 +356,7 @@ class Tensor:
         if x is None:
             raise AghError(-1, f"Broadcast not possible! {rhs.shape} -> {self.shape}")  # ops.rs:287-291
         if self.is_standard_layout() and x.is_standard_layout() and x.shape == rhs.shape:
-            check(self._fn("agh_scaled_add")(self._data_ptr(), alpha, x._data_ptr(), len(self)))
+            self._call("agh_scaled_add")(self._data_ptr(), alpha, x._data_ptr(), len(self))
             return
         if self.ndim > 4:
             raise AghError(-1, "scaled_add: more than 4 dimensions")
@@ -375,7 +364,7 @@ class Tensor:
         dims = [1] * pad + list(self.shape)
         sy = [0] * pad + list(self.strides)
         sx = [0] * pad + list(x.strides)
-        check(self._fn("agh_scaled_add_strided")(self._ptr(), self.offset, *sy, alpha, x._ptr(), x.offset, *sx, *dims))
+        self._call("agh_scaled_add_strided")(self._ptr(), self.offset, *sy, alpha, x._ptr(), x.offset, *sx, *dims)
 
     def add_assign(self, rhs):
         """`AddAssign` (src/tensor/ops.rs:245-255): `self.scaled_add(T::one(), &rhs)`."""
@@ -396,7 +385,7 @@ class Tensor:
         x = self.as_standard_layout()
         rows, cols = x.shape
         y = _uninit((cols,), self.dtype)
-        check(self._fn("agh_sum_axis0")(x._data_ptr(), y._ptr(), rows, cols))
+        self._call("agh_sum_axis0")(x._data_ptr(), y._ptr(), rows, cols)
         return y
 
     def cross_entropy_loss(self, target, out_ptr=None):
@@ -454,9 +443,9 @@ def gemm(alpha, a, b, beta, c, bias=None, relu=False):
     common = (m, k, n, alpha, a._ptr(), a.offset, a.strides[0], a.strides[1], b._ptr(), b.offset, b.strides[0],
               b.strides[1], beta, c._ptr(), c.offset, c.strides[0], c.strides[1])
     if bias is None and not relu:
-        check(getattr(lib, f"agh_gemm_{c.dtype}")(*common))
+        getattr(calls, f"agh_gemm_{c.dtype}")(*common)
     else:
         if bias is not None and (bias.dtype != c.dtype or bias.shape != (n,)):
             raise AghError(-1, f"bias must be a {c.dtype} vector of length {n}")
         bp, bo, bs_ = (bias._ptr(), bias.offset, bias.strides[0]) if bias is not None else (None, 0, 0)
-        check(getattr(lib, f"agh_gemm_{c.dtype}_bias_act")(*common, bp, bo, bs_, 1 if relu else 0))
+        getattr(calls, f"agh_gemm_{c.dtype}_bias_act")(*common, bp, bo, bs_, 1 if relu else 0)

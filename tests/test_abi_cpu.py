@@ -152,3 +152,30 @@ def test_rust_sys_crate_declares_the_header():
                 assert C.sizeof(ct) == C.sizeof(C.c_void_p) and not issubclass(ct, (C.c_int64, C.c_size_t, C.c_float)) or ct is C.c_void_p, (name, t, ct)
             else:
                 assert ct is kind[t] or (C.sizeof(ct) == C.sizeof(kind[t]) and ct._type_ == kind[t]._type_), (name, t, ct)
+
+
+def test_native_calls_mean_what_the_ctypes_calls_mean():
+    """The calls without ctypes: errors carry the entry's code and message, arguments that are no plain numbers (a ctypes pointer, a bool, a
+    numpy integer, too few) do what ctypes makes of them, integers wrap to their width; a Buffer owns what its `ptr` says."""
+    from autograph_amd import AghError, Buffer, _ffi
+    gemm = _ffi.calls.agh_gemm_f32
+    args = [1, 1, 1, 1.0, None, 0, 1, 1, None, 0, 1, 1, 0.0, None, 0, 1, 1]
+    for a in (args, args[:4] + [C.c_void_p(None)] + args[5:], [True] + args[1:], [np.int64(1)] + args[1:]):
+        with pytest.raises(AghError) as e:
+            gemm(*a)
+        assert e.value.code == -2 and "agh_init" in str(e.value)  # no device here
+    for a in (args[:-1], args[:3] + ["1.0"] + args[4:], [1.0] + args[1:]):
+        with pytest.raises((TypeError, C.ArgumentError)):
+            gemm(*a)
+    with pytest.raises(AghError):
+        gemm(2**64 + 1, *args[1:])
+    for size in (16, np.int64(16), True):
+        with pytest.raises(AghError):
+            Buffer(size)
+    for size in (1.5, "16", None):
+        with pytest.raises((TypeError, C.ArgumentError)):
+            Buffer(size)
+    b = Buffer.__new__(Buffer)  # what a failed allocation leaves: nothing is owned, dropping it frees nothing
+    b.ptr = None
+    b.note = "instances take attributes"
+    del b
