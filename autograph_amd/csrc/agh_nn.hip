@@ -1153,6 +1153,91 @@ __global__ __launch_bounds__(kThreads) void max_pool2_backward_kernel(T *__restr
         }
 }
 
+// Square windows of S x S cells, S = 2 or 3 (rows of no whole vectors, odd widths, any stride forward, disjoint backward): U windows a thread, a
+// grid's width apart, all of their cells requested before the first is compared, two neighbouring cells of a row at a time at any
+// element address.  The kernels above, which take any window, compare cell by cell as the loop's loads arrive and find their plane with a
+// 64-bit division.  What bounds it: the L1s, which every row of a window asks for lines that its neighbours share.  Both
+// directions with the clone in between, us: f32 60 x 130 x 90 x 90 in 3 x 3 330 -> 224, bf16 219 -> 142; 22 x 212 x 95 x 95 in 2 x 2 f32 213 -> 154, bf16
+// 127 -> 76.
+template <typename T> struct Pair;
+template <> struct Pair<float> { typedef float type __attribute__((ext_vector_type(2), aligned(4))); };
+template <> struct Pair<uint16_t> { typedef uint16_t type __attribute__((ext_vector_type(2), aligned(2))); };
+constexpr int kPoolU = 2;
+
+template <typename T, int S>
+__device__ __forceinline__ void window_load(const T *src, int iw, T (&v)[S * S]) {
+#pragma unroll
+    for (int i = 0; i < S; ++i) {
+        const typename Pair<T>::type q = *(const typename Pair<T>::type *)(src + (size_t)i * iw);
+        v[i * S] = q.x;
+        v[i * S + 1] = q.y;
+        if constexpr (S == 3) v[i * S + 2] = src[(size_t)i * iw + 2];
+    }
+}
+// the cell of the first strict maximum (a comparison with NaN is false, as in the loop of the general kernels)
+template <typename T, int N>
+__device__ __forceinline__ int window_argmax(const T (&v)[N], T &best) {
+    best = v[0];
+    float mf = Elem<T>::raw(v[0]);
+    int am = 0;
+#pragma unroll
+    for (int k = 1; k < N; ++k) {
+        const float vf = Elem<T>::raw(v[k]);
+        if (vf > mf) { mf = vf; best = v[k]; am = k; }
+    }
+    return am;
+}
+
+template <typename T, int S>
+__global__ __launch_bounds__(kThreads) void max_pool2_square_kernel(const T *__restrict__ x, T *__restrict__ y, PoolParams p, uint32_t total) {
+    const uint32_t e0 = blockIdx.x * (kThreads * kPoolU) + threadIdx.x;
+    T v[kPoolU][S * S];
+#pragma unroll
+    for (int u = 0; u < kPoolU; ++u) {
+        uint32_t row, plane, ho, wo;
+        p.div_ow.divmod(min(e0 + u * kThreads, total - 1), row, wo);
+        p.div_oh.divmod(row, plane, ho);
+        window_load<T, S>(x + ((size_t)plane * p.ih + (size_t)ho * p.sh) * p.iw + (size_t)wo * p.sw, p.iw, v[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < kPoolU; ++u) {
+        T m;
+        window_argmax(v[u], m);
+        if (e0 + u * kThreads < total) y[e0 + u * kThreads] = m;
+    }
+}
+
+template <typename T, int S>
+__global__ __launch_bounds__(kThreads) void max_pool2_backward_square_kernel(T *__restrict__ dx, const T *__restrict__ dy, PoolParams p, uint32_t total) {
+    const uint32_t e0 = blockIdx.x * (kThreads * kPoolU) + threadIdx.x;
+    T v[kPoolU][S * S], g[kPoolU];
+    T *win[kPoolU];
+#pragma unroll
+    for (int u = 0; u < kPoolU; ++u) {
+        const uint32_t e = min(e0 + u * kThreads, total - 1);
+        uint32_t row, plane, ho, wo;
+        p.div_ow.divmod(e, row, wo);
+        p.div_oh.divmod(row, plane, ho);
+        win[u] = dx + ((size_t)plane * p.ih + (size_t)ho * p.sh) * p.iw + (size_t)wo * p.sw;
+        g[u] = dy[e];
+        window_load<T, S>(win[u], p.iw, v[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < kPoolU; ++u) {
+        if (e0 + u * kThreads >= total) break;
+        T m;
+        const int am = window_argmax(v[u], m);
+        const T gv = Elem<T>::from_f32(0.0f + Elem<T>::raw(g[u]));  // `0 + dy` in T, as the host's `+=` on the zeroed cell computes it
+        auto cell = [&](int k) { return k == am ? gv : Elem<T>::zero(); };
+#pragma unroll
+        for (int i = 0; i < S; ++i) {
+            T *dst = win[u] + (size_t)i * p.iw;
+            *(typename Pair<T>::type *)dst = typename Pair<T>::type{cell(i * S), cell(i * S + 1)};
+            if constexpr (S == 3) dst[2] = cell(i * S + 2);
+        }
+    }
+}
+
 // 2x2 windows, stride 2, rows of whole 16-byte vectors: a work item is one 16-byte vector from each of the two
 // rows of a row pair (4 f32 / 8 bf16 elements: 2 / 4 neighbouring windows), so every load instruction of a wave
 // covers 1 KB of the row pair's memory, and the 8 bytes of results leave as one store.  The grid is sized to
@@ -1381,8 +1466,13 @@ int max_pool2_launch(const char *name, const void *x, void *y, int64_t bc, int64
         AGH_LAUNCH_CHECK(name);
         return AGH_OK;
     }
-    hipLaunchKernelGGL(max_pool2_kernel<T>, dim3((unsigned)blocks), dim3(kThreads), 0, stream(), (const T *)x,
-                       (T *)y, p, total);
+    if (h == w && (h == 2 || h == 3) && total < 0x7FFFFFFFull - kThreads * kPoolU) {
+        const dim3 grid((unsigned)((total + kThreads * kPoolU - 1) / (kThreads * kPoolU)));
+        if (h == 2) hipLaunchKernelGGL((max_pool2_square_kernel<T, 2>), grid, dim3(kThreads), 0, stream(), (const T *)x, (T *)y, p, (uint32_t)total);
+        else hipLaunchKernelGGL((max_pool2_square_kernel<T, 3>), grid, dim3(kThreads), 0, stream(), (const T *)x, (T *)y, p, (uint32_t)total);
+    } else
+        hipLaunchKernelGGL(max_pool2_kernel<T>, dim3((unsigned)blocks), dim3(kThreads), 0, stream(), (const T *)x,
+                           (T *)y, p, total);
     AGH_LAUNCH_CHECK(name);
     return AGH_OK;
 }
@@ -1409,8 +1499,13 @@ int max_pool2_backward_launch(const char *name, void *dx, const void *dy, int64_
     } else if (sh >= h && sw >= w) {
         size_t blocks = (total + kThreads - 1) / kThreads;
         if (blocks > 0x7FFFFFFFull) return fail(AGH_ERANGE, "%s: too many elements", name);
-        hipLaunchKernelGGL(max_pool2_backward_kernel<T>, dim3((unsigned)blocks), dim3(kThreads), 0, stream(),
-                           (T *)dx, (const T *)dy, p, total);
+        if (h == w && (h == 2 || h == 3) && total < 0x7FFFFFFFull - kThreads * kPoolU) {
+            const dim3 grid((unsigned)((total + kThreads * kPoolU - 1) / (kThreads * kPoolU)));
+            if (h == 2) hipLaunchKernelGGL((max_pool2_backward_square_kernel<T, 2>), grid, dim3(kThreads), 0, stream(), (T *)dx, (const T *)dy, p, (uint32_t)total);
+            else hipLaunchKernelGGL((max_pool2_backward_square_kernel<T, 3>), grid, dim3(kThreads), 0, stream(), (T *)dx, (const T *)dy, p, (uint32_t)total);
+        } else
+            hipLaunchKernelGGL(max_pool2_backward_kernel<T>, dim3((unsigned)blocks), dim3(kThreads), 0, stream(),
+                               (T *)dx, (const T *)dy, p, total);
     } else {
         size_t blocks = ((size_t)bc + 63) / 64;
         if (blocks > 0x7FFFFFFFull) return fail(AGH_ERANGE, "%s: too many planes", name);

@@ -1478,3 +1478,27 @@ def test_gemm_f32_operands_at_any_address(ag, monkeypatch, m, k, n):
                 assert np.abs(C.into_array() - want).max() <= 1e-5 * np.sqrt(k) * (np.abs(ar) @ np.abs(br)).max()
                 fused = view(ar, ta).dot(view(br, tb), bias=ag.Tensor.from_array(bias), relu=True).into_array()
                 assert np.array_equal(fused, orc.relu(orc.bias_add_rows(plain, bias))), (cfg, splits, ta, tb)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("shape,size,strides", [
+    ((1, 1, 2, 2), 2, 2), ((1, 1, 3, 3), 3, 3), ((3, 5, 17, 23), 2, 2), ((2, 3, 31, 35), 3, 3), ((1, 7, 9, 12), 3, 4), ((2, 2, 11, 13), 2, 3),
+    ((5, 3, 7, 259), 2, 2), ((1, 2, 513, 5), 3, 3), ((4, 4, 12, 10), 3, 2), ((3, 1, 9, 9), 2, 1),
+])
+def test_max_pool2_square_windows(ag, dtype, shape, size, strides):
+    """2 x 2 and 3 x 3 windows on rows of no whole vectors: one window, odd sizes and offsets, strides beyond the window (cells between them keep
+    x) and, forward, below it, batches that end inside a workgroup; ties, NaN, infinities and signed zeros among the values, bit for bit."""
+    bits = np.uint32 if dtype == "f32" else np.uint16
+    rng = np.random.default_rng(shape[3])
+    x = rng.choice(np.array([-2, -1, -0.0, 0.0, 0.5, 0.5, 1, np.nan, np.inf, -np.inf], np.float32), shape, p=[.1, .1, .1, .1, .2, .1, .1, .05, .1, .05])
+    x = to_dtype(x, dtype)
+    opts = ag.MaxPool2Options((size, size), (strides, strides))
+    flat = ag.Tensor.from_array(np.concatenate([np.zeros(1, x.dtype), x.ravel()]))   # the planes begin at an odd element
+    view = lambda: ag.Tensor(flat.buffer, shape, (shape[1] * shape[2] * shape[3], shape[2] * shape[3], shape[3], 1), 1, dtype)  # noqa: E731
+    y = view().max_pool2(opts).into_array()
+    assert np.array_equal(y.view(bits), orc.max_pool2(x, (size, size), (strides, strides)).view(bits))
+    dy = to_dtype(rng.standard_normal(y.shape), dtype)
+    dx = view()
+    dx.max_pool2_backward(ag.Tensor.from_array(dy), opts)
+    assert np.array_equal(dx.into_array().view(bits), orc.max_pool2_backward(x, dy, (size, size), (strides, strides)).view(bits))
+    assert flat.into_array()[0] == 0  # the element in front of the view
