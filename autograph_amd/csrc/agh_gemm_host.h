@@ -281,6 +281,21 @@ inline int plan_splits(int64_t tiles, int ktiles, int64_t cus, int kmin) {
     return (int)std::max<int64_t>(1, std::min(std::min(cus / tiles, (int64_t)(ktiles / kmin)), (int64_t)256));
 }
 
+// What split k costs and saves in bf16, in us, where every workgroup has a CU to itself: k-tiles a split, the second launch and the f32 partial sums
+// by the MB of C (as bf16).  Fitted to 420 products.  Splitting as far as the chip has CUs cost 2000x2048x1008 21.6 us where one split takes 16.2,
+// and 560x3344x2816 (53 k-tiles) gains: 26.3 / 24.5.
+struct Bf16SplitTime { double ktile, second, part_mb; };
+static const Bf16SplitTime kBf16SplitTimes[2] = {{0.44, 3.6, 1.0}, {0.95, 2.3, 0.88}};  // tiles of 128 x 128: whole vectors, any address
+inline double bf16_split_us(const Bf16SplitTime &t, int splits, int ktiles, double mb) {
+    return t.ktile * ((ktiles + splits - 1) / splits) + (splits > 1 ? t.second + t.part_mb * splits * mb : 0.0);
+}
+inline int bf16_best_splits(const Bf16SplitTime &t, int most, int ktiles, double mb) {
+    int best = 1;
+    for (int s = 2; s <= most; ++s)
+        if (bf16_split_us(t, s, ktiles, mb) < bf16_split_us(t, best, ktiles, mb)) best = s;
+    return best;
+}
+
 // Time in us of an f32 product on the direct-to-LDS kernels' 64 x 64 or 128 x 128 tiles, fitted to 450 products of 16 to 60000 x 16 to
 // 8192 x 16 to 8192 outside the small kernel's range (mean error 4 % with whole vectors, 6 % at any address): a launch, rounds of
 // workgroups of so many k-tiles and a store each, the bytes of C, and for split k the second launch and its partial sums.
@@ -463,6 +478,17 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
             cost = rounds == 1 ? (t.bp == 64 ? 0.52 * (kt + 5.0) : 0.95 * (kt + 3.0)) : (double)rounds * (t.bp == 64 ? 0.38 : 0.75) * (kt + 2.0);
         if (best < 0 || cost < best_cost) { best = i; best_cost = cost; }
     }
+    // Operands at any address, more 64 x 64 tiles than CUs and k in splits: 128 x 128 tiles that leave half of the chip idle are a poor second above,
+    // where a tile walks all of k (2661x7265x442 87 -> 47 us in three splits, 664x7239x1744 71 -> 40, 1248x8121x893 76 -> 51).  A tenth is left for the estimate's error
+    // (440x2952x3783 31.3 us on 64 x 64, 35.6 on 128 x 128 in two).  Not with the fixed scratch memory, nor where a capture cannot have more.
+    if (sizeof(T) == 2 && any_addr && best == 4 && batch == 1 && g.NP > 64 && g.NQ > 64 && !fixed_scratch && !setting("AGH_GEMM_SPLITS")) {
+        const int64_t tiles = (int64_t)((g.NP + 127) / 128) * ((g.NQ + 127) / 128), small = (int64_t)((g.NP + 63) / 64) * ((g.NQ + 63) / 64);
+        const int ktiles = (g.K + BK - 1) / BK, most = (int)std::min<int64_t>(cus / tiles, ktiles / 12);
+        const double mb = (double)g.NP * g.NQ * 2e-6;
+        const int s = ktiles >= 32 && small > cus ? bf16_best_splits(kBf16SplitTimes[1], most, ktiles, mb) : 1;
+        if (s > 1 && bf16_split_us(kBf16SplitTimes[1], s, ktiles, mb) + 3 * 0.95 < 0.9 * best_cost && workspace_ready((size_t)s * g.NQ * g.NPpad * sizeof(float)))
+            best = 3;
+    }
     if (forced_cfg >= 0) best = forced_cfg;
 
 #ifdef AGH_GEMM_WITH_F32_DIRECT
@@ -535,6 +561,8 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
     // at least four k-tiles a split; twelve for the bf16 128 x 128 direct tile, whose four-stage ring makes fewer,
     // longer splits the better trade (128x4096x4096: 17.0-17.2 us in 4 to 6 splits, 19.5 in 8)
     int splits = batch == 1 ? plan_splits(tiles, ktiles, cus, direct_ok && best == 3 ? 12 : 4) : 1;
+    if (sizeof(T) == 2 && direct_ok && best == 3 && splits > 1)
+        splits = bf16_best_splits(kBf16SplitTimes[any_addr], splits, ktiles, (double)g.NP * g.NQ * 2e-6);
     if (batch == 1) splits = env_int("AGH_GEMM_SPLITS", splits);
     if (splits < 1) splits = 1;
     if (splits > ktiles && ktiles > 0) splits = ktiles;

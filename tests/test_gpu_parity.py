@@ -1502,3 +1502,24 @@ def test_max_pool2_square_windows(ag, dtype, shape, size, strides):
     dx.max_pool2_backward(ag.Tensor.from_array(dy), opts)
     assert np.array_equal(dx.into_array().view(bits), orc.max_pool2_backward(x, dy, (size, size), (strides, strides)).view(bits))
     assert flat.into_array()[0] == 0  # the element in front of the view
+
+
+@pytest.mark.parametrize("m,k,n", [(1100, 4103, 1101), (2001, 3001, 301), (2000, 2048, 1008), (560, 3344, 1408), (1408, 4096, 1400)])
+def test_gemm_bf16_split_by_cost(ag, monkeypatch, m, k, n):
+    """bf16 products whose tiles leave CUs idle, at any address and of whole vectors: split k and 128 x 128 tiles as the estimate chooses them give
+    whole numbers exactly and agree with one split of 64 x 64 tiles within a rounding; the entry without allocations takes them too."""
+    rng = np.random.default_rng(k)
+    ai, bi = (to_dtype(rng.integers(-2, 3, s).astype(np.float32), "bf16") for s in ((m, k), (k, n)))
+    want = orc.f32_to_bf16((orc.bf16_to_f32(ai) @ orc.bf16_to_f32(bi)).astype(np.float32))
+    A, B = ag.Tensor.from_array(ai), ag.Tensor.from_array(bi)
+    assert np.array_equal(A.dot(B).into_array(), want)
+    out = ag.Tensor.zeros((m, n), "bf16")
+    ag._ffi.check(ag.lib.agh_gemm_bf16_noalloc(m, k, n, 1.0, A._ptr(), 0, k, 1, B._ptr(), 0, n, 1, 0.0, out._ptr(), 0, n, 1))
+    assert np.array_equal(out.into_array(), want)
+    a, b = (ag.Tensor.from_array(to_dtype(rng.standard_normal(s), "bf16")) for s in ((m, k), (k, n)))
+    got = orc.bf16_to_f32(a.dot(b).into_array())
+    monkeypatch.setenv("AGH_GEMM_CFG", "4")
+    monkeypatch.setenv("AGH_GEMM_SPLITS", "1")
+    one = orc.bf16_to_f32(a.dot(b).into_array())
+    # f32 sums of k products of unit variance in two orders, each rounded to bf16: a step of the larger magnitude and what the sums differ by
+    assert np.all(np.abs(got - one) <= 2.0**-7 * np.maximum(np.abs(got), np.abs(one)) + 8 * k * 2.0**-24)
