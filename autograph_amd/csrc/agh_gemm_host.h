@@ -480,13 +480,16 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
     }
     // Operands at any address, more 64 x 64 tiles than CUs and k in splits: 128 x 128 tiles that leave half of the chip idle are a poor second above,
     // where a tile walks all of k (2661x7265x442 87 -> 47 us in three splits, 664x7239x1744 71 -> 40, 1248x8121x893 76 -> 51).  A tenth is left for the estimate's error
-    // (440x2952x3783 31.3 us on 64 x 64, 35.6 on 128 x 128 in two).  Not with the fixed scratch memory, nor where a capture cannot have more.
-    if (sizeof(T) == 2 && any_addr && best == 4 && batch == 1 && g.NP > 64 && g.NQ > 64 && !fixed_scratch && !setting("AGH_GEMM_SPLITS")) {
+    // (440x2952x3783 31.3 us on 64 x 64, 35.6 on 128 x 128 in two).  Not where a capture cannot have the scratch memory for it; the fixed one holds
+    // a 128 x 128 tile of partial sums for each of 256 CUs, so agh_gemm_bf16_noalloc takes the same way and gives the same bits.
+    if (sizeof(T) == 2 && any_addr && best == 4 && batch == 1 && g.NP > 64 && g.NQ > 64 && !setting("AGH_GEMM_SPLITS")) {
         const int64_t tiles = (int64_t)((g.NP + 127) / 128) * ((g.NQ + 127) / 128), small = (int64_t)((g.NP + 63) / 64) * ((g.NQ + 63) / 64);
         const int ktiles = (g.K + BK - 1) / BK, most = (int)std::min<int64_t>(cus / tiles, ktiles / 12);
         const double mb = (double)g.NP * g.NQ * 2e-6;
         const int s = ktiles >= 32 && small > cus ? bf16_best_splits(kBf16SplitTimes[1], most, ktiles, mb) : 1;
-        if (s > 1 && bf16_split_us(kBf16SplitTimes[1], s, ktiles, mb) + 3 * 0.95 < 0.9 * best_cost && workspace_ready((size_t)s * g.NQ * g.NPpad * sizeof(float)))
+        const size_t bytes = (size_t)s * g.NQ * g.NPpad * sizeof(float);
+        if (s > 1 && bf16_split_us(kBf16SplitTimes[1], s, ktiles, mb) + 3 * 0.95 < 0.9 * best_cost &&
+            (fixed_scratch ? bytes <= (size_t)AGH_NOALLOC_SCRATCH_BYTES : workspace_ready(bytes)))
             best = 3;
     }
     if (forced_cfg >= 0) best = forced_cfg;
@@ -504,9 +507,13 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
             const double us64 = f32_tile_us(64, any_addr, g.NP, g.NQ, g.K, batch, cus, &s64);
             const double us128 = f32_tile_us(128, any_addr, g.NP, g.NQ, g.K, batch, cus, &s128);
             const int64_t tiles128 = (int64_t)((g.NP + 127) / 128) * ((g.NQ + 127) / 128) * batch;
-            if (any_addr) best = us128 < us64 ? 3 : 4;
-            else if (best == 4 && us128 < 0.97 * us64) best = 3;
-            else if (best == 3 && us64 < 0.97 * us128 && s64 >= s128) {
+            // (a capture that cannot have scratch memory for the splits of the other tile keeps the one it had)
+            const int64_t part = (int64_t)g.NQ * g.NPpad * (int64_t)sizeof(float);
+            const bool ready64 = s64 == 1 || workspace_ready((size_t)(s64 * part)), ready128 = s128 == 1 || workspace_ready((size_t)(s128 * part));
+            if (any_addr) {
+                if (us128 < us64 ? ready128 : ready64) best = us128 < us64 ? 3 : 4;
+            } else if (best == 4 && us128 < 0.97 * us64 && ready128) best = 3;
+            else if (best == 3 && us64 < 0.97 * us128 && s64 >= s128 && ready64) {
                 best = 4;
                 g.two_sums = tiles128 * s128 <= cus;
             }

@@ -1518,8 +1518,43 @@ def test_gemm_bf16_split_by_cost(ag, monkeypatch, m, k, n):
     assert np.array_equal(out.into_array(), want)
     a, b = (ag.Tensor.from_array(to_dtype(rng.standard_normal(s), "bf16")) for s in ((m, k), (k, n)))
     got = orc.bf16_to_f32(a.dot(b).into_array())
+    ag._ffi.check(ag.lib.agh_gemm_bf16_noalloc(m, k, n, 1.0, a._ptr(), 0, k, 1, b._ptr(), 0, n, 1, 0.0, out._ptr(), 0, n, 1))
+    assert np.array_equal(orc.bf16_to_f32(out.into_array()), got)  # the same plan
     monkeypatch.setenv("AGH_GEMM_CFG", "4")
     monkeypatch.setenv("AGH_GEMM_SPLITS", "1")
     one = orc.bf16_to_f32(a.dot(b).into_array())
     # f32 sums of k products of unit variance in two orders, each rounded to bf16: a step of the larger magnitude and what the sums differ by
     assert np.all(np.abs(got - one) <= 2.0**-7 * np.maximum(np.abs(got), np.abs(one)) + 8 * k * 2.0**-24)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,m,k,n", [("f32", 136, 7008, 3004), ("f32", 133, 7001, 3003), ("bf16", 664, 7239, 1744)])
+def test_gemm_captured_before_any_split_had_scratch(ag, dtype, m, k, n):
+    """A product that runs in splits of k where scratch memory can be had, and that the general tile choice does not split, can be captured
+    without any: it then keeps that choice.  The same product called eagerly takes the splits, and so does a capture after it."""
+    rng = np.random.default_rng(m)
+    ai, bi = (to_dtype(rng.integers(-1, 2, s).astype(np.float32), dtype) for s in ((m, k), (k, n)))
+    A, B = ag.Tensor.from_array(ai), ag.Tensor.from_array(bi)
+    want = ai @ bi if dtype == "f32" else orc.f32_to_bf16((orc.bf16_to_f32(ai) @ orc.bf16_to_f32(bi)).astype(np.float32))
+    out = ag.Tensor.zeros((m, n), dtype)
+    call = getattr(ag.lib, f"agh_gemm_{dtype}")
+
+    def dot():
+        ag._ffi.check(call(m, k, n, 1.0, A._ptr(), 0, k, 1, B._ptr(), 0, n, 1, 0.0, out._ptr(), 0, n, 1))
+
+    check = ag._ffi.check
+    check(ag.lib.agh_sync())
+    check(ag.lib.agh_cache_release())  # the library's scratch memory is handed back, unless a graph of an earlier test still names it
+    for _ in range(2):
+        graph = C.c_void_p()
+        check(ag.lib.agh_graph_begin())
+        dot()
+        check(ag.lib.agh_graph_end(C.byref(graph)))
+        for _ in range(3):
+            check(ag.lib.agh_memset(out._ptr(), 0, out.buffer.nbytes))
+            check(ag.lib.agh_graph_launch(graph))
+            check(ag.lib.agh_sync())
+            assert np.array_equal(out.into_array(), want)
+        check(ag.lib.agh_graph_destroy(graph))
+        dot()
+        assert np.array_equal(out.into_array(), want)
