@@ -349,8 +349,8 @@ int agh_lenet5_weight_grads_bf16(const void *a2, const void *a1, const void *f, 
                                  const void *target, void *loss, const void *x, const void *p1, const void *gm1, const void *gm2,
                                  void *dw1, void *dw2, int64_t bs);
 
-/* The whole step (autograph_backend.rs:70-86): forward, loss, gradients and the update of all six parameters, two launches up to a batch of
- * 256 and four beyond.  Same values and bits as the entry points above followed by agh_sgd_momentum_<T> (agh_scaled_add_<T> with
+/* The whole step (autograph_backend.rs:70-86): forward, loss, gradients and the update of all six parameters, two
+ * launches.  Same values and bits as the entry points above followed by agh_sgd_momentum_<T> (agh_scaled_add_<T> with
  * -learning_rate where velocities is null).  Arrays of device pointers, read before the call returns:
  *   params, velocities, grads   conv1 [6,1,5,5], conv2 [16,6,5,5], dense1 [256,128], dense2 [128,84], dense3 [84,10], its bias [10]
  *   saves                       c1, p1, c2, p2, d1, a1, d2, a2 as agh_lenet5_forward_train_<T> writes them, logits [bs,10]
