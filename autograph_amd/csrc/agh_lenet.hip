@@ -1,5 +1,6 @@
 // The LeNet5 of the reference's benchmark (benches/neural-network-benches/src/autograph_backend.rs:70-162): inference in one
 // launch, and the launches of its training step.
+#include <cstddef>
 #include <type_traits>
 
 #include "agh_internal.h"
@@ -1265,8 +1266,9 @@ int lenet5_weight_grads_entry(const char *name, const void *a2, const void *a1, 
 // gradients, adds the shares, and whoever finishes a gradient updates its parameter (nothing else reads the parameters there).  Every value is
 // rounded where the separate launches round it and summed in their order, so gradients, loss and parameters have their bits.  What bounds the
 // first launch is its chain of eighteen stages behind barriers, 40000 cycles in bf16, the longest 7000 (shares of the weight gradients), 4300
-// (staging), 3900 (col2im) and 3800 (conv2); a batch beyond 256 is several rounds of it, one workgroup per CU.  A captured step, bf16 /
-// f32: batch 100 42.3 -> 27.4 us / 42.7 -> 26.0, 400 70.8 -> 48.9 / 82.0 -> 45.5, 1000 109 -> 90 / 135 -> 82.
+// (staging), 3900 (col2im) and 3800 (conv2); a batch beyond 512 is several rounds of it, two workgroups per CU (one per CU, with
+// arrays of their own for everything: in brackets).  A captured step, five launches -> here, bf16 / f32: batch 100 42.3 -> 27.4 us / 42.7 -> 26.0,
+// 400 70.8 -> 40.7 (48.9) / 82.4 -> 38.5 (45.5), 1000 109.7 -> 70.9 (90) / 135.3 -> 65.8 (82), 2048 194 -> 127 (168) / 248 -> 117 (152).
 template <typename T>
 struct LenetStep {
     const T *x, *w1, *w2, *wd1, *wd2, *wd3, *b3;
@@ -1278,15 +1280,25 @@ struct LenetStep {
 };
 
 template <typename T, bool WHOLE>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void lenet5_step_image_kernel(LenetStep<T> a, LenetSaves<T> sv) {
-    __shared__ LenetForwardLds<T, 1> s;
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 4))) void lenet5_step_image_kernel(LenetStep<T> a, LenetSaves<T> sv) {
+    // Two workgroups fit a CU (LDS 81144 bytes in f32, 67952 in bf16; 128 registers): behind the dense layers' gradients the forward pass's last
+    // arrays (parts, wd2s, wd3s) are free.  There lie pm, gp1s behind it, and when pm has been read g1 and behind it q2 and q1, each written
+    // behind a barrier after the last read of what it replaces.
+    using Forward = LenetForwardLds<T, 1>;
+    constexpr int kFree = offsetof(Forward, parts), kPm = 64 * kPmPitch, kG1 = 576 * 6, kSize = sizeof(Forward);
+    constexpr int kBackward = kFree + (kPm + 864) * 4;
+    static_assert(kG1 + 24 * 150 <= kPm + 864 && kFree % 16 == 0, "g1, q2 and q1 fit where pm and gp1s were");
+    __shared__ __align__(16) unsigned char lds[kSize > kBackward ? kSize : kBackward];
+    Forward &s = *(Forward *)lds;
     __shared__ LenetStepLds st;
     __shared__ __align__(16) float gm2s[64 * 16];  // gradient of conv2's output, [y*8 + x][oc]
-    __shared__ __align__(8) float g1[576 * 6];     // of conv1's output, [y*24 + x][oc]
     __shared__ __align__(16) float gd1s[128], gd2s[84];
-    __shared__ float gls[16], gfs[256], gp1s[864];
-    __shared__ float pm[64 * kPmPitch];            // gm2 . W, every entry rounded to T
-    __shared__ float q2[16 * 150], q1[8 * 150];
+    __shared__ float gls[16];
+    float *const gfs = s.p2;                  // 256: gradient of the flattened features, for the features themselves
+    float *const pm = (float *)(lds + kFree);  // gm2 . W, every entry rounded to T
+    float *const gp1s = pm + kPm;             // 864: gradient of conv1's pooled output
+    float *const g1 = pm;                     // of conv1's output, [y*24 + x][oc]
+    float *const q2 = g1 + kG1, *const q1 = q2 + 16 * 150;
     constexpr int NT = 512;
     const int tid = threadIdx.x;
     const size_t b = blockIdx.x;
