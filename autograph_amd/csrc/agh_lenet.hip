@@ -125,7 +125,7 @@ __device__ __forceinline__ uint32_t lds_address_of(const void *p) {
     return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char *)p;
 }
 
-// waves_per_eu(2, 2): eight waves per workgroup are two per SIMD whatever the register count; without the hint the
+// waves_per_eu: eight waves per workgroup are two per SIMD, four where two workgroups of one image share a CU; without the hint the
 // compiler aimed the bf16 training instantiation at 128 registers and gave up the early weight loads for it (30 us
 // instead of 20)
 // IMGS images per workgroup.  4: a batch of a thousand is one round of 250 workgroups.  1 (batches up to 256, e.g. the
@@ -539,15 +539,15 @@ __device__ __forceinline__ void lenet5_forward_body(LenetForwardLds<T, IMGS> &s,
     }
 }
 
-template <typename T, bool SAVE, int IMGS>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void lenet5_forward_kernel(const T *__restrict__ x, const T *__restrict__ w1,
+template <typename T, bool SAVE, int IMGS, bool WHOLE>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, IMGS == 1 ? 4 : 2))) void lenet5_forward_kernel(const T *__restrict__ x, const T *__restrict__ w1,
                                                               const T *__restrict__ w2, const T *__restrict__ wd1,
                                                               const T *__restrict__ wd2, const T *__restrict__ wd3,
                                                               const T *__restrict__ b3, T *__restrict__ out, int bs,
                                                               LenetSaves<T> sv, int w23_aligned) {
     __shared__ LenetForwardLds<T, IMGS> s;
     float4 wreg[16];
-    lenet5_forward_body<T, SAVE, IMGS, false>(s, x, w1, w2, wd1, wd2, wd3, b3, out, bs, sv, w23_aligned, nullptr, wreg, [] {});
+    lenet5_forward_body<T, SAVE, IMGS, WHOLE>(s, x, w1, w2, wd1, wd2, wd3, b3, out, bs, sv, w23_aligned, nullptr, wreg, [] {});
 }
 
 // The input-gradient chain of a LeNet5 training step in one launch, one workgroup per image: cross-entropy backward,
@@ -1543,15 +1543,21 @@ int lenet5_forward_entry(const char *name, const void *x, const void *w1, const 
         sv = {(T *)saves[0], (T *)saves[1], (T *)saves[2], (T *)saves[3], (T *)saves[4], (T *)saves[5], (T *)saves[6], (T *)saves[7]};
     }
     // one image per workgroup while that still fits the chip in one round
-    const bool single = bs <= 256;  // measured: 7.0 against 11.2 us up to 256 images, 13.1 against 11.3 us at 384
-#define AGH_LENET(SAVEV, IMGSV) \
-    hipLaunchKernelGGL((lenet5_forward_kernel<T, SAVEV, IMGSV>), dim3((unsigned)((bs + IMGSV - 1) / IMGSV)), dim3(512), 0, stream(), \
+    const bool single = bs <= 256;  // measured: 7.0 against 11.2 us up to 256 images
+    // Two such workgroups share a CU.  Where they need few enough rounds (of 256 images: every further one costs a third of the time that a round of
+    // 1024 takes with four images a workgroup), they are faster up to a batch of 512, from 1025 to 1280 and from 2049 to 2304: f32 257 10.9 -> 9.1 us, 512
+    // 11.0 -> 9.6, 1025 20.5 -> 18.1, 2304 30.9 -> 30.8, bf16 12.8 -> 9.4, 12.9 -> 10.1, 24.2 -> 19.4, 36.2 -> 33.6; beyond: f32 600 11.0 / 12.7,
+    // 1536 21.0 / 21.7, bf16 1000 12.9 / 16.9.  Conv2's sums are one chain, as with four images a workgroup: the same bits.
+    const int64_t rounds1 = (bs + 255) / 256, rounds4 = (bs + 1023) / 1024;
+    const bool pairs = rounds1 <= 3 * rounds4 - (rounds4 < 3);
+#define AGH_LENET(SAVEV, IMGSV, WHOLEV) \
+    hipLaunchKernelGGL((lenet5_forward_kernel<T, SAVEV, IMGSV, WHOLEV>), dim3((unsigned)((bs + IMGSV - 1) / IMGSV)), dim3(512), 0, stream(), \
                        (const T *)x, (const T *)w1, (const T *)w2, (const T *)wd1, (const T *)wd2, (const T *)wd3, (const T *)b3, \
                        (T *)logits, (int)bs, sv, w23_aligned)
     if (saves) {
-        if (single) AGH_LENET(true, 1); else AGH_LENET(true, 4);
+        if (single) AGH_LENET(true, 1, false); else if (pairs) AGH_LENET(true, 1, true); else AGH_LENET(true, 4, false);
     } else {
-        if (single) AGH_LENET(false, 1); else AGH_LENET(false, 4);
+        if (single) AGH_LENET(false, 1, false); else if (pairs) AGH_LENET(false, 1, true); else AGH_LENET(false, 4, false);
     }
 #undef AGH_LENET
     AGH_LAUNCH_CHECK(name);

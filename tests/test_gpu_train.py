@@ -442,6 +442,22 @@ def test_lenet5_train_step_in_two_launches(ag, dtype, bs, momentum):
             ag._ffi.check(getattr(ag.lib, f"agh_lenet5_train_step_{dtype}")(tx._ptr(), tt.ptr, *args, 1.0, 0.1, 0.9, None, bs))
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_lenet5_logits_do_not_depend_on_the_batch_above_256(ag, dtype):
+    """One image or four a workgroup, by the rounds a batch takes: the logits of an image have the same bits on either side of every change."""
+    rng = np.random.default_rng(8)
+    params = [ag.Tensor.from_array(to_dtype(p, dtype)) for p in lenet_params(rng)]
+    x = to_dtype(rng.uniform(0, 1, (2432, 1, 28, 28)), dtype)
+
+    def logits(bs):
+        tx, out = ag.Tensor.from_array(x[:bs]), ag.Tensor.zeros((bs, 10), dtype)
+        ag._ffi.check(getattr(ag.lib, f"agh_lenet5_forward_{dtype}")(tx._ptr(), *[p._ptr() for p in params], out._ptr(), bs))
+        return out.into_array()
+    want = logits(2432)  # four a workgroup
+    for bs in (257, 511, 512, 513, 1024, 1025, 1280, 1281, 2048, 2049, 2304, 2305):
+        assert np.array_equal(logits(bs), want[:bs]), bs
+
+
 @pytest.mark.parametrize("fused_backward", [True, False])
 @pytest.mark.parametrize("fused_forward", [True, False])
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
