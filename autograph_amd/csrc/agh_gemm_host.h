@@ -507,11 +507,13 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
             const double us64 = f32_tile_us(64, any_addr, g.NP, g.NQ, g.K, batch, cus, &s64);
             const double us128 = f32_tile_us(128, any_addr, g.NP, g.NQ, g.K, batch, cus, &s128);
             const int64_t tiles128 = (int64_t)((g.NP + 127) / 128) * ((g.NQ + 127) / 128) * batch;
-            // (a capture that cannot have scratch memory for the splits of the other tile keeps the one it had)
+            // (A capture that cannot have scratch memory for the splits of the other tile keeps the one it had.  At any address that is 64 x 64,
+            // whatever the cost above says: it is split only where the element-wise loaders' choice is, and needs no more scratch memory, so no
+            // capture is refused that those could serve, 1279x1023x959 for one: one split there, three on 128 x 128.)
             const int64_t part = (int64_t)g.NQ * g.NPpad * (int64_t)sizeof(float);
             const bool ready64 = s64 == 1 || workspace_ready((size_t)(s64 * part)), ready128 = s128 == 1 || workspace_ready((size_t)(s128 * part));
             if (any_addr) {
-                if (us128 < us64 ? ready128 : ready64) best = us128 < us64 ? 3 : 4;
+                best = us128 < us64 && ready128 ? 3 : 4;
             } else if (best == 4 && us128 < 0.97 * us64 && ready128) best = 3;
             else if (best == 3 && us64 < 0.97 * us128 && s64 >= s128 && ready64) {
                 best = 4;

@@ -6,6 +6,7 @@ Bars: im2col / col2im / pooling / relu bit-exact; f32 gemm within 1e-5*sqrt(K) r
 bf16 gemm within 1 bf16 ulp + 1e-2 relative of an f32-accumulated reference.
 """
 import ctypes as C  # noqa: F401
+import gc
 import time
 
 import numpy as np
@@ -1527,34 +1528,55 @@ def test_gemm_bf16_split_by_cost(ag, monkeypatch, m, k, n):
     assert np.all(np.abs(got - one) <= 2.0**-7 * np.maximum(np.abs(got), np.abs(one)) + 8 * k * 2.0**-24)
 
 
-@pytest.mark.gpu
-@pytest.mark.parametrize("dtype,m,k,n", [("f32", 136, 7008, 3004), ("f32", 133, 7001, 3003), ("bf16", 664, 7239, 1744)])
-def test_gemm_captured_before_any_split_had_scratch(ag, dtype, m, k, n):
-    """A product that runs in splits of k where scratch memory can be had, and that the general tile choice does not split, can be captured
-    without any: it then keeps that choice.  The same product called eagerly takes the splits, and so does a capture after it."""
+@pytest.mark.parametrize("branch", [False, True])
+@pytest.mark.parametrize("dtype,m,k,n", [("f32", 136, 7008, 3004), ("f32", 133, 7001, 3003), ("f32", 1279, 1023, 959), ("f32", 1500, 1501, 1001),
+                                         ("bf16", 664, 7239, 1744)])
+def test_gemm_captured_before_any_split_had_scratch(ag, dtype, m, k, n, branch):
+    """A product that runs in splits of k where scratch memory can be had, and that takes one split on 64 x 64 tiles, can be captured
+    without any, on the main stream and in a branch (whose scratch memory is its own).  The same product called eagerly takes the splits, and
+    so does a capture after it."""
     rng = np.random.default_rng(m)
     ai, bi = (to_dtype(rng.integers(-1, 2, s).astype(np.float32), dtype) for s in ((m, k), (k, n)))
     A, B = ag.Tensor.from_array(ai), ag.Tensor.from_array(bi)
     want = ai @ bi if dtype == "f32" else orc.f32_to_bf16((orc.bf16_to_f32(ai) @ orc.bf16_to_f32(bi)).astype(np.float32))
     out = ag.Tensor.zeros((m, n), dtype)
     call = getattr(ag.lib, f"agh_gemm_{dtype}")
+    check, lib = ag._ffi.check, ag.lib
 
     def dot():
-        ag._ffi.check(call(m, k, n, 1.0, A._ptr(), 0, k, 1, B._ptr(), 0, n, 1, 0.0, out._ptr(), 0, n, 1))
+        if branch:
+            check(lib.agh_branch_begin())
+        try:
+            check(call(m, k, n, 1.0, A._ptr(), 0, k, 1, B._ptr(), 0, n, 1, 0.0, out._ptr(), 0, n, 1))
+        finally:
+            if branch:
+                check(lib.agh_branch_end())
+                check(lib.agh_branch_join())
 
-    check = ag._ffi.check
-    check(ag.lib.agh_sync())
-    check(ag.lib.agh_cache_release())  # the library's scratch memory is handed back, unless a graph of an earlier test still names it
-    for _ in range(2):
+    def scratch():
+        nbytes = C.c_size_t()
+        check(lib.agh_workspace_stats(C.byref(nbytes), None))
+        return nbytes.value
+
+    gc.collect()  # (a graph that an earlier test has dropped would keep the scratch memory it names)
+    check(lib.agh_sync())
+    check(lib.agh_cache_release())
+    for had in (False, True):
+        assert (scratch() > 0) == had, "no product has run yet that needs scratch memory" if not had else "the eager product took splits"
         graph = C.c_void_p()
-        check(ag.lib.agh_graph_begin())
-        dot()
-        check(ag.lib.agh_graph_end(C.byref(graph)))
-        for _ in range(3):
-            check(ag.lib.agh_memset(out._ptr(), 0, out.buffer.nbytes))
-            check(ag.lib.agh_graph_launch(graph))
-            check(ag.lib.agh_sync())
-            assert np.array_equal(out.into_array(), want)
-        check(ag.lib.agh_graph_destroy(graph))
+        check(lib.agh_graph_begin())
+        try:
+            try:
+                dot()
+            finally:
+                check(lib.agh_graph_end(C.byref(graph)))
+            for _ in range(3):
+                check(lib.agh_memset(out._ptr(), 0, out.buffer.nbytes))
+                check(lib.agh_graph_launch(graph))
+                check(lib.agh_sync())
+                assert np.array_equal(out.into_array(), want)
+        finally:
+            if graph:
+                check(lib.agh_graph_destroy(graph))
         dot()
         assert np.array_equal(out.into_array(), want)
