@@ -284,14 +284,16 @@ int conv2_taps16_try(const char *name, const void *x, const void *w, const void 
     }
     if (!tg || (!forced && us > limit_us)) return 1;
     const int64_t passes = (all_groups + groups - 1) / groups, units = taps * groups, steps = (units + 3) / 4;
-    const int64_t yh = pool ? oh / 2 : oh, yw = pool ? ow / 2 : ow, nall = pool ? yh * yw * 4 : npos;
     const int64_t pitch = groups * 16 + 16, tab_bytes = (steps + 1) * 16;
-    auto lds_bytes = [&]() { return rows * cols * pitch + tab_bytes; };
-    if (pool) {  // the tile's positions are fewer where its rows, less than three times as many, take too much of the LDS
-        auto pool_rows = [&]() { rows = (2 * std::min(yh - 1, (16 * tg - 1 + yw - 1) / yw) + 1) * sh + (fh - 1) * dh + 1; };
-        for (pool_rows(); tg > 1 && lds_bytes() > kTaps16PoolLds; pool_rows()) tg /= 2;
-        if (lds_bytes() > 160 * 1024) return 1;
-    }
+    auto lds_bytes = [&](int64_t r) { return r * cols * pitch + tab_bytes; };
+    // rows of a tile of 16 t windows
+    auto pool_rows = [&](int64_t t) { return (2 * std::min(oh / 2 - 1, (16 * t - 1 + ow / 2 - 1) / (ow / 2)) + 1) * sh + (fh - 1) * dh + 1; };
+    // A stride of four rows and more can make the windows' rows several times the plain positions': where even the smallest tile of them does not fit,
+    // neither call is taken here, since the fused one returns the bits of the plain one (one in a hundred shapes of strides 1 to 8 that would be).
+    if (oh >= 2 && ow >= 2 && lds_bytes(pool_rows(1)) > 160 * 1024) return 1;
+    const int64_t yh = pool ? oh / 2 : oh, yw = pool ? ow / 2 : ow, nall = pool ? yh * yw * 4 : npos;
+    if (pool)  // the tile's positions are fewer where its rows take too much of the LDS
+        for (rows = pool_rows(tg); tg > 1 && lds_bytes(rows) > kTaps16PoolLds; rows = pool_rows(tg)) tg /= 2;
     const int64_t ptiles = (nall + 64 * tg - 1) / (64 * tg), gx = bs * ptiles, gy = (n16 + nt - 1) / nt;
     const int64_t frags = n16 * passes * steps * 64;
     if (gx > 0x7FFFFFFF || gy > 65535 || frags > 0x7FFFFFFF) return 1;
@@ -310,7 +312,7 @@ int conv2_taps16_try(const char *name, const void *x, const void *w, const void 
     q.div_ptiles = FastDiv((uint32_t)ptiles); q.div_cols = FastDiv((uint32_t)cols); q.div_rows = FastDiv((uint32_t)rows);
     q.div_yw = FastDiv((uint32_t)yw); q.div_groups = FastDiv((uint32_t)groups); q.div_fw = FastDiv((uint32_t)fw);
     const dim3 grid((unsigned)gx, (unsigned)gy);
-    const size_t smem = (size_t)lds_bytes();
+    const size_t smem = (size_t)lds_bytes(rows);
 #define AGH_TAPS16(TGV, NTV) \
     case TGV * 8 + NTV: \
         return pool ? taps16_launch<TGV, NTV, true>(name, x, wp, bias, y, grid, smem, q) \

@@ -334,6 +334,30 @@ def test_conv2_fused_pool_out_of_staged_rows_equals_the_layers(ag, dtype, case):
         assert np.array_equal(got, want), (relu, np.mean(got != want))
 
 
+@pytest.mark.parametrize("case", [
+    # bs, ic, ih, iw, oc, filter, padding, stride: a fused pool's rows take more than a CU's LDS where the plain call's take less than 64 KB
+    (16, 8, 41, 405, 128, (1, 1), (0, 0), (4, 4)),
+    (30, 8, 115, 324, 32, (1, 1), (0, 0), (5, 3)),
+    (11, 64, 57, 79, 32, (2, 2), (1, 1), (8, 1)),
+    (16, 16, 66, 218, 128, (1, 1), (0, 0), (8, 1)),
+    (30, 8, 25, 324, 32, (1, 1), (0, 0), (4, 3)),      # just inside
+])
+def test_conv2_bf16_fused_pool_whose_rows_exceed_lds_equals_the_layers(ag, case):
+    """The same where the rows of a workgroup's windows are many times those of as many plain positions (a stride of four rows and more): both
+    calls take the same kernel, or neither.  Two terms that cancel make the order of the sums visible in bf16."""
+    bs, ic, ih, iw, oc, f, p, s = case
+    rng = np.random.default_rng(34)
+    x, w = rng.standard_normal((bs, ic, ih, iw)), rng.standard_normal((oc, ic) + f)
+    x[:, 0] *= 4096
+    x[:, ic - 1] = x[:, 0]
+    w[:, ic - 1, 0, 0] = -w[:, 0, 0, 0]
+    conv = ag.Conv2(ag.Tensor.from_array(to_dtype(w, "bf16")), None, p, s)
+    x = ag.Tensor.from_array(to_dtype(x, "bf16"))
+    want = ag.MaxPool2((2, 2)).forward(conv.forward(x)).into_array()
+    got = conv.forward(x, pool2x2=True).into_array()
+    assert np.array_equal(got, want), np.mean(got != want)
+
+
 def test_conv2_route_is_the_faster_one(ag, monkeypatch):
     """Conv2 out of staged rows or by im2col and a product, as chosen by size: within a quarter of the faster."""
     for bs, ic, h, oc, f, p, s, dtype in ((205, 3, 50, 128, 7, 3, 1, "bf16"), (4, 128, 81, 16, 7, 0, 1, "bf16"), (64, 3, 95, 64, 7, 3, 2, "f32"),
