@@ -671,6 +671,9 @@ int conv2_direct_entry(const char *name, const void *x, const void *w, const voi
     // the matrix-core kernel of any geometry, where it expects to need less time than what would run in its place; with the
     // pool, where the convolution alone would run on it (the fused call returns the same bits as the separate layers)
     const double taps_limit = taps_forced != 0 ? conv2_taps_limit<T>(shape) : 0.0;
+    // scratch memory that a capture cannot have for the bf16 kernel chosen: workspace() refuses it then, and says that the sequence has to run once eagerly
+    size_t lacking = 0;
+    void *unused = nullptr;
     const bool implicit_gemm_plain = pool2x2 && shape.unit() && conv2_mfma_takes<T>(x, w, bs, ic, ih, iw, oc, fh, fw, pw, oh, ow);
     if (sizeof(T) == 2 && (taps16_forced || (taps_forced < 0 && taps_limit >= kTapsLeastUs && !implicit_gemm_plain))) {
         double f32_us = 1e30;
@@ -684,8 +687,9 @@ int conv2_direct_entry(const char *name, const void *x, const void *w, const voi
         const int rc = !taps16_forced && limit < kTaps16LeastUs
                            ? 1
                            : conv2_taps16_try(name, x, w, bias, y, bs, ic, ih, iw, oc, fh, fw, ph, pw, sh, sw, dh, dw, oh, ow, act, pool2x2 != 0,
-                                              taps16_forced, limit);
+                                              taps16_forced, limit, lacking);
         if (rc != 1) return rc;
+        if (taps16_forced && lacking) return workspace(lacking, &unused);
         if (taps16_forced) return fail(AGH_ERANGE, "%s: AGH_CONV_TAPS=2, and that kernel does not take this shape", name);
     }
     if (taps_forced == 1 || (taps_limit >= kTapsLeastUs && !implicit_gemm_plain)) {
@@ -782,9 +786,11 @@ int conv2_direct_entry(const char *name, const void *x, const void *w, const voi
     }
 
     ConvParams p;
-    if (!conv2_lds_plan(shape, pool2x2 != 0, p, l))
+    if (!conv2_lds_plan(shape, pool2x2 != 0, p, l)) {
+        if (lacking) return workspace(lacking, &unused);
         return fail(AGH_ERANGE, "%s: image + filter bank (%lld bytes) do not fit in LDS; use im2col + gemm", name,
                     (long long)(l.w_bytes + l.img_bytes));
+    }
     const int oct = l.oct;
     const int64_t items = l.items, imgs = l.imgs, pix = (int64_t)p.yh * p.yw;
     p.act = act; p.has_bias = bias != nullptr;

@@ -253,7 +253,7 @@ static int taps16_launch(const char *name, const void *x, const void *wp, const 
 
 int conv2_taps16_try(const char *name, const void *x, const void *w, const void *bias, void *y, int64_t bs, int64_t ic, int64_t ih,
                      int64_t iw, int64_t oc, int64_t fh, int64_t fw, int64_t ph, int64_t pw, int64_t sh, int64_t sw, int64_t dh,
-                     int64_t dw, int64_t oh, int64_t ow, int act, bool pool, bool forced, double limit_us) {
+                     int64_t dw, int64_t oh, int64_t ow, int act, bool pool, bool forced, double limit_us, size_t &lacking) {
     const int64_t npos = oh * ow, taps = fh * fw, cols = (ow - 1) * sw + (fw - 1) * dw + 1, all_groups = (ic + 7) / 8;
     if (npos > ((int64_t)1 << 24) || ic * taps > ((int64_t)1 << 24) || oc * ic * taps > ((int64_t)1 << 28) || cols > (1 << 16)) return 1;
     const int64_t cus = compute_units() > 0 ? compute_units() : 256, n16 = (oc + 15) / 16;
@@ -298,8 +298,12 @@ int conv2_taps16_try(const char *name, const void *x, const void *w, const void 
     const int64_t frags = n16 * passes * steps * 64;
     if (gx > 0x7FFFFFFF || gy > 65535 || frags > 0x7FFFFFFF) return 1;
     void *wp = nullptr;
-    // (inside a capture the scratch memory cannot grow: the kernel without a packed bank is taken then)
-    if (!workspace_ready((size_t)frags * 16)) return 1;
+    // Inside a capture the scratch memory cannot grow.  The kernels that need none are left then: what they took without this one they take, the
+    // rest is refused.
+    if (!workspace_ready((size_t)frags * 16)) {
+        lacking = (size_t)frags * 16;
+        return 1;
+    }
     if (int rc = workspace((size_t)frags * 16, &wp)) return rc;
     hipLaunchKernelGGL(taps16_pack_kernel, dim3((unsigned)((frags + 255) / 256)), dim3(256), 0, stream(), (const uint16_t *)w, (uint4 *)wp, (int)oc,
                        (int)ic, (int)taps, (int)groups, (int)units, (int)steps, (int)passes, (uint32_t)frags);

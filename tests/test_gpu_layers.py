@@ -5,6 +5,7 @@ Mirrors conv2_im2col_<T>_<opts> (tests/integration_tests.rs:986-993, body :1182-
 checks the chain against the naive 7-deep loop on x, w = (1..=10).cycle() data.
 """
 import ctypes as C
+import gc
 import time
 
 import numpy as np
@@ -275,36 +276,83 @@ def test_conv2_taps_kernel_on_the_bf16_matrix_cores(ag, case, monkeypatch):
             assert np.array_equal(fused, ag.MaxPool2((2, 2)).forward(plain).into_array()), tile
 
 
-def test_conv2_taps_bf16_captured(ag):
-    """A convolution with a packed filter bank inside a captured graph: on the main stream the bits of the eager call at every replay; in a
-    branch, whose scratch memory may not be there yet and cannot grow, it is captured all the same (on the kernel without a bank)."""
+@pytest.mark.parametrize("shape,former", [
+    # bs, ic, ih, iw, oc, filter; the kernel without scratch memory that takes the shape where this one cannot be had (AGH_CONV_TAPS), if any
+    ((4, 32, 41, 41, 48, 5), "1"),      # the f32 matrix cores
+    ((58, 16, 8, 18, 32, 5), "0"),      # row tiles
+    ((10, 32, 38, 13, 48, 7), None),    # a program would take im2col and a product
+])
+def test_conv2_taps_bf16_captured(ag, monkeypatch, shape, former):
+    """A convolution with a packed filter bank inside a captured graph.  Run eagerly before, it has its scratch memory, on the main stream: the bits of
+    the eager call at every replay.  Without, as in a branch, which has its own, the kernel that needs none is captured; where there is none, the
+    capture is refused and the message says what to do."""
+    bs, ic, ih, iw, oc, f = shape
+    oh, ow = ih - f + 1, iw - f + 1
     rng = np.random.default_rng(39)
-    x = ag.Tensor.from_array(to_dtype(rng.standard_normal((4, 32, 41, 41)), "bf16"))
-    w = ag.Tensor.from_array(to_dtype(rng.standard_normal((48, 32, 5, 5)) * 0.05, "bf16"))
-    y, z = (ag.Tensor.uninit((4, 48, 37, 37), "bf16") for _ in range(2))
+    x = ag.Tensor.from_array(to_dtype(rng.standard_normal((bs, ic, ih, iw)), "bf16"))
+    w = ag.Tensor.from_array(to_dtype(rng.standard_normal((oc, ic, f, f)) * 0.05, "bf16"))
+    y, z = (ag.Tensor.uninit((bs, oc, oh, ow), "bf16") for _ in range(2))
     check, lib = ag._ffi.check, ag.lib
 
-    def call(out):
-        check(lib.agh_conv2_direct_bf16(x._data_ptr(), w._data_ptr(), None, out._ptr(), 4, 32, 41, 41, 48, 5, 5, 0, 0, 1, 1, 1, 1, 0, 0))
+    def call(out, route=""):
+        monkeypatch.setenv("AGH_CONV_TAPS", route)
+        check(lib.agh_conv2_direct_bf16(x._data_ptr(), w._data_ptr(), None, out._ptr(), bs, ic, ih, iw, oc, f, f, 0, 0, 1, 1, 1, 1, 0, 0))
+
+    def captured_without():
+        if former is None:
+            with pytest.raises(ag.AghError, match="run the sequence once eagerly"):
+                call(z)
+        else:
+            call(z)
+
+    def scratch():
+        nbytes = C.c_size_t()
+        check(lib.agh_workspace_stats(C.byref(nbytes), None))
+        return nbytes.value
+
+    def replay(body, outputs):
+        graph = C.c_void_p()
+        check(lib.agh_graph_begin())
+        try:
+            try:
+                body()
+            finally:
+                check(lib.agh_graph_end(C.byref(graph)))
+            for _ in range(3 if outputs else 0):
+                for out, _ in outputs:
+                    check(lib.agh_memset(out._ptr(), 0, out.buffer.nbytes))
+                check(lib.agh_graph_launch(graph))
+                check(lib.agh_sync())
+                for out, want in outputs:
+                    assert np.array_equal(out.into_array(), want)
+        finally:
+            if graph:
+                check(lib.agh_graph_destroy(graph))
+
+    def both():
+        check(lib.agh_branch_begin())
+        try:
+            captured_without()
+        finally:
+            check(lib.agh_branch_end())
+        call(y)
+        check(lib.agh_branch_join())
+
+    gc.collect()  # (a graph that an earlier test has dropped would keep the scratch memory it names)
+    check(lib.agh_sync())
+    check(lib.agh_cache_release())
+    without = []
+    if former is not None:
+        call(z, former)
+        without = [(z, z.into_array())]
+    assert scratch() == 0
+    replay(captured_without, without)
     call(y)
     want = y.into_array()
-    graph = C.c_void_p()
-    check(lib.agh_graph_begin())
-    check(lib.agh_branch_begin())
-    call(z)
-    check(lib.agh_branch_end())
-    call(y)
-    check(lib.agh_branch_join())
-    check(lib.agh_graph_end(C.byref(graph)))
-    for _ in range(3):
-        for t in (y, z):
-            check(lib.agh_memset(t._ptr(), 0, t.buffer.nbytes))
-        check(lib.agh_graph_launch(graph))
-        check(lib.agh_sync())
-        assert np.array_equal(y.into_array(), want)
-        got, ref = as_f32(z.into_array()), as_f32(want)
-        assert np.all(np.abs(got - ref) <= 2.0**-7 * np.abs(ref) + 1e-4)  # another order of sums of 800 terms below 1, one rounding
-    check(lib.agh_graph_destroy(graph))
+    assert scratch() > 0
+    call(y, "2")
+    assert np.array_equal(y.into_array(), want)
+    replay(both, [(y, want)] + without)
 
 
 CONV_TAPS_POOL = [
