@@ -43,8 +43,14 @@ bool convert(PyObject *o, A &out) {
         out = (A)(uintptr_t)PyLong_AsUnsignedLongLongMask(o);
     } else if constexpr (std::is_floating_point<A>::value) {
         if (PyFloat_CheckExact(o)) out = (A)PyFloat_AS_DOUBLE(o);
-        else if (PyLong_CheckExact(o)) out = (A)PyLong_AsDouble(o);
-        else return false;
+        else if (PyLong_CheckExact(o)) {
+            const double d = PyLong_AsDouble(o);
+            if (d == -1.0 && PyErr_Occurred()) {  // too large: ctypes refuses it in its own words
+                PyErr_Clear();
+                return false;
+            }
+            out = (A)d;
+        } else return false;
     } else {
         if (!PyLong_CheckExact(o)) return false;
         out = (A)PyLong_AsUnsignedLongLongMask(o);
@@ -56,7 +62,6 @@ template <typename... A, size_t... I>
 PyObject *call(int (*fn)(A...), const char *name, PyObject *const *args, Py_ssize_t n, std::index_sequence<I...>) {
     std::tuple<A...> v;
     if (n == (Py_ssize_t)sizeof...(A) && (convert(args[I], std::get<I>(v)) && ...)) {
-        if (PyErr_Occurred()) return nullptr;  // (an integer too large for a double)
         int rc;
         Py_BEGIN_ALLOW_THREADS
         rc = fn(std::get<I>(v)...);

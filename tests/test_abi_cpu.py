@@ -167,6 +167,11 @@ def test_native_calls_mean_what_the_ctypes_calls_mean():
     for a in (args[:-1], args[:3] + ["1.0"] + args[4:], [1.0] + args[1:]):
         with pytest.raises((TypeError, C.ArgumentError)):
             gemm(*a)
+    for a in (args[:3] + [10**400] + args[4:], args[:3] + [10**400, C.c_void_p(None)] + args[5:]):  # an integer that no float holds
+        with pytest.raises(C.ArgumentError):
+            gemm(*a)
+    with pytest.raises(AghError):
+        gemm(*args[:3], 10**300, *args[4:])
     with pytest.raises(AghError):
         gemm(2**64 + 1, *args[1:])
     for size in (16, np.int64(16), True):
