@@ -143,4 +143,4 @@ try:
     from . import _calls as calls
 except ImportError as e:
     raise ImportError(f"autograph_amd._calls: {e}; build it with `make -C {os.path.join(_HERE, 'csrc')}`") from e
-calls.setup(AghError, _through_ctypes)
+calls.setup(AghError, _through_ctypes, lambda name: C.cast(getattr(lib, name), ptr).value)

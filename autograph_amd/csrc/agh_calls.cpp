@@ -4,6 +4,9 @@
 // A call converts its arguments as the ctypes table does (integers wrap to their width, floats are cast, None is a null pointer), releases the
 // GIL and raises AghError for a status other than 0.  Whatever is not a plain int, float or None (a ctypes object, an array, a wrong type) goes
 // through the ctypes function of the same name, so every call means what it means there.
+//
+// The module is not linked to the library: setup() takes the entry points' addresses from the handle that ctypes has opened, so that there is one
+// instance of the library, with its streams, caches and scratch memory, whatever the loader's search path holds.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -19,11 +22,34 @@
 
 namespace {
 
-PyObject *g_error = nullptr;     // AghError(code, message)
+#define AGH_CALLS(X)                                                                                                                     \
+    X(agh_gemm_f32) X(agh_gemm_bf16) X(agh_gemm_f32_bias_act) X(agh_gemm_bf16_bias_act) X(agh_gemm_f32_batched) X(agh_gemm_bf16_batched) \
+    X(agh_im2col_conv2_f32) X(agh_im2col_conv2_bf16) X(agh_col2im_conv2_f32) X(agh_col2im_conv2_bf16)                                    \
+    X(agh_conv2_direct_f32) X(agh_conv2_direct_bf16) X(agh_conv2_backward_input_f32) X(agh_conv2_backward_input_bf16)                    \
+    X(agh_max_pool2_f32) X(agh_max_pool2_bf16) X(agh_max_pool2_backward_f32) X(agh_max_pool2_backward_bf16)                              \
+    X(agh_relu_f32) X(agh_relu_bf16) X(agh_relu_backward_f32) X(agh_relu_backward_bf16)                                                  \
+    X(agh_assign_f32) X(agh_assign_bf16) X(agh_scaled_add_f32) X(agh_scaled_add_bf16)                                                    \
+    X(agh_scaled_add_strided_f32) X(agh_scaled_add_strided_bf16) X(agh_sum_axis0_f32) X(agh_sum_axis0_bf16)                              \
+    X(agh_lenet5_forward_f32) X(agh_lenet5_forward_bf16) X(agh_memcpy_d2d) X(agh_graph_launch)
+
+// every entry point used here, as setup() has found it
+struct Entries {
+#define AGH_ENTRY(name) decltype(&::name) name;
+    AGH_CALLS(AGH_ENTRY) AGH_ENTRY(agh_malloc) AGH_ENTRY(agh_free) AGH_ENTRY(agh_last_error_string)
+#undef AGH_ENTRY
+};
+Entries g_entries = {};
+PyObject *g_error = nullptr;     // AghError(code, message); null before setup()
 PyObject *g_fallback = nullptr;  // callable (name, args): the same call through ctypes
 
+bool ready() {
+    if (!g_error) PyErr_SetString(PyExc_RuntimeError, "_calls.setup has not been called");
+    return g_error != nullptr;
+}
+
 int raise_status(int code) {
-    PyObject *e = PyObject_CallFunction(g_error, "iN", code, PyUnicode_DecodeUTF8(agh_last_error_string(), (Py_ssize_t)strlen(agh_last_error_string()), "replace"));
+    const char *text = g_entries.agh_last_error_string();
+    PyObject *e = PyObject_CallFunction(g_error, "iN", code, PyUnicode_DecodeUTF8(text, (Py_ssize_t)strlen(text), "replace"));
     if (e) {
         PyErr_SetObject(g_error, e);
         Py_DECREF(e);
@@ -60,6 +86,7 @@ bool convert(PyObject *o, A &out) {
 
 template <typename... A, size_t... I>
 PyObject *call(int (*fn)(A...), const char *name, PyObject *const *args, Py_ssize_t n, std::index_sequence<I...>) {
+    if (!ready()) return nullptr;
     std::tuple<A...> v;
     if (n == (Py_ssize_t)sizeof...(A) && (convert(args[I], std::get<I>(v)) && ...)) {
         int rc;
@@ -99,7 +126,7 @@ void release(BufferObject *b) {
         void *mem = (void *)(uintptr_t)PyLong_AsUnsignedLongLongMask(ptr);
         if (mem) {
             Py_BEGIN_ALLOW_THREADS
-            agh_free(mem);
+            g_entries.agh_free(mem);
             Py_END_ALLOW_THREADS
         }
     }
@@ -108,6 +135,7 @@ void release(BufferObject *b) {
 int buffer_init(PyObject *self, PyObject *args, PyObject *kwargs) {
     static const char *names[] = {"nbytes", nullptr};
     PyObject *nbytes;
+    if (!ready()) return -1;
     if (!PyArg_ParseTupleAndKeywords(args, kwargs, "O", const_cast<char **>(names), &nbytes)) return -1;
     PyObject *whole = PyNumber_Index(nbytes);  // (a TypeError for a float or a text)
     if (!whole) return -1;
@@ -117,14 +145,14 @@ int buffer_init(PyObject *self, PyObject *args, PyObject *kwargs) {
     void *mem = nullptr;
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = agh_malloc(&mem, bytes);
+    rc = g_entries.agh_malloc(&mem, bytes);
     Py_END_ALLOW_THREADS
     if (rc != 0) return raise_status(rc);
     release(b);
     if (mem) {
         b->ptr = PyLong_FromVoidPtr(mem);
         if (!b->ptr) {
-            agh_free(mem);
+            g_entries.agh_free(mem);
             return -1;
         }
     } else {
@@ -146,9 +174,24 @@ PyMemberDef buffer_members[] = {{"ptr", T_OBJECT, offsetof(BufferObject, ptr), 0
                                 {nullptr, 0, 0, 0, nullptr}};
 PyTypeObject BufferType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
+// setup(AghError, fallback, address): address(name) is the entry point's in the library that ctypes has opened
 PyObject *setup(PyObject *, PyObject *args) {
-    PyObject *error, *fallback;
-    if (!PyArg_ParseTuple(args, "OO", &error, &fallback)) return nullptr;
+    PyObject *error, *fallback, *address;
+    if (!PyArg_ParseTuple(args, "OOO", &error, &fallback, &address)) return nullptr;
+    Entries entries;
+    auto find = [&](const char *name, auto &entry) {
+        PyObject *at = PyObject_CallFunction(address, "s", name);
+        if (!at) return false;
+        entry = (std::remove_reference_t<decltype(entry)>)PyLong_AsVoidPtr(at);
+        Py_DECREF(at);
+        if (!entry && !PyErr_Occurred()) PyErr_Format(PyExc_ImportError, "%s: no address", name);
+        return entry != nullptr;
+    };
+#define AGH_FIND(name) \
+    if (!find(#name, entries.name)) return nullptr;
+    AGH_CALLS(AGH_FIND) AGH_FIND(agh_malloc) AGH_FIND(agh_free) AGH_FIND(agh_last_error_string)
+#undef AGH_FIND
+    g_entries = entries;
     Py_INCREF(error);
     Py_XSETREF(g_error, error);
     Py_INCREF(fallback);
@@ -157,20 +200,11 @@ PyObject *setup(PyObject *, PyObject *args) {
 }
 
 #define AGH_CALL(name) \
-    PyObject *py_##name(PyObject *, PyObject *const *args, Py_ssize_t n) { return call_any(name, #name, args, n); }
-#define AGH_CALLS(X)                                                                                                                     \
-    X(agh_gemm_f32) X(agh_gemm_bf16) X(agh_gemm_f32_bias_act) X(agh_gemm_bf16_bias_act) X(agh_gemm_f32_batched) X(agh_gemm_bf16_batched) \
-    X(agh_im2col_conv2_f32) X(agh_im2col_conv2_bf16) X(agh_col2im_conv2_f32) X(agh_col2im_conv2_bf16)                                    \
-    X(agh_conv2_direct_f32) X(agh_conv2_direct_bf16) X(agh_conv2_backward_input_f32) X(agh_conv2_backward_input_bf16)                    \
-    X(agh_max_pool2_f32) X(agh_max_pool2_bf16) X(agh_max_pool2_backward_f32) X(agh_max_pool2_backward_bf16)                              \
-    X(agh_relu_f32) X(agh_relu_bf16) X(agh_relu_backward_f32) X(agh_relu_backward_bf16)                                                  \
-    X(agh_assign_f32) X(agh_assign_bf16) X(agh_scaled_add_f32) X(agh_scaled_add_bf16)                                                    \
-    X(agh_scaled_add_strided_f32) X(agh_scaled_add_strided_bf16) X(agh_sum_axis0_f32) X(agh_sum_axis0_bf16)                              \
-    X(agh_lenet5_forward_f32) X(agh_lenet5_forward_bf16) X(agh_memcpy_d2d) X(agh_graph_launch)
+    PyObject *py_##name(PyObject *, PyObject *const *args, Py_ssize_t n) { return call_any(g_entries.name, #name, args, n); }
 AGH_CALLS(AGH_CALL)
 
 #define AGH_METHOD(name) {#name, (PyCFunction)(void (*)(void))py_##name, METH_FASTCALL, nullptr},
-PyMethodDef methods[] = {AGH_CALLS(AGH_METHOD){"setup", setup, METH_VARARGS, "setup(AghError, fallback)"}, {nullptr, nullptr, 0, nullptr}};
+PyMethodDef methods[] = {AGH_CALLS(AGH_METHOD){"setup", setup, METH_VARARGS, "setup(AghError, fallback, address)"}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_calls", "Calls of the C ABI of libautograph_hip.so", -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

@@ -184,3 +184,19 @@ def test_native_calls_mean_what_the_ctypes_calls_mean():
     b.ptr = None
     b.note = "instances take attributes"
     del b
+
+
+def test_one_instance_of_the_library(tmp_path):
+    """The calls without ctypes reach the library that ctypes has opened, not another one that the loader's search path holds."""
+    import shutil
+    import subprocess
+    import sys
+
+    from autograph_amd import _ffi
+    shutil.copy(_ffi.LIB_PATH, tmp_path / os.path.basename(_ffi.LIB_PATH))
+    program = ("import autograph_amd\n"
+               "print(len({line.split()[-1] for line in open('/proc/self/maps') if line.rstrip().endswith('/libautograph_hip.so')}))\n")
+    env = dict(os.environ, LD_LIBRARY_PATH=os.pathsep.join(filter(None, (str(tmp_path), os.environ.get("LD_LIBRARY_PATH")))))
+    out = subprocess.run([sys.executable, "-c", program], env=env, cwd=ROOT, check=True,
+                         capture_output=True, text=True).stdout
+    assert out.strip() == "1"
