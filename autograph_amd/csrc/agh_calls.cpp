@@ -25,7 +25,7 @@ namespace {
 #define AGH_CALLS(X)                                                                                                                     \
     X(agh_gemm_f32) X(agh_gemm_bf16) X(agh_gemm_f32_bias_act) X(agh_gemm_bf16_bias_act) X(agh_gemm_f32_batched) X(agh_gemm_bf16_batched) \
     X(agh_im2col_conv2_f32) X(agh_im2col_conv2_bf16) X(agh_col2im_conv2_f32) X(agh_col2im_conv2_bf16)                                    \
-    X(agh_conv2_direct_f32) X(agh_conv2_direct_bf16) X(agh_conv2_backward_input_f32) X(agh_conv2_backward_input_bf16)                    \
+    X(agh_conv2_direct_f32) X(agh_conv2_direct_bf16)                                                                                     \
     X(agh_max_pool2_f32) X(agh_max_pool2_bf16) X(agh_max_pool2_backward_f32) X(agh_max_pool2_backward_bf16)                              \
     X(agh_relu_f32) X(agh_relu_bf16) X(agh_relu_backward_f32) X(agh_relu_backward_bf16)                                                  \
     X(agh_assign_f32) X(agh_assign_bf16) X(agh_scaled_add_f32) X(agh_scaled_add_bf16)                                                    \
