@@ -5,6 +5,7 @@ this module raises.
 """
 import ctypes as C
 import os
+import sys
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libautograph_hip.so")
@@ -142,5 +143,5 @@ def _through_ctypes(name, args):
 try:
     from . import _calls as calls
 except ImportError as e:
-    raise ImportError(f"autograph_amd._calls: {e}; build it with `make -C {os.path.join(_HERE, 'csrc')}`") from e
+    raise ImportError(f"autograph_amd._calls: {e}; build it with `make -C {os.path.join(_HERE, 'csrc')} PYTHON={sys.executable} calls`") from e
 calls.setup(AghError, _through_ctypes, lambda name: C.cast(getattr(lib, name), ptr).value)

@@ -200,3 +200,15 @@ def test_one_instance_of_the_library(tmp_path):
     out = subprocess.run([sys.executable, "-c", program], env=env, cwd=ROOT, check=True,
                          capture_output=True, text=True).stdout
     assert out.strip() == "1"
+
+
+def test_library_is_built_without_python():
+    """`make lib`, and `make` where there are no Python headers, build the library and not the package's extension."""
+    import subprocess
+
+    def commands(*args):
+        return subprocess.run(["make", "-n", "-B", "-C", os.path.join(ROOT, "autograph_amd", "csrc"), *args], check=True, capture_output=True, text=True).stdout
+    for args in (("lib",), ("PYTHON=false",)):
+        text = commands(*args)
+        assert "-o ../lib/libautograph_hip.so" in text and "agh_calls.cpp -o" not in text, args
+    assert "agh_calls.cpp -o ../_calls." in commands()
