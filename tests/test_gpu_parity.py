@@ -1154,6 +1154,42 @@ def test_max_pool2_reference_cases(ag, dtype):
         assert np.array_equal(dx.into_array(), orc.max_pool2_backward(x, dy, (2, 2)))
 
 
+@pytest.mark.parametrize("m,k,n", [(33, 65, 35), (130, 131, 67), (65, 97, 129)])
+@pytest.mark.parametrize("rows", ["n", "m", "neither"])
+def test_gemm_f32_batches_at_any_address(ag, monkeypatch, m, k, n, rows):
+    """The same form over a batch, whose matrices start at odd elements: C with rows of n, with rows of m (as a convolution writes NCHW) and with no
+    unit stride, so that both operands come first, exchanged and not; a shared B, alpha, beta, bias along n and relu.  Whole numbers exactly, and
+    nothing of C outside its matrices is written."""
+    nb, lib, check = 3, ag.lib, ag._ffi.check
+    rng = np.random.default_rng(k)
+    rsc, csc = {"n": (n, 1), "m": (1, m), "neither": (2 * n, 2)}[rows]
+    span = (m - 1) * rsc + (n - 1) * csc + 1
+    for ta, tb, shared in ((False, False, False), (True, False, True), (False, True, False), (True, True, True)):
+        a, b = (rng.integers(-8, 9, s).astype(np.float32) for s in ((nb, m, k), (1 if shared else nb, k, n)))
+        bias = rng.integers(-8, 9, n).astype(np.float32)
+        sa, sb, sc = m * k + 3, 0 if shared else k * n + 1, span + 5
+
+        def flat(mats, step, transposed):
+            out = np.full(1 + step * len(mats) + mats[0].size, np.inf, np.float32)
+            for i, x in enumerate(mats):
+                out[1 + i * step:1 + i * step + x.size] = (x.T if transposed else x).ravel()
+            return ag.Tensor.from_array(out)
+        A, B, bias_t = flat(a, sa, ta), flat(b, sb, tb), ag.Tensor.from_array(bias)
+        c0 = rng.integers(-8, 9, 3 + sc * nb).astype(np.float32)
+        want = c0.copy()
+        cells = np.arange(m)[:, None] * rsc + np.arange(n)[None, :] * csc
+        for i in range(nb):
+            at = 3 + i * sc + cells
+            want[at] = np.maximum(2 * (a[i] @ b[0 if shared else i]) - 3 * c0[at] + bias, 0)
+        for cfg in ("3", "4", ""):
+            monkeypatch.setenv("AGH_GEMM_CFG", cfg)
+            monkeypatch.setenv("AGH_GEMM_SMALL", "0")
+            out = ag.Tensor.from_array(c0)
+            check(lib.agh_gemm_f32_batched(nb, m, k, n, 2.0, A._ptr(), 1, *((1, m) if ta else (k, 1)), sa, B._ptr(), 1, *((1, k) if tb else (n, 1)), sb,
+                                           -3.0, out._ptr(), 3, rsc, csc, sc, bias_t._ptr(), 0, 1, 1))
+            assert np.array_equal(out.into_array(), want), (cfg, ta, tb, shared)
+
+
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("shape,size,strides", [
     ((1000, 6, 24, 24), (2, 2), (2, 2)), ((1000, 16, 8, 8), (2, 2), (2, 2)), ((100, 6, 24, 24), (2, 2), (2, 2)),
@@ -1505,10 +1541,12 @@ def test_max_pool2_square_windows(ag, dtype, shape, size, strides):
     assert flat.into_array()[0] == 0  # the element in front of the view
 
 
-@pytest.mark.parametrize("m,k,n", [(1100, 4103, 1101), (2001, 3001, 301), (2000, 2048, 1008), (560, 3344, 1408), (1408, 4096, 1400)])
-def test_gemm_bf16_split_by_cost(ag, monkeypatch, m, k, n):
-    """bf16 products whose tiles leave CUs idle, at any address and of whole vectors: split k and 128 x 128 tiles as the estimate chooses them give
-    whole numbers exactly and agree with one split of 64 x 64 tiles within a rounding; the entry without allocations takes them too."""
+@pytest.mark.parametrize("m,k,n,cfg,splits", [(1100, 4103, 1101, "3", 3), (2001, 3001, 301, "4", 1), (2000, 2048, 1008, "3", 1), (560, 3344, 1408, "4", 1),
+                                              (560, 3344, 2816, "3", 2), (1408, 4096, 1400, "3", 2), (664, 7239, 1744, "3", 3)])
+def test_gemm_bf16_split_by_cost(ag, monkeypatch, m, k, n, cfg, splits):
+    """bf16 products whose tiles leave CUs idle, at any address and of whole vectors: split k and 128 x 128 tiles as the estimate chooses them (the bits
+    of that plan forced, which those of another number of splits are not) give whole numbers exactly and agree with one split of 64 x 64 tiles
+    within a rounding; the entry without allocations takes them too."""
     rng = np.random.default_rng(k)
     ai, bi = (to_dtype(rng.integers(-2, 3, s).astype(np.float32), "bf16") for s in ((m, k), (k, n)))
     want = orc.f32_to_bf16((orc.bf16_to_f32(ai) @ orc.bf16_to_f32(bi)).astype(np.float32))
@@ -1521,6 +1559,10 @@ def test_gemm_bf16_split_by_cost(ag, monkeypatch, m, k, n):
     got = orc.bf16_to_f32(a.dot(b).into_array())
     ag._ffi.check(ag.lib.agh_gemm_bf16_noalloc(m, k, n, 1.0, a._ptr(), 0, k, 1, b._ptr(), 0, n, 1, 0.0, out._ptr(), 0, n, 1))
     assert np.array_equal(orc.bf16_to_f32(out.into_array()), got)  # the same plan
+    monkeypatch.setenv("AGH_GEMM_CFG", cfg)
+    for other in (0, 1):
+        monkeypatch.setenv("AGH_GEMM_SPLITS", str(splits + other))
+        assert np.array_equal(orc.bf16_to_f32(a.dot(b).into_array()), got) == (other == 0), (splits, other)
     monkeypatch.setenv("AGH_GEMM_CFG", "4")
     monkeypatch.setenv("AGH_GEMM_SPLITS", "1")
     one = orc.bf16_to_f32(a.dot(b).into_array())
