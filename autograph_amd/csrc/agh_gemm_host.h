@@ -282,18 +282,19 @@ inline int plan_splits(int64_t tiles, int ktiles, int64_t cus, int kmin) {
 }
 
 // What split k costs and saves in bf16, in us, where every workgroup has a CU to itself: k-tiles a split, the second launch and the f32 partial sums
-// by the MB of C (as bf16).  Fitted to 420 products.  Splitting as far as the chip has CUs cost 2000x2048x1008 21.6 us where one split takes 16.2,
-// and 560x3344x2816 (53 k-tiles) gains: 26.3 / 24.5.
+// by the MB of C (as bf16).  Fitted to 420 products on tiles of 128 x 128, of whole vectors and at any address.
 struct Bf16SplitTime { double ktile, second, part_mb; };
-static const Bf16SplitTime kBf16SplitTimes[2] = {{0.44, 3.6, 1.0}, {0.95, 2.3, 0.88}};  // tiles of 128 x 128: whole vectors, any address
+static const Bf16SplitTime kBf16Split = {0.44, 3.6, 1.0}, kBf16SplitAny = {0.95, 2.3, 0.88};
 inline double bf16_split_us(const Bf16SplitTime &t, int splits, int ktiles, double mb) {
     return t.ktile * ((ktiles + splits - 1) / splits) + (splits > 1 ? t.second + t.part_mb * splits * mb : 0.0);
 }
-inline int bf16_best_splits(const Bf16SplitTime &t, int most, int ktiles, double mb) {
-    int best = 1;
-    for (int s = 2; s <= most; ++s)
-        if (bf16_split_us(t, s, ktiles, mb) < bf16_split_us(t, best, ktiles, mb)) best = s;
-    return best;
+// Whether a product of whole vectors that would have two splits takes one: the estimate has to be well below, since a k-tile is 0.44 to 0.75 us by
+// sizes and strides.  One split / two: where the second launch adds single elements (rows of C no multiple of four), below 0.86 of the
+// estimate 0.68 to 0.98 of the time over 80 products (728x2016x2215, B transposed, 18.0 / 24.6; 2160x2472x827 at 0.88 29.8 / 29.4); where it
+// adds vectors, below 0.77 0.74 to 1.02 over 25 (2000x2048x1008 16.2 / 20.7), from there to 0.8 up to 1.09 and beyond up to 1.26
+// (1656x2616x792 27.9 / 22.2, 440x2952x3784 28.4 / 23.7).  Three and more splits are never that far above.
+inline bool bf16_one_split(int ktiles, double mb, bool by_vectors) {
+    return bf16_split_us(kBf16Split, 1, ktiles, mb) < (by_vectors ? 0.77 : 0.86) * bf16_split_us(kBf16Split, 2, ktiles, mb);
 }
 
 // Time in us of an f32 product on the direct-to-LDS kernels' 64 x 64 or 128 x 128 tiles, fitted to 450 products of 16 to 60000 x 16 to
@@ -484,11 +485,10 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
     // a 128 x 128 tile of partial sums for each of 256 CUs, so agh_gemm_bf16_noalloc takes the same way and gives the same bits.
     if (sizeof(T) == 2 && any_addr && best == 4 && batch == 1 && g.NP > 64 && g.NQ > 64 && !setting("AGH_GEMM_SPLITS")) {
         const int64_t tiles = (int64_t)((g.NP + 127) / 128) * ((g.NQ + 127) / 128), small = (int64_t)((g.NP + 63) / 64) * ((g.NQ + 63) / 64);
-        const int ktiles = (g.K + BK - 1) / BK, most = (int)std::min<int64_t>(cus / tiles, ktiles / 12);
+        const int ktiles = (g.K + BK - 1) / BK, s = ktiles >= 32 && small > cus ? (int)std::min<int64_t>(cus / tiles, ktiles / 12) : 1;
         const double mb = (double)g.NP * g.NQ * 2e-6;
-        const int s = ktiles >= 32 && small > cus ? bf16_best_splits(kBf16SplitTimes[1], most, ktiles, mb) : 1;
         const size_t bytes = (size_t)s * g.NQ * g.NPpad * sizeof(float);
-        if (s > 1 && bf16_split_us(kBf16SplitTimes[1], s, ktiles, mb) + 3 * 0.95 < 0.9 * best_cost &&
+        if (s > 1 && bf16_split_us(kBf16SplitAny, s, ktiles, mb) + 3 * 0.95 < 0.9 * best_cost &&
             (fixed_scratch ? bytes <= (size_t)AGH_NOALLOC_SCRATCH_BYTES : workspace_ready(bytes)))
             best = 3;
     }
@@ -570,8 +570,7 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
     // at least four k-tiles a split; twelve for the bf16 128 x 128 direct tile, whose four-stage ring makes fewer,
     // longer splits the better trade (128x4096x4096: 17.0-17.2 us in 4 to 6 splits, 19.5 in 8)
     int splits = batch == 1 ? plan_splits(tiles, ktiles, cus, direct_ok && best == 3 ? 12 : 4) : 1;
-    if (sizeof(T) == 2 && direct_ok && best == 3 && splits > 1)
-        splits = bf16_best_splits(kBf16SplitTimes[any_addr], splits, ktiles, (double)g.NP * g.NQ * 2e-6);
+    if (sizeof(T) == 2 && direct_ok && !any_addr && best == 3 && splits == 2 && bf16_one_split(ktiles, (double)g.NP * g.NQ * 2e-6, vec_store)) splits = 1;
     if (batch == 1) splits = env_int("AGH_GEMM_SPLITS", splits);
     if (splits < 1) splits = 1;
     if (splits > ktiles && ktiles > 0) splits = ktiles;

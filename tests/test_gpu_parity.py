@@ -1541,24 +1541,34 @@ def test_max_pool2_square_windows(ag, dtype, shape, size, strides):
     assert flat.into_array()[0] == 0  # the element in front of the view
 
 
-@pytest.mark.parametrize("m,k,n,cfg,splits", [(1100, 4103, 1101, "3", 3), (2001, 3001, 301, "4", 1), (2000, 2048, 1008, "3", 1), (560, 3344, 1408, "4", 1),
-                                              (560, 3344, 2816, "3", 2), (1408, 4096, 1400, "3", 2), (664, 7239, 1744, "3", 3)])
-def test_gemm_bf16_split_by_cost(ag, monkeypatch, m, k, n, cfg, splits):
+@pytest.mark.parametrize("m,k,n,tb,cfg,splits", [
+    (1100, 4103, 1101, False, "3", 3), (2001, 3001, 301, False, "4", 1), (664, 7239, 1744, False, "3", 3),    # at any address
+    (560, 3344, 1408, False, "4", 1), (560, 3344, 2816, False, "3", 2), (1408, 4096, 1400, False, "3", 2),
+    (2000, 2048, 1008, False, "3", 1), (440, 2952, 3784, False, "3", 2), (1656, 2616, 792, False, "3", 2),    # one split pays, or does not
+    (728, 2016, 2215, True, "3", 1), (2160, 2472, 827, True, "3", 2),                                         # and in odd rows of C
+])
+def test_gemm_bf16_split_by_cost(ag, monkeypatch, m, k, n, tb, cfg, splits):
     """bf16 products whose tiles leave CUs idle, at any address and of whole vectors: split k and 128 x 128 tiles as the estimate chooses them (the bits
     of that plan forced, which those of another number of splits are not) give whole numbers exactly and agree with one split of 64 x 64 tiles
     within a rounding; the entry without allocations takes them too."""
     rng = np.random.default_rng(k)
+
+    def right(values):
+        return ag.Tensor.from_array(np.ascontiguousarray(values.T)).t() if tb else ag.Tensor.from_array(values)
+
+    def noalloc(a, b):
+        out = ag.Tensor.zeros((m, n), "bf16")
+        ag._ffi.check(ag.lib.agh_gemm_bf16_noalloc(m, k, n, 1.0, a._ptr(), 0, k, 1, b._ptr(), 0, *b.strides, 0.0, out._ptr(), 0, n, 1))
+        return out.into_array()
     ai, bi = (to_dtype(rng.integers(-2, 3, s).astype(np.float32), "bf16") for s in ((m, k), (k, n)))
     want = orc.f32_to_bf16((orc.bf16_to_f32(ai) @ orc.bf16_to_f32(bi)).astype(np.float32))
-    A, B = ag.Tensor.from_array(ai), ag.Tensor.from_array(bi)
+    A, B = ag.Tensor.from_array(ai), right(bi)
     assert np.array_equal(A.dot(B).into_array(), want)
-    out = ag.Tensor.zeros((m, n), "bf16")
-    ag._ffi.check(ag.lib.agh_gemm_bf16_noalloc(m, k, n, 1.0, A._ptr(), 0, k, 1, B._ptr(), 0, n, 1, 0.0, out._ptr(), 0, n, 1))
-    assert np.array_equal(out.into_array(), want)
-    a, b = (ag.Tensor.from_array(to_dtype(rng.standard_normal(s), "bf16")) for s in ((m, k), (k, n)))
+    assert np.array_equal(noalloc(A, B), want)
+    ar, br = (to_dtype(rng.standard_normal(s), "bf16") for s in ((m, k), (k, n)))
+    a, b = ag.Tensor.from_array(ar), right(br)
     got = orc.bf16_to_f32(a.dot(b).into_array())
-    ag._ffi.check(ag.lib.agh_gemm_bf16_noalloc(m, k, n, 1.0, a._ptr(), 0, k, 1, b._ptr(), 0, n, 1, 0.0, out._ptr(), 0, n, 1))
-    assert np.array_equal(orc.bf16_to_f32(out.into_array()), got)  # the same plan
+    assert np.array_equal(orc.bf16_to_f32(noalloc(a, b)), got)  # the same plan
     monkeypatch.setenv("AGH_GEMM_CFG", cfg)
     for other in (0, 1):
         monkeypatch.setenv("AGH_GEMM_SPLITS", str(splits + other))
