@@ -1154,6 +1154,24 @@ def test_max_pool2_reference_cases(ag, dtype):
         assert np.array_equal(dx.into_array(), orc.max_pool2_backward(x, dy, (2, 2)))
 
 
+@pytest.mark.parametrize("m,k,n,ta,tb,direct", [
+    (397, 96, 2373, True, True, False), (391, 68, 7423, False, False, False), (2523, 324, 2492, True, True, False),     # whole vectors along k, short
+    (146, 672, 6485, True, True, False), (458, 2652, 3216, True, True, True), (1230, 1276, 961, False, False, True),    # and long
+    (4523, 122, 217, True, True, False), (2339, 93, 1744, False, False, False), (2061, 131, 1097, True, True, True),    # none along k
+    (1526, 84, 223, True, True, True), (146, 673, 6484, True, True, True), (1999, 2047, 1001, False, True, True),
+])
+def test_gemm_f32_at_any_address_where_it_pays(ag, monkeypatch, m, k, n, ta, tb, direct):
+    """Which products of no whole vectors take the direct-to-LDS kernel's form for them: the bits are those of the route forced, not of the other."""
+    rng = np.random.default_rng(m)
+    a, b = rng.uniform(-1, 1, (m, k)).astype(np.float32), rng.uniform(-1, 1, (k, n)).astype(np.float32)
+    A = ag.Tensor.from_array(np.ascontiguousarray(a.T)).t() if ta else ag.Tensor.from_array(a)
+    B = ag.Tensor.from_array(np.ascontiguousarray(b.T)).t() if tb else ag.Tensor.from_array(b)
+    got = A.dot(B).into_array()
+    assert_f32_gemm_close(got, a, b)
+    monkeypatch.setenv("AGH_GEMM_DIRECT", "0")
+    assert np.array_equal(got, A.dot(B).into_array()) == (not direct)
+
+
 @pytest.mark.parametrize("m,k,n", [(33, 65, 35), (130, 131, 67), (65, 97, 129)])
 @pytest.mark.parametrize("rows", ["n", "m", "neither"])
 def test_gemm_f32_batches_at_any_address(ag, monkeypatch, m, k, n, rows):
