@@ -512,9 +512,10 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
 #ifdef AGH_GEMM_WITH_F32_DIRECT
     if constexpr (sizeof(T) == 4) {
         // 64 x 64 or 128 x 128: by fitted times.  The cost above counts a round of 144 to 256 tiles of 128 x 128 like a full one, and those
-        // tiles as if they always shared a CU: 1132x272x3944 44 -> 32 us on 64 x 64, 3632x1008x64 21 -> 12; 133x7001x3003 123 -> 97 on
-        // 128 x 128.  No product's sums get longer by it: where 128 x 128 would be two sums (one workgroup per CU) or more splits of k,
-        // 64 x 64 is taken with two sums, or not at all.
+        // tiles as if they always shared a CU: 1132x272x3944 44 -> 32 us on 64 x 64, 136x7008x3004 126 -> 96 on 128 x 128.  (Six per cent are left to
+        // the estimate: of nine products that it puts 3 to 6 % faster on 128 x 128 five were slower, 6328x4296x168 148 / 153.)  No product's
+        // sums get longer by it: where 128 x 128 would be two sums (one workgroup per CU) or more splits of k, 64 x 64 is taken with two
+        // sums, or not at all.
         const bool f32_direct = (any_addr || !any_scalar) && g.K > 0 && env_int("AGH_GEMM_DIRECT", 1) != 0;
         if (f32_direct && forced_cfg < 0 && (best == 3 || best == 4) && !(any_addr && skinny) && !setting("AGH_GEMM_SPLITS") &&
             !setting("AGH_GEMM_KSPLIT")) {
@@ -529,7 +530,7 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
             const bool ready64 = s64 == 1 || workspace_ready((size_t)(s64 * part)), ready128 = s128 == 1 || workspace_ready((size_t)(s128 * part));
             if (any_addr) {
                 best = us128 < us64 && ready128 ? 3 : 4;
-            } else if (best == 4 && us128 < 0.97 * us64 && ready128) best = 3;
+            } else if (best == 4 && us128 < 0.94 * us64 && ready128) best = 3;
             else if (best == 3 && us64 < 0.97 * us128 && s64 >= s128 && ready64) {
                 best = 4;
                 g.two_sums = tiles128 * s128 <= cus;

@@ -1172,6 +1172,19 @@ def test_gemm_f32_at_any_address_where_it_pays(ag, monkeypatch, m, k, n, ta, tb,
     assert np.array_equal(got, A.dot(B).into_array()) == (not direct)
 
 
+@pytest.mark.parametrize("m,k,n,ta,cfg", [(1336, 6040, 1008, True, "4"), (136, 7008, 3004, False, "3"), (1104, 6424, 1552, True, "4")])
+def test_gemm_f32_tile_by_fitted_times(ag, monkeypatch, m, k, n, ta, cfg):
+    """64 x 64 tiles or 128 x 128 in splits, on both sides of what the estimate is trusted with: the bits of the tile forced, not of the other."""
+    rng = np.random.default_rng(m)
+    a, b = rng.uniform(-1, 1, (m, k)).astype(np.float32), rng.uniform(-1, 1, (k, n)).astype(np.float32)
+    A, B = ag.Tensor.from_array(np.ascontiguousarray(a.T)).t() if ta else ag.Tensor.from_array(a), ag.Tensor.from_array(b)
+    got = A.dot(B).into_array()
+    assert_f32_gemm_close(got, a, b)
+    for forced in ("3", "4"):
+        monkeypatch.setenv("AGH_GEMM_CFG", forced)
+        assert np.array_equal(got, A.dot(B).into_array()) == (forced == cfg), forced
+
+
 @pytest.mark.parametrize("m,k,n", [(33, 65, 35), (130, 131, 67), (65, 97, 129)])
 @pytest.mark.parametrize("rows", ["n", "m", "neither"])
 def test_gemm_f32_batches_at_any_address(ag, monkeypatch, m, k, n, rows):
