@@ -495,15 +495,17 @@ int gemm_entry(const char *name, int64_t m, int64_t k, int64_t n, float alpha, c
         if (best < 0 || cost < best_cost) { best = i; best_cost = cost; }
     }
     // Operands at any address, more 64 x 64 tiles than CUs and k in splits: 128 x 128 tiles that leave half of the chip idle are a poor second above,
-    // where a tile walks all of k (2661x7265x442 87 -> 47 us in three splits, 664x7239x1744 71 -> 40, 1248x8121x893 76 -> 51).  A tenth is left for the estimate's error
-    // (440x2952x3783 31.3 us on 64 x 64, 35.6 on 128 x 128 in two).  Not where a capture cannot have the scratch memory for it; the fixed one holds
-    // a 128 x 128 tile of partial sums for each of 256 CUs, so agh_gemm_bf16_noalloc takes the same way and gives the same bits.
+    // where a tile walks all of k (2661x7265x442 84 -> 44 us in three splits, 664x7239x1744 70 -> 40, 1248x8121x893 86 -> 56).  A sixth is left for the
+    // estimate's error and at least 40 k-tiles are asked for: over 70 such products 0.51 to 0.93 of the time, but of 30 others within that
+    // sixth or shorter eight were slower (8005x3321x241 38.2 / 42.6, 2658x3539x763, both transposed, 38.9 / 43.1, 2516x2262x406 21.1 / 22.1).  Not
+    // where a capture cannot have the scratch memory for it; the fixed one holds a 128 x 128 tile of partial sums for each of 256 CUs, so
+    // agh_gemm_bf16_noalloc takes the same way and gives the same bits.
     if (sizeof(T) == 2 && any_addr && best == 4 && batch == 1 && g.NP > 64 && g.NQ > 64 && !setting("AGH_GEMM_SPLITS")) {
         const int64_t tiles = (int64_t)((g.NP + 127) / 128) * ((g.NQ + 127) / 128), small = (int64_t)((g.NP + 63) / 64) * ((g.NQ + 63) / 64);
-        const int ktiles = (g.K + BK - 1) / BK, s = ktiles >= 32 && small > cus ? (int)std::min<int64_t>(cus / tiles, ktiles / 12) : 1;
+        const int ktiles = (g.K + BK - 1) / BK, s = ktiles >= 40 && small > cus ? (int)std::min<int64_t>(cus / tiles, ktiles / 12) : 1;
         const double mb = (double)g.NP * g.NQ * 2e-6;
         const size_t bytes = (size_t)s * g.NQ * g.NPpad * sizeof(float);
-        if (s > 1 && bf16_split_us(kBf16SplitAny, s, ktiles, mb) + 3 * 0.95 < 0.9 * best_cost &&
+        if (s > 1 && bf16_split_us(kBf16SplitAny, s, ktiles, mb) + 3 * 0.95 < 0.83 * best_cost &&
             (fixed_scratch ? bytes <= (size_t)AGH_NOALLOC_SCRATCH_BYTES : workspace_ready(bytes)))
             best = 3;
     }

@@ -1574,6 +1574,7 @@ def test_max_pool2_square_windows(ag, dtype, shape, size, strides):
 
 @pytest.mark.parametrize("m,k,n,tb,cfg,splits", [
     (1100, 4103, 1101, False, "3", 3), (2001, 3001, 301, False, "4", 1), (664, 7239, 1744, False, "3", 3),    # at any address
+    (505, 3106, 3302, True, "4", 1), (823, 2891, 1731, False, "4", 1), (2516, 2262, 406, False, "4", 1),    # the estimate close, k short
     (560, 3344, 1408, False, "4", 1), (560, 3344, 2816, False, "3", 2), (1408, 4096, 1400, False, "3", 2),
     (2000, 2048, 1008, False, "3", 1), (440, 2952, 3784, False, "3", 2), (1656, 2616, 792, False, "3", 2),    # one split pays, or does not
     (728, 2016, 2215, True, "3", 1), (2160, 2472, 827, True, "3", 2),                                         # and in odd rows of C
