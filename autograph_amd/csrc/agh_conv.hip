@@ -681,13 +681,16 @@ int conv2_direct_entry(const char *name, const void *x, const void *w, const voi
             conv2_taps_try<T>(name, x, w, bias, y, bs, ic, ih, iw, oc, fh, fw, ph, pw, sh, sw, dh, dw, oh, ow, act, false, false, 0.0, &f32_us);
         // Where the f32 kernel would be taken otherwise, its second launch (the packed bank, 3 us of a program's time) has to be worth it:
         // two microseconds and a quarter of a time that is on the safe side (12 x 12 pixels, 32 to 16 channels, 3 x 3: 10.4 us there, 13.7 here).
-        // Over 250 shapes the choice is 6 % behind the best of the three, two are 4 and 6 % slower than before.  Against im2col and a product a
-        // tenth is left for the estimate's error (33 x 128 x 12 x 76 to 256, 3 x 3: 75 us there, 83 here).
-        const double limit = f32_us <= taps_limit ? 0.75 * f32_us - 2.0 : 0.9 * taps_limit;
+        // Against im2col and a product a tenth is left for the estimate's error (33 x 128 x 12 x 76 to 256, 3 x 3: 74 us there, 83 here), and four tenths
+        // where the filter bank streams through workgroups that take up to twice the estimate, or few of them through little work (7 x 256 x 47 x
+        // 74 to 256, 5 x 5: 241 us there, 317 here; 2 x 256 x 17 x 9 to 96, 3 x 3: 20 and 28).  Of 240 shapes that were measured and the rule takes against
+        // im2col none is slower than it was there, 0.19 to 0.99 of the time.
+        const bool against_f32 = f32_us <= taps_limit;
+        const double limit = against_f32 ? 0.75 * f32_us - 2.0 : 0.9 * taps_limit, wary_limit = against_f32 ? limit : 0.6 * taps_limit;
         const int rc = !taps16_forced && limit < kTaps16LeastUs
                            ? 1
                            : conv2_taps16_try(name, x, w, bias, y, bs, ic, ih, iw, oc, fh, fw, ph, pw, sh, sw, dh, dw, oh, ow, act, pool2x2 != 0,
-                                              taps16_forced, limit, lacking);
+                                              taps16_forced, limit, wary_limit, lacking);
         if (rc != 1) return rc;
         if (taps16_forced && lacking) return workspace(lacking, &unused);
         if (taps16_forced) return fail(AGH_ERANGE, "%s: AGH_CONV_TAPS=2, and that kernel does not take this shape", name);

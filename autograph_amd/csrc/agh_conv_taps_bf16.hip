@@ -253,7 +253,7 @@ static int taps16_launch(const char *name, const void *x, const void *wp, const 
 
 int conv2_taps16_try(const char *name, const void *x, const void *w, const void *bias, void *y, int64_t bs, int64_t ic, int64_t ih,
                      int64_t iw, int64_t oc, int64_t fh, int64_t fw, int64_t ph, int64_t pw, int64_t sh, int64_t sw, int64_t dh,
-                     int64_t dw, int64_t oh, int64_t ow, int act, bool pool, bool forced, double limit_us, size_t &lacking) {
+                     int64_t dw, int64_t oh, int64_t ow, int act, bool pool, bool forced, double limit_us, double wary_limit_us, size_t &lacking) {
     const int64_t npos = oh * ow, taps = fh * fw, cols = (ow - 1) * sw + (fw - 1) * dw + 1, all_groups = (ic + 7) / 8;
     if (npos > ((int64_t)1 << 24) || ic * taps > ((int64_t)1 << 24) || oc * ic * taps > ((int64_t)1 << 28) || cols > (1 << 16)) return 1;
     const int64_t cus = compute_units() > 0 ? compute_units() : 256, n16 = (oc + 15) / 16;
@@ -282,8 +282,12 @@ int conv2_taps16_try(const char *name, const void *x, const void *w, const void 
             if (!tg || cost < us) { us = cost; tg = t; nt = n; rows = r; groups = gr; }
         }
     }
-    if (!tg || (!forced && us > limit_us)) return 1;
+    if (!tg) return 1;
     const int64_t passes = (all_groups + groups - 1) / groups, units = taps * groups, steps = (units + 3) / 4;
+    // Channels in passes or more than 36 steps: the bank streams from the L2s.  The estimate is up to half too low where a workgroup takes 64 channels
+    // or passes are many, and says little where there are few workgroups.
+    const bool streams = passes > 1 || steps > 36, few = bs * ((npos + 64 * tg - 1) / (64 * tg)) * ((n16 + nt - 1) / nt) * 4 < cus;
+    if (!forced && us > (streams && (nt == 4 || passes > 4 || few) ? wary_limit_us : limit_us)) return 1;
     const int64_t pitch = groups * 16 + 16, tab_bytes = (steps + 1) * 16;
     auto lds_bytes = [&](int64_t r) { return r * cols * pitch + tab_bytes; };
     // rows of a tile of 16 t windows

@@ -42,12 +42,12 @@ template <typename T>
 int conv2_taps_try(const char *name, const void *x, const void *w, const void *bias, void *y, int64_t bs, int64_t ic, int64_t ih,
                    int64_t iw, int64_t oc, int64_t fh, int64_t fw, int64_t ph, int64_t pw, int64_t sh, int64_t sw, int64_t dh,
                    int64_t dw, int64_t oh, int64_t ow, int act, bool pool, bool forced, double limit_us, double *estimate_us = nullptr);
-// The same on the bf16 matrix cores (agh_conv_taps_bf16.hip).  It needs scratch memory: where a capture cannot have it, 1, and `lacking` says how
+// The same on the bf16 matrix cores (agh_conv_taps_bf16.hip); wary_limit_us instead of limit_us where its estimate is least good.  It needs scratch memory: where a capture cannot have it, 1, and `lacking` says how
 // many bytes.
 constexpr double kTaps16LeastUs = 6.4;  // what no shape is expected to need less than there
 int conv2_taps16_try(const char *name, const void *x, const void *w, const void *bias, void *y, int64_t bs, int64_t ic, int64_t ih,
                      int64_t iw, int64_t oc, int64_t fh, int64_t fw, int64_t ph, int64_t pw, int64_t sh, int64_t sw, int64_t dh,
-                     int64_t dw, int64_t oh, int64_t ow, int act, bool pool, bool forced, double limit_us, size_t &lacking);
+                     int64_t dw, int64_t oh, int64_t ow, int act, bool pool, bool forced, double limit_us, double wary_limit_us, size_t &lacking);
 
 // Variables AGH_* that force a choice (measurements, tests) are read at every call; looked up one by one they cost a call of a small
 // product a quarter of its host time.  The first one that a call asks for walks the environment once and notes the few entries that begin

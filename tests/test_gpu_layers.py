@@ -280,7 +280,7 @@ def test_conv2_taps_kernel_on_the_bf16_matrix_cores(ag, case, monkeypatch):
     # bs, ic, ih, iw, oc, filter; the kernel without scratch memory that takes the shape where this one cannot be had (AGH_CONV_TAPS), if any
     ((4, 32, 41, 41, 48, 5), "1"),      # the f32 matrix cores
     ((58, 16, 8, 18, 32, 5), "0"),      # row tiles
-    ((10, 32, 38, 13, 48, 7), None),    # a program would take im2col and a product
+    ((22, 64, 21, 43, 48, 3), None),    # a program would take im2col and a product
 ])
 def test_conv2_taps_bf16_captured(ag, monkeypatch, shape, former):
     """A convolution with a packed filter bank inside a captured graph.  Run eagerly before, it has its scratch memory, on the main stream: the bits of
@@ -404,6 +404,23 @@ def test_conv2_bf16_fused_pool_whose_rows_exceed_lds_equals_the_layers(ag, case)
     want = ag.MaxPool2((2, 2)).forward(conv.forward(x)).into_array()
     got = conv.forward(x, pool2x2=True).into_array()
     assert np.array_equal(got, want), np.mean(got != want)
+
+
+@pytest.mark.parametrize("case,taken", [
+    ((7, 256, 47, 74, 256, 5, 2, 1), False), ((2, 256, 17, 9, 96, 3, 1, 1), False), ((5, 128, 24, 24, 96, 3, 0, 2), False),   # channels in passes, many steps
+    ((149, 32, 32, 23, 48, 7, 3, 1), True), ((126, 32, 76, 76, 48, 3, 1, 1), True), ((132, 128, 30, 30, 16, 7, 0, 1), True),
+    ((25, 128, 21, 37, 48, 5, 2, 1), True),
+])
+def test_conv2_bf16_route(ag, monkeypatch, case, taken):
+    """Which bf16 convolutions run out of staged rows on the bf16 matrix cores and which by im2col and a product: the bits of that route."""
+    bs, ic, h, w, oc, f, p, s = case
+    rng = np.random.default_rng(36)
+    x = ag.Tensor.from_array(to_dtype(rng.standard_normal((bs, ic, h, w)), "bf16"))
+    conv = ag.Conv2(ag.Tensor.from_array(to_dtype(rng.standard_normal((oc, ic, f, f)) * (2 / (ic * f * f)) ** 0.5, "bf16")), None, (p, p), (s, s))
+    got = conv.forward(x).into_array()
+    assert np.array_equal(got, conv.forward(x, algorithm="im2col").into_array()) == (not taken)
+    monkeypatch.setenv("AGH_CONV_TAPS", "2")
+    assert np.array_equal(got, conv.forward(x).into_array()) == taken
 
 
 def test_conv2_route_is_the_faster_one(ag, monkeypatch):
