@@ -272,18 +272,22 @@ inline bool short_and_narrow(const Args &g, int64_t batch, int64_t cus, int lp) 
 // Products at any address that the f32 kernel's form for them serves better than the element-wise loaders.
 // Up to k = 64 it does not: two k-tiles are all filling, and those loaders read only what there is (3889x18x648 7.9 / 10.7 us,
 // 37905x32x448 28.6 / 37.9, 3460x57x1352 15.2 / 18.5; 584x107x2002 16.4 / 13.3, 5088x95x642 21.8 / 20.2).
-// Nor, with more 64 x 64 tiles than CUs, where one operand's unit stride is along k and the other's along its rows: the element-wise loaders, four
-// workgroups a CU, are good at that.  Up to k = 128 some were slower here (6697x70x1384, both transposed, 33.4 / 38.2 us; 2339x93x1744 19.3 / 21.0).
-// With whole vectors along k and none along the rows, up to k = 512 one in three of 189 (7649x80x788 21.9 / 28.6; 391x68x7423, neither transposed, 18.2 /
-// 22.8; 2870x280x5883 130 / 139) and as fast all together; beyond it, 82 products of 0.75 to 0.98 of the time, those only whose tiles of 32 x 128 or
-// 128 x 32 need fewer rounds (146x672x6485 25.3 / 35.8).
+// Nor, with more 64 x 64 tiles than CUs,
+//   where tiles of 32 x 128 or 128 x 32, which only those loaders have, need 0.8 of the rounds or fewer: over 270 such products as fast all together,
+//   0.5 to 1.4 of the time one by one, and 65 to 96 rows or columns against any number on the whole slower (70x80x39588, left transposed, 15.7 /
+//   21.7; 146x672x6485, both, 25.3 / 35.8; 3704x1694x525, both, 99.7 / 117);
+//   up to k = 128 where one operand's unit stride is along k and the other's along its rows, which those loaders, four workgroups a CU, are good at
+//   (6697x70x1384, both transposed, 33.4 / 38.2; 2339x93x1744 19.3 / 21.0);
+//   up to k = 512 where moreover the operand along k is of whole vectors: one in three of 189 products slower (7649x80x788 21.9 / 28.6; 391x68x7423,
+//   neither transposed, 18.2 / 22.8; 2870x280x5883 130 / 139) and as fast all together; beyond it 82 products of 0.75 to 0.98 of the time.
 inline bool f32_any_pays(const Args &g, int64_t batch, int64_t cus, int lp, int lq, int lp_any, int lq_any) {
     if (g.K <= 64) return false;
     auto rounds = [&](int bp, int bq) { return ((int64_t)((g.NP + bp - 1) / bp) * ((g.NQ + bq - 1) / bq) * batch + cus - 1) / cus; };
-    if (lp_any == lq_any || rounds(64, 64) <= 1) return true;
-    if (g.K <= 128) return false;
+    if (rounds(64, 64) <= 1) return true;
+    if (std::min(rounds(32, 128), rounds(128, 32)) * 5 <= rounds(64, 64) * 4) return false;
+    if (lp_any == lq_any) return true;
     const bool whole_along_k = (lp_any == LD_K ? lp : lq) != LD_S;  // (the other operand has none then, or this is not asked)
-    return !whole_along_k || (g.K > 512 && std::min(rounds(32, 128), rounds(128, 32)) * 5 >= rounds(64, 64) * 4);
+    return g.K > (whole_along_k ? 512 : 128);
 }
 
 // Optional override for experiments: AGH_GEMM_CFG=<config id>, AGH_GEMM_SPLITS=<n>.

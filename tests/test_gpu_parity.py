@@ -1158,7 +1158,9 @@ def test_max_pool2_reference_cases(ag, dtype):
     (397, 96, 2373, True, True, False), (391, 68, 7423, False, False, False), (2523, 324, 2492, True, True, False),     # whole vectors along k, short
     (146, 672, 6485, True, True, False), (458, 2652, 3216, True, True, True), (1230, 1276, 961, False, False, True),    # and long
     (4523, 122, 217, True, True, False), (2339, 93, 1744, False, False, False), (2061, 131, 1097, True, True, True),    # none along k
-    (1526, 84, 223, True, True, True), (146, 673, 6484, True, True, True), (1999, 2047, 1001, False, True, True),
+    (1526, 84, 223, True, True, True), (200, 673, 6484, True, True, True), (1999, 2047, 1001, False, True, True),
+    (70, 76, 10088, True, False, False), (70, 80, 39588, True, False, False), (67, 133, 27416, False, False, False), (3704, 1694, 525, True, True, False),    # 32-row tiles, fewer rounds
+    (75, 69, 10907, False, True, True), (129, 85, 10001, False, True, True),
 ])
 def test_gemm_f32_at_any_address_where_it_pays(ag, monkeypatch, m, k, n, ta, tb, direct):
     """Which products of no whole vectors take the direct-to-LDS kernel's form for them: the bits are those of the route forced, not of the other."""
