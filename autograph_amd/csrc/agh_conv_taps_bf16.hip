@@ -8,12 +8,13 @@
 // channels zero) and 16 bytes of padding.  A unit is eight channels of one tap, a step of v_mfma_f32_16x16x32_bf16 four units, one per
 // 16-lane group: the A operand is one 16-byte LDS read per lane at the position's base + the unit's offset (a table in LDS), whatever
 // the stride, and the B operand one 16-byte load of a copy of the filter bank in fragment order (as large as the bank; it stays in
-// the L2s).  Channels that do not fit into half a CU's LDS are taken in passes.  Both operands of a step are requested one step (A) and
-// kAhead steps (B) before it.
-// What bounds it: staging (2-byte reads) and the waits of few workgroups; the products are a third of a large launch.  Against the f32 matrix
-// cores or im2col and a product, whichever it was (calls of a Python program, us): 149 x 32 x 32 x 23 to 48, 7 x 7 201 -> 30; 132 x 128 x 30 x 30
-// to 16, 7 x 7 453 -> 71; 126 x 32 x 76 x 76 to 48, 3 x 3 323 -> 66; 214 x 24 x 53 x 53 to 64, 3 x 3 stride 2 75 -> 32; 102 x 3 x 76 x 76 to 96, 7 x 7
-// 145 -> 78.
+// the L2s).  Channels whose rows do not fit into 64 KB of LDS, which leaves a CU two workgroups, are taken in passes.  Both operands of a step are
+// requested one step (A) and kAhead steps (B) before it.
+// What bounds it: latencies, of staging (2-byte reads) and of the bank's reads, with two workgroups a CU.  No unit is busy (counters of the first, third and
+// fourth shape below: matrix pipes 18, 11 and 23 % of a launch, LDS 16, 11 and 21 % with half of it conflicts, L1s half an access a cycle; a wave waits
+// for two thirds of its cycles).  Against the f32 matrix cores or im2col and a product, whichever it was (calls of a Python program, us):
+// 149 x 32 x 32 x 23 to 48, 7 x 7 with padding 213 -> 35; 132 x 128 x 30 x 30 to 16, 7 x 7 317 -> 59; 126 x 32 x 76 x 76 to 48, 3 x 3 with padding 334 -> 67;
+// 102 x 3 x 76 x 76 to 96, 7 x 7 with padding 172 -> 78.
 #include <algorithm>
 #include <type_traits>
 

@@ -33,10 +33,11 @@
 //
 // W = 1 is the form for operands at any element address, k and row counts of any size (unit stride along k or along rows
 // is all that is asked): the direct loads take 4 bytes a lane instead of 16, four of them a 1 KB image, and put every element where
-// the 16-byte load would have.  The matrix pipes bound it like the form above (a 64 x 64 k-tile is 1024 matrix cycles and 64
-// loads of 256 bytes), where the element-wise loaders of agh_gemm_kernel.h spend as long on addresses, conditions and LDS
-// writes: 4099x4101x4103 2011 -> 1470 us, 1999x2047x1001 131 -> 89, 133x7001x3003 249 -> 112, 2632x323x6065 179 -> 138.  What is left
-// to the aligned form (1190, 73, 97, 104 us) are the loads: 256 a k-tile of 128 x 128 through the CU's one address path.
+// the 16-byte load would have.  The matrix pipes bound it like the form above, if less (63, 61, 61 and 53 % busy over the products below, their neighbours of
+// whole vectors 78, 68, 70 and 66 %), where the element-wise loaders of agh_gemm_kernel.h spend as long on addresses, conditions and LDS
+// writes: 4099x4101x4103 2010 -> 1475 us, 1999x2047x1001 131 -> 92, 133x7001x3003 249 -> 111, 2632x323x6065 179 -> 130.  What is left to the
+// neighbours (1176, 73, 96, 104 us) are four times as many loads to issue, 128 a k-tile of 128 x 128 and 64 of 64 x 64; the L1s see no more accesses
+// (6 or 7 for 256 bytes that start anywhere).
 #pragma once
 #include "agh_gemm_bf16_dl.h"
 

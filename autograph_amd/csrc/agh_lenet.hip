@@ -1040,8 +1040,8 @@ int lenet5_dense_grads_entry(const char *name, const void *a2, const void *a1, c
 // The weight gradients of the two convolutions of a LeNet5 training step without their patch matrices:
 // dw2[oc][ci][fi][fj] = sum over images and output positions of gm2[(y, x)][oc] * p1[ci][y + fi][x + fj] (the product
 // gm2^T . im2col(p1) of layer.rs:990-1003), dw1 likewise from gm1 and x.  One workgroup per image forms the image's f32
-// partial sums from operands staged in LDS; a second launch adds the partials in image order and rounds once to T, as
-// the split-K GEMM does.
+// partial sums from operands staged in LDS; a second launch adds the partials (by quarters of the batch, two interleaved sums each, then these
+// eight) and rounds once to T, as the split-K GEMM does.
 constexpr int kLenetPartPitch = 2560;  // per image: 2400 entries of dw2, 150 of dw1
 // 512 threads: one image's partial sums out of LDS: g2 [y*8 + x][oc] and g1 [y*24 + x][oc] the gradients of the convolutions' outputs, p1s and
 // xs their inputs; q2 and q1 take the second half of conv2's positions and conv1's eight row groups.  On v_mfma_f32_16x16x4_f32 (lane (g, i):
